@@ -201,8 +201,9 @@ def prepare(case, seed):
             ctx.mark_step_begin()
             fbcache.set_first_hidden_states_residual(prev)
             if not seer:
-                fbcache.set_hidden_states_residual(x.randn(*shape))
-                fbcache.set_encoder_hidden_states_residual(x.randn(*state["text"].shape))
+                state["rest"], state["rest_text"] = x.randn(*shape), x.randn(*state["text"].shape)
+                fbcache.set_hidden_states_residual(state["rest"])
+                fbcache.set_encoder_hidden_states_residual(state["rest_text"])
         state["context"] = ctx
         if seer:
             state["seer"] = TaylorSeer(n_derivatives=2, skip_interval_steps=3)
@@ -258,6 +259,71 @@ def _cache_step(state):
         rest, _ = torch.ops.para_attn.fbcache_first_residual_diff(before, after, None)
         fbcache.set_hidden_states_residual(rest)
         return residual, hit, rest
+
+
+# ---------------------------------------------------------------------------------------------------------
+# the same in 64 bits
+# ---------------------------------------------------------------------------------------------------------
+def _attention64(q, k, v, keep=None, causal=False):
+    """(out, lse) in 64 bits, a head and a slice of the query rows at a time.  ``keep(b, h, r0, r1)``: what is added to
+    the scores of those rows, or where boolean which of them are kept."""
+    B, H, Sq, D = q.shape
+    Skv = k.shape[2]
+    out = torch.empty(B, H, Sq, D, dtype=torch.float64, device=q.device)
+    lse = torch.empty(B, H, Sq, dtype=torch.float64, device=q.device)
+    rows = max(1, (1 << 28) // Skv)
+    for b in range(B):
+        for h in range(H):
+            kt, vh = k[b, h].double().t().contiguous(), v[b, h].double()
+            for r0 in range(0, Sq, rows):
+                r1 = min(Sq, r0 + rows)
+                s = q[b, h, r0:r1].double() @ kt
+                s *= 1.0 / math.sqrt(D)
+                if causal:
+                    at = torch.arange(Skv, device=q.device)
+                    s.masked_fill_(at[None, :] > at[r0:r1, None], -math.inf)
+                if keep is not None:
+                    m = keep(b, h, r0, r1)
+                    if m.dtype == torch.bool:
+                        s.masked_fill_(~m, -math.inf)
+                    else:
+                        s += m.double()
+                top = s.amax(-1, keepdim=True)
+                s.sub_(top).exp_()
+                total = s.sum(-1, keepdim=True)
+                out[b, h, r0:r1] = (s @ vh) / total
+                lse[b, h, r0:r1] = (top + total.log())[:, 0]
+    return out, lse
+
+
+def exact(case, seed):
+    state = prepare(case, seed)
+    kind = case["kind"]
+    if kind == "self":
+        out, lse = _attention64(state["q"], state["k"], state["v"], causal=case["causal"])
+        return (out, lse) if case["lse"] else out
+    if kind == "cross":
+        bias = state["bias"]
+        return _attention64(state["q"], state["k"], state["v"], None if bias is None else lambda b, h, r0, r1: bias[b, 0])[0]
+    if kind == "masked":
+        mask = state["mask"]
+
+        def keep(b, h, r0, r1):
+            m = mask[b if mask.shape[0] > 1 else 0, h if mask.shape[1] > 1 else 0]
+            return m[r0:r1] if m.shape[0] > 1 else m
+
+        out, lse = _attention64(state["q"], state["k"], state["v"], keep)
+        return out if case["mask"] in ("prefix", "holes") else (out, lse)
+    if kind == "sparse":
+        mask, block = state["mask"], case["block"]
+        at = torch.arange(case["blocks"] * block, device=mask.device) // block
+        return _attention64(state["q"], state["k"], state["v"], lambda b, h, r0, r1: (mask[h] if mask.dim() == 3 else mask)[at[r0:r1]][:, at])
+    if kind == "ring":
+        return _attention64(state["q"], torch.cat(state["k"], 2), torch.cat(state["v"], 2))
+    residual = state["after"].double() - state["before"].double()
+    if case["step"] == "hit":
+        return residual, None, state["after"].double() + state["rest"].double(), state["text"].double() + state["rest_text"].double()
+    return residual, None, -residual if case["step"] == "miss" else None  # the second residual is taken the other way round
 
 
 # ---------------------------------------------------------------------------------------------------------
