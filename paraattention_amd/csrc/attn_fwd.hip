@@ -124,11 +124,12 @@ struct AttnParams {
   float* acc_out;
   float* acc_lse;
   int acc_first;
-  // attn_fwd_kernel only: an attention mask, one element per (batch, head, query, key) reached through four
+  // attn_fwd_kernel, and the pipelined kernels with PM: an attention mask, one element per (batch, head, query, key) reached through four
   // strides in elements (0 on broadcast dimensions).  MASK_BOOL: bytes, 0 = the key is dropped for that query;
   // MASK_F32 / MASK_ACT: a bias added to the scaled score (fp32, or the activation type).
   const void* mask;
   int64_t ms_b, ms_h, ms_q, ms_k;
+  int mask_kind;  // MASK_*
   // dense kernels: with `gate` set the launch leaves at once unless bit *gate of gate_mask is set (a decision taken on
   // the device by an earlier launch of the same stream, e.g. whether a key mask is a prefix)
   const int* gate;
@@ -579,6 +580,101 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_fwd_kernel(const AttnParams 
 
 
 // ---------------------------------------------------------------------------------------------
+// Attention masks in the pipelined kernels (template parameter PM).  The per-score mask of attn_fwd_kernel costs a
+// 64-bit address, a bounds test and a load per score; most masks in use select or bias whole keys, the same for every
+// query row of a workgroup, and then one load per lane and 64-key tile holds all of it:
+//   PM_KEYS     boolean, no query dimension
+//   PM_KEYBIAS  additive, no query dimension
+// Each wavefront lays the tile's 64 values down in its own 256 bytes of LDS and reads them back in the accumulator's
+// order (8 broadcast reads, one instruction per score); a tile that drops no key, or whose biases are all zero, costs
+// nothing beyond the vote that says so.  Measured against the per-score kernel (attn_fwd_kernel<MASK>, register-staged
+// tiles): two samples x 24 heads x 7800 rows against 256 keys with a bias 171 -> 104 us (0.47 PFLOP/s; bound by what a
+// workgroup does around its four key tiles), 24 heads x 4352 tokens with holes in the key mask, scan and two empty
+// launches included there, 390..545 -> 236 us (0.98 PFLOP/s, what the unmasked call of that size reaches).
+// The element of tile j + 2 is fetched while tile j + 1 is masked, so its latency is covered by the wait for the
+// tile copies at the top of every iteration.
+// ---------------------------------------------------------------------------------------------
+constexpr int PM_NONE = 0, PM_KEYS = 1, PM_KEYBIAS = 2;
+constexpr int PM_SLOT_BYTES = 256;  // LDS per wavefront, behind the K and V tiles
+// The running maximum of a masked row before its first kept key.  Finite, so that -inf scores against it give
+// exp2(-inf) = 0 instead of NaN; below every finite score, so that the first kept key raises it.
+constexpr float PM_NO_MAX = -3.402823466e38f;
+
+template <typename T, int PM>
+struct TileMask {
+  const char* base;  // this (batch, head)'s mask elements
+  int64_t step;      // bytes per key
+  uint32_t last, raw;
+  int lane, hh;
+  bool act;  // 16-bit elements in the activation type
+  float per_scale;
+  float* slot;
+  __device__ __forceinline__ void init(const AttnParams& p, int batch, int head, int lane_, char* lds) {
+    lane = lane_;
+    hh = lane_ >> 5;
+    last = (uint32_t)(p.Skv - 1);
+    const int64_t at = batch * p.ms_b + head * p.ms_h;
+    act = PM == PM_KEYBIAS && p.mask_kind == MASK_ACT;
+    const int bytes = PM == PM_KEYS ? 1 : act ? 2 : 4;
+    base = (const char*)p.mask + at * bytes;
+    step = p.ms_k * bytes;
+    per_scale = 1.0f / (p.scale_log2 * LN2);  // bias / scale, so that (s + that) * c = s * c + bias * log2(e)
+    slot = (float*)lds;
+  }
+  // PM_KEYS: keys up to and including the last one kept, found from the end (every wavefront for itself, 256 keys a
+  // step); the keys behind it are not walked at all, as with per-batch key counts
+  __device__ __forceinline__ int kept_end(int Skv) const {
+    int end = 0;
+    for (int top = Skv; top > 0 && end == 0; top -= 256) {
+      int best = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int key = top - 64 * (i + 1) + lane;
+        if (key >= 0 && *(const uint8_t*)(base + (int64_t)key * step) != 0) best = best > key + 1 ? best : key + 1;
+      }
+#pragma unroll
+      for (int d = 32; d > 0; d >>= 1) { const int o = __shfl_xor(best, d); best = o > best ? o : best; }
+      end = __builtin_amdgcn_readfirstlane(best);
+    }
+    return end;
+  }
+  // the element of key n0 + lane (any key for a tile that does not exist or ends early: those scores are dropped)
+  __device__ __forceinline__ void fetch(uint32_t n0) {
+    uint32_t key = n0 + lane;
+    key = key < last ? key : last;
+    const char* at = base + (int64_t)key * step;
+    if constexpr (PM == PM_KEYS) raw = *(const uint8_t*)at;
+    else if (act) raw = *(const uint16_t*)at;
+    else raw = *(const uint32_t*)at;
+  }
+  __device__ __forceinline__ void apply(floatx16& a0, floatx16& a1) const {
+    // what a lane lays down for its key: the bias, or the largest value a score may keep (-inf drops it whatever it is,
+    // also where a dropped key's row holds no numbers)
+    float b;
+    if constexpr (PM == PM_KEYS) {
+      if (!__any(raw == 0)) return;
+      b = raw != 0 ? INFINITY : -INFINITY;
+    } else {
+      b = (act ? T::lo(raw) : __uint_as_float(raw)) * per_scale;
+      if (!__any((__float_as_uint(b) << 1) != 0)) return;
+    }
+    __builtin_amdgcn_wave_barrier();
+    slot[lane] = b;
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      const floatx4 x = *(const floatx4*)(slot + 8 * a + 4 * hh), y = *(const floatx4*)(slot + 32 + 8 * a + 4 * hh);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        a0[4 * a + i] = PM == PM_KEYS ? fminf(a0[4 * a + i], x[i]) : a0[4 * a + i] + x[i];
+        a1[4 * a + i] = PM == PM_KEYS ? fminf(a1[4 * a + i], y[i]) : a1[4 * a + i] + y[i];
+      }
+    }
+  }
+};
+
+
+// ---------------------------------------------------------------------------------------------
 // head_dim 128: the tuned kernel.
 //
 // K and V tiles (64 keys x 256 B) go from global memory straight into LDS
@@ -940,7 +1036,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_fwd_d128_kernel(const AttnPa
 // workgroups in several key shares (AttnParams::split_*), fold the result into a running
 // (out, lse) pair (acc_*), or apply torch's causal mask (causal).
 // ---------------------------------------------------------------------------------------------
-template <typename T, bool SPARSE, int NW, bool BOUNDED = false, bool PAIR = false>
+template <typename T, bool SPARSE, int NW, bool BOUNDED = false, bool PAIR = false, int PM = PM_NONE>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_kernel(const AttnParams p) {
   typedef typename T::vec8 vec8;
   constexpr int DC = 8, DB = 4;
@@ -989,6 +1085,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
   int row_begin, row_end;
   TileIter it;
   decode_block<SPARSE>(p, qt, head, batch, row_begin, row_end, it);
+  TileMask<T, PM> tm;
+  if constexpr (PM != PM_NONE) tm.init(p, batch, head, lane, (char*)smem + 4 * TILE_BYTES + wave * PM_SLOT_BYTES);
+  if constexpr (PM == PM_KEYS) it.init_dense(__builtin_amdgcn_readfirstlane(tm.kept_end(p.Skv)));
   // Keys in segments (the blocks of a ring sweep, StreamPlan::kseg / vseg): the sweep below runs once per
   // segment, with the softmax state carried over in registers.  A key share of a split piece is then a run of
   // whole segments; with one segment it is a range of key tiles.
@@ -1096,7 +1195,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
   for (int i = 0; i < DB; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
-  float m_run = BOUNDED ? 0.f : -INFINITY, l_run = 0.f;
+  float m_run = BOUNDED ? 0.f : PM != PM_NONE ? PM_NO_MAX : -INFINITY, l_run = 0.f;
   const float c = p.scale_log2;
 
   // window of tiles j (being consumed), j+1 and j+2: (first key or OOB, valid keys)
@@ -1260,6 +1359,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
       __builtin_amdgcn_sched_barrier(0);
     }
     if (an) {
+      if constexpr (PM != PM_NONE) {
+        tm.apply(sn0, sn1);
+        if (n_nx2 != OOB) tm.fetch(n_nx2);  // (without the branch the compiler spills 70 registers here)
+      }
       if (v_nxt < BN || on_diagonal(n_nxt)) mask_tail(sn0, sn1, v_nxt, n_nxt);  // ragged, absent or diagonal tile j+1
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -1372,6 +1475,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
       }
 #pragma unroll
       for (int dc = 0; dc < DC; ++dc) sn1 = T::mfma32(f[dc], qf[dc], sn1);
+      if constexpr (PM != PM_NONE) {
+        tm.fetch(n_cur);
+        tm.apply(sn0, sn1);
+        tm.fetch(n_nxt);
+      }
       if (v_cur < BN || on_diagonal(n_cur)) mask_tail(sn0, sn1, v_cur, n_cur);
       if constexpr (!BOUNDED) {
         float m2 = fmaxf(sn0[0], sn1[0]);
@@ -1493,7 +1601,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
 // ---------------------------------------------------------------------------------------------
 constexpr int TILE64_BYTES = BN * 128;
 
-template <typename T, bool SPARSE, int NW, bool BOUNDED = false>
+template <typename T, bool SPARSE, int NW, bool BOUNDED = false, int PM = PM_NONE>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_kernel(const AttnParams p) {
   // BOUNDED and the flag: as in attn_fwd_d128_pipe_kernel
   if constexpr (!SPARSE) {
@@ -1528,6 +1636,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
   int row_begin, row_end;
   TileIter it;
   decode_block<SPARSE>(p, qt, head, batch, row_begin, row_end, it);
+  TileMask<T, PM> tm;
+  if constexpr (PM != PM_NONE) tm.init(p, batch, head, lane, (char*)smem + 4 * TILE64_BYTES + wave * PM_SLOT_BYTES);
+  if constexpr (PM == PM_KEYS) it.init_dense(__builtin_amdgcn_readfirstlane(tm.kept_end(p.Skv)));
 
   const uint16_t* qbase = (const uint16_t*)p.q + batch * p.qs_b + head * p.qs_h;
   const char* kbytes = (const char*)((const uint16_t*)p.k + batch * p.ks_b + head * p.ks_h);
@@ -1605,7 +1716,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
   for (int i = 0; i < DB; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
-  float m_run = BOUNDED ? 0.f : -INFINITY, l_run = 0.f;
+  float m_run = BOUNDED ? 0.f : PM != PM_NONE ? PM_NO_MAX : -INFINITY, l_run = 0.f;
   const float c = p.scale_log2;
 
   uint32_t n_cur, n_nxt, n_nx2;
@@ -1670,6 +1781,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
     for (int g = 0; g < 8; ++g) {
       if (g & 1) sn1 = T::mfma32(f[g], qf[g >> 1], sn1);
       else sn0 = T::mfma32(f[g], qf[g >> 1], sn0);
+    }
+    if constexpr (PM != PM_NONE) {
+      tm.fetch(n_cur);
+      tm.apply(sn0, sn1);
+      tm.fetch(n_nxt);
     }
     if (v_cur < BN || on_diagonal(n_cur)) mask_tail(sn0, sn1, v_cur, n_cur);
     if constexpr (!BOUNDED) {
@@ -1737,6 +1853,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
       else if (g < 2 * IPW) dma_v1(par ^ 1, n_nxt, g - IPW);  // V(j+1) takes the buffer V(j-1) has left
       f[g] = read_vt(tV, g >> 2, (g >> 1) & 1, g & 1);         // V(j) in the order stage B consumes it
       __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (PM != PM_NONE) {
+      tm.apply(sn0, sn1);
+      if (n_nx2 != OOB) tm.fetch(n_nx2);  // (without the branch the compiler spills 70 registers here)
     }
     if (v_nxt < BN || on_diagonal(n_nxt)) mask_tail(sn0, sn1, v_nxt, n_nxt);
     __builtin_amdgcn_sched_barrier(0);
@@ -3938,6 +4058,13 @@ static size_t split_ws_bytes(const SplitPlan& pl, int bm) {
   return pl.s > 1 ? (size_t)pl.tiles * pl.s * bm * (128 + 1) * sizeof(float) : 0;
 }
 
+// Whether the pipelined kernels take the call: K and V below 4 GiB per head (32-bit buffer offsets).
+static bool pipe_fits(const AttnParams& p, int D) {
+  if ((D != 128 && D != 64) || p.Skv <= 0) return false;
+  if ((uint64_t)(p.Skv - 1) * (uint64_t)p.ks_s * 2 + 256 >= PIPE_OOB || (uint64_t)(p.Skv - 1) * (uint64_t)p.vs_s * 2 + 256 >= PIPE_OOB) return false;
+  return !tuning().no_pipe;  // test aid: the kernels without offset limits
+}
+
 // Picks the kernel, the query rows per workgroup and the key-split tail.  The pipelined
 // head_dim-128 kernel needs K and V to span less than 4 GiB (32-bit buffer offsets).  128 rows = 4
 // wavefronts, two workgroups per CU; 256 rows = 8 wavefronts sharing one K/V stream (half the tile
@@ -3952,10 +4079,7 @@ static void choose_kernel(AttnParams& p, int D, int q_block, bool dense, size_t 
   p.split_s = 0;
   auto finish = [&] { p.n_qtiles = (p.Sq + p.bm - 1) / p.bm; };
   if (D != 128 && D != 64) return finish();
-  if (p.Skv <= 0 || (uint64_t)(p.Skv - 1) * (uint64_t)p.ks_s * 2 + 256 >= PIPE_OOB ||
-      (uint64_t)(p.Skv - 1) * (uint64_t)p.vs_s * 2 + 256 >= PIPE_OOB)
-    return finish();
-  if (tuning().no_pipe) return finish();  // test aid: the kernels without offset limits
+  if (!pipe_fits(p, D)) return finish();
   p.pipe = 1;
   const int forced = tuning().forced_bm;  // tuning aid
   if (D == 64) {  // no key split at head_dim 64; 128 rows unless asked otherwise
@@ -4523,6 +4647,44 @@ static int launch_masked(const AttnParams& p, int mask_kind, hipStream_t stream)
   return PA_OK;
 }
 
+// A pipelined kernel with its mask handling PM, planned by choose_kernel like a dense call with per-batch key counts.
+template <typename T, int D, int PM, int NW>
+static int launch_masked_pipe_nw(const AttnParams& p, hipStream_t stream) {
+  int64_t nblocks = (int64_t)p.B * p.H * p.n_qtiles;
+  if (p.split_s > 1) nblocks = (int64_t)p.split_main + (int64_t)p.split_tiles * p.split_s;
+  const size_t smem = 4 * (D == 128 ? TILE_BYTES : TILE64_BYTES) + NW * PM_SLOT_BYTES;
+  const void* fn;
+  if constexpr (D == 128) fn = (const void*)attn_fwd_d128_pipe_kernel<T, false, NW, false, false, PM>;
+  else fn = (const void*)attn_fwd_d64_pipe_kernel<T, false, NW, false, PM>;
+  static bool attr_done[PA_MAX_DEVICES] = {};  // benign race: the call is idempotent
+  const int dev = current_device();
+  if (dev < 0 || !attr_done[dev]) {
+    hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    if (e != hipSuccess) PA_FAIL(PA_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
+    if (dev >= 0) attr_done[dev] = true;
+  }
+  if constexpr (D == 128)
+    hipLaunchKernelGGL((attn_fwd_d128_pipe_kernel<T, false, NW, false, false, PM>), dim3((unsigned)nblocks), dim3(64 * NW), smem, stream, p);
+  else
+    hipLaunchKernelGGL((attn_fwd_d64_pipe_kernel<T, false, NW, false, PM>), dim3((unsigned)nblocks), dim3(64 * NW), smem, stream, p);
+  PA_CHECK_LAUNCH("masked attention kernel");
+  if constexpr (D == 128) {
+    if (p.split_s > 1) {
+      const int64_t rows = (int64_t)p.split_tiles * p.bm;
+      hipLaunchKernelGGL((attn_split_merge_kernel<T>), dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, stream, p);
+      PA_CHECK_LAUNCH("attention split merge kernel");
+    }
+  }
+  return PA_OK;
+}
+
+template <typename T, int D>
+static int launch_masked_pipe(const AttnParams& p, hipStream_t stream) {
+  const bool keys = p.mask_kind == MASK_BOOL;
+  if (p.bm == 256) return keys ? launch_masked_pipe_nw<T, D, PM_KEYS, 8>(p, stream) : launch_masked_pipe_nw<T, D, PM_KEYBIAS, 8>(p, stream);
+  return keys ? launch_masked_pipe_nw<T, D, PM_KEYS, 4>(p, stream) : launch_masked_pipe_nw<T, D, PM_KEYBIAS, 4>(p, stream);
+}
+
 // Whether a dense call with per-batch key counts that leave nearly all keys would go to the resident-workgroup
 // kernel: where that kernel takes the shape with `ws_avail` bytes of workspace and the launch is long enough for its
 // advantage over the kernel with one workgroup per query tile to outweigh a third, empty launch: from 512 key-tile
@@ -4549,6 +4711,9 @@ static size_t mask_scan_bytes(int B, int Skv) {
   return (((size_t)B + 1 + (size_t)3 * B * mask_chunks(Skv)) * sizeof(int32_t) + 255) & ~(size_t)255;
 }
 
+// From this size on a boolean key mask is scanned on the device and the kept keys of one with holes are gathered.
+constexpr double GATHER_FLOP = 3.0e11;
+
 // pa_attn_fwd_masked's workspace when it gathers the kept keys of a mask with holes: the scan's words, dense copies
 // of K and V [B][H][Skv][D], then the workspace of the dense launches.
 struct MaskedLayout {
@@ -4570,7 +4735,7 @@ extern "C" size_t pa_attn_fwd_masked_workspace_bytes(int B, int H, int Sq, int S
   if (H <= 0 || Sq <= 0 || Skv <= 0 || (D != 128 && D != 64)) return mask_scan_bytes(B, Skv > 0 ? Skv : 1) + dense;
   // room to gather the kept keys of a mask with holes (from 3e11 flop on; see pa_attn_fwd_masked), and for the dense
   // launches over the gathered copies, whose strides are those of contiguous tensors
-  if (4.0 * B * H * (double)Sq * (double)Skv * D < 3.0e11) return mask_scan_bytes(B, Skv > 0 ? Skv : 1) + dense;
+  if (4.0 * B * H * (double)Sq * (double)Skv * D < GATHER_FLOP) return mask_scan_bytes(B, Skv > 0 ? Skv : 1) + dense;
   const int64_t cs[3] = {(int64_t)H * Skv * D, (int64_t)Skv * D, D};
   const size_t dense_c = pa_attn_fwd_workspace_bytes(B, H, Sq, Skv, D, cs, cs);
   return masked_layout(B, H, Skv, D).dense + (dense > dense_c ? dense : dense_c);
@@ -4599,11 +4764,28 @@ extern "C" int pa_attn_fwd_masked(const void* q, const void* k, const void* v, v
   p.n_qtiles = (Sq + BM - 1) / BM;
   p.mask = mask;
   p.ms_b = mask_strides[0]; p.ms_h = mask_strides[1]; p.ms_q = mask_strides[2]; p.ms_k = mask_strides[3];
+  p.mask_kind = mask_kind;
+  // A mask without a query dimension (key padding, boolean or as a bias; also one per head) runs in the pipelined
+  // kernels: one launch, no scan.  Boolean ones from GATHER_FLOP on that are the same for every head go on below
+  // instead, where a mask with holes costs what its kept keys cost and the resident-workgroup kernel may serve it.
+  const bool no_query_dim = any && (Sq == 1 || p.ms_q == 0);
+  auto masked_pipe = [&](void* ws, size_t ws_bytes) {
+    choose_kernel(p, D, 256, true, ws ? ws_bytes : 0, nullptr);
+    if (p.split_s > 1) {
+      p.ws_out = (float*)ws;
+      p.ws_lse = p.ws_out + (size_t)p.split_tiles * p.split_s * p.bm * 128;
+    }
+    if (dtype == PA_DTYPE_BF16) return D == 128 ? launch_masked_pipe<BF16, 128>(p, st) : launch_masked_pipe<BF16, 64>(p, st);
+    return D == 128 ? launch_masked_pipe<F16, 128>(p, st) : launch_masked_pipe<F16, 64>(p, st);
+  };
+  const bool pipe_takes = no_query_dim && pipe_fits(p, D);
   // A boolean mask that only selects keys (the same for every head and query row; what the text padding of
   // video DiTs looks like) is usually a prefix per batch element.  Whether it is, is found out on the device: a
   // small scan writes the kept-key counts and a flag, then both the dense launch (counts as kv_len) and the
   // masked launch are enqueued, and the one the flag does not select leaves at once.  Nothing is read back.
   const bool key_only = mask_kind == MASK_BOOL && (H == 1 || p.ms_h == 0) && (Sq == 1 || p.ms_q == 0);
+  const double flops = 4.0 * B * H * (double)Sq * (double)Skv * D;
+  if (pipe_takes && (!key_only || flops < GATHER_FLOP)) return masked_pipe(workspace, workspace_bytes);
   const size_t scan = mask_scan_bytes(B, Skv > 0 ? Skv : 1);
   if (key_only && any && workspace && workspace_bytes >= scan) {
     int32_t* words = (int32_t*)workspace;
@@ -4615,8 +4797,7 @@ extern "C" int pa_attn_fwd_masked(const void* q, const void* k, const void* v, v
     // rows are gathered into dense copies, on which the fast kernels run with the counts as kv_len.  From 3e11 flop
     // on (0.3 ms), where a handful of launches that return at once no longer count, and where the workspace has room.
     const MaskedLayout lay = masked_layout(B, H, Skv, D);
-    const double flops = 4.0 * B * H * (double)Sq * (double)Skv * D;
-    const bool gather = flops >= 3.0e11 && workspace_bytes >= lay.dense;
+    const bool gather = flops >= GATHER_FLOP && workspace_bytes >= lay.dense;
     const size_t dense_off = gather ? lay.dense : scan;
     char* const dense_ws = (char*)workspace + dense_off;
     const size_t dense_bytes = workspace_bytes - dense_off;
@@ -4681,6 +4862,7 @@ extern "C" int pa_attn_fwd_masked(const void* q, const void* k, const void* v, v
     return attn_fwd_dense(q, k, v, out, lse, dtype, B, H, Sq, Skv, D, q_strides, k_strides, v_strides, out_strides,
                           scale, nullptr, 0, nullptr, 0, stream);
   }
+  if (pipe_takes) return masked_pipe(nullptr, 0);  // the workspace's first words are in use
   if (dtype == PA_DTYPE_BF16) return D == 128 ? launch_masked<BF16, 128>(p, mask_kind, st) : launch_masked<BF16, 64>(p, mask_kind, st);
   return D == 128 ? launch_masked<F16, 128>(p, mask_kind, st) : launch_masked<F16, 64>(p, mask_kind, st);
 }

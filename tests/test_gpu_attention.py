@@ -275,6 +275,45 @@ def test_general_masks_vs_f64(cuda, D, dtype):
         op(qd, kd, vd, torch.ones(B, Skv, dtype=torch.bool, device=cuda))  # [2,333] is not [Sq,Skv]
 
 
+@pytest.mark.parametrize("D", [128, 64])
+@pytest.mark.parametrize("bm", [128, 256])
+@pytest.mark.parametrize("Skv", [1, 64, 65, 255, 320])
+def test_key_only_masks_in_the_pipelined_kernels(cuda, tuning, D, bm, Skv):
+    """Masks without a query dimension at the edges of the 64-key tiles and of the 256-key steps in which the last kept
+    key is looked for: boolean (holes; the last key kept, or none in the second batch element; rows of dropped keys
+    that hold no numbers), one per head, on strided memory; additive in fp32 and the activation type, -inf and the
+    type's lowest value among the biases.  Tolerances of the unmasked kernels: the mask adds one fp32 operation."""
+    tuning("bm", bm)
+    B, H, Sq = 2, 3, 290
+    q, k, v = inputs.qkv(B, H, Sq, Skv, D, seed=Skv + D)
+    op = torch.ops.para_attn.attention_forward_with_lse
+    g = torch.Generator().manual_seed(Skv)
+    qn, kn, vn = q.float().numpy(), k.float().numpy(), v.float().numpy()
+    for shape in ((B, 1, 1, Skv), (1, H, 1, Skv)):
+        keep = torch.rand(shape, generator=g) < 0.6
+        keep[0, 0, 0, Skv - 1] = True
+        if shape[0] == B:
+            keep[1] = False
+        ref_out, ref_lse = oattn.sdpa_lse_f64(qn, kn, vn, None, np.broadcast_to(keep.numpy(), (B, H, Sq, Skv)))
+        kd = k.clone()
+        if shape[1] == 1:
+            kd.masked_fill_(~keep.expand(B, H, 1, Skv).transpose(2, 3), float("nan"))
+        strided = torch.zeros((*shape, 3), dtype=torch.bool, device=cuda)[..., 1]
+        strided.copy_(keep)
+        for m in (keep.to(cuda), strided):
+            out, lse = op(q.to(cuda), kd.to(cuda), v.to(cuda), m)
+            _check(out, lse, ref_out, ref_lse, f"key mask {shape}")
+        for dt in (torch.float32, q.dtype):
+            for low in (float("-inf"), torch.finfo(dt).min):
+                bias = (0.5 * torch.randn(shape, generator=g)).to(dt)
+                # the oracle takes no bias: it comes as one more column of q and k
+                qb = np.concatenate([qn, np.ones((B, H, Sq, 1))], -1)
+                kb = np.concatenate([kn, np.broadcast_to(math.sqrt(D) * bias.double().numpy(), (B, H, 1, Skv)).swapaxes(2, 3)], -1)
+                ref_out, ref_lse = oattn.sdpa_lse_f64(qb, kb, vn, 1.0 / math.sqrt(D), np.broadcast_to(keep.numpy(), (B, H, Sq, Skv)))
+                out, lse = op(q.to(cuda), k.to(cuda), v.to(cuda), bias.masked_fill(~keep, low).to(cuda))
+                _check(out, lse, ref_out, ref_lse, f"key bias {shape} {dt} {low}")
+
+
 def test_key_masks_take_the_fast_kernels_when_prefixes(cuda, tuning):
     """A key-only boolean mask is scanned on the device: prefixes run the dense kernels with per-batch key counts
     (here with the key-split tail and the score bound in play), anything else the per-score kernel; both give the
