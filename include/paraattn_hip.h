@@ -134,6 +134,23 @@ PA_API int pa_attn_fwd_lse_ws(const void* q, const void* k, const void* v, void*
                        float scale, const int32_t* kv_len, int is_causal, void* workspace,
                        size_t workspace_bytes, void* stream);
 
+/*
+ * Dense attention forward, optionally is_causal, for rows of D columns with D a
+ * multiple of 8 up to 96 other than 64 (and values as wide as the keys), read
+ * and written where they lie (the reference's aten kernels take any head_dim,
+ * src/para_attn/ops/__init__.py:58-109).  pa_attn_fwd_narrow_plan tells whether
+ * a call is taken (1) and the workspace it wants, 0 where zero-padded copies in
+ * pa_attn_fwd_lse_ws are the way (K or V of 2 GiB and more per head; up to 56
+ * columns, calls of 1e12 flop and more, whose softmax without a running maximum
+ * is worth the copies).  A null or short workspace is not an error, as there.
+ */
+PA_API int pa_attn_fwd_narrow_plan(int B, int H, int Sq, int Skv, int D, const int64_t k_strides[3],
+                       const int64_t v_strides[3], int is_causal, size_t* workspace_bytes);
+PA_API int pa_attn_fwd_narrow(const void* q, const void* k, const void* v, void* out, float* lse, int dtype,
+                       int B, int H, int Sq, int Skv, int D, const int64_t q_strides[3],
+                       const int64_t k_strides[3], const int64_t v_strides[3], const int64_t out_strides[3],
+                       float scale, int is_causal, void* workspace, size_t workspace_bytes, void* stream);
+
 /* kinds of attention mask taken by pa_attn_fwd_masked */
 #define PA_MASK_BOOL 1 /* bytes; 0 = the key is dropped for that query */
 #define PA_MASK_F32 2  /* fp32 bias added to the scaled score */
@@ -160,9 +177,11 @@ PA_API int pa_attn_fwd_lse_ws(const void* q, const void* k, const void* v, void*
  * is one of 3e11 flop or more, the kept K and V rows are gathered into dense
  * copies in the workspace, as the reference's attention_forward_sparse_kv
  * does with index_select (ops/__init__.py:276-296), and the same kernels run
- * on the copies.  Smaller calls with such a mask, and every other mask, run a
- * kernel that reads the mask per score.  The choice is made on the device:
- * nothing is read back, so the call can be captured in a HIP graph.
+ * on the copies.  Smaller calls with such a mask, and additive masks without a
+ * query dimension, run in the fast kernels too, which then load the mask once
+ * per key; every other mask runs a kernel that reads it per score.  The choice
+ * is made on the device: nothing is read back, so the call can be captured in a
+ * HIP graph.
  * workspace: pa_attn_fwd_masked_workspace_bytes() bytes (16-byte aligned, any
  * contents; from 3e11 flop on it includes the copies of K and V); null or
  * short is not an error: the per-score kernel runs where there is no room.

@@ -53,6 +53,11 @@ SIGNATURES = {
         [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _strides, _strides, _strides, _strides, _f, _vp, _i,
          _vp, _sz, _vp],
     ),
+    "pa_attn_fwd_narrow_plan": (_i, [_i, _i, _i, _i, _i, _strides, _strides, _i, ctypes.POINTER(_sz)]),
+    "pa_attn_fwd_narrow": (
+        _i,
+        [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _strides, _strides, _strides, _strides, _f, _i, _vp, _sz, _vp],
+    ),
     "pa_attn_fwd_masked": (
         _i,
         [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _strides, _strides, _strides, _strides, _f,

@@ -130,6 +130,7 @@ struct AttnParams {
   const void* mask;
   int64_t ms_b, ms_h, ms_q, ms_k;
   int mask_kind;  // MASK_*
+  int dt;  // columns of q, k, v and out that exist: head_dim (pipelined kernels built for narrower rows; 128 or 64 otherwise)
   // dense kernels: with `gate` set the launch leaves at once unless bit *gate of gate_mask is set (a decision taken on
   // the device by an earlier launch of the same stream, e.g. whether a key mask is a prefix)
   const int* gate;
@@ -693,6 +694,8 @@ constexpr int TILE_BYTES = BN * 256;  // one K or V tile at head_dim 128
 // Buffer offset that is out of range for every tensor the pipelined kernel accepts (its host side
 // refuses K or V extents of this size or more and takes the kernel above instead).
 constexpr uint32_t PIPE_OOB = 0xfffff000u;
+// Offset of the columns that narrow rows do not have; K and V extents stay below NARROW_LIMIT there.
+constexpr uint32_t NARROW_OOB = 0x80000000u, NARROW_LIMIT = 0x7fff0000u;
 
 typedef __attribute__((address_space(3))) char lds_char;
 typedef const __attribute__((address_space(1))) char glb_char;
@@ -1036,10 +1039,11 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_fwd_d128_kernel(const AttnPa
 // workgroups in several key shares (AttnParams::split_*), fold the result into a running
 // (out, lse) pair (acc_*), or apply torch's causal mask (causal).
 // ---------------------------------------------------------------------------------------------
-template <typename T, bool SPARSE, int NW, bool BOUNDED = false, bool PAIR = false, int PM = PM_NONE>
+template <typename T, bool SPARSE, int NW, bool BOUNDED = false, bool PAIR = false, int PM = PM_NONE, int W = 128>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_kernel(const AttnParams p) {
   typedef typename T::vec8 vec8;
-  constexpr int DC = 8, DB = 4;
+  constexpr int DC = W / 16, DB = W / 32;
+  static_assert(W == 128 || (W == 96 && !SPARSE && !PAIR && !BOUNDED), "row widths this kernel is written for");
   constexpr int IPW = 16 / NW;  // copy instructions per wavefront and K (V) tile
   // With a score bound on record the launch comes twice, once per variant, and the one the flag (computed on
   // the device just before) does not select leaves at once.  BOUNDED: exp2(score) cannot overflow or vanish, so
@@ -1122,7 +1126,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
     int r = row_ok ? my_row : (row_end - 1);
     const uint16_t* qp = qbase + (int64_t)r * p.qs_s + 8 * hh;
 #pragma unroll
-    for (int dc = 0; dc < DC; ++dc) qf[dc] = *(const vec8*)(qp + 16 * dc);
+    for (int dc = 0; dc < DC; ++dc) {
+      if (!(W < 128) || 16 * dc + 8 * hh < p.dt) qf[dc] = *(const vec8*)(qp + 16 * dc);
+      else qf[dc] = vec8{};  // the row ends here
+    }
     // no wait here: the loads overlap the first tile copies, whose wait in front of the first barrier covers them
   }
 
@@ -1136,7 +1143,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
   auto make_rsrc = [&](const char* base, uint32_t row_bytes, int n_keys) {
     u32x4 r;
     const uint64_t a = (uint64_t)base;
-    const uint64_t nbytes = (uint64_t)(n_keys - 1) * row_bytes + 256;  // start of the last row + one row
+    const uint64_t nbytes = (uint64_t)(n_keys - 1) * row_bytes + ((W < 128) ? 2 * p.dt : 256);  // start of the last row + one row
     r[0] = __builtin_amdgcn_readfirstlane((uint32_t)a);
     r[1] = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu);
     r[2] = __builtin_amdgcn_readfirstlane((uint32_t)nbytes);
@@ -1147,8 +1154,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
   u32x4 vrs = make_rsrc(vbytes, vs_bytes, p.Skv);
   const int dma_row = 4 * wave + (lane >> 4);
   const int dma_pc = lane & 15;
-  const uint32_t k_off0 = dma_row * ks_bytes + 16 * (dma_pc ^ (dma_row & 15));
-  const uint32_t v_off0 = dma_row * vs_bytes + 16 * (dma_pc ^ (4 * (dma_row & 3)));
+  // narrow rows: the chunks that do not exist come from beyond the descriptor's bound, as zeros (with extents below 2 GiB
+  // NARROW_OOB is out of range behind every tile's offset, also where the sum wraps around for a tile that does not exist)
+  const int k_chunk = dma_pc ^ (dma_row & 15), v_chunk = dma_pc ^ (4 * (dma_row & 3));
+  const uint32_t k_off0 = (W < 128) && 8 * k_chunk >= p.dt ? NARROW_OOB : dma_row * ks_bytes + 16 * k_chunk;
+  const uint32_t v_off0 = (W < 128) && 8 * v_chunk >= p.dt ? NARROW_OOB : dma_row * vs_bytes + 16 * v_chunk;
   const uint32_t lds_k = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_char*)sK + wave * 1024);
   const uint32_t lds_v = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_char*)sV + wave * 1024);
   constexpr uint32_t OOB = PIPE_OOB;  // first key of a tile that does not exist; also its soffset
@@ -1282,7 +1292,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
     // first fragments of K(j+1) on their way while the maximum is settled
     if (an) {
 #pragma unroll
-      for (int dc = 0; dc < DC; ++dc) f[dc] = read_k(tKn, dc & 1, dc >> 1);
+      for (int g = 0; g < 8; ++g) f[g] = read_k(tKn, g & 1, g >> 1);
     }
 
     if (!BOUNDED && ac) {
@@ -1335,6 +1345,51 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
     };
 #pragma unroll
     for (int r = 0; r < 16; ++r) sn0[r] = sn1[r] = 0.f;
+    if constexpr (W < 128) {
+      // The same pipeline for rows of up to 96 columns: 12 MFMAs in either stage.  Operand i (K(j+1) first, then V(j)
+      // in the order of use) sits in ring slot i % 8 and is fetched when MFMA i - 8 has issued.
+      constexpr int NA = 2 * DC, NB = 4 * DB;
+      auto fetch = [&](int i) {
+        if (i < NA) f[i & 7] = read_k(tKn, i & 1, i >> 1);
+        else if (i < NA + NB) f[i & 7] = read_vt(tV, (i - NA) / (2 * DB), (i - NA) / DB % 2, (i - NA) % DB);
+      };
+#pragma unroll
+      for (int i = 0; i < NA; ++i) {
+        if (i & 1) sn1 = T::mfma32(f[i & 7], qf[i >> 1], sn1);
+        else sn0 = T::mfma32(f[i & 7], qf[i >> 1], sn0);
+        if (i < IPW) dma_k1(par, n_nx2, i);
+        else if (i < 2 * IPW) dma_v1(par ^ 1, n_nxt, i - IPW);
+        fetch(i + 8);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (v_nxt < BN || on_diagonal(n_nxt)) mask_tail(sn0, sn1, v_nxt, n_nxt);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int n = 0; n < 6; ++n) expo_slot(n);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (NW == 4) __builtin_amdgcn_s_setprio(1);
+      __builtin_amdgcn_sched_barrier(0);
+      // four softmax slots under every three MFMAs: the 16 keys of the next three are packed when they are reached
+      float mxa = fmaxf(sn0[0], sn0[1]), mxb = fmaxf(sn1[0], sn1[1]);
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        const int i = NA + j, t = j / (2 * DB), cc = j / DB % 2, db = j % DB;
+        const uint32_t* pk = t == 0 ? pk0 : pk1;
+        u32x4 bw = {pk[4 * cc], pk[4 * cc + 1], pk[4 * cc + 2], pk[4 * cc + 3]};
+        o[db] = T::mfma32(f[i & 7], __builtin_bit_cast(vec8, bw), o[db]);
+        fetch(i + 8);
+#pragma unroll
+        for (int n = 4 * j / 3; n < 4 * (j + 1) / 3; ++n) expo_slot(6 + n);
+#pragma unroll
+        for (int n = 2 + 14 * j / NB; n < 2 + 14 * (j + 1) / NB; ++n) {
+          mxa = fmaxf(mxa, sn0[n]);
+          mxb = fmaxf(mxb, sn1[n]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      l_run += lsum;
+      mx = across(fmaxf(mxa, mxb));
+    } else {
 #pragma unroll
     for (int g = 0; g < 8; ++g) {
       // the two halves of S(j+1) alternate, so that no MFMA waits for the one just issued
@@ -1425,6 +1480,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
     }
     if (ac) l_run += lsum;
     if (!BOUNDED && an) mx = across(fmaxf(mxa, mxb));
+    }
 
     // slide the tile window
     n_cur = n_nxt;
@@ -1577,7 +1633,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
         u32x2 w;
         w[0] = T::pack2(o[db][4 * a] * inv, o[db][4 * a + 1] * inv);
         w[1] = T::pack2(o[db][4 * a + 2] * inv, o[db][4 * a + 3] * inv);
-        *(u32x2*)(op + 32 * db + 8 * a + 4 * hh) = w;
+        if (W == 128 || 32 * db + 8 * a < p.dt) *(u32x2*)(op + 32 * db + 8 * a + 4 * hh) = w;
       }
     if (p.lse != nullptr && hh == 0) {
       float lse = l_tot > 0.f ? (m_run + __builtin_amdgcn_logf(l_tot)) * LN2 : -INFINITY;
@@ -1601,7 +1657,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
 // ---------------------------------------------------------------------------------------------
 constexpr int TILE64_BYTES = BN * 128;
 
-template <typename T, bool SPARSE, int NW, bool BOUNDED = false, int PM = PM_NONE>
+template <typename T, bool SPARSE, int NW, bool BOUNDED = false, int PM = PM_NONE, bool NARROW = false>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_kernel(const AttnParams p) {
   // BOUNDED and the flag: as in attn_fwd_d128_pipe_kernel
   if constexpr (!SPARSE) {
@@ -1652,7 +1708,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
     int r = row_ok ? my_row : (row_end - 1);
     const uint16_t* qp = qbase + (int64_t)r * p.qs_s + 8 * hh;
 #pragma unroll
-    for (int dc = 0; dc < DC; ++dc) qf[dc] = *(const vec8*)(qp + 16 * dc);
+    for (int dc = 0; dc < DC; ++dc) {
+      if (!NARROW || 16 * dc + 8 * hh < p.dt) qf[dc] = *(const vec8*)(qp + 16 * dc);
+      else qf[dc] = vec8{};  // the row ends here
+    }
     // no wait here: the loads overlap the first tile copies, whose wait in front of the first barrier covers them
   }
 
@@ -1661,7 +1720,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
   auto make_rsrc = [&](const char* base, uint32_t row_bytes) {
     u32x4 r;
     const uint64_t a = (uint64_t)base;
-    const uint64_t nbytes = (uint64_t)(p.Skv - 1) * row_bytes + 128;  // start of the last row + one row
+    const uint64_t nbytes = (uint64_t)(p.Skv - 1) * row_bytes + (NARROW ? 2 * p.dt : 128);  // start of the last row + one row
     r[0] = __builtin_amdgcn_readfirstlane((uint32_t)a);
     r[1] = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu);
     r[2] = __builtin_amdgcn_readfirstlane((uint32_t)nbytes);
@@ -1672,8 +1731,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
   const u32x4 vrs = make_rsrc(vbytes, vs_bytes);
   const int dma_row = 8 * wave + (lane >> 3);
   const int dma_pc = lane & 7;
-  const uint32_t k_off0 = dma_row * ks_bytes + 16 * (dma_pc ^ ((dma_row >> 1) & 7));
-  const uint32_t v_off0 = dma_row * vs_bytes + 16 * (dma_pc ^ (4 * ((dma_row >> 1) & 1)));
+  // narrow rows: the chunks that do not exist come from beyond the descriptor's bound, as zeros (with extents below 2 GiB
+  // NARROW_OOB is out of range behind every tile's offset, also where the sum wraps around for a tile that does not exist)
+  const int k_chunk = dma_pc ^ ((dma_row >> 1) & 7), v_chunk = dma_pc ^ (4 * ((dma_row >> 1) & 1));
+  const uint32_t k_off0 = NARROW && 8 * k_chunk >= p.dt ? NARROW_OOB : dma_row * ks_bytes + 16 * k_chunk;
+  const uint32_t v_off0 = NARROW && 8 * v_chunk >= p.dt ? NARROW_OOB : dma_row * vs_bytes + 16 * v_chunk;
   const uint32_t lds_k = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_char*)sK + wave * 1024);
   const uint32_t lds_v = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_char*)sV + wave * 1024);
   constexpr uint32_t OOB = PIPE_OOB;
@@ -1931,7 +1993,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
         u32x2 w;
         w[0] = T::pack2(o[db][4 * a] * inv, o[db][4 * a + 1] * inv);
         w[1] = T::pack2(o[db][4 * a + 2] * inv, o[db][4 * a + 3] * inv);
-        *(u32x2*)(op + 32 * db + 8 * a + 4 * hh) = w;
+        if (!NARROW || 32 * db + 8 * a < p.dt) *(u32x2*)(op + 32 * db + 8 * a + 4 * hh) = w;
       }
     if (p.lse != nullptr && hh == 0) {
       float lse = l_tot > 0.f ? (m_run + __builtin_amdgcn_logf(l_tot)) * LN2 : -INFINITY;
@@ -3339,7 +3401,7 @@ __global__ __launch_bounds__(256) void attn_split_merge_kernel(const AttnParams 
   const int64_t r = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
   const int c8 = (threadIdx.x & 15) * 8;
   const int tl = (int)(r / p.bm), local = (int)(r % p.bm);
-  if (tl >= p.split_tiles) return;
+  if (tl >= p.split_tiles || c8 >= p.dt) return;
   const int tile = p.split_main + tl;
   const int qt = tile % p.n_qtiles, bh = tile / p.n_qtiles;
   const int head = bh % p.H, batch = bh / p.H;
@@ -3845,6 +3907,7 @@ static void fill_params(AttnParams& p, const void* q, const void* k, const void*
   p.acc_out = nullptr; p.acc_lse = nullptr; p.acc_first = 0;
   p.split_main = 0; p.split_tiles = 0; p.split_s = 0; p.ws_out = nullptr; p.ws_lse = nullptr;
   p.bound_flag = nullptr;
+  p.dt = 128; p.mask_kind = MASK_NONE;
   p.mask = nullptr; p.ms_b = p.ms_h = p.ms_q = p.ms_k = 0;
   p.gate = nullptr; p.gate_mask = 0;
   p.st = StreamPlan{};
@@ -4647,15 +4710,15 @@ static int launch_masked(const AttnParams& p, int mask_kind, hipStream_t stream)
   return PA_OK;
 }
 
-// A pipelined kernel with its mask handling PM, planned by choose_kernel like a dense call with per-batch key counts.
-template <typename T, int D, int PM, int NW>
-static int launch_masked_pipe_nw(const AttnParams& p, hipStream_t stream) {
+// A pipelined kernel with its mask handling PM, or for rows narrower than D (W < D), planned by choose_kernel like a dense call with per-batch key counts.
+template <typename T, int D, int PM, int NW, int W = D>
+static int launch_pipe_variant(const AttnParams& p, hipStream_t stream) {
   int64_t nblocks = (int64_t)p.B * p.H * p.n_qtiles;
   if (p.split_s > 1) nblocks = (int64_t)p.split_main + (int64_t)p.split_tiles * p.split_s;
-  const size_t smem = 4 * (D == 128 ? TILE_BYTES : TILE64_BYTES) + NW * PM_SLOT_BYTES;
+  const size_t smem = 4 * (D == 128 ? TILE_BYTES : TILE64_BYTES) + (PM == PM_NONE ? 0 : NW * PM_SLOT_BYTES);
   const void* fn;
-  if constexpr (D == 128) fn = (const void*)attn_fwd_d128_pipe_kernel<T, false, NW, false, false, PM>;
-  else fn = (const void*)attn_fwd_d64_pipe_kernel<T, false, NW, false, PM>;
+  if constexpr (D == 128) fn = (const void*)attn_fwd_d128_pipe_kernel<T, false, NW, false, false, PM, W>;
+  else fn = (const void*)attn_fwd_d64_pipe_kernel<T, false, NW, false, PM, (W < 64)>;
   static bool attr_done[PA_MAX_DEVICES] = {};  // benign race: the call is idempotent
   const int dev = current_device();
   if (dev < 0 || !attr_done[dev]) {
@@ -4664,10 +4727,10 @@ static int launch_masked_pipe_nw(const AttnParams& p, hipStream_t stream) {
     if (dev >= 0) attr_done[dev] = true;
   }
   if constexpr (D == 128)
-    hipLaunchKernelGGL((attn_fwd_d128_pipe_kernel<T, false, NW, false, false, PM>), dim3((unsigned)nblocks), dim3(64 * NW), smem, stream, p);
+    hipLaunchKernelGGL((attn_fwd_d128_pipe_kernel<T, false, NW, false, false, PM, W>), dim3((unsigned)nblocks), dim3(64 * NW), smem, stream, p);
   else
-    hipLaunchKernelGGL((attn_fwd_d64_pipe_kernel<T, false, NW, false, PM>), dim3((unsigned)nblocks), dim3(64 * NW), smem, stream, p);
-  PA_CHECK_LAUNCH("masked attention kernel");
+    hipLaunchKernelGGL((attn_fwd_d64_pipe_kernel<T, false, NW, false, PM, (W < 64)>), dim3((unsigned)nblocks), dim3(64 * NW), smem, stream, p);
+  PA_CHECK_LAUNCH("attention kernel (masked or narrow rows)");
   if constexpr (D == 128) {
     if (p.split_s > 1) {
       const int64_t rows = (int64_t)p.split_tiles * p.bm;
@@ -4681,8 +4744,62 @@ static int launch_masked_pipe_nw(const AttnParams& p, hipStream_t stream) {
 template <typename T, int D>
 static int launch_masked_pipe(const AttnParams& p, hipStream_t stream) {
   const bool keys = p.mask_kind == MASK_BOOL;
-  if (p.bm == 256) return keys ? launch_masked_pipe_nw<T, D, PM_KEYS, 8>(p, stream) : launch_masked_pipe_nw<T, D, PM_KEYBIAS, 8>(p, stream);
-  return keys ? launch_masked_pipe_nw<T, D, PM_KEYS, 4>(p, stream) : launch_masked_pipe_nw<T, D, PM_KEYBIAS, 4>(p, stream);
+  if (p.bm == 256) return keys ? launch_pipe_variant<T, D, PM_KEYS, 8>(p, stream) : launch_pipe_variant<T, D, PM_KEYBIAS, 8>(p, stream);
+  return keys ? launch_pipe_variant<T, D, PM_KEYS, 4>(p, stream) : launch_pipe_variant<T, D, PM_KEYBIAS, 4>(p, stream);
+}
+
+// Rows of D columns, D a multiple of 8 up to 96, unmasked or is_causal, read and written where they lie: the kernels
+// built for 64 and 128 columns with the columns that do not exist as zeros in LDS (the copies' descriptor gives them),
+// from 65 columns on with 12 MFMAs per stage and tile instead of 16.
+template <typename T>
+static int launch_narrow(const AttnParams& p, hipStream_t stream) {
+  if (p.dt > 64) return p.bm == 256 ? launch_pipe_variant<T, 128, PM_NONE, 8, 96>(p, stream) : launch_pipe_variant<T, 128, PM_NONE, 4, 96>(p, stream);
+  return p.bm == 256 ? launch_pipe_variant<T, 64, PM_NONE, 8, 32>(p, stream) : launch_pipe_variant<T, 64, PM_NONE, 4, 32>(p, stream);
+}
+
+// The plan of such a call; false: the pipelined kernels do not take it, or zero-padded copies in the kernels for 64
+// columns are faster (where their softmax without a running maximum applies).
+static bool plan_narrow(AttnParams& p, int D, size_t ws_avail, size_t* ws_need) {
+  const int built = D > 64 ? 128 : 64;
+  if (D % 8 || D < 8 || D > 96 || D == 64 || !pipe_fits(p, built)) return false;
+  if ((uint64_t)(p.Skv - 1) * (uint64_t)p.ks_s * 2 + 256 >= NARROW_LIMIT || (uint64_t)(p.Skv - 1) * (uint64_t)p.vs_s * 2 + 256 >= NARROW_LIMIT) return false;
+  if (built == 64 && bound_wanted(p.B, p.H, p.Sq, p.Skv, 64)) return false;
+  choose_kernel(p, built, 256, true, ws_avail, ws_need);
+  p.dt = D;
+  return true;
+}
+
+extern "C" int pa_attn_fwd_narrow_plan(int B, int H, int Sq, int Skv, int D, const int64_t k_strides[3], const int64_t v_strides[3],
+                                       int is_causal, size_t* workspace_bytes) {
+  if (workspace_bytes) *workspace_bytes = 0;
+  if (B <= 0 || H <= 0 || Sq <= 0 || Skv <= 0 || !k_strides || !v_strides) return 0;
+  const int64_t zero[3] = {0, 0, 0};
+  AttnParams p;
+  fill_params(p, nullptr, nullptr, nullptr, nullptr, nullptr, B, H, Sq, Skv, zero, k_strides, v_strides, zero, 1.f);
+  p.causal = is_causal != 0;
+  size_t need = 0;
+  if (!plan_narrow(p, D, 0, &need)) return 0;
+  if (workspace_bytes) *workspace_bytes = need;
+  return 1;
+}
+
+extern "C" int pa_attn_fwd_narrow(const void* q, const void* k, const void* v, void* out, float* lse, int dtype, int B, int H,
+                                  int Sq, int Skv, int D, const int64_t q_strides[3], const int64_t k_strides[3],
+                                  const int64_t v_strides[3], const int64_t out_strides[3], float scale, int is_causal,
+                                  void* workspace, size_t workspace_bytes, void* stream) {
+  int rc = check_common(q, k, v, out, dtype, B, H, Sq, Skv, D > 64 ? 128 : 64, q_strides, k_strides, v_strides, out_strides, scale);
+  if (rc) return rc;
+  if (workspace && ((uintptr_t)workspace) % 16) PA_FAIL(PA_ERR_WORKSPACE, "attention workspace not 16-byte aligned");
+  AttnParams p;
+  fill_params(p, q, k, v, out, lse, B, H, Sq, Skv, q_strides, k_strides, v_strides, out_strides, scale);
+  p.causal = is_causal != 0;
+  if (B <= 0 || H <= 0 || Sq <= 0 || !plan_narrow(p, D, workspace ? workspace_bytes : 0, nullptr))
+    PA_FAIL(PA_ERR_UNSUPPORTED, "pa_attn_fwd_narrow does not take this call (pa_attn_fwd_narrow_plan tells)");
+  if (p.split_s > 1) {
+    p.ws_out = (float*)workspace;
+    p.ws_lse = p.ws_out + (size_t)p.split_tiles * p.split_s * p.bm * 128;
+  }
+  return dtype == PA_DTYPE_BF16 ? launch_narrow<BF16>(p, (hipStream_t)stream) : launch_narrow<F16>(p, (hipStream_t)stream);
 }
 
 // Whether a dense call with per-batch key counts that leave nearly all keys would go to the resident-workgroup

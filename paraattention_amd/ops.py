@@ -55,7 +55,7 @@ def _kernel_ready(t):
 
 def _native_head_dims(query, value):
     """The kernels are built for head_dim 64 and 128 with values as wide as the keys; anything else up to 128 runs
-    through them zero-padded (``_pad_head_dims``)."""
+    through them on narrower rows (``_narrow_forward``) or zero-padded (``_pad_head_dims``)."""
     return query.shape[-1] == value.shape[-1] and query.shape[-1] in (64, 128)
 
 
@@ -63,7 +63,8 @@ def _pad_head_dims(query, key, value, scale):
     """q, k, v with head_dim zero-padded to 64 or 128 and the scale of the true head_dim.  Zero columns add nothing
     to q.k, and the padded columns of v give output columns that are dropped, so the result is that of the unpadded
     problem: head_dim 32, 40, 72, 80, 96 ... and values narrower or wider than the keys (which aten's kernels behind
-    src/para_attn/ops/__init__.py:58-109 take directly) at the price of one copy of each operand."""
+    src/para_attn/ops/__init__.py:58-109 take directly) at the price of one copy of each operand; multiples of 8 up to
+    96 without a mask come here only where ``_narrow_forward`` leaves them to it."""
     D, Dv = query.shape[-1], value.shape[-1]
     to = 64 if max(D, Dv) <= 64 else 128
     if scale is None:
@@ -150,6 +151,33 @@ def _dense_forward(query, key, value, scale, want_lse, kv_len=None, is_causal=Fa
     return out, lse
 
 
+def _narrow_forward(query, key, value, scale, want_lse, is_causal):
+    """head_dim 72, 80, 96, 40 ...: the kernels that read and write such rows where they lie (pa_attn_fwd_narrow), or
+    None where the call goes through zero-padded copies."""
+    B, H, Sq, D = query.shape
+    Skv = key.shape[2]
+    if value.shape[-1] != D or D % 8 or D > 96:
+        return None
+    _same_device(query, key=key, value=value)
+    q, k, v = _kernel_ready(query), _kernel_ready(key), _kernel_ready(value)
+    ks, vs = _lib.strides3(k), _lib.strides3(v)
+    lib = _lib.load()
+    with torch.cuda.device(q.device):
+        ws_bytes = ctypes.c_size_t()
+        if not lib.pa_attn_fwd_narrow_plan(B, H, Sq, Skv, D, ks, vs, 1 if is_causal else 0, ctypes.byref(ws_bytes)):
+            return None
+        out = _out_like(query, value)
+        lse = _lse_like(query) if want_lse else None
+        ws = torch.empty(ws_bytes.value, dtype=torch.uint8, device=q.device) if ws_bytes.value else None
+        rc = lib.pa_attn_fwd_narrow(
+            _ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(lse), _DTYPE_CODE[q.dtype], B, H, Sq, Skv, D,
+            _lib.strides3(q), ks, vs, _lib.strides3(out), float(1.0 / math.sqrt(D) if scale is None else scale),
+            1 if is_causal else 0, _ptr(ws), ws_bytes.value, _stream_ptr(q.device),
+        )
+    _lib.check(rc, "pa_attn_fwd_narrow")
+    return out, lse
+
+
 def _accumulate_forward(acc_out, acc_lse, query, key, value, scale, first, final):
     """One fused ring step (pa_attn_fwd_accumulate); returns the 16-bit output if ``final``."""
     B, H, Sq, D = query.shape
@@ -211,6 +239,10 @@ def _masked_forward(query, key, value, attn_mask, scale, want_lse, is_causal=Fal
     the host: whether a key mask is a prefix is settled on the device (pa_attn_fwd_masked), so masked calls can
     be captured in a HIP graph like the unmasked ones."""
     if not _native_head_dims(query, value):
+        if attn_mask is None:
+            res = _narrow_forward(query, key, value, scale, want_lse, is_causal)
+            if res is not None:
+                return res
         q, k, v, scale = _pad_head_dims(query, key, value, scale)
         out, lse = _masked_forward(q, k, v, attn_mask, scale, want_lse, is_causal)
         return out[..., : value.shape[-1]].contiguous(), lse

@@ -314,6 +314,35 @@ def test_key_only_masks_in_the_pipelined_kernels(cuda, tuning, D, bm, Skv):
                 _check(out, lse, ref_out, ref_lse, f"key bias {shape} {dt} {low}")
 
 
+@pytest.mark.parametrize("D", [8, 40, 56, 72, 80, 96])
+@pytest.mark.parametrize("bm", [0, 128, 256])
+@pytest.mark.parametrize("Sq,Skv", [(1, 1), (130, 65), (290, 320), (257, 4130)])
+def test_narrow_rows_in_place(cuda, tuning, D, bm, Sq, Skv):
+    """head_dims between the two the kernels are built for, read and written where they lie: [B,H,S,D] and [B,S,H,D]
+    memory, operands that end with their storage and sit in a sea of NaN (nothing may be read between or behind the
+    rows), is_causal, and (4130 keys, few query tiles) key-split partial results of fewer than 128 columns."""
+    tuning("bm", bm)
+    B, H = 2, 3
+    q, k, v = inputs.qkv(B, H, Sq, Skv, D, seed=D + Skv)
+    qn, kn, vn = q.float().numpy(), k.float().numpy(), v.float().numpy()
+    op = torch.ops.para_attn.attention_forward_with_lse
+
+    def among_nans(t, bshd):
+        wide = torch.full((B, t.shape[2], H, D + 8) if bshd else (B, H, t.shape[2], D + 8), float("nan"), dtype=t.dtype, device=cuda)
+        view = wide[..., 8:].transpose(1, 2) if bshd else wide[..., 8:]
+        return view.copy_(t)
+
+    for causal in (False, True):
+        keep = oattn.causal_keep(Sq, Skv) if causal else None
+        ref_out, ref_lse = oattn.sdpa_lse_f64(qn, kn, vn, None, keep)
+        for bshd in (False, True):
+            out, lse = op(among_nans(q, bshd), among_nans(k, bshd), among_nans(v, bshd), is_causal=causal)
+            assert out.is_contiguous()
+            _check(out, lse, ref_out, ref_lse, f"narrow rows, causal={causal} bshd={bshd}")
+        out, lse = op(q.to(cuda), k.to(cuda), v.to(cuda), is_causal=causal)
+        _check(out, lse, ref_out, ref_lse, f"narrow rows, contiguous, causal={causal}")
+
+
 def test_key_masks_take_the_fast_kernels_when_prefixes(cuda, tuning):
     """A key-only boolean mask is scanned on the device: prefixes run the dense kernels with per-batch key counts
     (here with the key-split tail and the score bound in play), anything else the per-score kernel; both give the
