@@ -97,6 +97,7 @@ struct AttnParams {
   int bm;            // query rows per workgroup (32 per wavefront)
   int pipe;          // head_dim 128: 1 = pipelined kernel, 0 = the one without 32-bit offset limits
   const int32_t* kv_len;  // dense: optional per-batch key count
+  int heads_first;  // pipelined dense kernels: the heads are the fastest grid index, not the query tiles
   int causal;             // dense: query row i sees keys 0..i only (torch's is_causal, top-left aligned)
   // block-sparse only
   const int32_t* runs;  // count[Hm*nSeg] then range[Hm*nSeg][cap][2]
@@ -257,8 +258,7 @@ __device__ __forceinline__ void decode_block(const AttnParams& p, int qt, int he
     const int cnt = p.runs[sidx];
     it.init_list(p.runs + (size_t)p.Hm * nseg + (size_t)sidx * p.cap * 2, cnt, p.Skv, p.pair != 0);
   } else {
-    // causal: a workgroup's work grows with its row index, so the longest ones are started first
-    if (p.causal) qt = p.n_qtiles - 1 - qt;
+    if (p.causal) qt = p.n_qtiles - 1 - qt;  // a workgroup's work grows with its row index: the longest ones first
     row_begin = qt * p.bm;
     row_end = row_begin + p.bm < p.Sq ? row_begin + p.bm : p.Sq;
     int len = p.Skv;
@@ -604,7 +604,7 @@ constexpr float PM_NO_MAX = -3.402823466e38f;
 template <typename T, int PM>
 struct TileMask {
   const char* base;  // this (batch, head)'s mask elements
-  int64_t step;      // bytes per key
+  uint32_t step;     // bytes per key; all of them span less than 2 GiB
   uint32_t last, raw;
   int lane, hh;
   bool act;  // 16-bit elements in the activation type
@@ -618,7 +618,7 @@ struct TileMask {
     act = PM == PM_KEYBIAS && p.mask_kind == MASK_ACT;
     const int bytes = PM == PM_KEYS ? 1 : act ? 2 : 4;
     base = (const char*)p.mask + at * bytes;
-    step = p.ms_k * bytes;
+    step = (uint32_t)(p.ms_k * bytes);
     per_scale = 1.0f / (p.scale_log2 * LN2);  // bias / scale, so that (s + that) * c = s * c + bias * log2(e)
     slot = (float*)lds;
   }
@@ -631,7 +631,7 @@ struct TileMask {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int key = top - 64 * (i + 1) + lane;
-        if (key >= 0 && *(const uint8_t*)(base + (int64_t)key * step) != 0) best = best > key + 1 ? best : key + 1;
+        if (key >= 0 && *(const uint8_t*)(base + (uint32_t)key * step) != 0) best = best > key + 1 ? best : key + 1;
       }
 #pragma unroll
       for (int d = 32; d > 0; d >>= 1) { const int o = __shfl_xor(best, d); best = o > best ? o : best; }
@@ -643,7 +643,7 @@ struct TileMask {
   __device__ __forceinline__ void fetch(uint32_t n0) {
     uint32_t key = n0 + lane;
     key = key < last ? key : last;
-    const char* at = base + (int64_t)key * step;
+    const char* at = base + key * step;
     if constexpr (PM == PM_KEYS) raw = *(const uint8_t*)at;
     else if (act) raw = *(const uint16_t*)at;
     else raw = *(const uint32_t*)at;
@@ -1082,8 +1082,13 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
       tile = p.split_main + piece_slot % p.split_tiles;
     }
   }
-  const int qt = tile % p.n_qtiles;
-  const int bh = tile / p.n_qtiles;
+  int qt = tile % p.n_qtiles, bh = tile / p.n_qtiles;
+  if constexpr (!SPARSE) {
+    if (p.heads_first) {
+      qt = tile / (p.B * p.H);
+      bh = tile - qt * (p.B * p.H);
+    }
+  }
   const int head = bh % p.H;
   const int batch = bh / p.H;
   int row_begin, row_end;
@@ -1679,14 +1684,26 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
   const int hh = lane >> 5;
 
   int tile = blockIdx.x;
+  int piece_slot = -1;  // >= 0: this workgroup computes one key share of a split query tile
+  if constexpr (!SPARSE) {
+    if (p.split_s > 1 && tile >= p.split_main) {
+      piece_slot = tile - p.split_main;
+      tile = p.split_main + piece_slot % p.split_tiles;
+    }
+  }
   if constexpr (SPARSE) {
     if (p.xcd_chunk > 0) {  // one contiguous eighth of the (head, query tile) list per XCD
       tile = (tile & 7) * p.xcd_chunk + (tile >> 3);
       if (tile >= p.B * p.H * p.n_qtiles) return;
     }
   }
-  const int qt = tile % p.n_qtiles;
-  const int bh = tile / p.n_qtiles;
+  int qt = tile % p.n_qtiles, bh = tile / p.n_qtiles;
+  if constexpr (!SPARSE) {
+    if (p.heads_first) {
+      qt = tile / (p.B * p.H);
+      bh = tile - qt * (p.B * p.H);
+    }
+  }
   const int head = bh % p.H;
   const int batch = bh / p.H;
   int row_begin, row_end;
@@ -1695,6 +1712,15 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
   TileMask<T, PM> tm;
   if constexpr (PM != PM_NONE) tm.init(p, batch, head, lane, (char*)smem + 4 * TILE64_BYTES + wave * PM_SLOT_BYTES);
   if constexpr (PM == PM_KEYS) it.init_dense(__builtin_amdgcn_readfirstlane(tm.kept_end(p.Skv)));
+
+  if constexpr (!SPARSE) {
+    if (piece_slot >= 0) {
+      const int piece = piece_slot / p.split_tiles, len = it.end;
+      const int nkt = (len + BN - 1) / BN;
+      const int t0 = (int)((int64_t)piece * nkt / p.split_s), t1 = (int)((int64_t)(piece + 1) * nkt / p.split_s);
+      it.init_range(t0 * BN, t1 * BN < len ? t1 * BN : len);
+    }
+  }
 
   const uint16_t* qbase = (const uint16_t*)p.q + batch * p.qs_b + head * p.qs_h;
   const char* kbytes = (const char*)((const uint16_t*)p.k + batch * p.ks_b + head * p.ks_h);
@@ -1984,6 +2010,23 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
     l_tot = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
   }
   const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
+  if constexpr (!SPARSE) {
+    if (piece_slot >= 0) {  // partial result of one key share: fp32, into the workspace (rows of 128, 64 of them used)
+      if (row_ok) {
+        const int64_t wrow = (int64_t)piece_slot * p.bm + (my_row - row_begin);
+        float* wp = p.ws_out + wrow * 128;
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+          for (int a = 0; a < 4; ++a) {
+            float4 w = {o[db][4 * a] * inv, o[db][4 * a + 1] * inv, o[db][4 * a + 2] * inv, o[db][4 * a + 3] * inv};
+            *(float4*)(wp + 32 * db + 8 * a + 4 * hh) = w;
+          }
+        if (hh == 0) p.ws_lse[wrow] = l_tot > 0.f ? (m_run + __builtin_amdgcn_logf(l_tot)) * LN2 : -INFINITY;
+      }
+      return;
+    }
+  }
   if (row_ok) {
     uint16_t* op = (uint16_t*)p.out + batch * p.os_b + head * p.os_h + (int64_t)my_row * p.os_s;
 #pragma unroll
@@ -3903,7 +3946,7 @@ static void fill_params(AttnParams& p, const void* q, const void* k, const void*
   p.Hm = 0; p.nQ = 0; p.cap = 0; p.q_lo = 0; p.q_block = 0; p.pair = 0; p.tiles_left = 0; p.tiles_per_block = 0;
   p.bm = BM; p.pipe = 0;
   p.xcd_chunk = 0;
-  p.causal = 0;
+  p.causal = 0; p.heads_first = 0;
   p.acc_out = nullptr; p.acc_lse = nullptr; p.acc_first = 0;
   p.split_main = 0; p.split_tiles = 0; p.split_s = 0; p.ws_out = nullptr; p.ws_lse = nullptr;
   p.bound_flag = nullptr;
@@ -3917,9 +3960,9 @@ template <typename T, int D, bool SPARSE>
 static int launch_attn(const AttnParams& p, hipStream_t stream) {
   int64_t nblocks = (int64_t)p.B * p.H * p.n_qtiles;
   if (nblocks == 0) return PA_OK;
-  // only the head_dim-128 pipelined kernel folds into a running pair or splits keys; the others would
-  // store through the (absent) plain output
-  if ((p.acc_out != nullptr || p.split_s > 1) && !(D == 128 && p.pipe && !SPARSE))
+  // only the head_dim-128 pipelined kernel folds into a running pair, only the dense pipelined kernels split keys; the
+  // others would store through the (absent) plain output
+  if ((p.acc_out != nullptr && !(D == 128 && p.pipe && !SPARSE)) || (p.split_s > 1 && !(p.pipe && !SPARSE)))
     PA_FAIL(PA_ERR_UNSUPPORTED, "accumulation / key split reached a kernel that has neither");
   if (p.out == nullptr && p.acc_out == nullptr) PA_FAIL(PA_ERR_INVALID, "null output pointer");
   if (p.split_s > 1) nblocks = (int64_t)p.split_main + (int64_t)p.split_tiles * p.split_s;
@@ -3996,7 +4039,7 @@ static int launch_attn(const AttnParams& p, hipStream_t stream) {
       hipLaunchKernelGGL((attn_fwd_kernel<T, D, SPARSE>), dim3((unsigned)nblocks), dim3(NTHREADS), smem, stream, p);
   }
   PA_CHECK_LAUNCH("attention kernel");
-  if constexpr (D == 128 && !SPARSE) {
+  if constexpr (!SPARSE) {
     if (p.split_s > 1) {
       const int64_t rows = (int64_t)p.split_tiles * p.bm;
       hipLaunchKernelGGL((attn_split_merge_kernel<T>), dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, stream, p);
@@ -4022,16 +4065,18 @@ struct SplitPlan {
 // dealing of workgroups to 8 XCDs) are MI355X's: 256 compute units in 8 XCDs.  On a device that reports another
 // compute-unit count the launches fall back to plain plans: no key split priced by those constants, no XCD order.
 static bool mi355x_layout() { return device_cus() == 256; }
-static SplitPlan plan_split(int64_t n_tiles, int slots, int kv_tiles, int bm, bool allow) {
+static SplitPlan plan_split(int64_t n_tiles, int slots, int kv_tiles, int bm, bool allow, double tile_us = 1.75, bool pairs = false) {
   if (slots <= 0) return {0, 1, 1.0};  // no device to ask: no estimate, no split
   SplitPlan best = {0, 1, (double)((n_tiles + slots - 1) / slots)};
+  // pairs: two places per compute unit; a last round of one workgroup per unit runs 1.5 times as fast
+  if (pairs && n_tiles % slots != 0 && n_tiles % slots <= slots / 2) best.rounds -= 0.33;
   if (!allow || n_tiles % slots == 0) return best;
   SplitPlan found = best;
   double best_found = best.rounds;
   // one round in microseconds (a key tile takes a workgroup about 1.75 us), to price the merge launch in
   // rounds: about 8 us of launch gap plus its partials at 3 TB/s (measured: 17.7 us for 46 MB; at 4608 keys
   // that is 0.13 of a round and the split loses, at 119k keys 0.03 and it wins)
-  const double round_us = ((double)kv_tiles + 4.0) * 1.75;
+  const double round_us = ((double)kv_tiles + 4.0) * tile_us;
   for (int extra = 0; extra < 2; ++extra) {
     const int64_t T = n_tiles % slots + (int64_t)extra * slots;
     if (T > n_tiles || T * 8 > 0x7fffffffLL) break;
@@ -4145,9 +4190,33 @@ static void choose_kernel(AttnParams& p, int D, int q_block, bool dense, size_t 
   if (!pipe_fits(p, D)) return finish();
   p.pipe = 1;
   const int forced = tuning().forced_bm;  // tuning aid
-  if (D == 64) {  // no key split at head_dim 64; 128 rows unless asked otherwise
+  const int n_cus = device_cus();
+  // is_causal: workgroups differ in length.  Where the query tiles of one head do not fill the chip the heads are the
+  // fastest grid index, so that the longest workgroups of all heads start first; in the order of the heads the last
+  // heads' longest ones start when the rest is done (24 heads x 4096 tokens, head_dim 64: 97 -> 76 us; head_dim 128 160 -> 110 us, 12 heads x 16384 tokens 912 -> 792).  Where they do,
+  // the order of the heads keeps the resident workgroups on one head's K and V.
+  auto order = [&] {
+    finish();
+    p.heads_first = dense && p.causal && n_cus > 0 && (int64_t)p.n_qtiles * p.bm < (int64_t)2 * n_cus * 128;
+  };
+  // head_dim 64: 128 rows unless asked otherwise, and the key-split tail beyond one round of workgroups (48 heads x
+  // 17776 tokens, 6672 workgroups on 512 places: 3.99 -> 3.84 ms; 3 heads x 24000: 0.58 -> 0.47 ms)
+  if (D == 64) {
+    p.dt = 64;
     if (forced == 256 && (dense || q_block % 256 == 0)) p.bm = 256;
-    return finish();
+    order();
+    const bool may = dense && n_cus > 0 && mi355x_layout() && !p.causal && !tuning().no_split && (ws_needed != nullptr || ws_bytes > 0);
+    const int64_t tiles = (int64_t)p.B * p.H * p.n_qtiles;
+    const int slots = p.bm == 256 ? n_cus : 2 * n_cus;
+    if (!may || tiles <= slots) return;
+    SplitPlan pl = plan_split(tiles, slots, (p.Skv + BN - 1) / BN, p.bm, true, 1.0, p.bm == 128);
+    if (ws_needed) *ws_needed = split_ws_bytes(pl, p.bm);
+    else if (pl.s > 1 && split_ws_bytes(pl, p.bm) <= ws_bytes) {
+      p.split_s = pl.s;
+      p.split_tiles = pl.tiles;
+      p.split_main = (int)(tiles - pl.tiles);
+    }
+    return;
   }
   if (!dense) {  // block-sparse: workgroups differ in length, no split
     // query blocks that are multiples of 256 rows take 256-row workgroups where there are two or more of them per
@@ -4184,7 +4253,7 @@ static void choose_kernel(AttnParams& p, int D, int q_block, bool dense, size_t 
   if (forced == 256) use256 = true;
   const SplitPlan& pl = use256 ? p256 : p128;
   p.bm = use256 ? 256 : 128;
-  finish();
+  order();
   if (ws_needed) *ws_needed = split_ws_bytes(pl, p.bm);
   if (pl.s > 1 && !ws_needed) {
     p.split_s = pl.s;
@@ -4731,12 +4800,10 @@ static int launch_pipe_variant(const AttnParams& p, hipStream_t stream) {
   else
     hipLaunchKernelGGL((attn_fwd_d64_pipe_kernel<T, false, NW, false, PM, (W < 64)>), dim3((unsigned)nblocks), dim3(64 * NW), smem, stream, p);
   PA_CHECK_LAUNCH("attention kernel (masked or narrow rows)");
-  if constexpr (D == 128) {
-    if (p.split_s > 1) {
-      const int64_t rows = (int64_t)p.split_tiles * p.bm;
-      hipLaunchKernelGGL((attn_split_merge_kernel<T>), dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, stream, p);
-      PA_CHECK_LAUNCH("attention split merge kernel");
-    }
+  if (p.split_s > 1) {
+    const int64_t rows = (int64_t)p.split_tiles * p.bm;
+    hipLaunchKernelGGL((attn_split_merge_kernel<T>), dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, stream, p);
+    PA_CHECK_LAUNCH("attention split merge kernel");
   }
   return PA_OK;
 }
@@ -4895,7 +4962,7 @@ extern "C" int pa_attn_fwd_masked(const void* q, const void* k, const void* v, v
     if (dtype == PA_DTYPE_BF16) return D == 128 ? launch_masked_pipe<BF16, 128>(p, st) : launch_masked_pipe<BF16, 64>(p, st);
     return D == 128 ? launch_masked_pipe<F16, 128>(p, st) : launch_masked_pipe<F16, 64>(p, st);
   };
-  const bool pipe_takes = no_query_dim && pipe_fits(p, D);
+  const bool pipe_takes = no_query_dim && pipe_fits(p, D) && (int64_t)(Skv - 1) * (p.ms_k > 0 ? p.ms_k : 1) < (int64_t)1 << 29;  // TileMask::step
   // A boolean mask that only selects keys (the same for every head and query row; what the text padding of
   // video DiTs looks like) is usually a prefix per batch element.  Whether it is, is found out on the device: a
   // small scan writes the kept-key counts and a flag, then both the dense launch (counts as kv_len) and the

@@ -343,6 +343,34 @@ def test_narrow_rows_in_place(cuda, tuning, D, bm, Sq, Skv):
         _check(out, lse, ref_out, ref_lse, f"narrow rows, contiguous, causal={causal}")
 
 
+@pytest.mark.parametrize("D,bound", [(64, -1), (64, 1), (40, -1)])
+def test_key_split_tail_head_dim_64(cuda, tuning, D, bound):
+    """33 heads x 16 query tiles leave 16 of 528 workgroups to a last round of 512 places: at head_dim 64 (and on narrow
+    rows) they are computed as key shares and folded.  The head that holds them against the oracle, the others bit for
+    bit against the launch without the split; unmasked, with and without a score bound, and under a key mask whose
+    last shares are empty in part."""
+    tuning("bound", bound)
+    B, H, Sq, Skv = 1, 33, 2048 - 5, 8192 + 3
+    q, k, v = inputs.qkv(B, H, Sq, Skv, D, seed=D)
+    dev = [t.to(cuda) for t in (q, k, v)]
+    op = torch.ops.para_attn.attention_forward_with_lse
+    keep = torch.rand(Skv, generator=torch.Generator().manual_seed(1)) < 0.7
+    keep[5000:] = False
+    last = [t[:, -1:].float().numpy() for t in (q, k, v)]
+    for mask in (None, keep):
+        if mask is not None and D == 40:
+            continue  # (masked narrow rows run padded)
+        m = None if mask is None else mask.to(cuda)[None, None, None, :]
+        ref_out, ref_lse = oattn.sdpa_lse_f64(*last, None, None if mask is None else mask.numpy())
+        tuning("no_split", 0)
+        out, lse = op(*dev, m)
+        tuning("no_split", 1)
+        out1, lse1 = op(*dev, m)
+        _check(out[:, -1:], lse[:, -1:], ref_out, ref_lse, f"split tail, masked={mask is not None}")
+        assert torch.equal(out[:, :-1], out1[:, :-1]) and torch.equal(lse[:, :-1], lse1[:, :-1])
+        assert not torch.equal(lse[:, -1], lse1[:, -1])  # another order of sums: the split was taken
+
+
 def test_key_masks_take_the_fast_kernels_when_prefixes(cuda, tuning):
     """A key-only boolean mask is scanned on the device: prefixes run the dense kernels with per-batch key counts
     (here with the key-split tail and the score bound in play), anything else the per-score kernel; both give the
