@@ -156,7 +156,11 @@ def set_tuning(name, value):
     check(load().pa_set_tuning(name.encode(), int(value)), "pa_set_tuning")
 
 
+_I64x3 = _i64 * 3  # one array type for all calls: ctypes takes 1 us to make one
+
+
 def strides3(t):
     """(batch, head, seq) strides of a 4-D tensor as a C int64[3]; size-1 dims get stride 0."""
-    st = [0 if t.shape[d] == 1 else t.stride(d) for d in range(3)]
-    return (ctypes.c_int64 * 3)(*st)
+    b, h, s, _ = t.stride()
+    nb, nh, ns, _ = t.shape
+    return _I64x3(0 if nb == 1 else b, 0 if nh == 1 else h, 0 if ns == 1 else s)

@@ -34,12 +34,31 @@ from . import _lib
 _DTYPE_CODE = {torch.bfloat16: _lib.PA_DTYPE_BF16, torch.float16: _lib.PA_DTYPE_F16, torch.float32: _lib.PA_DTYPE_F32}
 
 
+# What every call passes through before its launch costs more than the launch if it is spelled out (small calls: 38 us
+# of host work, 24 of them here, against 5 us for a launch): raw pointers and streams travel as Python integers, and
+# the device is switched only where it is not the current one.
 def _stream_ptr(device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
+
+
+class _StayOnDevice:
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return False
+
+
+_STAY = _StayOnDevice()
+
+
+def _on(device):
+    """Context in which ``device`` is the current one."""
+    return _STAY if torch._C._cuda_getDevice() == device.index else torch.cuda.device(device)
 
 
 def _ptr_array(tensors):
@@ -48,9 +67,17 @@ def _ptr_array(tensors):
 
 def _kernel_ready(t):
     """Rows must be unit-stride and 16-byte aligned for the kernels' vector loads."""
-    if t.stride(-1) != 1 or any(t.shape[d] > 1 and t.stride(d) % 8 for d in range(t.ndim - 1)) or t.data_ptr() % 16:
-        return t.contiguous()
-    return t
+    return t if _vector_rows(t) and t.data_ptr() % 16 == 0 else t.contiguous()
+
+
+def _vector_rows(t):
+    *lead, last = t.stride()
+    if last != 1:
+        return False
+    for n, step in zip(t.shape, lead):
+        if step % 8 and n > 1:
+            return False
+    return True
 
 
 def _native_head_dims(query, value):
@@ -82,7 +109,7 @@ def _out_like(query, value=None):
     if value is not None and not _native_head_dims(query, value):
         return torch.empty((*query.shape[:3], value.shape[-1]), dtype=query.dtype, device=query.device)
     out = torch.empty_like(query)
-    if out.stride(-1) != 1 or any(out.shape[d] > 1 and out.stride(d) % 8 for d in range(out.ndim - 1)):
+    if not _vector_rows(out):
         out = torch.empty(query.shape, dtype=query.dtype, device=query.device)
     return out
 
@@ -96,9 +123,10 @@ def _same_device(ref, **operands):
     """The kernels take raw pointers, so an operand on another device (a CPU mask beside GPU activations) must stop
     here with an error, as it does in the aten ops the reference calls, and not at a memory fault on the GPU.
     Every function below that hands a tensor's pointer to the library runs its tensors through this first."""
+    device = ref.device
     for name, t in operands.items():
-        if t is not None and t.device != ref.device:
-            raise ValueError(f"{name} is on {t.device} but must be on {ref.device}: all operands must share one device")
+        if t is not None and t.device != device:
+            raise ValueError(f"{name} is on {t.device} but must be on {device}: all operands must share one device")
 
 
 def _check_sdpa_args(query, key, value, dropout_p, is_causal, attn_mask=None, causal_ok=False, any_head_dim=False):
@@ -136,7 +164,7 @@ def _dense_forward(query, key, value, scale, want_lse, kv_len=None, is_causal=Fa
     if scale is None:
         scale = 1.0 / math.sqrt(D)
     lib = _lib.load()
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         # scratch for the score bound and the key-split tail of the launch (torch's caching allocator:
         # no hipMalloc in the steady state); its lifetime on the launch stream is the allocator's business
         ks, vs = _lib.strides3(k), _lib.strides3(v)
@@ -162,7 +190,7 @@ def _narrow_forward(query, key, value, scale, want_lse, is_causal):
     q, k, v = _kernel_ready(query), _kernel_ready(key), _kernel_ready(value)
     ks, vs = _lib.strides3(k), _lib.strides3(v)
     lib = _lib.load()
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         ws_bytes = ctypes.c_size_t()
         if not lib.pa_attn_fwd_narrow_plan(B, H, Sq, Skv, D, ks, vs, 1 if is_causal else 0, ctypes.byref(ws_bytes)):
             return None
@@ -194,7 +222,7 @@ def _accumulate_forward(acc_out, acc_lse, query, key, value, scale, first, final
     if scale is None:
         scale = 1.0 / math.sqrt(D)
     lib = _lib.load()
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         ks, vs = _lib.strides3(k), _lib.strides3(v)
         ws_bytes = lib.pa_attn_fwd_workspace_bytes(B, H, Sq, Skv, D, ks, vs)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
@@ -258,7 +286,7 @@ def _masked_forward(query, key, value, attn_mask, scale, want_lse, is_causal=Fal
     if scale is None:
         scale = 1.0 / math.sqrt(D)
     lib = _lib.load()
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         ks, vs = _lib.strides3(k), _lib.strides3(v)
         ws_bytes = lib.pa_attn_fwd_masked_workspace_bytes(B, H, Sq, Skv, D, ks, vs)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
@@ -365,7 +393,7 @@ def _merge_launch(acc_out, acc_lse, blk_out, blk_lse, out, lse_out):
     D = acc_out.shape[-1]
     rows = acc_out.numel() // D if D else 0
     lib = _lib.load()
-    with torch.cuda.device(acc_out.device):
+    with _on(acc_out.device):
         rc = lib.pa_merge_lse(
             _ptr(acc_out), _DTYPE_CODE[acc_out.dtype], _ptr(acc_lse),
             _ptr(blk_out), _DTYPE_CODE[blk_out.dtype], _ptr(blk_lse),
@@ -519,7 +547,7 @@ def attention_forward_sweep(
     if scale is None:
         scale = 1.0 / math.sqrt(D)
     lib = _lib.load()
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         kst, vst = _lib.strides3(ks[0]), _lib.strides3(vs[0])
         ws_bytes = lib.pa_attn_fwd_sweep_workspace_bytes(B, H, Sq, n, blk, D, kst, vst)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
@@ -605,7 +633,7 @@ def attention_forward_block_sparse(
     ws = torch.empty((ws_bytes + 3) // 4, dtype=torch.int32, device=q.device)
     if scale is None:
         scale = 1.0 / math.sqrt(D)
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         rc = lib.pa_attn_fwd_blocksparse(
             _ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(lse), _DTYPE_CODE[q.dtype], B, H, Sq, Skv, D,
             _lib.strides3(q), _lib.strides3(k), _lib.strides3(v), _lib.strides3(out), float(scale),
@@ -648,7 +676,7 @@ def block_sparse_key_runs(block_mask: torch.Tensor, seq_kv: int, kv_lo: int = 0,
     ws = torch.zeros(_runs_words(Hm, nQ, nK), dtype=torch.int32, device=block_mask.device)
     ws_bytes = ws.numel() * 4
     mask_u8 = block_mask.contiguous().view(torch.uint8)
-    with torch.cuda.device(block_mask.device):
+    with _on(block_mask.device):
         rc = lib.pa_blocksparse_build_runs(
             _ptr(mask_u8), Hm, nQ, nK, seq_kv, kv_lo, kv_block, _ptr(ws), ws_bytes, _stream_ptr(block_mask.device)
         )
@@ -692,7 +720,7 @@ def attention_forward_block_sparse_runs(
     q, out, lse = _sparse_outputs(query)
     if scale is None:
         scale = 1.0 / math.sqrt(D)
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         rc = lib.pa_attn_fwd_blocksparse_runs(
             _ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(lse), _DTYPE_CODE[q.dtype], B, H, Sq, Skv, D,
             _lib.strides3(q), _lib.strides3(k), _lib.strides3(v), _lib.strides3(out), float(scale),
@@ -745,7 +773,7 @@ _fb_workspaces = {}
 
 def _fb_workspace(device):
     """Zero-initialised ticket/partials buffer, one per (device, stream)."""
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream)
+    key = (device.index, _stream_ptr(device))
     ws = _fb_workspaces.get(key)
     if ws is None:
         nbytes = _lib.load().pa_fbcache_workspace_bytes()
@@ -803,7 +831,7 @@ def fbcache_residual_diff(prev: torch.Tensor, cur: torch.Tensor) -> torch.Tensor
     ratio = torch.empty((), dtype=prev.dtype, device=prev.device)
     ws = _fb_workspace(prev.device)
     lib = _lib.load()
-    with torch.cuda.device(prev.device):
+    with _on(prev.device):
         rc = lib.pa_fbcache_absdiff_ratio(
             _ptr(prev), _ptr(cur), _DTYPE_CODE[prev.dtype], pr[0], pr[1], pr[2], pr[3], cr[2], cr[3],
             _ptr(ratio), None, _ptr(ws), ws.numel() * 8, _stream_ptr(prev.device),
@@ -832,10 +860,13 @@ def fbcache_first_residual_diff(
     h, h0 = hidden.contiguous(), hidden0.contiguous()
     pv = prev.contiguous() if prev is not None else None
     resid = torch.empty(h.shape, dtype=h.dtype, device=h.device)
-    ratio = torch.full((), float("inf"), dtype=h.dtype, device=h.device)
+    # with something to compare the kernel writes the ratio; filling it first would be one more launch per step
+    ratio = torch.empty((), dtype=h.dtype, device=h.device)
+    if pv is None or pv.numel() == 0:
+        ratio.fill_(float("inf"))
     ws = _fb_workspace(h.device)
     lib = _lib.load()
-    with torch.cuda.device(h.device):
+    with _on(h.device):
         rc = lib.pa_fbcache_residual_ratio(
             _ptr(h), _ptr(h0), _ptr(pv), _ptr(resid), _DTYPE_CODE[h.dtype], h.numel(), _ptr(ratio), None,
             _ptr(ws), ws.numel() * 8, _stream_ptr(h.device),
@@ -858,7 +889,7 @@ def fbcache_apply_residual(residual: torch.Tensor, hidden: torch.Tensor) -> torc
     r, h = residual.contiguous(), hidden.contiguous()
     out = torch.empty(h.shape, dtype=h.dtype, device=h.device)
     lib = _lib.load()
-    with torch.cuda.device(h.device):
+    with _on(h.device):
         rc = lib.pa_fbcache_apply_residual(_ptr(r), _ptr(h), _ptr(out), _DTYPE_CODE[h.dtype], h.numel(), _stream_ptr(h.device))
     _lib.check(rc, "pa_fbcache_apply_residual")
     return out
@@ -896,7 +927,7 @@ def taylorseer_derivatives(y: torch.Tensor, prev: List[torch.Tensor], window: fl
     ts = _flat_same([y] + list(prev), "taylorseer_derivatives")
     cur = [torch.empty(y.shape, dtype=y.dtype, device=y.device) for _ in range(n)]
     lib = _lib.load()
-    with torch.cuda.device(y.device):
+    with _on(y.device):
         rc = lib.pa_taylorseer_update(
             _ptr(ts[0]), _ptr_array(ts[1:]), _ptr_array(cur), n, _DTYPE_CODE[y.dtype], y.numel(), float(window),
             _stream_ptr(y.device),
@@ -925,7 +956,7 @@ def taylorseer_value(derivs: List[torch.Tensor], elapsed: int, hidden: Optional[
     coef = (ctypes.c_float * m)(*[1 / math.factorial(i) for i in range(m)])
     pw = (ctypes.c_float * m)(*[float(elapsed**i) for i in range(m)])
     lib = _lib.load()
-    with torch.cuda.device(d0.device):
+    with _on(d0.device):
         rc = lib.pa_taylorseer_value(
             _ptr_array(ts[:m]), m, coef, pw, _ptr(ts[m]) if hidden is not None else None, _ptr(out),
             _DTYPE_CODE[d0.dtype], d0.numel(), _stream_ptr(d0.device),
