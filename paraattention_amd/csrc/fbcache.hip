@@ -204,16 +204,57 @@ __global__ __launch_bounds__(FB_THREADS) void fbcache_strided_kernel(
   const int64_t n = n_rows * row_len;
   const int64_t stride = (int64_t)gridDim.x * FB_THREADS;
   float sd = 0.f, sa = 0.f;
-  for (int64_t i = (int64_t)blockIdx.x * FB_THREADS + threadIdx.x; i < n; i += stride) {
-    const int64_t r = i / row_len;
-    const int64_t col = i - r * row_len;
-    const float x = Act<DT>::load1(prev, r * prs + col * pcs);
-    const float y = Act<DT>::load1(cur, r * crs + col * ccs);
-    sd += fabsf(Act<DT>::round1(x - y));
-    sa += fabsf(x);
+  // Row and column advance by the stride's own quotient and remainder (a 64-bit division per element was most of this
+  // kernel's time), and UNROLL elements are in flight per thread; the order of the sums is that of the plain loop.
+  constexpr int UNROLL = 8;
+  int64_t i = (int64_t)blockIdx.x * FB_THREADS + threadIdx.x;
+  int64_t r = i / row_len, col = i - r * row_len;
+  const int64_t dr = stride / row_len, dc = stride - dr * row_len;
+  while (i < n) {
+    float x[UNROLL], y[UNROLL];
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      x[u] = y[u] = 0.f;  // adds nothing past the end
+      if (i < n) {
+        x[u] = Act<DT>::load1(prev, r * prs + col * pcs);
+        y[u] = Act<DT>::load1(cur, r * crs + col * ccs);
+      }
+      i += stride;
+      r += dr;
+      col += dc;
+      if (col >= row_len) {
+        col -= row_len;
+        ++r;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      sd += fabsf(Act<DT>::round1(x[u] - y[u]));
+      sa += fabsf(x[u]);
+    }
   }
   finish<DT>(sd, sa, (double)n, ws, ratio_out, stats_out);
 }
+
+// a - b (SUB) or a + b of one 16-byte vector, every element rounded to the activation type
+template <int DT, bool SUB>
+__device__ __forceinline__ u32x4 combine_vec(const u32x4& a, const u32x4& b) {
+  auto f = [](float x, float y) { return SUB ? x - y : x + y; };
+  u32x4 r;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if constexpr (DT == PA_DTYPE_F32) r[k] = __float_as_uint(f(__uint_as_float(a[k]), __uint_as_float(b[k])));
+    else if constexpr (DT == PA_DTYPE_BF16) r[k] = BF16::pack2(f(BF16::lo(a[k]), BF16::lo(b[k])), f(BF16::hi(a[k]), BF16::hi(b[k])));
+    else r[k] = F16::pack2(f(F16::lo(a[k]), F16::lo(b[k])), f(F16::hi(a[k]), F16::hi(b[k])));
+  }
+  return r;
+}
+
+// The two kernels below are bound by HBM.  Four vectors of every operand in flight per thread and streaming stores, one
+// workgroup per CU: at 32760 x 5120 bf16 resid against prev 266 -> 215 us (6.2 TB/s), apply 233 -> 161 us (6.2 TB/s;
+// one vector at a time kept 2 MB of loads in flight on the whole chip).  Two to sixteen workgroups per CU are slower
+// (179 .. 240 us apply), as are eight vectors (162) and larger workgroups.
+constexpr int FB_UNROLL = 4;
 
 // resid = hidden - hidden0 (rounded, stored); reduction against prev if given.
 template <int DT, bool HAVE_PREV>
@@ -229,27 +270,26 @@ __global__ __launch_bounds__(FB_THREADS) void fbcache_residual_kernel(
   const int64_t n_vec = n / VEC;
   const int64_t stride = (int64_t)gridDim.x * FB_THREADS;
   float sd = 0.f, sa = 0.f;
-  for (int64_t i = (int64_t)blockIdx.x * FB_THREADS + threadIdx.x; i < n_vec; i += stride) {
-    const u32x4 h = __builtin_nontemporal_load(hv + i);
-    const u32x4 h0 = __builtin_nontemporal_load(h0v + i);
-    u32x4 r;
-    if constexpr (DT == PA_DTYPE_F32) {
+  int64_t i = (int64_t)blockIdx.x * FB_THREADS + threadIdx.x;
+  for (; i + (FB_UNROLL - 1) * stride < n_vec; i += FB_UNROLL * stride) {
+    u32x4 h[FB_UNROLL], h0[FB_UNROLL], pr[FB_UNROLL];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) r[k] = __float_as_uint(__uint_as_float(h[k]) - __uint_as_float(h0[k]));
-    } else if constexpr (DT == PA_DTYPE_BF16) {
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-        r[k] = BF16::pack2(BF16::lo(h[k]) - BF16::lo(h0[k]), BF16::hi(h[k]) - BF16::hi(h0[k]));
-    } else {
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-        r[k] = F16::pack2(F16::lo(h[k]) - F16::lo(h0[k]), F16::hi(h[k]) - F16::hi(h0[k]));
+    for (int u = 0; u < FB_UNROLL; ++u) {
+      h[u] = __builtin_nontemporal_load(hv + i + u * stride);
+      h0[u] = __builtin_nontemporal_load(h0v + i + u * stride);
+      if constexpr (HAVE_PREV) pr[u] = __builtin_nontemporal_load(pv + i + u * stride);
     }
-    rv[i] = r;  // re-read by the next step: keep it cacheable
-    if constexpr (HAVE_PREV) {
-      const u32x4 pr = __builtin_nontemporal_load(pv + i);
-      accum_vec<DT>(pr, r, sd, sa);
+#pragma unroll
+    for (int u = 0; u < FB_UNROLL; ++u) {
+      const u32x4 r = combine_vec<DT, true>(h[u], h0[u]);
+      __builtin_nontemporal_store(r, rv + i + u * stride);
+      if constexpr (HAVE_PREV) accum_vec<DT>(pr[u], r, sd, sa);
     }
+  }
+  for (; i < n_vec; i += stride) {
+    const u32x4 r = combine_vec<DT, true>(__builtin_nontemporal_load(hv + i), __builtin_nontemporal_load(h0v + i));
+    __builtin_nontemporal_store(r, rv + i);
+    if constexpr (HAVE_PREV) accum_vec<DT>(__builtin_nontemporal_load(pv + i), r, sd, sa);
   }
   if (blockIdx.x == 0 && threadIdx.x < (int)(n - n_vec * VEC)) {
     const int64_t j = n_vec * VEC + threadIdx.x;
@@ -274,24 +314,19 @@ __global__ __launch_bounds__(FB_THREADS) void fbcache_apply_kernel(const void* r
   u32x4* ov = (u32x4*)out;
   const int64_t n_vec = n / VEC;
   const int64_t stride = (int64_t)gridDim.x * FB_THREADS;
-  for (int64_t i = (int64_t)blockIdx.x * FB_THREADS + threadIdx.x; i < n_vec; i += stride) {
-    const u32x4 r = __builtin_nontemporal_load(rv + i);
-    const u32x4 h = __builtin_nontemporal_load(hv + i);
-    u32x4 o;
-    if constexpr (DT == PA_DTYPE_F32) {
+  int64_t i = (int64_t)blockIdx.x * FB_THREADS + threadIdx.x;
+  for (; i + (FB_UNROLL - 1) * stride < n_vec; i += FB_UNROLL * stride) {
+    u32x4 r[FB_UNROLL], h[FB_UNROLL];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) o[k] = __float_as_uint(__uint_as_float(r[k]) + __uint_as_float(h[k]));
-    } else if constexpr (DT == PA_DTYPE_BF16) {
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-        o[k] = BF16::pack2(BF16::lo(r[k]) + BF16::lo(h[k]), BF16::hi(r[k]) + BF16::hi(h[k]));
-    } else {
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-        o[k] = F16::pack2(F16::lo(r[k]) + F16::lo(h[k]), F16::hi(r[k]) + F16::hi(h[k]));
+    for (int u = 0; u < FB_UNROLL; ++u) {
+      r[u] = __builtin_nontemporal_load(rv + i + u * stride);
+      h[u] = __builtin_nontemporal_load(hv + i + u * stride);
     }
-    ov[i] = o;
+#pragma unroll
+    for (int u = 0; u < FB_UNROLL; ++u) __builtin_nontemporal_store(combine_vec<DT, false>(r[u], h[u]), ov + i + u * stride);
   }
+  for (; i < n_vec; i += stride)
+    __builtin_nontemporal_store(combine_vec<DT, false>(__builtin_nontemporal_load(rv + i), __builtin_nontemporal_load(hv + i)), ov + i);
   if (blockIdx.x == 0 && threadIdx.x < (int)(n - n_vec * VEC)) {
     const int64_t j = n_vec * VEC + threadIdx.x;
     const float s = Act<DT>::round1(Act<DT>::load1(resid, j) + Act<DT>::load1(hidden, j));
