@@ -193,6 +193,17 @@ PA_API int pa_attn_fwd_masked(const void* q, const void* k, const void* v, void*
                        const void* mask, int mask_kind, const int64_t mask_strides[4],
                        void* workspace, size_t workspace_bytes, void* stream);
 
+/*
+ * The workspace of one masked call whose mask is known: what
+ * pa_attn_fwd_masked_workspace_bytes says, or, for a boolean mask with a query
+ * dimension (strides as pa_attn_fwd_masked takes them), the room in which it is
+ * packed to one bit per score and the key tiles that nothing keeps are left
+ * out.  With less the per-score kernel runs.
+ */
+PA_API size_t pa_attn_fwd_masked_call_workspace_bytes(int B, int H, int Sq, int Skv, int D,
+                       const int64_t k_strides[3], const int64_t v_strides[3], int mask_kind,
+                       const int64_t mask_strides[4]);
+
 PA_API size_t pa_attn_fwd_masked_workspace_bytes(int B, int H, int Sq, int Skv, int D,
                                           const int64_t k_strides[3], const int64_t v_strides[3]);
 

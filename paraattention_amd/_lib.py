@@ -64,6 +64,7 @@ SIGNATURES = {
          _vp, _i, _strides, _vp, _sz, _vp],
     ),
     "pa_attn_fwd_masked_workspace_bytes": (_sz, [_i, _i, _i, _i, _i, _strides, _strides]),
+    "pa_attn_fwd_masked_call_workspace_bytes": (_sz, [_i, _i, _i, _i, _i, _strides, _strides, _i, _strides]),
     "pa_attn_fwd_lse_noalloc": (
         _i,
         [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _strides, _strides, _strides, _strides, _f, _vp, _i, _vp],

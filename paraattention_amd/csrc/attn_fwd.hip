@@ -131,6 +131,8 @@ struct AttnParams {
   const void* mask;
   int64_t ms_b, ms_h, ms_q, ms_k;
   int mask_kind;  // MASK_*
+  const uint64_t* mask_words;  // PM_BITS: [masks][Sq][key tiles], bit k: key k of the tile is kept
+  int64_t mw_b, mw_h;          // rows between two batch elements' (heads') words, 0 on broadcast dimensions
   int dt;  // columns of q, k, v and out that exist: head_dim (pipelined kernels built for narrower rows; 128 or 64 otherwise)
   // dense kernels: with `gate` set the launch leaves at once unless bit *gate of gate_mask is set (a decision taken on
   // the device by an earlier launch of the same stream, e.g. whether a key mask is a prefix)
@@ -586,16 +588,20 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_fwd_kernel(const AttnParams 
 // query row of a workgroup, and then one load per lane and 64-key tile holds all of it:
 //   PM_KEYS     boolean, no query dimension
 //   PM_KEYBIAS  additive, no query dimension
-// Each wavefront lays the tile's 64 values down in its own 256 bytes of LDS and reads them back in the accumulator's
+//   PM_BITS     boolean with a query dimension, packed by pack_mask_kernel: one 64-bit word per query row and key tile,
+//               and for every 128 query rows the list of the key tiles that any of them keeps (the others are not walked)
+// Without a query dimension each wavefront lays the tile's 64 values down in its own 256 bytes of LDS and reads them back in the accumulator's
 // order (8 broadcast reads, one instruction per score); a tile that drops no key, or whose biases are all zero, costs
 // nothing beyond the vote that says so.  Measured against the per-score kernel (attn_fwd_kernel<MASK>, register-staged
 // tiles): two samples x 24 heads x 7800 rows against 256 keys with a bias 171 -> 104 us (0.47 PFLOP/s; bound by what a
 // workgroup does around its four key tiles), 24 heads x 4352 tokens with holes in the key mask, scan and two empty
-// launches included there, 390..545 -> 236 us (0.98 PFLOP/s, what the unmasked call of that size reaches).
+// launches included there, 390..545 -> 236 us (0.98 PFLOP/s, what the unmasked call of that size reaches); three packed samples
+behind a common prefix, 2 x 24 heads x 8000 tokens 6.65 -> 0.88 ms, 16 heads x 3000 326 -> 94 us (about half the key tiles
+are kept by no row of a query tile there or more; the rest is the packed words instead of a byte load per score).
 // The element of tile j + 2 is fetched while tile j + 1 is masked, so its latency is covered by the wait for the
 // tile copies at the top of every iteration.
 // ---------------------------------------------------------------------------------------------
-constexpr int PM_NONE = 0, PM_KEYS = 1, PM_KEYBIAS = 2;
+constexpr int PM_NONE = 0, PM_KEYS = 1, PM_KEYBIAS = 2, PM_BITS = 3;
 constexpr int PM_SLOT_BYTES = 256;  // LDS per wavefront, behind the K and V tiles
 // The running maximum of a masked row before its first kept key.  Finite, so that -inf scores against it give
 // exp2(-inf) = 0 instead of NaN; below every finite score, so that the first kept key raises it.
@@ -610,9 +616,14 @@ struct TileMask {
   bool act;  // 16-bit elements in the activation type
   float per_scale;
   float* slot;
-  __device__ __forceinline__ void init(const AttnParams& p, int batch, int head, int lane_, char* lds) {
+  uint64_t word;  // PM_BITS: this lane's query row against the tile's keys
+  __device__ __forceinline__ void init(const AttnParams& p, int batch, int head, int lane_, char* lds, int row) {
     lane = lane_;
     hh = lane_ >> 5;
+    if constexpr (PM == PM_BITS) {
+      base = (const char*)(p.mask_words + ((int64_t)batch * p.mw_b + (int64_t)head * p.mw_h + row) * ((p.Skv + BN - 1) / BN));
+      return;
+    }
     last = (uint32_t)(p.Skv - 1);
     const int64_t at = batch * p.ms_b + head * p.ms_h;
     act = PM == PM_KEYBIAS && p.mask_kind == MASK_ACT;
@@ -641,6 +652,10 @@ struct TileMask {
   }
   // the element of key n0 + lane (any key for a tile that does not exist or ends early: those scores are dropped)
   __device__ __forceinline__ void fetch(uint32_t n0) {
+    if constexpr (PM == PM_BITS) {
+      word = ((const uint64_t*)base)[n0 / BN];
+      return;
+    }
     uint32_t key = n0 + lane;
     key = key < last ? key : last;
     const char* at = base + key * step;
@@ -649,6 +664,18 @@ struct TileMask {
     else raw = *(const uint32_t*)at;
   }
   __device__ __forceinline__ void apply(floatx16& a0, floatx16& a1) const {
+    if constexpr (PM == PM_BITS) {
+      if (__any(word != ~(uint64_t)0)) {
+        const uint32_t lo = (uint32_t)word >> (4 * hh), hi = (uint32_t)(word >> 32) >> (4 * hh);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const uint32_t bit = 1u << (8 * (r >> 2) + (r & 3));
+          if (!(lo & bit)) a0[r] = -INFINITY;
+          if (!(hi & bit)) a1[r] = -INFINITY;
+        }
+      }
+      return;
+    }
     // what a lane lays down for its key: the bias, or the largest value a score may keep (-inf drops it whatever it is,
     // also where a dropped key's row holds no numbers)
     float b;
@@ -1095,7 +1122,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
   TileIter it;
   decode_block<SPARSE>(p, qt, head, batch, row_begin, row_end, it);
   TileMask<T, PM> tm;
-  if constexpr (PM != PM_NONE) tm.init(p, batch, head, lane, (char*)smem + 4 * TILE_BYTES + wave * PM_SLOT_BYTES);
+  if constexpr (PM != PM_NONE) tm.init(p, batch, head, lane, (char*)smem + 4 * TILE_BYTES + wave * PM_SLOT_BYTES, min(row_begin + wave * 32 + l32, row_end - 1));
+  if constexpr (PM == PM_BITS) {  // the key tiles this query tile keeps, as build_runs_kernel lists them
+    const int nseg = p.nQ + 2, sidx = (int)((batch * p.mw_b + head * p.mw_h) / p.Sq) * nseg + 1 + qt;
+    it.init_list(p.runs + (size_t)p.Hm * nseg + (size_t)sidx * p.cap * 2, p.runs[sidx], p.Skv, false);
+  }
   if constexpr (PM == PM_KEYS) it.init_dense(__builtin_amdgcn_readfirstlane(tm.kept_end(p.Skv)));
   // Keys in segments (the blocks of a ring sweep, StreamPlan::kseg / vseg): the sweep below runs once per
   // segment, with the softmax state carried over in registers.  A key share of a split piece is then a run of
@@ -1539,7 +1570,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
       if constexpr (PM != PM_NONE) {
         tm.fetch(n_cur);
         tm.apply(sn0, sn1);
-        tm.fetch(n_nxt);
+        if (n_nxt != OOB) tm.fetch(n_nxt);
       }
       if (v_cur < BN || on_diagonal(n_cur)) mask_tail(sn0, sn1, v_cur, n_cur);
       if constexpr (!BOUNDED) {
@@ -1710,7 +1741,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
   TileIter it;
   decode_block<SPARSE>(p, qt, head, batch, row_begin, row_end, it);
   TileMask<T, PM> tm;
-  if constexpr (PM != PM_NONE) tm.init(p, batch, head, lane, (char*)smem + 4 * TILE64_BYTES + wave * PM_SLOT_BYTES);
+  if constexpr (PM != PM_NONE) tm.init(p, batch, head, lane, (char*)smem + 4 * TILE64_BYTES + wave * PM_SLOT_BYTES, min(row_begin + wave * 32 + l32, row_end - 1));
+  if constexpr (PM == PM_BITS) {  // the key tiles this query tile keeps, as build_runs_kernel lists them
+    const int nseg = p.nQ + 2, sidx = (int)((batch * p.mw_b + head * p.mw_h) / p.Sq) * nseg + 1 + qt;
+    it.init_list(p.runs + (size_t)p.Hm * nseg + (size_t)sidx * p.cap * 2, p.runs[sidx], p.Skv, false);
+  }
   if constexpr (PM == PM_KEYS) it.init_dense(__builtin_amdgcn_readfirstlane(tm.kept_end(p.Skv)));
 
   if constexpr (!SPARSE) {
@@ -1873,7 +1908,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
     if constexpr (PM != PM_NONE) {
       tm.fetch(n_cur);
       tm.apply(sn0, sn1);
-      tm.fetch(n_nxt);
+      if (n_nxt != OOB) tm.fetch(n_nxt);
     }
     if (v_cur < BN || on_diagonal(n_cur)) mask_tail(sn0, sn1, v_cur, n_cur);
     if constexpr (!BOUNDED) {
@@ -3950,7 +3985,7 @@ static void fill_params(AttnParams& p, const void* q, const void* k, const void*
   p.acc_out = nullptr; p.acc_lse = nullptr; p.acc_first = 0;
   p.split_main = 0; p.split_tiles = 0; p.split_s = 0; p.ws_out = nullptr; p.ws_lse = nullptr;
   p.bound_flag = nullptr;
-  p.dt = 128; p.mask_kind = MASK_NONE;
+  p.dt = 128; p.mask_kind = MASK_NONE; p.mask_words = nullptr; p.mw_b = p.mw_h = 0;
   p.mask = nullptr; p.ms_b = p.ms_h = p.ms_q = p.ms_k = 0;
   p.gate = nullptr; p.gate_mask = 0;
   p.st = StreamPlan{};
@@ -4784,7 +4819,7 @@ template <typename T, int D, int PM, int NW, int W = D>
 static int launch_pipe_variant(const AttnParams& p, hipStream_t stream) {
   int64_t nblocks = (int64_t)p.B * p.H * p.n_qtiles;
   if (p.split_s > 1) nblocks = (int64_t)p.split_main + (int64_t)p.split_tiles * p.split_s;
-  const size_t smem = 4 * (D == 128 ? TILE_BYTES : TILE64_BYTES) + (PM == PM_NONE ? 0 : NW * PM_SLOT_BYTES);
+  const size_t smem = 4 * (D == 128 ? TILE_BYTES : TILE64_BYTES) + (PM == PM_NONE || PM == PM_BITS ? 0 : NW * PM_SLOT_BYTES);
   const void* fn;
   if constexpr (D == 128) fn = (const void*)attn_fwd_d128_pipe_kernel<T, false, NW, false, false, PM, W>;
   else fn = (const void*)attn_fwd_d64_pipe_kernel<T, false, NW, false, PM, (W < 64)>;
@@ -4869,6 +4904,98 @@ extern "C" int pa_attn_fwd_narrow(const void* q, const void* k, const void* v, v
   return dtype == PA_DTYPE_BF16 ? launch_narrow<BF16>(p, (hipStream_t)stream) : launch_narrow<F16>(p, (hipStream_t)stream);
 }
 
+// A boolean mask with a query dimension as 64-bit words per query row and key tile, and for every 128 query rows and key
+// tile whether any of them keeps a key of it.  One workgroup = 128 rows x 512 keys; a lane turns 8 keys into a byte.
+// Bound by the mask's bytes: 8000 x 8000 keys are read once, an eighth of that is written.
+__global__ __launch_bounds__(256) void pack_mask_kernel(const uint8_t* mask, int64_t mb, int64_t mh, int64_t mq, int64_t mk, int n_heads,
+                                                        int Sq, int Skv, uint8_t* words, uint8_t* live) {
+  __shared__ uint64_t s_any[4];
+  const int nkt = (Skv + BN - 1) / BN;
+  const int m = blockIdx.z, batch = m / n_heads, head = m - batch * n_heads;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int key = blockIdx.x * 512 + lane * 8;
+  const uint8_t* src = mask + batch * mb + head * mh;
+  uint32_t any = 0;
+  for (int i = 0; i < 32; ++i) {
+    const int row = blockIdx.y * 128 + wave * 32 + i;
+    if (row >= Sq) break;
+    const uint8_t* at = src + (int64_t)row * mq + (int64_t)key * mk;
+    uint32_t bits = 0;
+    if (mk == 1 && key + 8 <= Skv) {
+      uint64_t x;
+      __builtin_memcpy(&x, at, 8);  // (any alignment)
+      x |= x >> 4;
+      x |= x >> 2;
+      x |= x >> 1;
+      bits = (uint32_t)(((x & 0x0101010101010101ull) * 0x0102040810204080ull) >> 56);
+    } else {
+      for (int k = 0; k < 8; ++k)
+        if (key + k < Skv && at[k * mk] != 0) bits |= 1u << k;
+    }
+    any |= bits;
+    if (key < nkt * BN) words[((int64_t)m * Sq + row) * nkt * 8 + (key >> 3)] = (uint8_t)bits;
+  }
+  const uint64_t w = __ballot(any != 0);
+  if (lane == 0) s_any[wave] = w;
+  __syncthreads();
+  if (threadIdx.x < 8) {
+    const int kt = blockIdx.x * 8 + threadIdx.x;
+    const uint64_t all = s_any[0] | s_any[1] | s_any[2] | s_any[3];
+    if (kt < nkt) live[((int64_t)m * gridDim.y + blockIdx.y) * nkt + kt] = ((all >> (8 * threadIdx.x)) & 0xff) != 0;
+  }
+}
+
+// pa_attn_fwd_masked's workspace for such a mask: the words, the live tiles, build_runs_kernel's lists of them.
+struct BitsLayout {
+  int64_t masks;
+  int nQ, nK, cap;
+  size_t live, runs, bytes;
+};
+static BitsLayout bits_layout(int B, int H, int Sq, int Skv, const int64_t ms[4]) {
+  auto up = [](size_t n) { return (n + 255) & ~(size_t)255; };
+  BitsLayout l;
+  l.masks = (int64_t)(ms[0] != 0 ? B : 1) * (ms[1] != 0 ? H : 1);
+  l.nQ = (Sq + 127) / 128;
+  l.nK = (Skv + BN - 1) / BN;
+  l.cap = l.nK / 2 + 3;
+  l.live = up((size_t)l.masks * Sq * l.nK * 8);
+  l.runs = l.live + up((size_t)l.masks * l.nQ * l.nK);
+  l.bytes = l.runs + up((size_t)l.masks * (l.nQ + 2) * (1 + 2 * (size_t)l.cap) * sizeof(int32_t));
+  return l;
+}
+// Boolean masks with a query dimension that go this way (and not to the per-score kernel): grids of the two preparing
+// launches within bounds.
+static bool bits_take(const AttnParams& p, int D, int mask_kind, const int64_t ms[4]) {
+  if (mask_kind != MASK_BOOL || p.Sq <= 1 || ms[2] == 0 || !pipe_fits(p, D)) return false;
+  const BitsLayout l = bits_layout(p.B, p.H, p.Sq, p.Skv, ms);
+  return l.masks <= 65535 && l.nQ <= 65535 && l.masks * (l.nQ + 2) < 0x7fffffffLL;
+}
+
+template <typename T, int D>
+static int launch_masked_bits(AttnParams p, const int64_t ms[4], void* ws, hipStream_t stream) {
+  const BitsLayout l = bits_layout(p.B, p.H, p.Sq, p.Skv, ms);
+  uint8_t* const live = (uint8_t*)ws + l.live;
+  int32_t* const runs = (int32_t*)((char*)ws + l.runs);
+  const int n_heads = ms[1] != 0 ? p.H : 1;
+  hipLaunchKernelGGL(pack_mask_kernel, dim3((l.nK + 7) / 8, l.nQ, (unsigned)l.masks), dim3(256), 0, stream, (const uint8_t*)p.mask, p.ms_b, p.ms_h,
+                     p.ms_q, p.ms_k, n_heads, p.Sq, p.Skv, (uint8_t*)ws, live);
+  PA_CHECK_LAUNCH("mask packing kernel");
+  hipLaunchKernelGGL(build_runs_kernel, dim3((unsigned)(l.masks * (l.nQ + 2))), dim3(64), 0, stream, (const uint8_t*)live, (int)l.masks, l.nQ, l.nK,
+                     p.Skv, 0, BN, l.cap, runs, (int32_t*)nullptr);
+  PA_CHECK_LAUNCH("mask runs kernel");
+  p.mask_words = (const uint64_t*)ws;
+  p.mw_h = ms[1] != 0 ? p.Sq : 0;
+  p.mw_b = ms[0] != 0 ? (int64_t)n_heads * p.Sq : 0;
+  p.runs = runs;
+  p.Hm = (int)l.masks;
+  p.nQ = l.nQ;
+  p.cap = l.cap;
+  p.bm = 128;
+  p.n_qtiles = l.nQ;
+  p.split_s = 0;
+  return launch_pipe_variant<T, D, PM_BITS, 4>(p, stream);
+}
+
 // Whether a dense call with per-batch key counts that leave nearly all keys would go to the resident-workgroup
 // kernel: where that kernel takes the shape with `ws_avail` bytes of workspace and the launch is long enough for its
 // advantage over the kernel with one workgroup per query tile to outweigh a third, empty launch: from 512 key-tile
@@ -4925,6 +5052,18 @@ extern "C" size_t pa_attn_fwd_masked_workspace_bytes(int B, int H, int Sq, int S
   return masked_layout(B, H, Skv, D).dense + (dense > dense_c ? dense : dense_c);
 }
 
+extern "C" size_t pa_attn_fwd_masked_call_workspace_bytes(int B, int H, int Sq, int Skv, int D, const int64_t k_strides[3],
+                                                          const int64_t v_strides[3], int mask_kind, const int64_t mask_strides[4]) {
+  size_t need = pa_attn_fwd_masked_workspace_bytes(B, H, Sq, Skv, D, k_strides, v_strides);
+  if (B <= 0 || H <= 0 || Sq <= 0 || Skv <= 0 || (D != 128 && D != 64) || !k_strides || !v_strides || !mask_strides) return need;
+  const int64_t zero[3] = {0, 0, 0};
+  AttnParams p;
+  fill_params(p, nullptr, nullptr, nullptr, nullptr, nullptr, B, H, Sq, Skv, zero, k_strides, v_strides, zero, 1.f);
+  int64_t eff[4];
+  for (int i = 0; i < 4; ++i) eff[i] = (i == 0 && B == 1) || (i == 1 && H == 1) ? 0 : mask_strides[i];
+  return bits_take(p, D, mask_kind, eff) ? bits_layout(B, H, Sq, Skv, eff).bytes : need;
+}
+
 extern "C" int pa_attn_fwd_masked(const void* q, const void* k, const void* v, void* out, float* lse,
                                   int dtype, int B, int H, int Sq, int Skv, int D,
                                   const int64_t q_strides[3], const int64_t k_strides[3],
@@ -4970,6 +5109,13 @@ extern "C" int pa_attn_fwd_masked(const void* q, const void* k, const void* v, v
   const bool key_only = mask_kind == MASK_BOOL && (H == 1 || p.ms_h == 0) && (Sq == 1 || p.ms_q == 0);
   const double flops = 4.0 * B * H * (double)Sq * (double)Skv * D;
   if (pipe_takes && (!key_only || flops < GATHER_FLOP)) return masked_pipe(workspace, workspace_bytes);
+  // a boolean mask with a query dimension (packed samples, windows): words and lists of live tiles, then one launch
+  int64_t eff[4];  // strides, 0 where the dimension is 1
+  for (int i = 0; i < 4; ++i) eff[i] = (i == 0 && B == 1) || (i == 1 && H == 1) ? 0 : mask_strides[i];
+  if (any && workspace && bits_take(p, D, mask_kind, eff) && workspace_bytes >= bits_layout(B, H, Sq, Skv, eff).bytes) {
+    if (dtype == PA_DTYPE_BF16) return D == 128 ? launch_masked_bits<BF16, 128>(p, eff, workspace, st) : launch_masked_bits<BF16, 64>(p, eff, workspace, st);
+    return D == 128 ? launch_masked_bits<F16, 128>(p, eff, workspace, st) : launch_masked_bits<F16, 64>(p, eff, workspace, st);
+  }
   const size_t scan = mask_scan_bytes(B, Skv > 0 ? Skv : 1);
   if (key_only && any && workspace && workspace_bytes >= scan) {
     int32_t* words = (int32_t*)workspace;
@@ -5088,7 +5234,8 @@ extern "C" int pa_attn_fwd_lse_noalloc(const void* q, const void* k, const void*
   // (the plan with one tail range per workgroup: the one a call falls back to when the workspace cannot hold the
   // partial results of drawn ranges, which take four times as many)
   const size_t need = shaped ? dense_ws_need(B, H, Sq, Skv, D, k_strides, v_strides, is_causal ? 2 : kv_len != nullptr ? 1 : 0, false) : 0;
-  if (need > (size_t)PA_NOALLOC_SCRATCH_BYTES)
+  // (head_dim 64 runs without its key split where that does not fit)
+  if (need > (size_t)PA_NOALLOC_SCRATCH_BYTES && D != 64)
     PA_FAIL(PA_ERR_WORKSPACE, "this problem's launch plan needs %zu bytes of scratch, the static buffer holds %zu: "
             "call pa_attn_fwd_lse_ws with a workspace of your own", need, (size_t)PA_NOALLOC_SCRATCH_BYTES);
   void* ws = nullptr;

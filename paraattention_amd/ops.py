@@ -288,7 +288,7 @@ def _masked_forward(query, key, value, attn_mask, scale, want_lse, is_causal=Fal
     lib = _lib.load()
     with _on(q.device):
         ks, vs = _lib.strides3(k), _lib.strides3(v)
-        ws_bytes = lib.pa_attn_fwd_masked_workspace_bytes(B, H, Sq, Skv, D, ks, vs)
+        ws_bytes = lib.pa_attn_fwd_masked_call_workspace_bytes(B, H, Sq, Skv, D, ks, vs, kind, mstrides)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
         rc = lib.pa_attn_fwd_masked(
             _ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(lse), _DTYPE_CODE[q.dtype], B, H, Sq, Skv, D,

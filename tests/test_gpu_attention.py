@@ -371,6 +371,36 @@ def test_key_split_tail_head_dim_64(cuda, tuning, D, bound):
         assert not torch.equal(lse[:, -1], lse1[:, -1])  # another order of sums: the split was taken
 
 
+@pytest.mark.parametrize("D", [128, 64])
+@pytest.mark.parametrize("Sq,Skv", [(2, 64), (128, 65), (129, 513), (300, 1100)])
+@pytest.mark.parametrize("shape", ["b1", "1h", "bh"])
+def test_masks_with_a_query_dimension(cuda, D, Sq, Skv, shape):
+    """Boolean masks per query row, packed to words of 64 keys: key tiles that a query tile drops as a whole (the first,
+    the last, a run in the middle, all of them), rows that keep nothing, keys that every row drops and whose rows hold
+    no numbers, and masks on transposed and on misaligned memory."""
+    B, H = 2, 3
+    q, k, v = inputs.qkv(B, H, Sq, Skv, D, seed=Skv + D)
+    mB, mH = (B if "b" in shape else 1), (H if "h" in shape else 1)
+    g = torch.Generator().manual_seed(Skv)
+    keep = torch.rand((mB, mH, Sq, Skv), generator=g) < 0.5
+    keep[:, :, :, :64] &= torch.arange(Sq)[:, None] >= 128       # the first key tile: dropped by the first query tile
+    keep[:, :, :128, 192:512] = False
+    keep[0, 0, :, (Skv - 1) // 64 * 64:] = False                 # the last one: dropped by all rows of one mask
+    keep[-1, -1, 128:] = False                                   # query tiles that keep nothing
+    keep[:, :, Sq - 1] = False
+    dropped = torch.rand(Skv, generator=g) < 0.1
+    keep[..., dropped] = False
+    kd = k.masked_fill(dropped[None, None, :, None], float("nan"))
+    ref_out, ref_lse = oattn.sdpa_lse_f64(q.float().numpy(), k.float().numpy(), v.float().numpy(), None, np.broadcast_to(keep.numpy(), (B, H, Sq, Skv)))
+    m = keep.to(cuda)
+    flipped = m.transpose(2, 3).contiguous().transpose(2, 3)
+    shifted = torch.zeros((mB, mH, Sq, Skv + 3), dtype=torch.bool, device=cuda)[..., 3:].copy_(m)
+    op = torch.ops.para_attn.attention_forward_with_lse
+    for what, mask in (("plain", m), ("transposed", flipped), ("misaligned", shifted)):
+        out, lse = op(q.to(cuda), kd.to(cuda), v.to(cuda), mask)
+        _check(out, lse, ref_out, ref_lse, f"{what} mask {shape}")
+
+
 def test_key_masks_take_the_fast_kernels_when_prefixes(cuda, tuning):
     """A key-only boolean mask is scanned on the device: prefixes run the dense kernels with per-batch key counts
     (here with the key-split tail and the score bound in play), anything else the per-score kernel; both give the
