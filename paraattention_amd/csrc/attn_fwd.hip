@@ -596,8 +596,8 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_fwd_kernel(const AttnParams 
 // tiles): two samples x 24 heads x 7800 rows against 256 keys with a bias 171 -> 104 us (0.47 PFLOP/s; bound by what a
 // workgroup does around its four key tiles), 24 heads x 4352 tokens with holes in the key mask, scan and two empty
 // launches included there, 390..545 -> 236 us (0.98 PFLOP/s, what the unmasked call of that size reaches); three packed samples
-behind a common prefix, 2 x 24 heads x 8000 tokens 6.65 -> 0.88 ms, 16 heads x 3000 326 -> 94 us (about half the key tiles
-are kept by no row of a query tile there or more; the rest is the packed words instead of a byte load per score).
+// behind a common prefix, 2 x 24 heads x 8000 tokens 6.65 -> 0.88 ms, 16 heads x 3000 326 -> 94 us (about half the key tiles
+// are kept by no row of a query tile there; the rest is the packed words instead of a byte load per score).
 // The element of tile j + 2 is fetched while tile j + 1 is masked, so its latency is covered by the wait for the
 // tile copies at the top of every iteration.
 // ---------------------------------------------------------------------------------------------
