@@ -177,11 +177,12 @@ PA_API int pa_attn_fwd_narrow(const void* q, const void* k, const void* v, void*
  * is one of 3e11 flop or more, the kept K and V rows are gathered into dense
  * copies in the workspace, as the reference's attention_forward_sparse_kv
  * does with index_select (ops/__init__.py:276-296), and the same kernels run
- * on the copies.  Smaller calls with such a mask, and additive masks without a
- * query dimension, run in the fast kernels too, which then load the mask once
- * per key; every other mask runs a kernel that reads it per score.  The choice
- * is made on the device: nothing is read back, so the call can be captured in a
- * HIP graph.
+ * on the copies.  Smaller calls with such a mask, and additive masks, run in
+ * the fast kernels too; so do boolean masks with a query dimension, packed to
+ * bits first.  What is left (additive masks whose keys are not adjacent in
+ * memory, K or V of 4 GiB and more per head, no room for the bits) runs a kernel
+ * that reads the mask per score.  The choice is made on the device: nothing is
+ * read back, so the call can be captured in a HIP graph.
  * workspace: pa_attn_fwd_masked_workspace_bytes() bytes (16-byte aligned, any
  * contents; from 3e11 flop on it includes the copies of K and V); null or
  * short is not an error: the per-score kernel runs where there is no room.

@@ -401,6 +401,34 @@ def test_masks_with_a_query_dimension(cuda, D, Sq, Skv, shape):
         _check(out, lse, ref_out, ref_lse, f"{what} mask {shape}")
 
 
+@pytest.mark.parametrize("D", [128, 64])
+@pytest.mark.parametrize("Sq,Skv", [(2, 1), (129, 64), (130, 131)])
+def test_biases_with_a_query_dimension(cuda, D, Sq, Skv):
+    """Additive masks per query row, fp32 and in the activation type: full and ragged key tiles, rows that begin at any
+    element, memory that ends with the last bias, -inf among them, and keys that are not adjacent (the per-score
+    kernel).  Against the masked fp64 softmax with the bias added to the scores."""
+    B, H = 2, 3
+    q, k, v = inputs.qkv(B, H, Sq, Skv, D, seed=Skv + D)
+    qn, kn, vn = (t.double().numpy() for t in (q, k, v))
+    op = torch.ops.para_attn.attention_forward_with_lse
+    g = torch.Generator().manual_seed(Skv)
+    for shape in ((1, H, Sq, Skv), (B, 1, Sq, Skv)):
+        for dt in (torch.float32, q.dtype):
+            bias = torch.randn(shape, generator=g).masked_fill_(torch.rand(shape, generator=g) < 0.2, float("-inf"))
+            bias[..., 0] = 0.25
+            bias = bias.to(dt)
+            s = np.einsum("bhqd,bhkd->bhqk", qn, kn) / math.sqrt(D) + bias.double().numpy()
+            m = s.max(-1, keepdims=True)
+            p = np.exp(s - m)
+            ref_out, ref_lse = (p @ vn) / p.sum(-1, keepdims=True), (m + np.log(p.sum(-1, keepdims=True)))[..., 0]
+            plain = bias.to(cuda)
+            shifted = torch.full((*shape[:3], Skv + 1), float("nan"), dtype=dt, device=cuda)[..., 1:].copy_(plain)
+            apart = torch.full((*shape, 2), float("nan"), dtype=dt, device=cuda)[..., 0].copy_(plain)
+            for what, mask in (("plain", plain), ("shifted", shifted), ("keys apart", apart)):
+                out, lse = op(q.to(cuda), k.to(cuda), v.to(cuda), mask)
+                _check(out, lse, ref_out, ref_lse, f"{what} bias {shape} {dt}")
+
+
 def test_key_masks_take_the_fast_kernels_when_prefixes(cuda, tuning):
     """A key-only boolean mask is scanned on the device: prefixes run the dense kernels with per-batch key counts
     (here with the key-split tail and the score bound in play), anything else the per-score kernel; both give the
