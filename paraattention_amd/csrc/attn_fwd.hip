@@ -636,9 +636,37 @@ struct TileMask {
     per_scale = 1.0f / (p.scale_log2 * LN2);  // bias / scale, so that (s + that) * c = s * c + bias * log2(e)
     slot = (float*)lds;
   }
-  // PM_KEYS: keys up to and including the last one kept, found from the end (every wavefront for itself, 256 keys a
-  // step); the keys behind it are not walked at all, as with per-batch key counts
+  // PM_KEYS: keys up to and including the last one kept, found from the end (every wavefront for itself); the keys behind
+  // it are not walked at all, as with per-batch key counts.  A step costs 0.6 .. 1.2 us whatever it looks at: adjacent
+  // mask bytes 16 per lane, 1024 keys first and 4096 a step from then on; others a byte per lane and load, 256 keys a step.
+  // The caller bounds the steps (kept_end_steps).
   __device__ __forceinline__ int kept_end(int Skv) const {
+    if (step == 1 && Skv >= 16) {
+      // keys of the 16 from `key` on (from the first one on for a lane before it: what it sees twice changes nothing)
+      auto last_of = [&](int key) {
+        key = key > 0 ? key : 0;
+        u32x4 w;
+        __builtin_memcpy(&w, base + (uint32_t)key, 16);  // (any alignment)
+        int n = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (w[i] != 0) n = key + 4 * i + 4 - (__builtin_clz(w[i]) >> 3);
+        return n;
+      };
+      auto highest = [](int n) {
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) n = max(n, __shfl_xor(n, d));
+        return __builtin_amdgcn_readfirstlane(n);
+      };
+      int end = highest(last_of(Skv - 1024 + 16 * lane));
+      for (int top = Skv - 1024; top > 0 && end == 0; top -= 4096) {
+        int n = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) n = max(n, last_of(top - 1024 * (i + 1) + 16 * lane));
+        end = highest(n);
+      }
+      return end;
+    }
     int end = 0;
     for (int top = Skv; top > 0 && end == 0; top -= 256) {
       int best = 0;
@@ -5076,6 +5104,15 @@ static size_t mask_scan_bytes(int B, int Skv) {
 // From this size on a boolean key mask is scanned on the device and the kept keys of one with holes are gathered.
 constexpr double GATHER_FLOP = 3.0e11;
 
+// Below it the workgroups look for the last kept key themselves (TileMask::kept_end), unless that may take more steps of
+// 0.6 .. 1.2 us than the scan with its empty launch costs: beyond 37888 adjacent keys, or 2560 others.  24 heads x 256 rows,
+// 700 kept of 32768 keys: 50 us with the scan, 33 without (the host's time); 8 heads x 256 rows, 4000 kept of 65536: 54 with,
+// 60 without; 1000 kept of 1M keys: 47 with, 2320 where every workgroup walked 256 keys a step.
+constexpr int KEPT_END_STEPS = 10;
+static int64_t kept_end_steps(int Skv, int64_t key_stride) {
+  return key_stride == 1 ? ((int64_t)Skv - 1024 + 4095) / 4096 + 1 : ((int64_t)Skv + 255) / 256;
+}
+
 // pa_attn_fwd_masked's workspace when it gathers the kept keys of a mask with holes: the scan's words, dense copies
 // of K and V [B][H][Skv][D], then the workspace of the dense launches.
 struct MaskedLayout {
@@ -5159,7 +5196,7 @@ extern "C" int pa_attn_fwd_masked(const void* q, const void* k, const void* v, v
   // masked launch are enqueued, and the one the flag does not select leaves at once.  Nothing is read back.
   const bool key_only = mask_kind == MASK_BOOL && (H == 1 || p.ms_h == 0) && (Sq == 1 || p.ms_q == 0);
   const double flops = 4.0 * B * H * (double)Sq * (double)Skv * D;
-  if (pipe_takes && (!key_only || flops < GATHER_FLOP)) return masked_pipe(workspace, workspace_bytes);
+  if (pipe_takes && (!key_only || (flops < GATHER_FLOP && kept_end_steps(Skv, p.ms_k) <= KEPT_END_STEPS))) return masked_pipe(workspace, workspace_bytes);
   // a boolean mask with a query dimension (packed samples, windows): words and lists of live tiles, then one launch
   int64_t eff[4];  // strides, 0 where the dimension is 1
   for (int i = 0; i < 4; ++i) eff[i] = (i == 0 && B == 1) || (i == 1 && H == 1) ? 0 : mask_strides[i];
@@ -5177,6 +5214,8 @@ extern "C" int pa_attn_fwd_masked(const void* q, const void* k, const void* v, v
     return D == 128 ? launch_pipe_variant<F16, 128, PM_BIAS, 4>(p, st) : launch_pipe_variant<F16, 64, PM_BIAS, 4>(p, st);
   }
   const size_t scan = mask_scan_bytes(B, Skv > 0 ? Skv : 1);
+  void* other_ws = nullptr;  // what the launch after the scan may use: the room of those that the flag does not select
+  size_t other_bytes = 0;
   if (key_only && any && workspace && workspace_bytes >= scan) {
     int32_t* words = (int32_t*)workspace;
     const int* flag = words + B;  // bit 0: prefixes; bit 1: at least 7/8 of the keys kept everywhere
@@ -5247,12 +5286,14 @@ extern "C" int pa_attn_fwd_masked(const void* q, const void* k, const void* v, v
     }
     p.gate = flag;
     p.gate_mask = HOLES_FEWER | HOLES_MOST;
+    other_ws = dense_ws;
+    other_bytes = dense_bytes;
   }
   if (!any) {  // no rows, or no keys: the dense path writes what an empty softmax gives
     return attn_fwd_dense(q, k, v, out, lse, dtype, B, H, Sq, Skv, D, q_strides, k_strides, v_strides, out_strides,
                           scale, nullptr, 0, nullptr, 0, stream);
   }
-  if (pipe_takes) return masked_pipe(nullptr, 0);  // the workspace's first words are in use
+  if (pipe_takes) return masked_pipe(other_ws, other_bytes);
   if (dtype == PA_DTYPE_BF16) return D == 128 ? launch_masked<BF16, 128>(p, mask_kind, st) : launch_masked<BF16, 64>(p, mask_kind, st);
   return D == 128 ? launch_masked<F16, 128>(p, mask_kind, st) : launch_masked<F16, 64>(p, mask_kind, st);
 }

@@ -314,6 +314,57 @@ def test_key_only_masks_in_the_pipelined_kernels(cuda, tuning, D, bm, Skv):
                 _check(out, lse, ref_out, ref_lse, f"key bias {shape} {dt} {low}")
 
 
+@pytest.mark.parametrize("Skv", [15, 16, 17, 1023, 1025, 5121, 9300, 37888, 37889])
+def test_last_kept_key_of_long_masks(cuda, Skv):
+    """The last kept key at the edges of the steps in which it is looked for (16 adjacent keys per lane, 1024 and then 4096
+    a step; 256 a step on strided memory; from 37889 keys on, or 2561 strided ones, the scan of the whole mask), with and without a hole,
+    the same for all heads or one per head.  No key behind it may count, none before it be lost."""
+    B, H, Sq, D = 1, 2, 3, 64
+    q, k, v = inputs.qkv(B, H, Sq, Skv, D, seed=Skv)
+    dev = [t.to(cuda) for t in (q, k, v)]
+    op = torch.ops.para_attn.attention_forward_with_lse
+    lasts = sorted({n for e in (0, 15, 16, 1023, 1024, 5119, 5120) for n in (e, Skv - 1 - e) if 0 <= n < Skv})
+    for i, last in enumerate(lasts):
+        keep = torch.arange(Skv) <= last
+        if i % 2:
+            keep[last // 2] = last == 0
+        ref_out, ref_lse = oattn.sdpa_lse_f64(q.float().numpy(), k.float().numpy(), v.float().numpy(), None, keep.numpy())
+        m = keep.to(cuda)[None, None, None, :]
+        strided = torch.zeros(1, 1, 1, Skv, 2, dtype=torch.bool, device=cuda)[..., 1].copy_(m)
+        shifted = torch.ones(1, 1, 1, Skv + 3, dtype=torch.bool, device=cuda)[..., 3:].copy_(m)
+        for what, mask in (("plain", m), ("strided", strided), ("misaligned", shifted), ("per head", m.repeat(1, H, 1, 1))):
+            out, lse = op(*dev, mask)
+            _check(out, lse, ref_out, ref_lse, f"{what}, last kept key {last}")
+
+
+@pytest.mark.parametrize("D", [128, 64])
+def test_a_long_dropped_tail_costs_no_walk(cuda, D):
+    """1000 kept of 262144 keys take about as long as a call on those 1000 keys (a bound of five times; walking the rest of the
+    mask in every workgroup took more than twenty)."""
+    H, Sq, Skv, kept = 2, 256, 262144, 1000
+    q = torch.randn(1, H, Sq, D, dtype=torch.bfloat16, device=cuda)
+    k, v = (torch.randn(1, H, Skv, D, dtype=torch.bfloat16, device=cuda) for _ in range(2))
+    mask = (torch.arange(Skv, device=cuda) < kept)[None, None, None, :]
+    op = torch.ops.para_attn.attention_forward_with_lse
+
+    def best_of_five(f):
+        times = []
+        for _ in range(6):  # the first one warms up
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(20):
+                got = f()
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b) / 20)
+        return min(times[1:]), got
+
+    plain, want = best_of_five(lambda: op(q, k[:, :, :kept], v[:, :, :kept]))
+    masked, got = best_of_five(lambda: op(q, k, v, mask))
+    assert (got[0].float() - want[0].float()).abs().max().item() <= OUT_ATOL and (got[1] - want[1]).abs().max().item() <= LSE_ATOL
+    assert masked < 5 * plain, f"{masked * 1e3:.0f} us against {plain * 1e3:.0f} us without the dropped keys"
+
+
 @pytest.mark.parametrize("D", [8, 40, 56, 72, 80, 96])
 @pytest.mark.parametrize("bm", [0, 128, 256])
 @pytest.mark.parametrize("Sq,Skv", [(1, 1), (130, 65), (290, 320), (257, 4130)])
