@@ -111,9 +111,9 @@ PA_API int pa_attn_fwd_lse(const void* q, const void* k, const void* v, void* ou
  * brings it.  With a workspace of at least pa_attn_fwd_workspace_bytes() bytes
  * (device memory, 16-byte aligned, contents irrelevant before and after) the
  * head_dim-128 kernels cut the query tiles that do not fill a round of the
- * chip's compute units into ranges of key tiles, one per compute unit, and fold
- * their partial results with the same log-sum-exp merge as pa_merge_lse, which
- * removes the idle tail of the launch.
+ * chip's compute units into ranges of key tiles, one per compute unit (head_dim
+ * 64: into equal key shares), and fold their partial results with the same
+ * log-sum-exp merge as pa_merge_lse, which removes the idle tail of the launch.
  * On launches of 1e12 flop and more the first 8 KB of the workspace hold a bound
  * of the scores, computed on the device from the largest row norms of q and k
  * (two small launches that read q and k once): where no score can leave
@@ -218,12 +218,17 @@ PA_API size_t pa_attn_fwd_masked_workspace_bytes(int B, int H, int Sq, int Skv, 
  * arguments, kernels and results as pa_attn_fwd_lse_ws with a workspace of
  * pa_attn_fwd_workspace_bytes() bytes, except that large problems (see the knob
  * "stream_dyn") keep one tail range per workgroup, the plan pa_attn_fwd_lse_ws
- * itself falls back to when its workspace is too small for drawn ranges; there
- * the two entry points agree to rounding, not bit for bit.  A problem whose
- * launch plan needs more scratch than the buffer holds even so is refused with
- * PA_ERR_WORKSPACE (it is not run unsplit behind the caller's back).  Nothing in the buffer has to survive
- * between calls and nothing has to be cleared; but all calls on one GPU share
- * it, so calls that overlap on one GPU (two streams, two threads) race.
+ * itself falls back to when its workspace is too small for drawn ranges, and
+ * that head_dim 64 runs without the key-split tail that a workspace buys it
+ * (as pa_attn_fwd_lse does; no call of it needs more scratch than the score
+ * bound's words); there the two entry points agree to rounding, not bit for
+ * bit.  A head_dim-128 problem whose launch plan needs more scratch than the
+ * buffer holds even so is refused with PA_ERR_WORKSPACE (it is not run unsplit
+ * behind the caller's back).  Nothing in the buffer has to survive between
+ * calls and nothing has to be cleared; but all calls on one GPU that use it
+ * share it, so such calls race where they overlap (two streams, two threads):
+ * head_dim 128 whose launches cut their tail, and launches of 1e12 flop and
+ * more with the score bound.
  */
 #define PA_NOALLOC_SCRATCH_BYTES (80u << 20)
 PA_API int pa_attn_fwd_lse_noalloc(const void* q, const void* k, const void* v, void* out, float* lse,

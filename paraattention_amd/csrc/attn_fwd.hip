@@ -5334,9 +5334,12 @@ extern "C" int pa_attn_fwd_lse_noalloc(const void* q, const void* k, const void*
   const bool shaped = B > 0 && H > 0 && Sq > 0 && Skv > 0 && (D == 128 || D == 64) && k_strides && v_strides;
   // (the plan with one tail range per workgroup: the one a call falls back to when the workspace cannot hold the
   // partial results of drawn ranges, which take four times as many)
-  const size_t need = shaped ? dense_ws_need(B, H, Sq, Skv, D, k_strides, v_strides, is_causal ? 2 : kv_len != nullptr ? 1 : 0, false) : 0;
-  // (head_dim 64 runs without its key split where that does not fit)
-  if (need > (size_t)PA_NOALLOC_SCRATCH_BYTES && D != 64)
+  // (head_dim 64 without its key split, whose partial results calls that overlap would share: the score bound's words only,
+  // which hold no split)
+  size_t need = 0, lent = PA_NOALLOC_SCRATCH_BYTES;
+  if (shaped && D == 64) need = lent = bound_wanted(B, H, Sq, Skv, D) ? bound_ws_bytes(1) : 0;
+  else if (shaped) need = dense_ws_need(B, H, Sq, Skv, D, k_strides, v_strides, is_causal ? 2 : kv_len != nullptr ? 1 : 0, false);
+  if (need > (size_t)PA_NOALLOC_SCRATCH_BYTES)
     PA_FAIL(PA_ERR_WORKSPACE, "this problem's launch plan needs %zu bytes of scratch, the static buffer holds %zu: "
             "call pa_attn_fwd_lse_ws with a workspace of your own", need, (size_t)PA_NOALLOC_SCRATCH_BYTES);
   void* ws = nullptr;
@@ -5345,7 +5348,7 @@ extern "C" int pa_attn_fwd_lse_noalloc(const void* q, const void* k, const void*
     if (rc) return rc;
   }
   return attn_fwd_dense(q, k, v, out, lse, dtype, B, H, Sq, Skv, D, q_strides, k_strides, v_strides,
-                        out_strides, scale, kv_len, is_causal, ws, ws ? (size_t)PA_NOALLOC_SCRATCH_BYTES : 0, stream);
+                        out_strides, scale, kv_len, is_causal, ws, ws ? lent : 0, stream);
 }
 
 // The lists of paired query blocks (build_pair_runs_kernel): half the segments, up to nK + 2 ranges each.

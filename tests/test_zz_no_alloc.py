@@ -90,6 +90,27 @@ def test_noalloc_with_resident_workgroups(cuda, tuning):
         assert (lse[:, :1].cpu() - ref_lse).abs().max().item() <= 1e-3
 
 
+def test_noalloc_head_dim_64_keeps_its_keys_whole(cuda, tuning):
+    """At head_dim 64 the entry runs without the key-split tail: calls of it share no partial results (they may overlap),
+    and none is refused for a plan larger than the buffer.  Bit for bit the launch whose split is
+    switched off, which the launch with a workspace is not."""
+    lib = _lib.load()
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    # a few workgroups beyond a round of two per compute unit; and a split whose partial results would not fit the buffer
+    for H, Sq, Skv, fits in ((33, cus * 8 - 5, 8192 + 3, True), (3, cus * 160 - 5, 131072, False)):
+        q, k, v = (t.to(cuda) for t in inputs.qkv(1, H, Sq, Skv, 64, seed=Sq))
+        tuning("no_split", 1)
+        whole_out, whole_lse, _ = _call_ws(lib, q, k, v)
+        tuning("no_split", 0)
+        split_out, split_lse, need = _call_ws(lib, q, k, v)
+        assert need > 16384 and (need <= _lib.PA_NOALLOC_SCRATCH_BYTES) == fits and not torch.equal(split_lse, whole_lse), "meant to split"
+        rc, out, lse = _call_noalloc(lib, q, k, v)
+        assert rc == 0, lib.pa_last_error()
+        torch.cuda.synchronize()
+        assert torch.equal(out, whole_out) and torch.equal(lse, whole_lse), (H, Sq, Skv)
+        assert (out.float() - split_out.float()).abs().max().item() <= 2e-2 and (lse - split_lse).abs().max().item() <= 1e-3
+
+
 def test_noalloc_refuses_what_the_buffer_cannot_hold(cuda, tuning):
     lib = _lib.load()
     tuning("bm", 256)
