@@ -115,8 +115,9 @@ struct AttnParams {
   // score_bound_*_kernel), so the running maximum is not needed; null = not known, keep the maximum
   const int* bound_flag;
   int split_main, split_tiles, split_s;
-  float* ws_out;  // [split_s * split_tiles][bm][128]
+  float* ws_out;  // [split_s * split_tiles][bm][ws_cols]
   float* ws_lse;  // [split_s * split_tiles][bm]
+  int ws_cols;    // columns of a partial result: those the kernel is built for (128; 64 at head_dim 64 and below)
   // dense pipelined kernel only: ring accumulation.  With acc_out set, the result of this launch is
   // folded into the running pair (acc_out fp32 [B,H,Sq,128] contiguous, acc_lse [B,H,Sq]) by the
   // log-sum-exp merge instead of being stored on its own.  acc_first: the pair holds nothing yet
@@ -2125,10 +2126,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
   }
   const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
   if constexpr (!SPARSE) {
-    if (piece_slot >= 0) {  // partial result of one key share: fp32, into the workspace (rows of 128, 64 of them used)
+    if (piece_slot >= 0) {  // partial result of one key share: fp32, into the workspace
       if (row_ok) {
         const int64_t wrow = (int64_t)piece_slot * p.bm + (my_row - row_begin);
-        float* wp = p.ws_out + wrow * 128;
+        float* wp = p.ws_out + wrow * 64;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -3583,8 +3584,8 @@ __global__ __launch_bounds__(256) void attn_split_merge_kernel(const AttnParams 
     for (int i = 0; i < p.split_s; ++i) {
       const int64_t wrow = ((int64_t)i * p.split_tiles + tl) * p.bm + local;
       const float w = __expf(p.ws_lse[wrow] - m);  // an empty share has LSE -inf: weight 0
-      const float4 a = *(const float4*)(p.ws_out + wrow * 128 + c8);
-      const float4 b = *(const float4*)(p.ws_out + wrow * 128 + c8 + 4);
+      const float4 a = *(const float4*)(p.ws_out + wrow * p.ws_cols + c8);
+      const float4 b = *(const float4*)(p.ws_out + wrow * p.ws_cols + c8 + 4);
       den += w;
       acc[0] += w * a.x; acc[1] += w * a.y; acc[2] += w * a.z; acc[3] += w * a.w;
       acc[4] += w * b.x; acc[5] += w * b.y; acc[6] += w * b.z; acc[7] += w * b.w;
@@ -4062,7 +4063,7 @@ static void fill_params(AttnParams& p, const void* q, const void* k, const void*
   p.xcd_chunk = 0;
   p.causal = 0; p.heads_first = 0;
   p.acc_out = nullptr; p.acc_lse = nullptr; p.acc_first = 0;
-  p.split_main = 0; p.split_tiles = 0; p.split_s = 0; p.ws_out = nullptr; p.ws_lse = nullptr;
+  p.split_main = 0; p.split_tiles = 0; p.split_s = 0; p.ws_out = nullptr; p.ws_lse = nullptr; p.ws_cols = 128;
   p.bound_flag = nullptr;
   p.dt = 128; p.mask_kind = MASK_NONE; p.mask_words = nullptr; p.mw_b = p.mw_h = 0;
   p.mask = nullptr; p.ms_b = p.ms_h = p.ms_q = p.ms_k = 0;
@@ -4179,7 +4180,7 @@ struct SplitPlan {
 // dealing of workgroups to 8 XCDs) are MI355X's: 256 compute units in 8 XCDs.  On a device that reports another
 // compute-unit count the launches fall back to plain plans: no key split priced by those constants, no XCD order.
 static bool mi355x_layout() { return device_cus() == 256; }
-static SplitPlan plan_split(int64_t n_tiles, int slots, int kv_tiles, int bm, bool allow, double tile_us = 1.75, bool pairs = false) {
+static SplitPlan plan_split(int64_t n_tiles, int slots, int kv_tiles, int bm, bool allow, double tile_us = 1.75, bool pairs = false, int cols = 128) {
   if (slots <= 0) return {0, 1, 1.0};  // no device to ask: no estimate, no split
   SplitPlan best = {0, 1, (double)((n_tiles + slots - 1) / slots)};
   // pairs: two places per compute unit; a last round of one workgroup per unit runs 1.5 times as fast
@@ -4196,7 +4197,7 @@ static SplitPlan plan_split(int64_t n_tiles, int slots, int kv_tiles, int bm, bo
     if (T > n_tiles || T * 8 > 0x7fffffffLL) break;
     for (int s = 2; s <= 8 && kv_tiles / s >= 16; ++s) {
       const double share = ((double)kv_tiles / s + 4.0) / ((double)kv_tiles + 4.0);
-      const double merge_us = 8.0 + (double)T * s * bm * 129.0 * 4.0 / 3.0e6;
+      const double merge_us = 8.0 + (double)T * s * bm * (cols + 1) * 4.0 / 3.0e6;
       const double r = (double)((n_tiles - T) / slots) + (double)((T * s + slots - 1) / slots) * share + merge_us / round_us;
       if (r < best.rounds * 0.97 && r < best_found) { best_found = r; found = {(int)T, s, r}; }
     }
@@ -4276,8 +4277,12 @@ extern "C" int pa_set_tuning(const char* name, int value) {
 }
 
 // Bytes of workspace the key-split tail of the plan for bm rows per workgroup needs.
-static size_t split_ws_bytes(const SplitPlan& pl, int bm) {
-  return pl.s > 1 ? (size_t)pl.tiles * pl.s * bm * (128 + 1) * sizeof(float) : 0;
+static size_t split_ws_bytes(const SplitPlan& pl, int bm, int cols = 128) {
+  return pl.s > 1 ? (size_t)pl.tiles * pl.s * bm * (cols + 1) * sizeof(float) : 0;
+}
+static void lend_split_ws(AttnParams& p, void* ws) {
+  p.ws_out = (float*)ws;
+  p.ws_lse = p.ws_out + (size_t)p.split_tiles * p.split_s * p.bm * p.ws_cols;
 }
 
 // Whether the pipelined kernels take the call: K and V below 4 GiB per head (32-bit buffer offsets).
@@ -4316,16 +4321,17 @@ static void choose_kernel(AttnParams& p, int D, int q_block, bool dense, size_t 
   // head_dim 64: 128 rows unless asked otherwise, and the key-split tail beyond one round of workgroups (48 heads x
   // 17776 tokens, 6672 workgroups on 512 places: 3.99 -> 3.84 ms; 3 heads x 24000: 0.58 -> 0.47 ms)
   if (D == 64) {
-    p.dt = 64;
+    p.dt = p.ws_cols = 64;
     if (forced == 256 && (dense || q_block % 256 == 0)) p.bm = 256;
     order();
     const bool may = dense && n_cus > 0 && mi355x_layout() && !p.causal && !tuning().no_split && (ws_needed != nullptr || ws_bytes > 0);
     const int64_t tiles = (int64_t)p.B * p.H * p.n_qtiles;
     const int slots = p.bm == 256 ? n_cus : 2 * n_cus;
     if (!may || tiles <= slots) return;
-    SplitPlan pl = plan_split(tiles, slots, (p.Skv + BN - 1) / BN, p.bm, true, 1.0, p.bm == 128);
-    if (ws_needed) *ws_needed = split_ws_bytes(pl, p.bm);
-    else if (pl.s > 1 && split_ws_bytes(pl, p.bm) <= ws_bytes) {
+    // (a key tile takes a workgroup 1.04 us here: those 17776 tokens, 282 tiles in 13.2 rounds)
+    SplitPlan pl = plan_split(tiles, slots, (p.Skv + BN - 1) / BN, p.bm, true, 1.0, p.bm == 128, 64);
+    if (ws_needed) *ws_needed = split_ws_bytes(pl, p.bm, 64);
+    else if (pl.s > 1 && split_ws_bytes(pl, p.bm, 64) <= ws_bytes) {
       p.split_s = pl.s;
       p.split_tiles = pl.tiles;
       p.split_main = (int)(tiles - pl.tiles);
@@ -4722,7 +4728,7 @@ static int attn_fwd_dense(const void* q, const void* k, const void* v, void* out
     }
   }
   const size_t split_bytes = streamed ? stream_bytes
-                             : p.split_s > 1 ? (size_t)p.split_tiles * p.split_s * p.bm * (128 + 1) * sizeof(float) : 0;
+                             : p.split_s > 1 ? (size_t)p.split_tiles * p.split_s * p.bm * (p.ws_cols + 1) * sizeof(float) : 0;
   if (want_bound && p.pipe && (D == 64 || p.bm == 256) && ws_avail >= split_bytes + bound_bytes) {
     ws_base += bound_bytes;
     if (opts != nullptr && opts->bound_done != nullptr && *opts->bound_done) {
@@ -4752,10 +4758,7 @@ static int attn_fwd_dense(const void* q, const void* k, const void* v, void* out
     if (B == 0 || H == 0 || Sq == 0) return PA_OK;
     return dtype == PA_DTYPE_BF16 ? launch_stream<BF16>(p, (hipStream_t)stream) : launch_stream<F16>(p, (hipStream_t)stream);
   }
-  if (p.split_s > 1) {
-    p.ws_out = (float*)ws_base;
-    p.ws_lse = p.ws_out + (size_t)p.split_tiles * p.split_s * p.bm * 128;
-  }
+  if (p.split_s > 1) lend_split_ws(p, ws_base);
   return dispatch_attn<false>(p, dtype, D, (hipStream_t)stream);
 }
 
@@ -4976,10 +4979,7 @@ extern "C" int pa_attn_fwd_narrow(const void* q, const void* k, const void* v, v
   p.causal = is_causal != 0;
   if (B <= 0 || H <= 0 || Sq <= 0 || !plan_narrow(p, D, workspace ? workspace_bytes : 0, nullptr))
     PA_FAIL(PA_ERR_UNSUPPORTED, "pa_attn_fwd_narrow does not take this call (pa_attn_fwd_narrow_plan tells)");
-  if (p.split_s > 1) {
-    p.ws_out = (float*)workspace;
-    p.ws_lse = p.ws_out + (size_t)p.split_tiles * p.split_s * p.bm * 128;
-  }
+  if (p.split_s > 1) lend_split_ws(p, workspace);
   return dtype == PA_DTYPE_BF16 ? launch_narrow<BF16>(p, (hipStream_t)stream) : launch_narrow<F16>(p, (hipStream_t)stream);
 }
 
@@ -5182,10 +5182,7 @@ extern "C" int pa_attn_fwd_masked(const void* q, const void* k, const void* v, v
   const bool no_query_dim = any && (Sq == 1 || p.ms_q == 0);
   auto masked_pipe = [&](void* ws, size_t ws_bytes) {
     choose_kernel(p, D, 256, true, ws ? ws_bytes : 0, nullptr);
-    if (p.split_s > 1) {
-      p.ws_out = (float*)ws;
-      p.ws_lse = p.ws_out + (size_t)p.split_tiles * p.split_s * p.bm * 128;
-    }
+    if (p.split_s > 1) lend_split_ws(p, ws);
     if (dtype == PA_DTYPE_BF16) return D == 128 ? launch_masked_pipe<BF16, 128>(p, st) : launch_masked_pipe<BF16, 64>(p, st);
     return D == 128 ? launch_masked_pipe<F16, 128>(p, st) : launch_masked_pipe<F16, 64>(p, st);
   };

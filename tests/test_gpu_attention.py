@@ -2,6 +2,7 @@
 
 Tolerances are the ones the task states: bf16/fp16 output atol 2e-2 / rtol 2e-2, fp32 LSE 1e-3.
 """
+import ctypes
 import math
 
 import numpy as np
@@ -11,6 +12,7 @@ import torch
 import paraattention_amd  # noqa: F401
 from oracle import attention as oattn
 from oracle import inputs
+from paraattention_amd import _lib
 
 pytestmark = pytest.mark.gpu
 
@@ -420,6 +422,37 @@ def test_key_split_tail_head_dim_64(cuda, tuning, D, bound):
         _check(out[:, -1:], lse[:, -1:], ref_out, ref_lse, f"split tail, masked={mask is not None}")
         assert torch.equal(out[:, :-1], out1[:, :-1]) and torch.equal(lse[:, :-1], lse1[:, :-1])
         assert not torch.equal(lse[:, -1], lse1[:, -1])  # another order of sums: the split was taken
+
+
+@pytest.mark.parametrize("D", [64, 40])
+def test_partial_results_of_head_dim_64(cuda, D):
+    """A workspace of exactly the stated size, all of it NaN and with a NaN behind it: 16 query tiles in 8 key shares take
+    (64 + 1) floats per row and share, the result is the op's own, and nothing behind the workspace is touched."""
+    lib = _lib.load()
+    B, H, Sq, Skv = 1, 33, 2048 - 5, 8192 + 3
+    q, k, v = (t.to(cuda) for t in inputs.qkv(B, H, Sq, Skv, D, seed=D))
+    ks, vs = _lib.strides3(k), _lib.strides3(v)
+    if D == 64:
+        need = lib.pa_attn_fwd_call_workspace_bytes(B, H, Sq, Skv, D, ks, vs, 0, 0)
+    else:
+        room = ctypes.c_size_t()
+        assert lib.pa_attn_fwd_narrow_plan(B, H, Sq, Skv, D, ks, vs, 0, ctypes.byref(room)) == 1
+        need = room.value
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert need == 16 * 8 * 128 * (64 + 1) * 4
+    ws = torch.full((need // 4 + 64,), float("nan"), device=cuda)
+    out, lse = torch.empty_like(q), torch.empty(B, H, Sq, device=cuda)
+    sizes = (0, B, H, Sq, Skv, D, _lib.strides3(q), ks, vs, _lib.strides3(out), 1.0 / math.sqrt(D))
+    operands = [t.data_ptr() for t in (q, k, v, out, lse)]
+    stream = torch.cuda.current_stream().cuda_stream
+    if D == 64:
+        rc = lib.pa_attn_fwd_lse_ws(*operands, *sizes, None, 0, ws.data_ptr(), need, stream)
+    else:
+        rc = lib.pa_attn_fwd_narrow(*operands, *sizes, 0, ws.data_ptr(), need, stream)
+    assert rc == 0, lib.pa_last_error()
+    want_out, want_lse = torch.ops.para_attn.attention_forward_with_lse(q, k, v)
+    assert torch.equal(out, want_out) and torch.equal(lse, want_lse) and torch.isfinite(lse).all()
+    assert torch.isnan(ws[need // 4:]).all()
 
 
 @pytest.mark.parametrize("D", [128, 64])
