@@ -1771,7 +1771,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
 // ---------------------------------------------------------------------------------------------
 constexpr int TILE64_BYTES = BN * 128;
 
-template <typename T, bool SPARSE, int NW, bool BOUNDED = false, int PM = PM_NONE, bool NARROW = false>
+// CUT: the grid has key shares of split query tiles, or the heads as its fastest index.  A template argument and not a look
+// at the parameters, because a launch with neither -- cross-attention of many rows to a few hundred keys can never split --
+// pays their decode and epilogue in every short workgroup (33 scalar registers spilled against 24): 40 heads x 32760 rows
+// against 512 keys 244.9 -> 242.0 us without them, 24 x 17776 against 256 keys 56.6 -> 55.6, 16 heads x 3000 tokens 50.5 -> 49.7.
+template <typename T, bool SPARSE, int NW, bool BOUNDED = false, int PM = PM_NONE, bool NARROW = false, bool CUT = false>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_kernel(const AttnParams p) {
   // BOUNDED and the flag: as in attn_fwd_d128_pipe_kernel
   if constexpr (!SPARSE) {
@@ -1794,7 +1798,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
 
   int tile = blockIdx.x;
   int piece_slot = -1;  // >= 0: this workgroup computes one key share of a split query tile
-  if constexpr (!SPARSE) {
+  if constexpr (CUT) {
     if (p.split_s > 1 && tile >= p.split_main) {
       piece_slot = tile - p.split_main;
       tile = p.split_main + piece_slot % p.split_tiles;
@@ -1807,7 +1811,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
     }
   }
   int qt = tile % p.n_qtiles, bh = tile / p.n_qtiles;
-  if constexpr (!SPARSE) {
+  if constexpr (CUT) {
     if (p.heads_first) {
       qt = tile / (p.B * p.H);
       bh = tile - qt * (p.B * p.H);
@@ -1826,7 +1830,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
   }
   if constexpr (PM == PM_KEYS) it.init_dense(__builtin_amdgcn_readfirstlane(tm.kept_end(p.Skv)));
 
-  if constexpr (!SPARSE) {
+  if constexpr (CUT) {
     if (piece_slot >= 0) {
       const int piece = piece_slot / p.split_tiles, len = it.end;
       const int nkt = (len + BN - 1) / BN;
@@ -2125,7 +2129,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
     l_tot = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
   }
   const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
-  if constexpr (!SPARSE) {
+  if constexpr (CUT) {
     if (piece_slot >= 0) {  // partial result of one key share: fp32, into the workspace
       if (row_ok) {
         const int64_t wrow = (int64_t)piece_slot * p.bm + (my_row - row_begin);
@@ -4071,6 +4075,31 @@ static void fill_params(AttnParams& p, const void* q, const void* k, const void*
   p.st = StreamPlan{};
 }
 
+template <typename T, bool SPARSE, int NW, bool BOUNDED, int PM = PM_NONE, bool NARROW = false, bool CUT = false>
+static int launch_d64(const AttnParams& p, int64_t nblocks, hipStream_t stream) {
+  const size_t smem = 4 * TILE64_BYTES + (PM == PM_KEYS || PM == PM_KEYBIAS ? NW * PM_SLOT_BYTES : 0);
+  static bool attr_done[PA_MAX_DEVICES] = {};  // benign race: the call is idempotent
+  const int dev = current_device();
+  if (dev < 0 || !attr_done[dev]) {
+    hipError_t e = hipFuncSetAttribute((const void*)attn_fwd_d64_pipe_kernel<T, SPARSE, NW, BOUNDED, PM, NARROW, CUT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    if (e != hipSuccess) PA_FAIL(PA_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
+    if (dev >= 0) attr_done[dev] = true;
+  }
+  hipLaunchKernelGGL((attn_fwd_d64_pipe_kernel<T, SPARSE, NW, BOUNDED, PM, NARROW, CUT>), dim3((unsigned)nblocks), dim3(64 * NW), smem, stream, p);
+  PA_CHECK_LAUNCH("attention kernel (head_dim 64)");
+  return PA_OK;
+}
+
+template <typename T, bool SPARSE, bool BOUNDED>
+static int launch_d64_plain(const AttnParams& p, int64_t nblocks, hipStream_t stream) {
+  if constexpr (!SPARSE) {
+    if (p.split_s > 1 || p.heads_first)
+      return p.bm == 256 ? launch_d64<T, false, 8, BOUNDED, PM_NONE, false, true>(p, nblocks, stream)
+                         : launch_d64<T, false, 4, BOUNDED, PM_NONE, false, true>(p, nblocks, stream);
+  }
+  return p.bm == 256 ? launch_d64<T, SPARSE, 8, BOUNDED>(p, nblocks, stream) : launch_d64<T, SPARSE, 4, BOUNDED>(p, nblocks, stream);
+}
+
 template <typename T, int D, bool SPARSE>
 static int launch_attn(const AttnParams& p, hipStream_t stream) {
   int64_t nblocks = (int64_t)p.B * p.H * p.n_qtiles;
@@ -4091,47 +4120,44 @@ static int launch_attn(const AttnParams& p, hipStream_t stream) {
     else if (p.pipe) { fn = (const void*)attn_fwd_d128_pipe_kernel<T, SPARSE, 4>; slot = 1; }
     else { fn = (const void*)attn_fwd_d128_kernel<T, SPARSE>; slot = 0; }
   } else {
-    if (p.pipe && p.bm == 256) { fn = (const void*)attn_fwd_d64_pipe_kernel<T, SPARSE, 8>; slot = 2; smem = 4 * TILE64_BYTES; }
-    else if (p.pipe) { fn = (const void*)attn_fwd_d64_pipe_kernel<T, SPARSE, 4>; slot = 1; smem = 4 * TILE64_BYTES; }
-    else { fn = (const void*)attn_fwd_kernel<T, D, SPARSE>; slot = 0; smem = Smem<D>::BYTES; }
+    fn = (const void*)attn_fwd_kernel<T, D, SPARSE>;
+    slot = p.pipe ? 1 : 0;
+    smem = Smem<D>::BYTES;
   }
   // the attribute belongs to the function on one device: remembered per device and kernel variant
-  if (p.bound_flag != nullptr && (SPARSE || !(D == 128 ? slot == 2 : slot >= 1)))
+  if (p.bound_flag != nullptr && (SPARSE || slot != (D == 128 ? 2 : 1)))
     PA_FAIL(PA_ERR_UNSUPPORTED, "score bound reached a kernel that does not read it");
-  static bool attr_done[PA_MAX_DEVICES][6] = {};  // benign race: the call is idempotent
+  static bool attr_done[PA_MAX_DEVICES][5] = {};  // benign race: the call is idempotent
   const int dev = current_device();
-  if (dev < 0 || !attr_done[dev][slot]) {
+  if (!(D == 64 && p.pipe) && (dev < 0 || !attr_done[dev][slot])) {
     hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     if (e != hipSuccess) PA_FAIL(PA_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
     if (dev >= 0) attr_done[dev][slot] = true;
   }
   if constexpr (!SPARSE) {
     if (p.bound_flag != nullptr) {  // the variant without a running maximum first; one of the two returns at once
-      const void* fb;
-      if constexpr (D == 128) fb = (const void*)attn_fwd_d128_pipe_kernel<T, false, 8, true>;
-      else fb = slot == 2 ? (const void*)attn_fwd_d64_pipe_kernel<T, false, 8, true> : (const void*)attn_fwd_d64_pipe_kernel<T, false, 4, true>;
-      const int bslot = 3 + (D == 64 && slot == 1 ? 1 : 0);
-      if (dev < 0 || !attr_done[dev][bslot]) {
-        hipError_t e = hipFuncSetAttribute(fb, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        if (e != hipSuccess) PA_FAIL(PA_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
-        if (dev >= 0) attr_done[dev][bslot] = true;
-      }
-      if constexpr (D == 128)
+      if constexpr (D == 128) {
+        const void* fb = (const void*)attn_fwd_d128_pipe_kernel<T, false, 8, true>;
+        if (dev < 0 || !attr_done[dev][3]) {
+          hipError_t e = hipFuncSetAttribute(fb, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+          if (e != hipSuccess) PA_FAIL(PA_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
+          if (dev >= 0) attr_done[dev][3] = true;
+        }
         hipLaunchKernelGGL((attn_fwd_d128_pipe_kernel<T, false, 8, true>), dim3((unsigned)nblocks), dim3(512), smem, stream, p);
-      else if (slot == 2)
-        hipLaunchKernelGGL((attn_fwd_d64_pipe_kernel<T, false, 8, true>), dim3((unsigned)nblocks), dim3(512), smem, stream, p);
-      else
-        hipLaunchKernelGGL((attn_fwd_d64_pipe_kernel<T, false, 4, true>), dim3((unsigned)nblocks), dim3(256), smem, stream, p);
+      } else {
+        const int rc = launch_d64_plain<T, false, true>(p, nblocks, stream);
+        if (rc != PA_OK) return rc;
+      }
       PA_CHECK_LAUNCH("attention kernel (bounded scores)");
     }
   }
   if constexpr (D == 128 && SPARSE) {
     if (p.pair) {
       const void* fp = (const void*)attn_fwd_d128_pipe_kernel<T, true, 8, false, true>;
-      if (dev < 0 || !attr_done[dev][5]) {
+      if (dev < 0 || !attr_done[dev][4]) {
         hipError_t e = hipFuncSetAttribute(fp, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
         if (e != hipSuccess) PA_FAIL(PA_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
-        if (dev >= 0) attr_done[dev][5] = true;
+        if (dev >= 0) attr_done[dev][4] = true;
       }
       hipLaunchKernelGGL((attn_fwd_d128_pipe_kernel<T, true, 8, false, true>), dim3((unsigned)nblocks), dim3(512), smem, stream, p);
       PA_CHECK_LAUNCH("attention kernel (paired query blocks)");
@@ -4146,11 +4172,10 @@ static int launch_attn(const AttnParams& p, hipStream_t stream) {
     else
       hipLaunchKernelGGL((attn_fwd_d128_kernel<T, SPARSE>), dim3((unsigned)nblocks), dim3(NTHREADS), smem, stream, p);
   } else {
-    if (slot == 2)
-      hipLaunchKernelGGL((attn_fwd_d64_pipe_kernel<T, SPARSE, 8>), dim3((unsigned)nblocks), dim3(512), smem, stream, p);
-    else if (slot == 1)
-      hipLaunchKernelGGL((attn_fwd_d64_pipe_kernel<T, SPARSE, 4>), dim3((unsigned)nblocks), dim3(256), smem, stream, p);
-    else
+    if (p.pipe) {
+      const int rc = launch_d64_plain<T, SPARSE, false>(p, nblocks, stream);
+      if (rc != PA_OK) return rc;
+    } else
       hipLaunchKernelGGL((attn_fwd_kernel<T, D, SPARSE>), dim3((unsigned)nblocks), dim3(NTHREADS), smem, stream, p);
   }
   PA_CHECK_LAUNCH("attention kernel");
@@ -4901,22 +4926,21 @@ template <typename T, int D, int PM, int NW, int W = D>
 static int launch_pipe_variant(const AttnParams& p, hipStream_t stream) {
   int64_t nblocks = (int64_t)p.B * p.H * p.n_qtiles;
   if (p.split_s > 1) nblocks = (int64_t)p.split_main + (int64_t)p.split_tiles * p.split_s;
-  const size_t smem = 4 * (D == 128 ? TILE_BYTES : TILE64_BYTES) + (PM == PM_NONE || PM == PM_BITS || PM == PM_BIAS ? 0 : NW * PM_SLOT_BYTES);
-  const void* fn;
-  if constexpr (D == 128) fn = (const void*)attn_fwd_d128_pipe_kernel<T, false, NW, false, false, PM, W>;
-  else fn = (const void*)attn_fwd_d64_pipe_kernel<T, false, NW, false, PM, (W < 64)>;
-  static bool attr_done[PA_MAX_DEVICES] = {};  // benign race: the call is idempotent
-  const int dev = current_device();
-  if (dev < 0 || !attr_done[dev]) {
-    hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    if (e != hipSuccess) PA_FAIL(PA_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
-    if (dev >= 0) attr_done[dev] = true;
-  }
-  if constexpr (D == 128)
+  if constexpr (D == 128) {
+    const size_t smem = 4 * TILE_BYTES + (PM == PM_KEYS || PM == PM_KEYBIAS ? NW * PM_SLOT_BYTES : 0);
+    static bool attr_done[PA_MAX_DEVICES] = {};  // benign race: the call is idempotent
+    const int dev = current_device();
+    if (dev < 0 || !attr_done[dev]) {
+      hipError_t e = hipFuncSetAttribute((const void*)attn_fwd_d128_pipe_kernel<T, false, NW, false, false, PM, W>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+      if (e != hipSuccess) PA_FAIL(PA_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
+      if (dev >= 0) attr_done[dev] = true;
+    }
     hipLaunchKernelGGL((attn_fwd_d128_pipe_kernel<T, false, NW, false, false, PM, W>), dim3((unsigned)nblocks), dim3(64 * NW), smem, stream, p);
-  else
-    hipLaunchKernelGGL((attn_fwd_d64_pipe_kernel<T, false, NW, false, PM, (W < 64)>), dim3((unsigned)nblocks), dim3(64 * NW), smem, stream, p);
-  PA_CHECK_LAUNCH("attention kernel (masked or narrow rows)");
+    PA_CHECK_LAUNCH("attention kernel (masked or narrow rows)");
+  } else {  // (masks with a query dimension are planned without a split)
+    const int rc = launch_d64<T, false, NW, false, PM, (W < 64), PM != PM_BITS && PM != PM_BIAS>(p, nblocks, stream);
+    if (rc != PA_OK) return rc;
+  }
   if (p.split_s > 1) {
     const int64_t rows = (int64_t)p.split_tiles * p.bm;
     hipLaunchKernelGGL((attn_split_merge_kernel<T>), dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, stream, p);
