@@ -593,7 +593,8 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_fwd_kernel(const AttnParams 
 //               and for every 128 query rows the list of the key tiles that any of them keeps (the others are not walked)
 //   PM_BIAS     additive with a query dimension and adjacent keys: four keys per load, right where they are added (2 x 24
 //               heads x 2999 tokens, head_dim 64, fp32 bias per head 2.13 -> 0.49 ms; 16 heads x 2000, head_dim 128
-//               225 -> 139 us; bound by the latency of loads that no register is left to fetch ahead)
+//               225 -> 85 us, 139 of them while it spilled 9 registers; bound by the latency of loads that no register is
+//               left to fetch ahead: it takes 255 of 256)
 // Without a query dimension each wavefront lays the tile's 64 values down in its own 256 bytes of LDS and reads them back in the accumulator's
 // order (8 broadcast reads, one instruction per score); a tile that drops no key, or whose biases are all zero, costs
 // nothing beyond the vote that says so.  Measured against the per-score kernel (attn_fwd_kernel<MASK>, register-staged
@@ -632,7 +633,7 @@ struct TileMask {
     const int64_t at = batch * p.ms_b + head * p.ms_h;
     act = (PM == PM_KEYBIAS || PM == PM_BIAS) && p.mask_kind == MASK_ACT;
     const int bytes = PM == PM_KEYS ? 1 : act ? 2 : 4;
-    base = (const char*)p.mask + (PM == PM_BIAS ? at + row * p.ms_q : at) * bytes;
+    base = (const char*)p.mask + (PM == PM_BIAS ? at + row * p.ms_q + 4 * hh : at) * bytes;  // PM_BIAS: from the lane's own keys on
     step = (uint32_t)(p.ms_k * bytes);
     per_scale = 1.0f / (p.scale_log2 * LN2);  // bias / scale, so that (s + that) * c = s * c + bias * log2(e)
     slot = (float*)lds;
@@ -701,7 +702,7 @@ struct TileMask {
     if (nvalid <= 0) return;
     if (nvalid == BN) {
       if (act) {
-        const char* at = base + (n0 + 4 * hh) * 2;
+        const char* at = base + (uint64_t)n0 * 2;
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -715,7 +716,7 @@ struct TileMask {
             s[4 * a + 3] += T::hi(w[1]) * per_scale;
           }
       } else {
-        const char* at = base + (n0 + 4 * hh) * 4;
+        const char* at = base + (uint64_t)n0 * 4;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
           floatx4 w[4];
@@ -733,8 +734,8 @@ struct TileMask {
     // the ragged last tile: key by key, nothing past the last one is read
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const uint32_t n = n0 + 8 * (r >> 2) + 4 * hh + (r & 3);
-      const uint32_t k0 = n < last ? n : last, k1 = n + 32 < last ? n + 32 : last;
+      const int n = (int)n0 + 8 * (r >> 2) + (r & 3), end = (int)last - 4 * hh;  // (end < 0: the last key is another lane's)
+      const int k0 = min(n, end), k1 = min(n + 32, end);
       a0[r] += (act ? T::lo(((const uint16_t*)base)[k0]) : ((const float*)base)[k0]) * per_scale;
       a1[r] += (act ? T::lo(((const uint16_t*)base)[k1]) : ((const float*)base)[k1]) * per_scale;
     }
@@ -1148,6 +1149,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
   constexpr int DC = W / 16, DB = W / 32;
   static_assert(W == 128 || (W == 96 && !SPARSE && !PAIR && !BOUNDED), "row widths this kernel is written for");
   constexpr int IPW = 16 / NW;  // copy instructions per wavefront and K (V) tile
+  // is_causal, key shares, key segments and the fold into a running pair: masks with a query dimension are planned without
+  // them (compiled in all the same, they took registers that PM_BIAS spilled and read back in every tile)
+  constexpr bool ALL = !SPARSE && PM != PM_BITS && PM != PM_BIAS;
   // With a score bound on record the launch comes twice, once per variant, and the one the flag (computed on
   // the device just before) does not select leaves at once.  BOUNDED: exp2(score) cannot overflow or vanish, so
   // the reference point of the softmax stays 0 and row maxima, rescale checks and rescales are compiled out.
@@ -1179,14 +1183,14 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
       if (tile >= p.B * p.H * p.n_qtiles) return;
     }
   }
-  if constexpr (!SPARSE) {
+  if constexpr (ALL) {
     if (p.split_s > 1 && tile >= p.split_main) {
       piece_slot = tile - p.split_main;
       tile = p.split_main + piece_slot % p.split_tiles;
     }
   }
   int qt = tile % p.n_qtiles, bh = tile / p.n_qtiles;
-  if constexpr (!SPARSE) {
+  if constexpr (ALL) {
     if (p.heads_first) {
       qt = tile / (p.B * p.H);
       bh = tile - qt * (p.B * p.H);
@@ -1208,7 +1212,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
   // segment, with the softmax state carried over in registers.  A key share of a split piece is then a run of
   // whole segments; with one segment it is a range of key tiles.
   int seg_lo = 0, seg_hi = 1;
-  if constexpr (!SPARSE) {
+  if constexpr (ALL) {
     const int nseg = p.st.nseg > 1 ? p.st.nseg : 1;
     seg_hi = nseg;
     if (piece_slot >= 0) {
@@ -1360,11 +1364,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
   // causal: the tile starting at key n0 needs masking for this wavefront if it reaches past its first row
   auto on_diagonal = [&](uint32_t n0) {
     if constexpr (SPARSE) return false;
-    else return p.causal != 0 && n0 != OOB && (int)n0 + BN - 1 > wave_row0;
+    else return ALL && p.causal != 0 && n0 != OOB && (int)n0 + BN - 1 > wave_row0;
   };
   auto mask_tail = [&](floatx16& a0, floatx16& a1, int nvalid, uint32_t n0) {
     int lim = nvalid;
-    if constexpr (!SPARSE) {
+    if constexpr (ALL) {
       if (p.causal) lim = min(lim, my_row - (int)n0 + 1);  // keys up to the row's own index
     }
     lim -= 4 * hh;
@@ -1608,7 +1612,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
   // the copies' descriptors following their tile's segment, was measured: the bookkeeping that adds to every
   // iteration costs 4.5 % of the sweep, the drains it saves 2 %).
   for (int seg = seg_lo; seg < seg_hi; ++seg) {
-    if constexpr (!SPARSE) {
+    if constexpr (ALL) {
       if (p.st.nseg > 1) {  // this segment's keys and values, all of them
         const int64_t koff = (batch * p.ks_b + head * p.ks_h) * 2, voff = (batch * p.vs_b + head * p.vs_h) * 2;
         krs = make_rsrc((const char*)p.st.kseg[seg] + koff, ks_bytes, p.st.seg_len);
@@ -1681,7 +1685,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
     l_tot = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
   }
   const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
-  if constexpr (!SPARSE) {
+  if constexpr (ALL) {
     if (piece_slot >= 0) {  // partial result of one key share: fp32, into the workspace
       if (row_ok) {
         const int64_t wrow = (int64_t)piece_slot * p.bm + (my_row - row_begin);

@@ -45,6 +45,15 @@ def kernels():
     return found
 
 
+def test_pipelined_kernels_spill_no_vector_register(kernels):
+    attention = {n: k for n, k in kernels.items() if any(f"{kind}_kernel" in n for kind in ("pipe", "stream", "short"))}
+    # (the form with 64 rows per wavefront, which only a tuning knob reaches, spills and is slower for it)
+    attention = {n: k for n, k in attention.items() if not re.search(r"stream_kernelI.*ELb[01]ELi2ELb", n)}
+    assert len(attention) > 60
+    spilled = {n: k[".vgpr_spill_count"] for n, k in attention.items() if k[".vgpr_spill_count"] or k[".private_segment_fixed_size"]}
+    assert not spilled, spilled
+
+
 @pytest.mark.parametrize("T", ["4BF16", "3F16"])
 def test_unsplit_head_dim_64_kernels_pay_nothing_for_the_split(kernels, T):
     """The dense kernel of an unsplit launch spills fewer scalar registers than the one that decodes key shares, for both
