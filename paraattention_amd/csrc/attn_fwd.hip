@@ -595,8 +595,12 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_fwd_kernel(const AttnParams 
 //               heads x 2999 tokens, head_dim 64, fp32 bias per head 2.13 -> 0.49 ms; 16 heads x 2000, head_dim 128
 //               225 -> 85 us, 139 of them while it spilled 9 registers; bound by the latency of loads that no register is
 //               left to fetch ahead: it takes 255 of 256)
-// Without a query dimension each wavefront lays the tile's 64 values down in its own 256 bytes of LDS and reads them back in the accumulator's
-// order (8 broadcast reads, one instruction per score); a tile that drops no key, or whose biases are all zero, costs
+// Without a query dimension one vote of the wavefront holds a tile's 64 kept keys, and a tile's 64 biases are laid down in the
+// wavefront's own 256 bytes of LDS and read back in the accumulator's order (8 broadcast reads, one instruction per score).  A
+// choice by lane masks of the vote's bits costs head_dim 128 nothing against a minimum with -inf read back from LDS,
+// which would leave NaN to the compiler (24 heads x 4352 tokens, 30 % dropped at random: 257.6 and 256.7 us), and
+// head_dim 64 gains 3 % where a few tiles have holes and loses 4 where all have (128.9 and 133.1, 170.1 and 163.4); bits
+// read back from LDS cost 3 and 1 %.  A tile that drops no key, or whose biases are all zero, costs
 // nothing beyond the vote that says so.  Measured against the per-score kernel (attn_fwd_kernel<MASK>, register-staged
 // tiles): two samples x 24 heads x 7800 rows against 256 keys with a bias 171 -> 104 us (0.47 PFLOP/s; bound by what a
 // workgroup does around its four key tiles), 24 heads x 4352 tokens with holes in the key mask, scan and two empty
@@ -753,16 +757,24 @@ struct TileMask {
       }
       return;
     }
-    // what a lane lays down for its key: the bias, or the largest value a score may keep (-inf drops it whatever it is,
-    // also where a dropped key's row holds no numbers)
-    float b;
     if constexpr (PM == PM_KEYS) {
-      if (!__any(raw == 0)) return;
-      b = raw != 0 ? INFINITY : -INFINITY;
-    } else {
-      b = (act ? T::lo(raw) : __uint_as_float(raw)) * per_scale;
-      if (!__any((__float_as_uint(b) << 1) != 0)) return;
+      // One vote holds the tile.  Score r of a lane belongs to key n of the first half (n + 32 of the second), n + 4 in the upper
+      // 32 lanes: two bits of the vote, spread over the halves of a lane mask, choose between the score and -inf.  (A
+      // dropped key's score may be a NaN, of a row that holds no numbers, and this file is compiled without NaN
+      // semantics: no minimum with -inf has to drop it.)
+      const uint64_t kept = __ballot(raw != 0);
+      if (kept == ~(uint64_t)0) return;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int n = 8 * (r >> 2) + (r & 3);
+        auto lanes = [&](uint32_t w) { return (uint64_t)(uint32_t)((int32_t)(w << (31 - n)) >> 31) | (uint64_t)(uint32_t)((int32_t)(w << (27 - n)) >> 31) << 32; };
+        if (!__builtin_amdgcn_inverse_ballot_w64(lanes((uint32_t)kept))) a0[r] = -INFINITY;
+        if (!__builtin_amdgcn_inverse_ballot_w64(lanes((uint32_t)(kept >> 32)))) a1[r] = -INFINITY;
+      }
+      return;
     }
+    const float b = (act ? T::lo(raw) : __uint_as_float(raw)) * per_scale;  // what a lane lays down for its key
+    if (!__any((__float_as_uint(b) << 1) != 0)) return;
     __builtin_amdgcn_wave_barrier();
     slot[lane] = b;
     __builtin_amdgcn_wave_barrier();
@@ -771,8 +783,8 @@ struct TileMask {
       const floatx4 x = *(const floatx4*)(slot + 8 * a + 4 * hh), y = *(const floatx4*)(slot + 32 + 8 * a + 4 * hh);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        a0[4 * a + i] = PM == PM_KEYS ? fminf(a0[4 * a + i], x[i]) : a0[4 * a + i] + x[i];
-        a1[4 * a + i] = PM == PM_KEYS ? fminf(a1[4 * a + i], y[i]) : a1[4 * a + i] + y[i];
+        a0[4 * a + i] += x[i];
+        a1[4 * a + i] += y[i];
       }
     }
   }
@@ -4081,7 +4093,7 @@ static void fill_params(AttnParams& p, const void* q, const void* k, const void*
 
 template <typename T, bool SPARSE, int NW, bool BOUNDED, int PM = PM_NONE, bool NARROW = false, bool CUT = false>
 static int launch_d64(const AttnParams& p, int64_t nblocks, hipStream_t stream) {
-  const size_t smem = 4 * TILE64_BYTES + (PM == PM_KEYS || PM == PM_KEYBIAS ? NW * PM_SLOT_BYTES : 0);
+  const size_t smem = 4 * TILE64_BYTES + (PM == PM_KEYBIAS ? NW * PM_SLOT_BYTES : 0);
   static bool attr_done[PA_MAX_DEVICES] = {};  // benign race: the call is idempotent
   const int dev = current_device();
   if (dev < 0 || !attr_done[dev]) {
@@ -4931,7 +4943,7 @@ static int launch_pipe_variant(const AttnParams& p, hipStream_t stream) {
   int64_t nblocks = (int64_t)p.B * p.H * p.n_qtiles;
   if (p.split_s > 1) nblocks = (int64_t)p.split_main + (int64_t)p.split_tiles * p.split_s;
   if constexpr (D == 128) {
-    const size_t smem = 4 * TILE_BYTES + (PM == PM_KEYS || PM == PM_KEYBIAS ? NW * PM_SLOT_BYTES : 0);
+    const size_t smem = 4 * TILE_BYTES + (PM == PM_KEYBIAS ? NW * PM_SLOT_BYTES : 0);
     static bool attr_done[PA_MAX_DEVICES] = {};  // benign race: the call is idempotent
     const int dev = current_device();
     if (dev < 0 || !attr_done[dev]) {
