@@ -165,27 +165,33 @@ PA_API int pa_attn_fwd_narrow(const void* q, const void* k, const void* v, void*
  * a broadcast dimension.  A query row that keeps no key yields out = 0 and
  * lse = -inf.  Not causal (torch refuses a mask together with is_causal).
  *
- * A boolean mask that only selects keys (head and query strides 0: the text
+ * Masks without a query dimension (key padding, boolean or additive, also one
+ * per head) and additive masks with one run in the fast kernels, which read
+ * them as they go; boolean masks with a query dimension are packed to bits
+ * first, and key tiles that nothing keeps are left out.
+ * A boolean mask that is the same for every head and query row (the text
  * padding masks of src/para_attn/ops/__init__.py:248-299) is scanned on the
- * device; where it keeps a prefix of the keys in every batch element the fast
- * dense kernels run with the counts as kv_len (long launches whose prefixes
- * keep at least 7/8 of the keys everywhere: the kernel with resident
- * workgroups, which plain dense calls use).  Where it has holes (the mask of
- * the reference's sequence-parallel HunyuanVideo adapter, whose text padding
- * lies inside the gathered sequence:
- * context_parallel/diffusers_adapters/hunyuan_video.py:86-100) and the call
- * is one of 3e11 flop or more, the kept K and V rows are gathered into dense
- * copies in the workspace, as the reference's attention_forward_sparse_kv
- * does with index_select (ops/__init__.py:276-296), and the same kernels run
- * on the copies.  Smaller calls with such a mask, and additive masks, run in
- * the fast kernels too; so do boolean masks with a query dimension, packed to
- * bits first.  What is left (additive masks whose keys are not adjacent in
- * memory, K or V of 4 GiB and more per head, no room for the bits) runs a kernel
- * that reads the mask per score.  The choice is made on the device: nothing is
- * read back, so the call can be captured in a HIP graph.
- * workspace: pa_attn_fwd_masked_workspace_bytes() bytes (16-byte aligned, any
- * contents; from 3e11 flop on it includes the copies of K and V); null or
- * short is not an error: the per-score kernel runs where there is no room.
+ * device instead in calls of 3e11 flop and more, and where looking for its last
+ * kept key in every workgroup would take long (more than 37888 keys; 2560
+ * where they are not adjacent in memory): where it keeps a prefix of the keys
+ * in every batch element the fast dense kernels run with the counts as kv_len
+ * (long launches whose prefixes keep at least 7/8 of the keys everywhere: the
+ * kernel with resident workgroups, which plain dense calls use).  Where it has
+ * holes (the mask of the reference's sequence-parallel HunyuanVideo adapter,
+ * whose text padding lies inside the gathered sequence:
+ * context_parallel/diffusers_adapters/hunyuan_video.py:86-100) and the call is
+ * one of 3e11 flop or more, the kept K and V rows are gathered into dense
+ * copies in the workspace, as the reference's attention_forward_sparse_kv does
+ * with index_select (ops/__init__.py:276-296), and the same kernels run on the
+ * copies.  The choice is made on the device: nothing is read back, so the call
+ * can be captured in a HIP graph.
+ * A kernel that reads the mask per score takes what is left: additive masks
+ * with a query dimension whose keys are not adjacent in memory, K or V of 4 GiB
+ * and more per head, boolean masks with a query dimension and no room for the
+ * bits.
+ * workspace: pa_attn_fwd_masked_call_workspace_bytes() bytes (16-byte aligned,
+ * any contents); null or short is not an error: without room for them there
+ * are no bits, no scan, no gathered copies and no key split.
  */
 PA_API int pa_attn_fwd_masked(const void* q, const void* k, const void* v, void* out, float* lse,
                        int dtype, int B, int H, int Sq, int Skv, int D,

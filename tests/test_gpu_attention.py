@@ -513,10 +513,126 @@ def test_biases_with_a_query_dimension(cuda, D, Sq, Skv):
                 _check(out, lse, ref_out, ref_lse, f"{what} bias {shape} {dt}")
 
 
+def _every_mask(B, H, Sq, Skv, seed):
+    """name -> (mask, what it keeps [B|1,H|1,Sq|1,Skv], what it adds): every form a mask may take, small enough for the oracle."""
+    g = torch.Generator().manual_seed(seed)
+    pos = torch.arange(Skv)
+    prefix = (pos[None, :] < torch.tensor([Skv - 3, Skv // 3])[:B, None])[:, None, None, :]
+    holes = prefix & (pos % 7 != 3)
+    nothing = prefix.clone()
+    nothing[0] = False
+    rows = torch.rand(1, H, Sq, Skv, generator=g) < 0.4
+    rows[:, :, :, : Skv // 2] &= (torch.arange(Sq) >= Sq // 2)[:, None]
+    key_bias, row_bias = torch.randn(B, 1, 1, Skv, generator=g), torch.randn(1, H, Sq, Skv, generator=g)
+    row_bias[rows] = float("-inf")
+    row_bias[..., 0] = 0.5
+    return {"prefix": (prefix, prefix, None), "holes": (holes, holes, None), "nothing kept": (nothing, nothing, None),
+            "one per head": (rows[:, :, :1], rows[:, :, :1], None), "query dimension": (rows, rows, None),
+            "key bias": (key_bias, None, key_bias), "row bias": (row_bias, None, row_bias),
+            "16-bit row bias": (row_bias.bfloat16(), None, row_bias.bfloat16().float())}
+
+
+def _masked_oracle(q, k, v, keep, bias):
+    B, H, Sq, D = q.shape
+    if bias is None:
+        return oattn.sdpa_lse_f64(q.float().numpy(), k.float().numpy(), v.float().numpy(), None, np.broadcast_to(keep.numpy(), (B, H, Sq, k.shape[2])))
+    s = np.einsum("bhqd,bhkd->bhqk", q.double().numpy(), k.double().numpy()) / math.sqrt(D) + bias.double().numpy()
+    m = s.max(-1, keepdims=True)
+    p = np.exp(s - m)
+    return (p @ v.double().numpy()) / p.sum(-1, keepdims=True), (m + np.log(p.sum(-1, keepdims=True)))[..., 0]
+
+
+@pytest.mark.parametrize("D", [128, 64])
+@pytest.mark.parametrize("Sq,Skv", [(150, 333), (30, 8193)])
+def test_masks_in_the_kernels_without_offset_limits(cuda, tuning, D, Sq, Skv):
+    """The kernel that reads a mask per score, and the scan of key masks in front of it (one workgroup up to 8192 keys, chunks
+    beyond): what runs where the pipelined kernels do not take K and V, asked for by name."""
+    tuning("no_pipe", 1)
+    B, H = 2, 3
+    q, k, v = inputs.qkv(B, H, Sq, Skv, D, seed=Skv + D)
+    dev = [t.to(cuda) for t in (q, k, v)]
+    for name, (mask, keep, bias) in _every_mask(B, H, Sq, Skv, D).items():
+        out, lse = torch.ops.para_attn.attention_forward_with_lse(*dev, mask.to(cuda))
+        _check(out, lse, *_masked_oracle(q, k, v, keep, bias), name)
+
+
+def _masked_call(lib, q, k, v, mask, nbytes):
+    """pa_attn_fwd_masked with a workspace of nbytes, all ones in it and behind it (None: no workspace)."""
+    B, H, Sq, D = q.shape
+    Skv = k.shape[2]
+    out, lse = torch.empty_like(q), torch.empty(B, H, Sq, device=q.device)
+    kind = 1 if mask.dtype == torch.bool else 2 if mask.dtype == torch.float32 else 3
+    strides = (ctypes.c_int64 * 4)(*mask.expand(B, H, Sq, Skv).stride())
+    ws = torch.full(((nbytes or 0) + 256,), 255, dtype=torch.uint8, device=q.device)
+    rc = lib.pa_attn_fwd_masked(*(t.data_ptr() for t in (q, k, v, out, lse)), 0, B, H, Sq, Skv, D, *(_lib.strides3(t) for t in (q, k, v, out)),
+                                1.0 / math.sqrt(D), mask.data_ptr(), kind, strides, None if nbytes is None else ws.data_ptr(), nbytes or 0,
+                                torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, lib.pa_last_error()
+    assert (ws[nbytes or 0 :] == 255).all(), "written behind the workspace"
+    return out, lse
+
+
+@pytest.mark.parametrize("D", [128, 64])
+def test_masked_entry_with_little_or_no_workspace(cuda, D):
+    """pa_attn_fwd_masked with no workspace, one byte less than the call asks for, and what it asks for: every form of a mask
+    gives the oracle's result with each, and nothing behind the workspace is written."""
+    lib = _lib.load()
+    B, H, Sq, Skv = 2, 3, 150, 333
+    q, k, v = inputs.qkv(B, H, Sq, Skv, D, seed=D)
+    dev = [t.to(cuda) for t in (q, k, v)]
+    for name, (mask, keep, bias) in _every_mask(B, H, Sq, Skv, D).items():
+        ref = _masked_oracle(q, k, v, keep, bias)
+        md = mask.to(cuda)
+        kind = 1 if mask.dtype == torch.bool else 2 if mask.dtype == torch.float32 else 3
+        need = lib.pa_attn_fwd_masked_call_workspace_bytes(B, H, Sq, Skv, D, _lib.strides3(dev[1]), _lib.strides3(dev[2]), kind,
+                                                           (ctypes.c_int64 * 4)(*md.expand(B, H, Sq, Skv).stride()))
+        for nbytes in (None, 16, need - 1, need):
+            _check(*_masked_call(lib, *dev, md, nbytes), *ref, f"{name}, workspace {nbytes} of {need}")
+
+
+@pytest.mark.parametrize("D", [128, 64])
+def test_large_key_masks_without_room_for_the_gather(cuda, D):
+    """A call of 3e11 flop whose workspace holds the scan's words but not the copies of K and V: a prefix runs the dense kernels
+    behind the scan, a mask with holes the kernel behind them that the flag lets run, which may use what is left of
+    the workspace; without one the mask is looked at in the kernel.  A batch element that keeps nothing included."""
+    lib = _lib.load()
+    B, H, Sq, Skv = 2, 8 * 128 // D, 6300, 6311
+    q, k, v = inputs.qkv(B, H, Sq, Skv, D, seed=D)
+    dev = [t.to(cuda) for t in (q, k, v)]
+    assert 4.0 * B * H * Sq * Skv * D >= 3e11
+    ks, vs = _lib.strides3(dev[1]), _lib.strides3(dev[2])
+    need = lib.pa_attn_fwd_masked_workspace_bytes(B, H, Sq, Skv, D, ks, vs)
+    rows = torch.cat([torch.arange(0, 40), torch.arange(Sq - 40, Sq)])
+    heads = [0, H - 1]
+    pos = torch.arange(Skv)
+    for name, m in (("prefix", pos[None, :] < torch.tensor([Skv - 100, 700])[:, None]), ("holes", (pos % 5 != 2)[None, :].repeat(B, 1)),
+                    ("nothing", torch.stack([pos < 0, pos % 5 != 2]))):
+        mask = m[:, None, None, :].to(cuda)
+        ref = oattn.sdpa_lse_f64(q[:, heads][:, :, rows].float().numpy(), k[:, heads].float().numpy(), v[:, heads].float().numpy(), None, m[:, None, None, :].numpy())
+        for nbytes in (None, 4096, need // 4, need):
+            out, lse = _masked_call(lib, *dev, mask, nbytes)
+            _check(out[:, heads][:, :, rows.to(cuda)], lse[:, heads][:, :, rows.to(cuda)], *ref, f"{name}, workspace {nbytes} of {need}")
+
+
+def test_masks_with_key_rows_spread_over_4gib(cuda):
+    """K and V beyond the pipelined kernels' 32-bit offsets, under every form of a mask."""
+    B, H, Sq, Skv, D = 1, 1, 130, 4100, 128
+    q, k, v = inputs.qkv(B, H, Sq, Skv, D, seed=37)
+    stride = 1 << 19  # elements between consecutive key rows
+    big = torch.empty(2, Skv * stride, dtype=torch.bfloat16, device=cuda)
+    kd, vd = (big[i].as_strided((B, H, Skv, D), (0, 0, stride, 1)).copy_(t) for i, t in enumerate((k, v)))
+    for name, (mask, keep, bias) in _every_mask(B, H, Sq, Skv, D).items():
+        out, lse = torch.ops.para_attn.attention_forward_with_lse(q.to(cuda), kd, vd, mask.to(cuda))
+        _check(out, lse, *_masked_oracle(q, k, v, keep, bias), name)
+    del big, kd, vd
+    torch.cuda.empty_cache()
+
+
 def test_key_masks_take_the_fast_kernels_when_prefixes(cuda, tuning):
-    """A key-only boolean mask is scanned on the device: prefixes run the dense kernels with per-batch key counts
-    (here with the key-split tail and the score bound in play), anything else the per-score kernel; both give the
-    oracle's result and neither reads the mask on the host."""
+    """A key-only boolean mask below 3e11 flop: adjacent keys are looked at in the pipelined kernel; keys that lie apart (2597 of
+    them, too many steps for that) are scanned on the device, prefixes run the dense kernels with per-batch key
+    counts (here with the key-split tail and the score bound in play), masks with holes the pipelined kernel behind
+    the scan.  All give the oracle's result and none reads the mask on the host."""
     tuning("bound", 1)
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     B, H, D = 2, 4, 128
@@ -531,9 +647,12 @@ def test_key_masks_take_the_fast_kernels_when_prefixes(cuda, tuning):
     rows = torch.cat([torch.arange(0, 30), torch.arange(Sq - 300, Sq, 7)])
     for name, m in (("prefix", prefix), ("scattered", scattered)):
         ref_out, ref_lse = oattn.sdpa_lse_f64(q[:, :, rows].float().numpy(), k.float().numpy(), v.float().numpy(), None, m[:, None, None, :].numpy())
-        out, lse = torch.ops.para_attn.attention_forward_with_lse(qd, kd, vd, m[:, None, None, :].to(cuda))
-        _check(out[:, :, rows.to(cuda)], lse[:, :, rows.to(cuda)], ref_out, ref_lse, name)
-        assert torch.isfinite(lse).all()
+        adjacent = m[:, None, None, :].to(cuda)
+        apart = torch.zeros(B, 1, 1, Skv, 2, dtype=torch.bool, device=cuda)[..., 0].copy_(adjacent)
+        for mask in (adjacent, apart):
+            out, lse = torch.ops.para_attn.attention_forward_with_lse(qd, kd, vd, mask)
+            _check(out[:, :, rows.to(cuda)], lse[:, :, rows.to(cuda)], ref_out, ref_lse, name)
+            assert torch.isfinite(lse).all()
 
 
 @pytest.mark.parametrize("rounds", [-1, 6])
@@ -594,8 +713,8 @@ def test_long_launches_with_nearly_full_key_masks(cuda, rounds, tuning):
 @pytest.mark.parametrize("Sq,Skv", [(150, 333), (9000, 9011)])
 def test_key_masks_that_keep_nothing_in_one_batch_element(cuda, Sq, Skv):
     """A key mask that drops every key of one batch element (out = 0, LSE = -inf there, the oracle's convention), as a
-    prefix of length 0 and, with a hole in the other element, as a mask with holes; at a small size (the per-score
-    kernel for the mask with holes) and at one where the kept keys are gathered."""
+    prefix of length 0 and, with a hole in the other element, as a mask with holes; at a small size (the mask is
+    looked at in the pipelined kernel) and at one where the kept keys are gathered."""
     B, H, D = 2, 8, 128
     q, k, v = inputs.qkv(B, H, Sq, Skv, D, seed=61)
     qd, kd, vd = q.to(cuda), k.to(cuda), v.to(cuda)

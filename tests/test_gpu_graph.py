@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 def _eager(q, kb, vb, prev, cur, key_mask, block_mask):
     out, lse = torch.ops.para_attn.attention_forward_with_lse(q, kb[0], vb[0])
-    # masked calls: whether the key mask is a prefix is decided on the device, inside the captured work
+    # masked calls: where the mask ends, and whether it has holes, is found out on the device, inside the captured work
     mo, ml = torch.ops.para_attn.attention_forward_with_lse(q, kb[0], vb[0], key_mask)
     so = torch.ops.para_attn.attention_forward_sparse_kv(q, kb[0], vb[0], key_mask.expand(-1, -1, q.shape[2], -1))
     ro, rl = paraattention_amd.ring_sweep(q, kb, vb, fused=True)
@@ -43,7 +43,7 @@ def test_graph_replays_match_eager(cuda, tuning):
     block_mask = (torch.rand(8, 20, generator=torch.Generator().manual_seed(3)) < 0.5).to(cuda)  # 128-row x 128-key blocks
     _eager(q, kb, vb, prev, cur, key_mask, block_mask)  # warm-up outside capture (library load, function attributes)
     key_mask[..., 5] = False
-    _eager(q, kb, vb, prev, cur, key_mask, block_mask)  # and the per-score kernel's
+    _eager(q, kb, vb, prev, cur, key_mask, block_mask)  # and with a hole in the mask
     key_mask[..., 5] = True
     torch.cuda.synchronize()
     side = torch.cuda.Stream()
