@@ -305,13 +305,7 @@ __global__ __launch_bounds__(FB_THREADS) void fbcache_residual_kernel(
   if constexpr (HAVE_PREV) finish<DT>(sd, sa, (double)n, ws, ratio_out, stats_out);
 }
 
-// What follows the cached blocks reads the result at once, so it is left in the caches where they hold it beside the
-// operands: up to FB_STREAM_BYTES.  apply and a layer norm behind it, 4608 x 3072 bf16 35.1 -> 31.6 us, 17776 x 3072
-// 114.8 -> 96.5 (apply alone 52.0 and 50.4); at 32760 x 5120 336 streamed, 340 not (apply alone 162.6, 170.1).  The residual
-// is next read a whole step later and streams at every size.
-constexpr int64_t FB_STREAM_BYTES = (int64_t)128 << 20;
-
-template <int DT, bool STREAM>
+template <int DT>
 __global__ __launch_bounds__(FB_THREADS) void fbcache_apply_kernel(const void* resid, const void* hidden,
                                                                   void* out, int64_t n) {
   constexpr int VEC = Act<DT>::VEC;
@@ -320,10 +314,6 @@ __global__ __launch_bounds__(FB_THREADS) void fbcache_apply_kernel(const void* r
   u32x4* ov = (u32x4*)out;
   const int64_t n_vec = n / VEC;
   const int64_t stride = (int64_t)gridDim.x * FB_THREADS;
-  auto put = [&](int64_t at, const u32x4& x) {
-    if constexpr (STREAM) __builtin_nontemporal_store(x, ov + at);
-    else ov[at] = x;
-  };
   int64_t i = (int64_t)blockIdx.x * FB_THREADS + threadIdx.x;
   for (; i + (FB_UNROLL - 1) * stride < n_vec; i += FB_UNROLL * stride) {
     u32x4 r[FB_UNROLL], h[FB_UNROLL];
@@ -333,10 +323,10 @@ __global__ __launch_bounds__(FB_THREADS) void fbcache_apply_kernel(const void* r
       h[u] = __builtin_nontemporal_load(hv + i + u * stride);
     }
 #pragma unroll
-    for (int u = 0; u < FB_UNROLL; ++u) put(i + u * stride, combine_vec<DT, false>(r[u], h[u]));
+    for (int u = 0; u < FB_UNROLL; ++u) __builtin_nontemporal_store(combine_vec<DT, false>(r[u], h[u]), ov + i + u * stride);
   }
   for (; i < n_vec; i += stride)
-    put(i, combine_vec<DT, false>(__builtin_nontemporal_load(rv + i), __builtin_nontemporal_load(hv + i)));
+    __builtin_nontemporal_store(combine_vec<DT, false>(__builtin_nontemporal_load(rv + i), __builtin_nontemporal_load(hv + i)), ov + i);
   if (blockIdx.x == 0 && threadIdx.x < (int)(n - n_vec * VEC)) {
     const int64_t j = n_vec * VEC + threadIdx.x;
     const float s = Act<DT>::round1(Act<DT>::load1(resid, j) + Act<DT>::load1(hidden, j));
@@ -447,10 +437,7 @@ extern "C" int pa_fbcache_apply_residual(const void* resid, const void* hidden, 
   hipStream_t s = (hipStream_t)stream;
   FB_DISPATCH(dtype, {
     const int grid = fb_grid(n / Act<DT>::VEC / 2);
-    if (n * (int64_t)elem_size(dtype) > FB_STREAM_BYTES)
-      hipLaunchKernelGGL((fbcache_apply_kernel<DT, true>), dim3(grid), dim3(FB_THREADS), 0, s, resid, hidden, out, n);
-    else
-      hipLaunchKernelGGL((fbcache_apply_kernel<DT, false>), dim3(grid), dim3(FB_THREADS), 0, s, resid, hidden, out, n);
+    hipLaunchKernelGGL(fbcache_apply_kernel<DT>, dim3(grid), dim3(FB_THREADS), 0, s, resid, hidden, out, n);
   });
   PA_CHECK_LAUNCH("fbcache apply kernel");
   return PA_OK;
