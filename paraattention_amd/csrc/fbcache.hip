@@ -251,9 +251,13 @@ __device__ __forceinline__ u32x4 combine_vec(const u32x4& a, const u32x4& b) {
 }
 
 // The two kernels below are bound by HBM.  Four vectors of every operand in flight per thread and streaming stores, one
-// workgroup per CU: at 32760 x 5120 bf16 resid against prev 266 -> 215 us (6.2 TB/s), apply 233 -> 161 us (6.2 TB/s;
-// one vector at a time kept 2 MB of loads in flight on the whole chip).  Two to sixteen workgroups per CU are slower
-// (179 .. 240 us apply), as are eight vectors (162) and larger workgroups.
+// workgroup per CU: at 32760 x 5120 bf16 the call with resid against prev 280 -> 235 us (5.7 TB/s), apply 231 -> 162 us
+// (6.2 TB/s; one vector at a time kept 2 MB of loads in flight on the whole chip).  Two to sixteen workgroups per CU are
+// slower (179 .. 240 us apply), as are eight vectors (162) and larger workgroups.
+// Streaming stores cost what reads the result next: apply with a layer norm behind it takes 35.1 us at 4608 x 3072 and 114.8 at
+// 17776 x 3072, with cacheable stores 31.6 and 96.3 (37.5 and 121.9 before the four vectors).  But a result left in the
+// caches pushes out what a down-sampled comparison reads there: cached steps with every second column compared,
+// 6000 x 5120 to 12000 x 5120, take 1 .. 4 % longer, and beyond 128 MiB apply itself does (170 us).
 constexpr int FB_UNROLL = 4;
 
 // resid = hidden - hidden0 (rounded, stored); reduction against prev if given.

@@ -110,3 +110,17 @@ def test_fused_first_block_step(cuda, dtype):
         fbcache.set_first_hidden_states_residual(prev.to(cuda))
         r2, hit2 = fbcache.first_block_step(h.to(cuda), h0.to(cuda))
         assert hit2 is (want < 0.12)
+
+
+@pytest.mark.parametrize("n", [4 * 65536 * 8 - 1, 4 * 65536 * 8, 5 * 65536 * 8 + 13, (64 << 20), (64 << 20) + 1])
+def test_residual_and_apply_at_the_edges_of_their_loops(cuda, n):
+    """Four vectors per thread and step on a full grid (256 workgroups of 256 threads), the step that ends early, a remainder that
+    fills no vector, and 128 MiB with and without one: bit for bit what torch gives."""
+    g = torch.Generator(device=cuda).manual_seed(n % 1000)
+    h, h0, prev = (torch.randn(1, n, generator=g, device=cuda, dtype=torch.bfloat16) for _ in range(3))
+    resid, ratio = torch.ops.para_attn.fbcache_first_residual_diff(h, h0, prev)
+    assert torch.equal(resid, h - h0)
+    assert torch.equal(torch.ops.para_attn.fbcache_apply_residual(resid, h), resid + h)
+    if n < 1 << 22:
+        want, _, _ = ofb.residual_diff_ratio(prev.float().cpu().numpy(), resid.float().cpu().numpy())
+        assert ratio.item() == want
