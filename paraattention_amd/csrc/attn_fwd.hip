@@ -604,7 +604,8 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_fwd_kernel(const AttnParams 
 // nothing beyond the vote that says so.  Measured against the per-score kernel (attn_fwd_kernel<MASK>, register-staged
 // tiles): two samples x 24 heads x 7800 rows against 256 keys with a bias 171 -> 104 us (0.47 PFLOP/s; bound by what a
 // workgroup does around its four key tiles), 24 heads x 4352 tokens with holes in the key mask, scan and two empty
-// launches included there, 390..545 -> 236 us (0.98 PFLOP/s, what the unmasked call of that size reaches); three packed samples
+// launches included there, 390..700 -> 236 us (0.98 PFLOP/s, what the unmasked call of that size reaches, and what a mask that
+// keeps a prefix took before, in the fast kernels behind the scan); three packed samples
 // behind a common prefix, 2 x 24 heads x 8000 tokens 6.65 -> 0.88 ms, 16 heads x 3000 326 -> 94 us (about half the key tiles
 // are kept by no row of a query tile there; the rest is the packed words instead of a byte load per score).
 // The element of tile j + 2 is fetched while tile j + 1 is masked, so its latency is covered by the wait for the
@@ -4353,7 +4354,8 @@ static void choose_kernel(AttnParams& p, int D, int q_block, bool dense, size_t 
   const int n_cus = device_cus();
   // is_causal: workgroups differ in length.  Where the query tiles of one head do not fill the chip the heads are the
   // fastest grid index, so that the longest workgroups of all heads start first; in the order of the heads the last
-  // heads' longest ones start when the rest is done (24 heads x 4096 tokens, head_dim 64: 97 -> 76 us; head_dim 128 160 -> 110 us, 12 heads x 16384 tokens 912 -> 792).  Where they do,
+  // heads' longest ones start when the rest is done (24 heads x 4096 tokens, head_dim 64: 97 -> 76 us; head_dim 128 160 -> 106 us,
+  // 12 heads x 16384 tokens 912 -> 792, 40 x 16000 2444 -> 2289, 40 x 27000 6895 -> 6565).  Where they do, from 65536 rows on,
   // the order of the heads keeps the resident workgroups on one head's K and V.
   auto order = [&] {
     finish();
@@ -4403,7 +4405,9 @@ static void choose_kernel(AttnParams& p, int D, int q_block, bool dense, size_t 
   double r128 = p128.rounds, r256 = p256.rounds;
   if (cus > 0 && p128.s == 1 && n128 % (2 * cus) != 0 && n128 % (2 * cus) <= cus) r128 -= 0.33;
   // measured throughput of a full round of 256-row workgroups against one of 128-row workgroups:
-  // +4..10 % from 4608 keys up, -4 % at 512 keys
+  // +4..10 % from 4608 keys up, -4 % at 512 keys; the instance for 96 columns gains 1 .. 2.5 % from 4096 to 30000 tokens (2 x 16
+  // heads x 4096, head_dim 72: 191.5 against 193.8 us) and loses up to 6 at 1200 to 2500 (2 x 16 x 2500, head_dim 88, where the
+  // merge's price then tips the choice: 99.5 against 93.7)
   const double gain256 = !mi355x_layout() ? 1.0 : kv_tiles >= 32 ? 1.055 : 0.95;
   bool use256 = cus > 0 && n256 >= cus && r256 / gain256 < r128;
   // is_causal: workgroups differ in length and are started longest first, so whole rounds mean nothing; measured
