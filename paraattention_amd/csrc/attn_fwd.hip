@@ -9,6 +9,7 @@
 //   attn_fwd_d128_stream_kernel  the same pipeline, resident workgroups over a list of pieces (the dense default)
 //   attn_fwd_d128_short_kernel   the same pipeline for 449..512 keys per head (cross-attention to a text prompt)
 //   attn_fwd_d64_pipe_kernel   head_dim 64, the same pipeline (the default)
+// (attn_resident.hip holds another one, for keys that fit into LDS as a whole.)
 //
 // Both GEMMs run transposed so that the softmax needs no cross-lane traffic and
 // P never leaves registers:
@@ -38,6 +39,7 @@
 #include <atomic>
 #include <type_traits>
 
+#include "attn_resident.h"
 #include "pa_common.h"
 
 namespace pa {
@@ -4262,8 +4264,9 @@ static SplitPlan plan_split(int64_t n_tiles, int slots, int kv_tiles, int bm, bo
 //   PARAATTN_WAVE_ROWS=64    "wave_rows"     the resident-workgroup kernel as 4 wavefronts of 64 query rows instead of 8 of 32
 //   PARAATTN_SPARSE_ORDER=0  "sparse_order"  block-sparse: 0 = the query blocks of a head in their own order instead of longest list first
 //   PARAATTN_SHORT_KEYS=0|1  "short_keys"    never / wherever it applies the kernel for 449..512 keys (-1 = by the number of pieces)
+//   PARAATTN_RESIDENT=0|1    "resident"      never / wherever it applies the kernel that keeps all keys in LDS (-1 = by size)
 struct Tuning {
-  std::atomic<int> no_pipe, no_split, no_xcd_order, forced_bm, bound, stream, stream_even, stream_dyn, stream_solo, sparse_pair, wave_rows, short_keys, sparse_order;
+  std::atomic<int> no_pipe, no_split, no_xcd_order, forced_bm, bound, stream, stream_even, stream_dyn, stream_solo, sparse_pair, wave_rows, short_keys, sparse_order, resident;
 };
 static Tuning& tuning() {
   static Tuning t;
@@ -4290,6 +4293,8 @@ static Tuning& tuning() {
     const int sk = num("PARAATTN_SHORT_KEYS", -1);
     t.short_keys = sk == 0 || sk == 1 ? sk : -1;
     t.sparse_order = num("PARAATTN_SPARSE_ORDER", 1) != 0;
+    const int rs = num("PARAATTN_RESIDENT", -1);
+    t.resident = rs == 0 || rs == 1 ? rs : -1;
     return true;
   }();
   (void)init;
@@ -4314,6 +4319,7 @@ extern "C" int pa_set_tuning(const char* name, int value) {
   else if (!strcmp(name, "wave_rows")) t.wave_rows = value == 64 ? 64 : 0;
   else if (!strcmp(name, "short_keys")) t.short_keys = value == 0 || value == 1 ? value : -1;
   else if (!strcmp(name, "sparse_order")) t.sparse_order = value != 0;
+  else if (!strcmp(name, "resident")) t.resident = value == 0 || value == 1 ? value : -1;
   else PA_FAIL(PA_ERR_INVALID, "pa_set_tuning: unknown knob '%s'", name);
   return PA_OK;
 }
@@ -4639,6 +4645,24 @@ static int launch_short(const AttnParams& p, hipStream_t stream) {
   return PA_OK;
 }
 
+// The call as the kernel that keeps all keys in LDS takes it (attn_resident.hip), for a dense call or one with an additive
+// mask that has no query dimension.  Asking for another kernel by knob switches it off.
+static bool plan_resident_call(const AttnParams& p, int D, ResidentCall& c) {
+  int want = tuning().resident;
+  if (tuning().no_pipe || p.causal || p.kv_len != nullptr || p.gate != nullptr) return false;
+  if (want < 0 && (tuning().forced_bm != 0 || tuning().stream == 1 || tuning().short_keys == 1)) return false;
+  c.q = p.q; c.k = p.k; c.v = p.v; c.out = p.out; c.lse = p.lse;
+  c.B = p.B; c.H = p.H; c.Sq = p.Sq; c.Skv = p.Skv;
+  c.qs_b = p.qs_b; c.qs_h = p.qs_h; c.qs_s = p.qs_s;
+  c.ks_b = p.ks_b; c.ks_h = p.ks_h; c.ks_s = p.ks_s;
+  c.vs_b = p.vs_b; c.vs_h = p.vs_h; c.vs_s = p.vs_s;
+  c.os_b = p.os_b; c.os_h = p.os_h; c.os_s = p.os_s;
+  c.scale_log2 = p.scale_log2;
+  c.bias = p.mask; c.ms_b = p.ms_b; c.ms_h = p.ms_h; c.ms_k = p.ms_k;
+  c.bias_act = p.mask_kind == MASK_ACT;
+  return plan_resident(c, D, want);
+}
+
 template <typename T, int RB, bool KVLEN>
 static int launch_stream_rb(const AttnParams& p, hipStream_t stream) {
   const size_t smem = 4 * TILE_BYTES + 8 * 8192 + 16;  // two K and two V tiles, a staging area for outputs, two words
@@ -4746,6 +4770,8 @@ static int attn_fwd_dense(const void* q, const void* k, const void* v, void* out
   p.causal = is_causal != 0;
   p.gate = gate;
   p.gate_mask = gate_mask;
+  ResidentCall rcall;
+  if (!accumulate && !segs && plan_resident_call(p, D, rcall)) return launch_resident(rcall, dtype, D, (hipStream_t)stream);
   if (!accumulate && !segs && plan_short(p, D))
     return dtype == PA_DTYPE_BF16 ? launch_short<BF16>(p, (hipStream_t)stream) : launch_short<F16>(p, (hipStream_t)stream);
   const size_t ws_avail = workspace ? workspace_bytes : 0;
@@ -4891,6 +4917,8 @@ static size_t dense_ws_need(int B, int H, int Sq, int Skv, int D, const int64_t 
     fill_params(p, nullptr, nullptr, nullptr, nullptr, nullptr, B, H, Sq, Skv, zero, k_strides, v_strides, zero, 1.f);
     p.causal = plan == 2;
     size_t need = 0;
+    ResidentCall rcall;
+    if (plan == 0 && plan_resident_call(p, D, rcall)) continue;  // takes none
     if (plan != 0 || !plan_stream(p, D, nullptr, 0, true, &need, allow_drawn)) {
       need = 0;
       choose_kernel(p, D, 256, true, 0, &need);
@@ -5225,6 +5253,8 @@ extern "C" int pa_attn_fwd_masked(const void* q, const void* k, const void* v, v
   // instead, where a mask with holes costs what its kept keys cost and the resident-workgroup kernel may serve it.
   const bool no_query_dim = any && (Sq == 1 || p.ms_q == 0);
   auto masked_pipe = [&](void* ws, size_t ws_bytes) {
+    ResidentCall rcall;
+    if (mask_kind != MASK_BOOL && plan_resident_call(p, D, rcall)) return launch_resident(rcall, dtype, D, st);
     choose_kernel(p, D, 256, true, ws ? ws_bytes : 0, nullptr);
     if (p.split_s > 1) lend_split_ws(p, ws);
     if (dtype == PA_DTYPE_BF16) return D == 128 ? launch_masked_pipe<BF16, 128>(p, st) : launch_masked_pipe<BF16, 64>(p, st);

@@ -1061,6 +1061,67 @@ def test_short_key_kernel(cuda, dtype, tuning):
         assert torch.equal(out_d, want[0]) and torch.equal(lse_d, want[1]), (B, H, Sq, Skv)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D,most,most_biased", [(128, 288, 256), (64, 576, 512)])
+def test_resident_key_kernel(cuda, dtype, D, most, most_biased, tuning):
+    """The kernel that keeps all keys of a head in LDS, forced on: one key, one and several tiles of 64 keys, a last tile of 32,
+    ragged ones, the most keys it takes; query rows in parts of a 32-row block, fewer blocks than wavefronts and several
+    workgroups per head; both memory layouts; additive masks per batch element and per head.  Against the fp64 oracle, and
+    within rounding of the kernels that stream their keys."""
+    op = torch.ops.para_attn.attention_forward_with_lse
+    for Skv in (1, 31, 33, 64, 65, 96, 129, 257, most_biased, most):
+        for Sq in (1, 45, 300, 1061):
+            B, H = (2, 3) if Sq < 1000 else (1, 2)
+            q, k, v = inputs.qkv(B, H, Sq, Skv, D, seed=Sq + Skv, dtype=dtype)
+            dev = [t.to(cuda) if Sq % 2 else t.to(cuda).transpose(1, 2).contiguous().transpose(1, 2) for t in (q, k, v)]
+            g = torch.Generator().manual_seed(Skv)
+            pad = (torch.arange(Skv)[None] >= torch.tensor([max(1, Skv // 3), Skv])[:B, None])[:, None, None, :]
+            for mask in (None, pad.to(dtype) * -10000.0, torch.randn(1, H, 1, Skv, generator=g)):
+                m = None if mask is None else mask.to(cuda)
+                tuning("resident", 1)
+                out, lse = op(*dev, m)
+                tuning("resident", 0)
+                out0, lse0 = op(*dev, m)
+                qn, kn = q.double().numpy(), k.double().numpy()
+                if mask is not None:  # a bias per key is one more column of the keys
+                    bias = np.broadcast_to(mask.double().numpy()[:, :, 0, :, None], (B, H, Skv, 1))
+                    qn, kn = np.concatenate([qn, np.full((B, H, Sq, 1), math.sqrt(D))], -1), np.concatenate([kn, bias], -1)
+                ref_out, ref_lse = oattn.sdpa_lse_f64(qn, kn, v.double().numpy(), 1.0 / math.sqrt(D))
+                _check(out, lse, ref_out, ref_lse, f"resident keys {(B, H, Sq, Skv, D, dtype, None if mask is None else mask.shape)}")
+                assert (out.float() - out0.float()).abs().max().item() <= 2e-2 and (lse - lse0).abs().max().item() <= 1e-4
+
+
+@pytest.mark.parametrize("where", ["padding", "-inf", "lowest", "nan key", "nan value", "inf value", "inf key", "nan bias", "all lowest", "all -inf",
+                                   "first keys", "large scores"])
+@pytest.mark.parametrize("D", [128, 64])
+def test_resident_key_kernel_leaves_out_only_zeros(cuda, D, where, tuning):
+    """Key tiles so far below the others that their probabilities are zero are not computed; what a NaN or an infinity in them
+    does to a row, and masks of the type's lowest value, come out as in the kernels that compute them."""
+    B, H, Sq, Skv = 2, 2, 200, 256
+    for dtype in (torch.bfloat16, torch.float32):
+        q, k, v = (t.to(cuda) for t in inputs.qkv(B, H, Sq, Skv, D, seed=7))
+        pad = torch.arange(Skv, device=cuda)[None] >= torch.tensor([[40], [100]], device=cuda)
+        low = torch.finfo(dtype).min
+        m = torch.zeros(B, Skv, device=cuda, dtype=dtype).masked_fill(pad, {"-inf": -math.inf, "lowest": low}.get(where, -10000.0))[:, None, None, :]
+        if where == "nan key": k[0, 0, Skv - 1, 3] = math.nan
+        if where == "nan value": v[0, 0, Skv - 1, 3] = math.nan
+        if where == "inf value": v[0, 1, Skv - 2, 5] = math.inf
+        if where == "inf key": k[0, 1, Skv - 2, 5] = math.inf
+        if where == "nan bias": m[0, 0, 0, Skv - 1] = math.nan
+        if where == "all lowest": m[0] = low
+        if where == "all -inf": m[0] = -math.inf
+        if where == "first keys": m = m.flip(-1)
+        if where == "large scores": q, k = q * 60, k * 40  # scores reach across the padding
+        got = {}
+        for knob in (0, 1):
+            tuning("resident", knob)
+            got[knob] = torch.ops.para_attn.attention_forward_with_lse(q, k, v, m)
+        for a, b in zip(got[0], got[1]):
+            assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isinf(), b.isinf()), (where, dtype)
+            ok = a.isfinite()
+            assert torch.allclose(a[ok].float(), b[ok].float(), atol=2e-2, rtol=2e-2), (where, dtype)
+
+
 @pytest.mark.parametrize("scale", [1.0, 0.3])
 def test_short_key_kernel_large_logits(cuda, scale, tuning):
     """Logits of a few hundred through the kernel for short key sequences: the running maximum rises from tile to

@@ -63,3 +63,10 @@ def test_unsplit_head_dim_64_kernels_pay_nothing_for_the_split(kernels, T):
             name = f"attn_fwd_d64_pipe_kernelINS_{T}ELb0ELi{wavefronts}ELb{bounded}ELi0ELb0ELb%dEEEv"
             whole, cut = (next(k[".sgpr_spill_count"] for n, k in kernels.items() if name % c in n) for c in (0, 1))
             assert whole <= 24 and whole < cut, (name, whole, cut)
+
+
+def test_resident_key_kernels_spill_nothing(kernels):
+    resident = {n: k for n, k in kernels.items() if "attn_fwd_resident_kernel" in n}
+    assert len(resident) == 12  # two types, two head_dims; unmasked with a last tile of 64 or 32 keys, and with a bias
+    for n, k in resident.items():
+        assert not k[".vgpr_spill_count"] and not k[".sgpr_spill_count"] and not k[".private_segment_fixed_size"], n
