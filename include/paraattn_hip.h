@@ -435,12 +435,28 @@ PA_API int pa_fbcache_residual_ratio(const void* hidden, const void* hidden0, co
                               void* ratio_out, float* stats_out,
                               void* workspace, size_t workspace_bytes, void* stream);
 
+/* Only the residual; inf_out, where given, is one element of the type that becomes +inf (the ratio of a step without a previous one). */
+PA_API int pa_fbcache_residual(const void* hidden, const void* hidden0, void* resid_out, int dtype, int64_t n, void* inf_out, void* stream);
+
+/*
+ * pa_fbcache_residual_ratio against a down-sampled previous residual (src/para_attn/first_block_cache/utils.py:276-278, 289-295): hidden, hidden0 and
+ * resid_out are n_rows x row_len, prev is the contiguous n_rows x (row_len / step) tensor of every step-th column.  step: 2, 4 or 8 (fp32: 2
+ * or 4), row_len a multiple of 8 (fp32: 4); PA_ERR_UNSUPPORTED otherwise.
+ */
+PA_API int pa_fbcache_residual_ratio_strided(const void* hidden, const void* hidden0, const void* prev, void* resid_out, int dtype,
+                                             int64_t n_rows, int64_t row_len, int step, void* ratio_out, float* stats_out,
+                                             void* workspace, size_t workspace_bytes, void* stream);
+
 /*
  * Cache-hit path: out = resid + hidden (src/para_attn/first_block_cache/utils.py:237-259),
  * contiguous, n elements, rounded to dtype.  out may alias hidden.
  */
 PA_API int pa_fbcache_apply_residual(const void* resid, const void* hidden, void* out, int dtype,
                               int64_t n, void* stream);
+
+/* The same for two tensors of one type in one launch (hidden states and the text stream); neither may be empty. */
+PA_API int pa_fbcache_apply_residual2(const void* resid, const void* hidden, void* out, int64_t n, const void* resid2, const void* hidden2,
+                                      void* out2, int64_t n2, int dtype, void* stream);
 
 /*
  * TaylorSeer finite differences (src/para_attn/first_block_cache/taylorseer.py:29-38,

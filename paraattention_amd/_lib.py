@@ -102,6 +102,9 @@ SIGNATURES = {
     ),
     "pa_fbcache_workspace_bytes": (_sz, []),
     "pa_fbcache_residual_ratio": (_i, [_vp, _vp, _vp, _vp, _i, _i64, _vp, _vp, _vp, _sz, _vp]),
+    "pa_fbcache_residual": (_i, [_vp, _vp, _vp, _i, _i64, _vp, _vp]),
+    "pa_fbcache_residual_ratio_strided": (_i, [_vp, _vp, _vp, _vp, _i, _i64, _i64, _i, _vp, _vp, _vp, _sz, _vp]),
+    "pa_fbcache_apply_residual2": (_i, [_vp, _vp, _vp, _i64, _vp, _vp, _vp, _i64, _i, _vp]),
     "pa_fbcache_apply_residual": (_i, [_vp, _vp, _vp, _i, _i64, _vp]),
 }
 

@@ -271,15 +271,18 @@ def first_block_step(hidden_states, original_hidden_states, parallelized=False):
     """Residual of the first block plus the cache decision in one pass over memory
     (utils.py:359-366: ``hidden - original``, ``mark_step_begin``, ``get_can_use_cache``).
 
-    Returns (first_hidden_states_residual, can_use_cache).  Falls back to the
-    two-step form when down-sampling is on, since the stored residual then has
-    another shape than the fresh one.
+    Returns (first_hidden_states_residual, can_use_cache).  Takes the two-step form where the
+    stored residual has another shape than the fresh one; one down-sampled by a step
+    that divides the kernel's vectors is compared in the same pass too.
     """
     ctx = _ctx()
     ctx.mark_step_begin()
     threshold = ctx.get_residual_diff_threshold()
     gated = ctx.is_in_warmup() or threshold <= 0.0
     prev = None if gated else get_first_hidden_states_residual()
+    if prev is not None and not parallelized and ops.strided_residual_takes(hidden_states, prev, ctx.downsample_factor):
+        resid, ratio = ops.fbcache_first_residual_diff_strided(hidden_states, original_hidden_states, prev, ctx.downsample_factor)
+        return resid, ratio.item() < threshold
     if ctx.downsample_factor > 1 or (prev is not None and prev.shape != hidden_states.shape):
         resid, _ = ops.fbcache_first_residual_diff(hidden_states, original_hidden_states, None)
         return resid, (not gated) and get_can_use_cache(resid, parallelized=parallelized)
@@ -300,12 +303,14 @@ def apply_prev_hidden_states_residual(hidden_states, encoder_hidden_states=None)
         return ctx.get_taylorseer().approximate_value_plus(hidden_states), encoder_hidden_states
     res = ctx.get_buffer("hidden_states_residual")
     assert res is not None, "hidden_states_residual must be set before"
-    hidden_states = ops.fbcache_apply_residual(res, hidden_states)
-    if encoder_hidden_states is not None:
-        eres = ctx.get_buffer("encoder_hidden_states_residual")
-        assert eres is not None, "encoder_hidden_states_residual must be set before"
-        encoder_hidden_states = ops.fbcache_apply_residual(eres, encoder_hidden_states)
-    return hidden_states, encoder_hidden_states
+    if encoder_hidden_states is None:
+        return ops.fbcache_apply_residual(res, hidden_states), None
+    eres = ctx.get_buffer("encoder_hidden_states_residual")
+    assert eres is not None, "encoder_hidden_states_residual must be set before"
+    if hidden_states.dtype == encoder_hidden_states.dtype and hidden_states.device == encoder_hidden_states.device \
+            and hidden_states.numel() > 0 and encoder_hidden_states.numel() > 0:
+        return ops.fbcache_apply_residual_pair(res, hidden_states, eres, encoder_hidden_states)
+    return ops.fbcache_apply_residual(res, hidden_states), ops.fbcache_apply_residual(eres, encoder_hidden_states)
 
 
 @torch.compiler.disable

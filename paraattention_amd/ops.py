@@ -21,6 +21,7 @@ torch elementwise calls:
   block_sparse_key_runs, attention_forward_block_sparse_runs  (the same with the mask's run scan done once)
   fbcache_residual_diff                        (first_block_cache/utils.py:228-233)
   fbcache_first_residual_diff, fbcache_apply_residual (utils.py:359, 237-259)
+  fbcache_first_residual_diff_strided, fbcache_apply_residual_pair (the same down-sampled; both streams at once)
   taylorseer_derivatives, taylorseer_value     (first_block_cache/taylorseer.py:29-48)
 """
 import ctypes
@@ -860,12 +861,14 @@ def fbcache_first_residual_diff(
     h, h0 = hidden.contiguous(), hidden0.contiguous()
     pv = prev.contiguous() if prev is not None else None
     resid = torch.empty(h.shape, dtype=h.dtype, device=h.device)
-    # with something to compare the kernel writes the ratio; filling it first would be one more launch per step
-    ratio = torch.empty((), dtype=h.dtype, device=h.device)
-    if pv is None or pv.numel() == 0:
-        ratio.fill_(float("inf"))
-    ws = _fb_workspace(h.device)
+    ratio = torch.empty((), dtype=h.dtype, device=h.device)  # the kernel writes it: a fill would be one more launch per step
     lib = _lib.load()
+    if pv is None:
+        with _on(h.device):
+            rc = lib.pa_fbcache_residual(_ptr(h), _ptr(h0), _ptr(resid), _DTYPE_CODE[h.dtype], h.numel(), _ptr(ratio), _stream_ptr(h.device))
+        _lib.check(rc, "pa_fbcache_residual")
+        return resid, ratio
+    ws = _fb_workspace(h.device)
     with _on(h.device):
         rc = lib.pa_fbcache_residual_ratio(
             _ptr(h), _ptr(h0), _ptr(pv), _ptr(resid), _DTYPE_CODE[h.dtype], h.numel(), _ptr(ratio), None,
@@ -877,6 +880,43 @@ def fbcache_first_residual_diff(
 
 @torch.library.register_fake("para_attn::fbcache_first_residual_diff")
 def _(hidden, hidden0, prev=None):
+    return hidden.new_empty(hidden.shape), hidden.new_empty(())
+
+
+def strided_residual_takes(hidden, prev, step):
+    """Whether ``fbcache_first_residual_diff_strided`` compares ``prev`` with every ``step``-th column of a residual like ``hidden``."""
+    vec = 4 if hidden.dtype == torch.float32 else 8
+    return (step > 1 and vec % step == 0 and hidden.ndim > 0 and hidden.shape[-1] % vec == 0 and hidden.numel() > 0
+            and prev.dtype == hidden.dtype and prev.shape == (*hidden.shape[:-1], hidden.shape[-1] // step))
+
+
+@torch.library.custom_op("para_attn::fbcache_first_residual_diff_strided", mutates_args=(), device_types=("cuda",))
+def fbcache_first_residual_diff_strided(
+    hidden: torch.Tensor, hidden0: torch.Tensor, prev: torch.Tensor, step: int
+) -> Tuple[torch.Tensor, torch.Tensor]:
+    """``fbcache_first_residual_diff`` against a down-sampled previous residual: the ratio compares ``prev`` with
+    ``residual[..., ::step]`` (src/para_attn/first_block_cache/utils.py:276-278) in the pass that writes the residual."""
+    if hidden.shape != hidden0.shape or hidden.dtype != hidden0.dtype or hidden.dtype not in _DTYPE_CODE:
+        raise ValueError("hidden and hidden0 must share shape and a supported dtype")
+    if not strided_residual_takes(hidden, prev, step):
+        raise NotImplementedError(f"every {step}-th column of {tuple(hidden.shape)} {hidden.dtype} against {tuple(prev.shape)} {prev.dtype}")
+    _same_device(hidden, hidden0=hidden0, prev=prev)
+    h, h0, pv = hidden.contiguous(), hidden0.contiguous(), prev.contiguous()
+    resid = torch.empty(h.shape, dtype=h.dtype, device=h.device)
+    ratio = torch.empty((), dtype=h.dtype, device=h.device)
+    ws = _fb_workspace(h.device)
+    lib = _lib.load()
+    with _on(h.device):
+        rc = lib.pa_fbcache_residual_ratio_strided(
+            _ptr(h), _ptr(h0), _ptr(pv), _ptr(resid), _DTYPE_CODE[h.dtype], h.numel() // h.shape[-1], h.shape[-1], step, _ptr(ratio), None,
+            _ptr(ws), ws.numel() * 8, _stream_ptr(h.device),
+        )
+    _lib.check(rc, "pa_fbcache_residual_ratio_strided")
+    return resid, ratio
+
+
+@torch.library.register_fake("para_attn::fbcache_first_residual_diff_strided")
+def _(hidden, hidden0, prev, step):
     return hidden.new_empty(hidden.shape), hidden.new_empty(())
 
 
@@ -898,6 +938,35 @@ def fbcache_apply_residual(residual: torch.Tensor, hidden: torch.Tensor) -> torc
 @torch.library.register_fake("para_attn::fbcache_apply_residual")
 def _(residual, hidden):
     return hidden.new_empty(hidden.shape)
+
+
+@torch.library.custom_op("para_attn::fbcache_apply_residual_pair", mutates_args=(), device_types=("cuda",))
+def fbcache_apply_residual_pair(
+    residual: torch.Tensor, hidden: torch.Tensor, residual2: torch.Tensor, hidden2: torch.Tensor
+) -> Tuple[torch.Tensor, torch.Tensor]:
+    """(residual + hidden, residual2 + hidden2) in one launch: the two streams of a cache hit
+    (src/para_attn/first_block_cache/utils.py:245-259).  All four share one dtype; neither pair is empty."""
+    for r, h in ((residual, hidden), (residual2, hidden2)):
+        if r.shape != h.shape or r.dtype != h.dtype or h.dtype not in _DTYPE_CODE:
+            raise ValueError("residual and hidden must share shape and a supported dtype")
+    if hidden2.dtype != hidden.dtype:
+        raise ValueError("both pairs must share one dtype")
+    _same_device(hidden, residual=residual, hidden2=hidden2, residual2=residual2)
+    ts = [t.contiguous() for t in (residual, hidden, residual2, hidden2)]
+    outs = [torch.empty(t.shape, dtype=t.dtype, device=t.device) for t in (hidden, hidden2)]
+    lib = _lib.load()
+    with _on(hidden.device):
+        rc = lib.pa_fbcache_apply_residual2(
+            _ptr(ts[0]), _ptr(ts[1]), _ptr(outs[0]), hidden.numel(), _ptr(ts[2]), _ptr(ts[3]), _ptr(outs[1]), hidden2.numel(),
+            _DTYPE_CODE[hidden.dtype], _stream_ptr(hidden.device),
+        )
+    _lib.check(rc, "pa_fbcache_apply_residual2")
+    return outs[0], outs[1]
+
+
+@torch.library.register_fake("para_attn::fbcache_apply_residual_pair")
+def _(residual, hidden, residual2, hidden2):
+    return hidden.new_empty(hidden.shape), hidden2.new_empty(hidden2.shape)
 
 
 # ---------------------------------------------------------------------------------

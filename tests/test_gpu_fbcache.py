@@ -124,3 +124,45 @@ def test_residual_and_apply_at_the_edges_of_their_loops(cuda, n):
     if n < 1 << 22:
         want, _, _ = ofb.residual_diff_ratio(prev.float().cpu().numpy(), resid.float().cpu().numpy())
         assert ratio.item() == want
+
+
+@pytest.mark.parametrize("step", [2, 4, 8])
+@pytest.mark.parametrize("shape", [(1, 3, 8), (2, 257, 136), (1, 1500, 1920)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_down_sampled_comparison_in_the_residual_pass(cuda, dtype, shape, step):
+    """The residual compared with every step-th column of the previous one in the pass that writes it: residual bit for bit, ratio
+    bit for bit in 16 bits (fp32 means differ in the last bits with the order of the sums); 256 threads x 4 vectors x 256 workgroups and less."""
+    a, b = inputs.fbcache_pair(shape, seed=sum(shape) + step, noise=0.1, dtype=dtype)
+    hidden, prev = a + b, (b + 0.05 * a)[..., ::step].contiguous()
+    takes = paraattention_amd.ops.strided_residual_takes(hidden, prev, step)
+    assert takes == (shape[-1] % step == 0 and not (step == 8 and dtype == torch.float32))
+    if not takes:
+        with pytest.raises(NotImplementedError):
+            torch.ops.para_attn.fbcache_first_residual_diff_strided(hidden.to(cuda), a.to(cuda), prev.to(cuda), step)
+        return
+    resid, ratio = torch.ops.para_attn.fbcache_first_residual_diff_strided(hidden.to(cuda), a.to(cuda), prev.to(cuda), step)
+    want = hidden - a
+    assert torch.equal(resid.cpu(), want)
+    want_ratio, _, _ = ofb.residual_diff_ratio(prev.float().numpy(), want[..., ::step].contiguous().float().numpy(), NAMES[dtype])
+    if dtype == torch.float32:
+        assert abs(ratio.item() - want_ratio) <= 2e-6 * abs(want_ratio)
+    else:
+        assert ratio.item() == want_ratio
+    again = torch.ops.para_attn.fbcache_first_residual_diff_strided(hidden.to(cuda), a.to(cuda), prev.to(cuda), step)
+    assert again[1].item() == ratio.item()  # the workspace was left clean
+
+
+@pytest.mark.parametrize("sizes", [((1, 1, 1), (1, 1, 3)), ((1, 2000, 1920), (1, 7, 1920)), ((1, 5, 64), (2, 900, 520)), ((1, 333, 77), (1, 512, 77))])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_both_streams_in_one_launch(cuda, dtype, sizes):
+    """fbcache_apply_residual_pair against two eager additions: sizes that leave one workgroup to either tensor, ragged ends."""
+    g = torch.Generator().manual_seed(5)
+    ts = [torch.randn(s, generator=g).to(dtype).to(cuda) for s in (sizes[0], sizes[0], sizes[1], sizes[1])]
+    out, out2 = torch.ops.para_attn.fbcache_apply_residual_pair(*ts)
+    assert torch.equal(out, ts[0] + ts[1]) and torch.equal(out2, ts[2] + ts[3])
+
+
+def test_residual_without_a_previous_one(cuda):
+    a, b = (t.to(cuda) for t in inputs.fbcache_pair((2, 100, 61), seed=9))
+    resid, ratio = torch.ops.para_attn.fbcache_first_residual_diff(a, b, None)
+    assert torch.equal(resid, a - b) and ratio.item() == float("inf")
