@@ -141,6 +141,22 @@ def load():
     return _lib
 
 
+_host = None
+
+
+def host_calls():
+    """The module with the host side of the ordinary calls (csrc/host_calls.cpp), on top of the same library."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _host_calls
+        except ImportError as e:
+            raise ImportError(f"paraattention_amd/_host_calls.so cannot be loaded ({e}): build it with `make -C {os.path.join(_HERE, 'csrc')}`") from e
+        _host = _host_calls
+    return _host
+
+
 def check(rc, what):
     """Turn a PA_ERR_* return code into the exception the reference's op would raise."""
     if rc == PA_OK:

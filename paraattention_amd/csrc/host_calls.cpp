@@ -11,6 +11,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cmath>
+#include <vector>
 
 #include "../../include/paraattn_hip.h"
 
@@ -123,19 +124,14 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   }
   const Strides3 qs(q), ks(k), vs(v);
   const int dt = dtype_code(q.scalar_type());
+  size_t bytes = 0;
+  if (pm != nullptr) bytes = pa_attn_fwd_masked_call_workspace_bytes(B, H, Sq, Skv, D, ks.v, vs.v, kind, ms);
+  else if (native) bytes = pa_attn_fwd_call_workspace_bytes(B, H, Sq, Skv, D, ks.v, vs.v, 0, causal);
+  else if (!pa_attn_fwd_narrow_plan(B, H, Sq, Skv, D, ks.v, vs.v, causal, &bytes)) Py_RETURN_NONE;
   Tensor out, lse;
   int rc;
   {
     pybind11::gil_scoped_release no_gil;
-    size_t bytes = 0;
-    if (pm != nullptr) {
-      bytes = pa_attn_fwd_masked_call_workspace_bytes(B, H, Sq, Skv, D, ks.v, vs.v, kind, ms);
-    } else if (native) {
-      bytes = pa_attn_fwd_call_workspace_bytes(B, H, Sq, Skv, D, ks.v, vs.v, 0, causal);
-    } else if (!pa_attn_fwd_narrow_plan(B, H, Sq, Skv, D, ks.v, vs.v, causal, &bytes)) {
-      rc = -1;
-      goto done;
-    }
     // (rows of other head_dims come out contiguous, as from the zero-padded copies)
     out = native ? out_like(q) : at::empty(q.sizes(), q.options());
     if (want_lse) lse = at::empty({B, H, Sq}, q.options().dtype(at::kFloat));
@@ -150,9 +146,7 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     else
       rc = pa_attn_fwd_narrow(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), (float*)ptr(lse), dt, B, H, Sq, Skv, D, qs.v, ks.v, vs.v, os.v,
                               (float)scale, causal, ptr(ws), bytes, stream);
-  done:;
   }
-  if (rc < 0 && !out.defined()) Py_RETURN_NONE;
   if (rc != PA_OK) return PyLong_FromLong(rc);
   return pair(out, lse);
   END_HANDLE_TH_ERRORS
@@ -164,23 +158,36 @@ bool same_flat(const Tensor& a, const Tensor& b) {
 }
 bool flat_operand(const Tensor& a) { return plain(a) && dtype_code(a.scalar_type()) >= 0 && a.numel() > 0 && same_flat(a, a); }
 
-// fbcache_residual(hidden, hidden0, prev or None, workspace, stream) -> (residual, ratio)
+// fbcache_residual(hidden, hidden0, prev or None, step, workspace or None, stream) -> (residual, ratio): against prev, which holds every
+// step-th column (the caller has seen to the shapes where step > 1)
 PyObject* fbcache_residual(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   const Tensor *h, *h0, *prev, *ws;
-  if (nargs != 5 || !optional_tensor(args[0], &h) || !optional_tensor(args[1], &h0) || !optional_tensor(args[2], &prev) || !optional_tensor(args[3], &ws))
+  if (nargs != 6 || !optional_tensor(args[0], &h) || !optional_tensor(args[1], &h0) || !optional_tensor(args[2], &prev) || !optional_tensor(args[4], &ws))
     Py_RETURN_NONE;
-  if (!h || !h0 || !ws || !flat_operand(*h) || !same_flat(*h, *h0) || (prev && !same_flat(*h, *prev))) Py_RETURN_NONE;
-  void* const stream = PyLong_AsVoidPtr(args[4]);
+  const long step = PyLong_AsLong(args[3]);
+  void* const stream = PyLong_AsVoidPtr(args[5]);
   if (PyErr_Occurred()) return nullptr;
+  if (!h || !h0 || !flat_operand(*h) || !same_flat(*h, *h0)) Py_RETURN_NONE;
+  if (prev) {
+    if (!ws || !plain(*ws) || !flat_operand(*prev) || prev->scalar_type() != h->scalar_type() || prev->device() != h->device()) Py_RETURN_NONE;
+    if (step == 1 ? prev->sizes() != h->sizes() : step < 2 || h->dim() == 0 || prev->numel() * step != h->numel()) Py_RETURN_NONE;
+  }
   Tensor resid, ratio;
   int rc;
   {
     pybind11::gil_scoped_release no_gil;
     resid = at::empty(h->sizes(), h->options());
     ratio = at::empty({}, h->options());
-    rc = pa_fbcache_residual_ratio(h->data_ptr(), h0->data_ptr(), prev ? prev->data_ptr() : nullptr, resid.data_ptr(), dtype_code(h->scalar_type()),
-                                   h->numel(), ratio.data_ptr(), nullptr, ws->data_ptr(), ws->numel() * ws->element_size(), stream);
+    const int dt = dtype_code(h->scalar_type());
+    const size_t ws_bytes = prev ? ws->numel() * ws->element_size() : 0;
+    if (!prev) rc = pa_fbcache_residual(h->data_ptr(), h0->data_ptr(), resid.data_ptr(), dt, h->numel(), ratio.data_ptr(), stream);
+    else if (step == 1)
+      rc = pa_fbcache_residual_ratio(h->data_ptr(), h0->data_ptr(), prev->data_ptr(), resid.data_ptr(), dt, h->numel(), ratio.data_ptr(), nullptr,
+                                     ws->data_ptr(), ws_bytes, stream);
+    else
+      rc = pa_fbcache_residual_ratio_strided(h->data_ptr(), h0->data_ptr(), prev->data_ptr(), resid.data_ptr(), dt, h->numel() / h->size(-1), h->size(-1),
+                                             (int)step, ratio.data_ptr(), nullptr, ws->data_ptr(), ws_bytes, stream);
   }
   if (rc != PA_OK) return PyLong_FromLong(rc);
   return pair(resid, ratio);
@@ -206,12 +213,151 @@ PyObject* fbcache_apply(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
-PyMethodDef methods[] = {
-    {"attention", (PyCFunction)(void (*)(void))attention, METH_FASTCALL, nullptr},
-    {"fbcache_residual", (PyCFunction)(void (*)(void))fbcache_residual, METH_FASTCALL, nullptr},
-    {"fbcache_apply", (PyCFunction)(void (*)(void))fbcache_apply, METH_FASTCALL, nullptr},
-    {nullptr, nullptr, 0, nullptr},
-};
+// fbcache_apply_pair(residual, hidden, residual2, hidden2, stream) -> (residual + hidden, residual2 + hidden2)
+PyObject* fbcache_apply_pair(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  const Tensor *r, *h, *r2, *h2;
+  if (nargs != 5 || !optional_tensor(args[0], &r) || !optional_tensor(args[1], &h) || !optional_tensor(args[2], &r2) || !optional_tensor(args[3], &h2))
+    Py_RETURN_NONE;
+  if (!r || !h || !r2 || !h2 || !flat_operand(*h) || !flat_operand(*h2) || !same_flat(*h, *r) || !same_flat(*h2, *r2)) Py_RETURN_NONE;
+  if (h2->scalar_type() != h->scalar_type() || h2->device() != h->device()) Py_RETURN_NONE;
+  void* const stream = PyLong_AsVoidPtr(args[4]);
+  if (PyErr_Occurred()) return nullptr;
+  Tensor out, out2;
+  int rc;
+  {
+    pybind11::gil_scoped_release no_gil;
+    out = at::empty(h->sizes(), h->options());
+    out2 = at::empty(h2->sizes(), h2->options());
+    rc = pa_fbcache_apply_residual2(r->data_ptr(), h->data_ptr(), out.data_ptr(), h->numel(), r2->data_ptr(), h2->data_ptr(), out2.data_ptr(), h2->numel(),
+                                    dtype_code(h->scalar_type()), stream);
+  }
+  if (rc != PA_OK) return PyLong_FromLong(rc);
+  return pair(out, out2);
+  END_HANDLE_TH_ERRORS
+}
+
+// A sequence of tensors shaped like its first one, which is a flat operand
+bool flat_list(PyObject* list, std::vector<const Tensor*>& out) {
+  if (!PyList_Check(list) && !PyTuple_Check(list)) return false;
+  const Py_ssize_t n = PySequence_Fast_GET_SIZE(list);
+  PyObject** items = PySequence_Fast_ITEMS(list);
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    const Tensor* t;
+    if (!optional_tensor(items[i], &t) || !t) return false;
+    if (out.empty() ? !flat_operand(*t) : !same_flat(*out[0], *t)) return false;
+    out.push_back(t);
+  }
+  return true;
+}
+
+// taylorseer_value(derivs, elapsed, hidden or None, stream) -> value (+ hidden)
+PyObject* taylorseer_value(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  std::vector<const Tensor*> d;
+  const Tensor* h;
+  if (nargs != 4 || !flat_list(args[0], d) || d.empty() || d.size() > 16 || !optional_tensor(args[2], &h) || (h && !same_flat(*d[0], *h))) Py_RETURN_NONE;
+  const long elapsed = PyLong_AsLong(args[1]);
+  void* const stream = PyLong_AsVoidPtr(args[3]);
+  if (PyErr_Occurred()) return nullptr;
+  if (elapsed < -65536 || elapsed > 65536) Py_RETURN_NONE;
+  const int m = (int)d.size();
+  const void* src[16];
+  float coef[16], pw[16];
+  double factorial = 1, power = 1;  // (exact below 2^53, which is where this path ends)
+  for (int i = 0; i < m; ++i) {
+    if (i > 0) {
+      factorial *= i;
+      power *= (double)elapsed;
+    }
+    if (std::fabs(power) > 9e15) Py_RETURN_NONE;
+    src[i] = d[i]->data_ptr();
+    coef[i] = (float)(1.0 / factorial);
+    pw[i] = (float)power;
+  }
+  Tensor out;
+  int rc;
+  {
+    pybind11::gil_scoped_release no_gil;
+    out = at::empty(d[0]->sizes(), d[0]->options());
+    rc = pa_taylorseer_value(src, m, coef, pw, h ? h->data_ptr() : nullptr, out.data_ptr(), dtype_code(out.scalar_type()), out.numel(), stream);
+  }
+  if (rc != PA_OK) return PyLong_FromLong(rc);
+  return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
+}
+
+// taylorseer_derivatives(y, prev, window, stream) -> [x1, ..., xn]
+PyObject* taylorseer_derivatives(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  std::vector<const Tensor*> d;
+  const Tensor* y;
+  if (nargs != 4 || !optional_tensor(args[0], &y) || !y || !flat_operand(*y) || !flat_list(args[1], d) || d.empty() || d.size() > 16 || !same_flat(*y, *d[0]))
+    Py_RETURN_NONE;
+  const double window = PyFloat_AsDouble(args[2]);
+  void* const stream = PyLong_AsVoidPtr(args[3]);
+  if (PyErr_Occurred()) return nullptr;
+  const int n = (int)d.size();
+  const void* src[16];
+  void* dst[16];
+  std::vector<Tensor> cur(n);
+  int rc;
+  {
+    pybind11::gil_scoped_release no_gil;
+    for (int i = 0; i < n; ++i) {
+      cur[i] = at::empty(y->sizes(), y->options());
+      src[i] = d[i]->data_ptr();
+      dst[i] = cur[i].data_ptr();
+    }
+    rc = pa_taylorseer_update(y->data_ptr(), src, dst, n, dtype_code(y->scalar_type()), y->numel(), (float)window, stream);
+  }
+  if (rc != PA_OK) return PyLong_FromLong(rc);
+  PyObject* list = PyList_New(n);
+  if (!list) return nullptr;
+  for (int i = 0; i < n; ++i) PyList_SET_ITEM(list, i, THPVariable_Wrap(cur[i]));
+  return list;
+  END_HANDLE_TH_ERRORS
+}
+
+// block_sparse(query, key, value, block_mask, scale or None, stream) -> (out, lse): the mask covers all rows and keys
+PyObject* block_sparse(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  const Tensor *pq, *pk, *pv, *m;
+  if (nargs != 6 || !optional_tensor(args[0], &pq) || !optional_tensor(args[1], &pk) || !optional_tensor(args[2], &pv) || !optional_tensor(args[3], &m))
+    Py_RETURN_NONE;
+  if (!pq || !pk || !pv || !m || !attention_operands(*pq, *pk, *pv)) Py_RETURN_NONE;
+  const Tensor &q = *pq, &k = *pk, &v = *pv;
+  const int64_t B = q.size(0), H = q.size(1), Sq = q.size(2), D = q.size(3), Skv = k.size(2);
+  if (B > INT32_MAX || H > INT32_MAX || Sq > INT32_MAX || Skv > INT32_MAX || (D != 64 && D != 128)) Py_RETURN_NONE;
+  if (!plain(*m) || m->device() != q.device() || m->scalar_type() != at::kBool || m->dim() < 2 || m->dim() > 3 || !m->is_contiguous()) Py_RETURN_NONE;
+  const int64_t Hm = m->dim() == 3 ? m->size(0) : 1, nQ = m->size(-2), nK = m->size(-1);
+  if ((Hm != 1 && Hm != H) || nQ <= 0 || nK <= 0 || nQ > Sq || nK > Skv || Sq % nQ != 0 || Skv % nK != 0) Py_RETURN_NONE;
+  double scale = 1.0 / std::sqrt((double)D);
+  if (args[4] != Py_None) scale = PyFloat_AsDouble(args[4]);
+  void* const stream = PyLong_AsVoidPtr(args[5]);
+  if (PyErr_Occurred()) return nullptr;
+  const Strides3 qs(q), ks(k), vs(v);
+  Tensor out, lse;
+  int rc;
+  {
+    pybind11::gil_scoped_release no_gil;
+    const size_t bytes = pa_blocksparse_workspace_bytes((int)Hm, (int)nQ, (int)nK);
+    out = out_like(q);
+    lse = at::empty({B, H, Sq}, q.options().dtype(at::kFloat));
+    const Tensor ws = scratch((bytes + 3) / 4 * 4, q);
+    const Strides3 os(out);
+    rc = pa_attn_fwd_blocksparse(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), (float*)lse.data_ptr(), dtype_code(q.scalar_type()), B, H, Sq, Skv,
+                                 D, qs.v, ks.v, vs.v, os.v, (float)scale, (const uint8_t*)m->data_ptr(), (int)Hm, (int)nQ, (int)nK, 0, (int)(Sq / nQ), 0,
+                                 (int)(Skv / nK), (int32_t*)ptr(ws), bytes, stream);
+  }
+  if (rc != PA_OK) return PyLong_FromLong(rc);
+  return pair(out, lse);
+  END_HANDLE_TH_ERRORS
+}
+
+#define METHOD(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {METHOD(attention),        METHOD(block_sparse),     METHOD(fbcache_residual),       METHOD(fbcache_apply),
+                         METHOD(fbcache_apply_pair), METHOD(taylorseer_value), METHOD(taylorseer_derivatives), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_calls", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

@@ -162,13 +162,11 @@ class UnifiedAttnMode(_SdpaMode):
         self._attn_func = attn_func
 
     def _call(self, *args, **kwargs):
-        func = F.scaled_dot_product_attention
         method = self._parallel_method
-        if method in ("ulysses", "ring"):  # world size 1: both stages pass the call on
-            self._parallel_method = "ring" if method == "ulysses" else "none"
+        if method in ("ulysses", "ring"):  # world size 1: both stages pass the call on, straight to the last one
+            self._parallel_method = "none"
             try:
-                with self:
-                    return func(*args, **kwargs)
+                return self._call(*args, **kwargs)
             finally:
                 self._parallel_method = method
         if method != "none":

@@ -62,6 +62,20 @@ def _on(device):
     return _STAY if torch._C._cuda_getDevice() == device.index else torch.cuda.device(device)
 
 
+def _native(name, device, *args):
+    """The ordinary call in native code (csrc/host_calls.cpp), which takes operands that lie on the current device ready for the kernels;
+    None where it is another kind of call, to be looked at by the code below each use."""
+    index = device.index
+    if index is None or torch._C._cuda_getDevice() != index:
+        return None
+    if args[-1] is _fb_workspace:
+        args = (*args[:-1], _fb_workspace(device))
+    res = getattr(_lib.host_calls(), name)(*args, torch._C._cuda_getCurrentRawStream(index))
+    if type(res) is int:
+        _lib.check(res, name)
+    return res
+
+
 def _ptr_array(tensors):
     return (ctypes.c_void_p * len(tensors))(*[t.data_ptr() for t in tensors])
 
@@ -316,6 +330,10 @@ def attention_forward_with_lse(
 ) -> Tuple[torch.Tensor, torch.Tensor]:
     """out [B,H,Sq,D] in query's dtype and natural-log LSE [B,H,Sq] in fp32
     (src/para_attn/ops/__init__.py:160-179)."""
+    if dropout_p == 0.0:
+        res = _native("attention", query.device, query, key, value, attn_mask, scale, True, is_causal)
+        if res is not None:
+            return res
     _check_sdpa_args(query, key, value, dropout_p, is_causal, attn_mask, causal_ok=True, any_head_dim=True)
     out, lse = _masked_forward(query, key, value, attn_mask, scale, True, is_causal)
     return out, lse
@@ -338,6 +356,10 @@ def attention_forward(
     scale: Optional[float] = None,
 ) -> torch.Tensor:
     """Plain SDPA forward, no LSE (src/para_attn/ops/__init__.py:204-223)."""
+    if dropout_p == 0.0:
+        res = _native("attention", query.device, query, key, value, attn_mask, scale, False, is_causal)
+        if res is not None:
+            return res[0]
     _check_sdpa_args(query, key, value, dropout_p, is_causal, attn_mask, causal_ok=True, any_head_dim=True)
     out, _ = _masked_forward(query, key, value, attn_mask, scale, False, is_causal)
     return out
@@ -368,7 +390,8 @@ def attention_forward_sparse_kv(
     """
     _check_sdpa_args(query, key, value, dropout_p, is_causal, attn_mask, any_head_dim=True)
     if attn_mask is None:
-        return _masked_forward(query, key, value, None, scale, False)[0]
+        res = _native("attention", query.device, query, key, value, None, scale, False, False)
+        return (res if res is not None else _masked_forward(query, key, value, None, scale, False))[0]
     if attn_mask.dtype != torch.bool:
         raise AssertionError("attn_mask must be a boolean tensor")
     m = attn_mask
@@ -378,8 +401,9 @@ def attention_forward_sparse_kv(
         m = m.expand(query.shape[0], *m.shape[1:])
     while m.ndim > 2:
         m = m[:, 0]
-    out, _ = _masked_forward(query, key, value, m[:, None, None, :], scale, False)
-    return out
+    m = m[:, None, None, :]
+    res = _native("attention", query.device, query, key, value, m, scale, False, False)
+    return (res if res is not None else _masked_forward(query, key, value, m, scale, False))[0]
 
 
 @torch.library.register_fake("para_attn::attention_forward_sparse_kv")
@@ -617,6 +641,10 @@ def attention_forward_block_sparse(
     rows and keys outside those ranges are dense (:158-171, :178-189, :247-274).
     Identical to dense SDPA with -inf on the dropped tiles.
     """
+    if q_lo == 0 and kv_lo == 0 and q_hi < 0 and kv_hi < 0:
+        res = _native("block_sparse", query.device, query, key, value, block_mask, scale)
+        if res is not None:
+            return res
     _check_sdpa_args(query, key, value, 0.0, False)
     B, H, Sq, D = query.shape
     Skv = key.shape[2]
@@ -853,6 +881,9 @@ def fbcache_first_residual_diff(
     """(residual, ratio): residual = hidden - hidden0 (src/para_attn/first_block_cache/utils.py:359)
     and, in the same pass, the reduction of ``fbcache_residual_diff(prev, residual)``.
     Without ``prev`` the ratio is +inf (never similar)."""
+    res = _native("fbcache_residual", hidden.device, hidden, hidden0, prev, 1, _fb_workspace if prev is not None else None)
+    if res is not None:
+        return res
     if hidden.shape != hidden0.shape or hidden.dtype != hidden0.dtype or hidden.dtype not in _DTYPE_CODE:
         raise ValueError("hidden and hidden0 must share shape and a supported dtype")
     if prev is not None and (prev.shape != hidden.shape or prev.dtype != hidden.dtype):
@@ -900,6 +931,9 @@ def fbcache_first_residual_diff_strided(
         raise ValueError("hidden and hidden0 must share shape and a supported dtype")
     if not strided_residual_takes(hidden, prev, step):
         raise NotImplementedError(f"every {step}-th column of {tuple(hidden.shape)} {hidden.dtype} against {tuple(prev.shape)} {prev.dtype}")
+    res = _native("fbcache_residual", hidden.device, hidden, hidden0, prev, step, _fb_workspace)
+    if res is not None:
+        return res
     _same_device(hidden, hidden0=hidden0, prev=prev)
     h, h0, pv = hidden.contiguous(), hidden0.contiguous(), prev.contiguous()
     resid = torch.empty(h.shape, dtype=h.dtype, device=h.device)
@@ -923,6 +957,9 @@ def _(hidden, hidden0, prev, step):
 @torch.library.custom_op("para_attn::fbcache_apply_residual", mutates_args=(), device_types=("cuda",))
 def fbcache_apply_residual(residual: torch.Tensor, hidden: torch.Tensor) -> torch.Tensor:
     """``residual + hidden``, contiguous (src/para_attn/first_block_cache/utils.py:237-259)."""
+    res = _native("fbcache_apply", hidden.device, residual, hidden)
+    if res is not None:
+        return res
     if residual.shape != hidden.shape or residual.dtype != hidden.dtype or hidden.dtype not in _DTYPE_CODE:
         raise ValueError("residual and hidden must share shape and a supported dtype")
     _same_device(hidden, residual=residual)
@@ -946,6 +983,9 @@ def fbcache_apply_residual_pair(
 ) -> Tuple[torch.Tensor, torch.Tensor]:
     """(residual + hidden, residual2 + hidden2) in one launch: the two streams of a cache hit
     (src/para_attn/first_block_cache/utils.py:245-259).  All four share one dtype; neither pair is empty."""
+    res = _native("fbcache_apply_pair", hidden.device, residual, hidden, residual2, hidden2)
+    if res is not None:
+        return res
     for r, h in ((residual, hidden), (residual2, hidden2)):
         if r.shape != h.shape or r.dtype != h.dtype or h.dtype not in _DTYPE_CODE:
             raise ValueError("residual and hidden must share shape and a supported dtype")
@@ -993,6 +1033,9 @@ def taylorseer_derivatives(y: torch.Tensor, prev: List[torch.Tensor], window: fl
     n = len(prev)
     if n == 0:
         return []
+    res = _native("taylorseer_derivatives", y.device, y, prev, window)
+    if res is not None:
+        return res
     ts = _flat_same([y] + list(prev), "taylorseer_derivatives")
     cur = [torch.empty(y.shape, dtype=y.dtype, device=y.device) for _ in range(n)]
     lib = _lib.load()
@@ -1019,6 +1062,9 @@ def taylorseer_value(derivs: List[torch.Tensor], elapsed: int, hidden: Optional[
     m = len(derivs)
     if m == 0:
         raise ValueError("taylorseer_value: no stored derivative")
+    res = _native("taylorseer_value", derivs[0].device, derivs, elapsed, hidden)
+    if res is not None:
+        return res
     ts = _flat_same(list(derivs) + ([hidden] if hidden is not None else []), "taylorseer_value")
     d0 = ts[0]
     out = torch.empty(d0.shape, dtype=d0.dtype, device=d0.device)
