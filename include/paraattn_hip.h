@@ -75,6 +75,8 @@ PA_API const char* pa_last_error(void);
  *                                           longest list of key ranges first (1, the default)
  *   "short_keys"   PARAATTN_SHORT_KEYS=0|1  0 / 1: never / wherever it applies the kernel for 449..512 keys per head (head_dim 128,
  *                                           dense), -1 = where a workgroup gets two query tiles or more
+ *   "key_halves"   PARAATTN_KEY_HALVES=0|1  0 / 1: never / wherever it applies workgroups of 8 wavefronts on 128 query rows, 4 for either
+ *                                           half of the key tiles; -1 = where the grid leaves the chip room
  *   "resident"     PARAATTN_RESIDENT=0|1    0 / 1: never / wherever it applies the kernel that keeps all keys of a head in LDS (up to
  *                                           288 keys at head_dim 128, 576 at head_dim 64; less with an additive mask), -1 = where
  *                                           it is expected to be the fastest

@@ -112,6 +112,8 @@ struct AttnParams {
   // tile; the last split_tiles query tiles are computed by split_s workgroups each, over
   // consecutive shares of the key tiles, which leave normalised fp32 partial outputs and their
   // LSE in the workspace (piece-major) for attn_split_merge_kernel.  split_s <= 1: no split.
+  int n_wg;        // dense pipelined kernels with xcd_chunk: workgroups that have work
+  int key_halves;  // pipelined kernels: 128-row workgroups of 8 wavefronts, 4 for either half of the key tiles (template flag KS)
   int xcd_chunk;  // block-sparse pipelined kernel: ceil(workgroups / 8), 0 = plain order
   // 256-row dense kernel: *bound_flag != 0 says that no score can leave [-60, 60] in the log2 domain (see
   // score_bound_*_kernel), so the running maximum is not needed; null = not known, keep the maximum
@@ -613,6 +615,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_fwd_kernel(const AttnParams 
 // The element of tile j + 2 is fetched while tile j + 1 is masked, so its latency is covered by the wait for the
 // tile copies at the top of every iteration.
 // ---------------------------------------------------------------------------------------------
+constexpr int HALVES = 16;  // pipelined kernels, in the place of a number of wavefronts: 8, four for either half of the key tiles
 constexpr int PM_NONE = 0, PM_KEYS = 1, PM_KEYBIAS = 2, PM_BITS = 3, PM_BIAS = 4;
 constexpr int PM_SLOT_BYTES = 256;  // LDS per wavefront, behind the K and V tiles
 // The running maximum of a masked row before its first kept key.  Finite, so that -inf scores against it give
@@ -632,6 +635,8 @@ struct TileMask {
   __device__ __forceinline__ void init(const AttnParams& p, int batch, int head, int lane_, char* lds, int row) {
     lane = lane_;
     hh = lane_ >> 5;
+    raw = 0;
+    word = 0;
     if constexpr (PM == PM_BITS) {
       base = (const char*)(p.mask_words + ((int64_t)batch * p.mw_b + (int64_t)head * p.mw_h + row) * ((p.Skv + BN - 1) / BN));
       return;
@@ -1157,13 +1162,20 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_fwd_d128_kernel(const AttnPa
 // tile copies per flop).  Dense launches may compute the query tiles of the last round of
 // workgroups in several key shares (AttnParams::split_*), fold the result into a running
 // (out, lse) pair (acc_*), or apply torch's causal mask (causal).
+// KS (WAVES = HALVES): 8 wavefronts on 128 query rows, 4 for either half of the key tiles (they take the tiles in turn, each half with its own
+// buffers), folded in LDS at the end; for launches that give a compute unit one workgroup (take_halves): a step of two tiles takes
+// 1.65 us, two steps of one wavefront per SIMD 2.1.
 // ---------------------------------------------------------------------------------------------
-template <typename T, bool SPARSE, int NW, bool BOUNDED = false, bool PAIR = false, int PM = PM_NONE, int W = 128>
-__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_kernel(const AttnParams p) {
+template <typename T, bool SPARSE, int WAVES, bool BOUNDED = false, bool PAIR = false, int PM = PM_NONE, int W = 128>
+__global__ __launch_bounds__(WAVES == 4 ? 256 : 512, WAVES == 4 ? 2 : 1) void attn_fwd_d128_pipe_kernel(const AttnParams p) {
+  constexpr bool KS = WAVES == HALVES;
+  constexpr int NW = KS ? 8 : WAVES;
   typedef typename T::vec8 vec8;
   constexpr int DC = W / 16, DB = W / 32;
   static_assert(W == 128 || (W == 96 && !SPARSE && !PAIR && !BOUNDED), "row widths this kernel is written for");
-  constexpr int IPW = 16 / NW;  // copy instructions per wavefront and K (V) tile
+  static_assert(!KS || (!BOUNDED && !PAIR), "the two halves of the keys");
+  constexpr int NWG = KS ? NW / 2 : NW;  // wavefronts that share a tile
+  constexpr int IPW = 16 / NWG;  // copy instructions per wavefront and K (V) tile
   // is_causal, key shares, key segments and the fold into a running pair: masks with a query dimension are planned without
   // them (compiled in all the same, they took registers that PM_BIAS spilled and read back in every tile)
   constexpr bool ALL = !SPARSE && PM != PM_BITS && PM != PM_BIAS;
@@ -1176,14 +1188,14 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
   if constexpr (!SPARSE) {
     if (p.gate != nullptr && !gate_open(p.gate, p.gate_mask)) return;
   }
-  constexpr int RS = 4 * NW;    // tile rows between two of them
+  constexpr int RS = 4 * NWG;    // tile rows between two of them
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
-  char* const sK = (char*)smem;                    // [2][64][256 B]
-  char* const sV = (char*)smem + 2 * TILE_BYTES;   // [2][64][256 B]
-
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave_id = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = KS ? wave_id >> 2 : 0, wave = KS ? wave_id & 3 : wave_id;  // KS: which half of the keys; the row block
+  char* const sK = (char*)smem + group * (4 * TILE_BYTES);  // [2][64][256 B]
+  char* const sV = sK + 2 * TILE_BYTES;                     // [2][64][256 B]
   const int l32 = lane & 31;
   const int hh = lane >> 5;
 
@@ -1197,6 +1209,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
       tile = (tile & 7) * p.xcd_chunk + (tile >> 3);
       if (tile >= p.B * p.H * p.n_qtiles) return;
     }
+  } else if (p.xcd_chunk > 0) {
+    tile = (tile & 7) * p.xcd_chunk + (tile >> 3);
+    if (tile >= p.n_wg) return;
   }
   if constexpr (ALL) {
     if (p.split_s > 1 && tile >= p.split_main) {
@@ -1217,7 +1232,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
   TileIter it;
   decode_block<SPARSE>(p, qt, head, batch, row_begin, row_end, it);
   TileMask<T, PM> tm;
-  if constexpr (PM != PM_NONE) tm.init(p, batch, head, lane, (char*)smem + 4 * TILE_BYTES + wave * PM_SLOT_BYTES, min(row_begin + wave * 32 + l32, row_end - 1));
+  if constexpr (PM != PM_NONE) tm.init(p, batch, head, lane, (char*)smem + (KS ? 8 : 4) * TILE_BYTES + wave_id * PM_SLOT_BYTES, min(row_begin + wave * 32 + l32, row_end - 1));
   if constexpr (PM == PM_BITS) {  // the key tiles this query tile keeps, as build_runs_kernel lists them
     const int nseg = p.nQ + 2, sidx = (int)((batch * p.mw_b + head * p.mw_h) / p.Sq) * nseg + 1 + qt;
     it.init_list(p.runs + (size_t)p.Hm * nseg + (size_t)sidx * p.cap * 2, p.runs[sidx], p.Skv, false);
@@ -1336,7 +1351,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
   for (int i = 0; i < DB; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
-  float m_run = BOUNDED ? 0.f : PM != PM_NONE ? PM_NO_MAX : -INFINITY, l_run = 0.f;
+  float m_run = BOUNDED ? 0.f : PM != PM_NONE || KS ? PM_NO_MAX : -INFINITY, l_run = 0.f;
   const float c = p.scale_log2;
 
   // window of tiles j (being consumed), j+1 and j+2: (first key or OOB, valid keys)
@@ -1347,7 +1362,13 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
   // upper); a range's first key carries the bits in its two low bits (ranges begin at multiples of 4 there).
   int m_cur = 3, m_nxt = 3, m_nx2 = 3;
   const int my_bit = wave < NW / 2 ? 1 : 2;
-  auto pull = [&](uint32_t& n0, int& nv) {
+  // KS: the groups take the tiles of the list in turn; `ex` says whether the pair exists (of its two tiles the second may not)
+  bool e_cur = false, e_nxt = false, e_nx2 = false;
+  auto pull = [&](uint32_t& n0, int& nv, bool& ex) {
+    if constexpr (KS) {
+      ex = it.valid();
+      if (group != 0 && it.valid()) it.next();
+    }
     if constexpr (PAIR) {
       m_cur = m_nxt;
       m_nxt = m_nx2;
@@ -1364,13 +1385,16 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
       it.next();
       n0 = (uint32_t)a;
       nv = b;
+      if constexpr (KS) {
+        if (group == 0 && it.valid()) it.next();
+      }
     } else {
       n0 = OOB;
       nv = 0;
       if constexpr (PAIR) m_nx2 = 0;
     }
   };
-  bool have = false;
+  bool have = false, any_key = false;
 
   // -inf on the keys past the end of a ragged tile: register r of this lane is key
   // 8*(r/4) + r%4 + 4*hh of the first half (+32 for the second); constants against one per-lane
@@ -1619,8 +1643,12 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
     v_cur = v_nxt;
     n_nxt = n_nx2;
     v_nxt = v_nx2;
-    pull(n_nx2, v_nx2);
-    have = n_cur != OOB;
+    if constexpr (KS) {
+      e_cur = e_nxt;
+      e_nxt = e_nx2;
+    }
+    pull(n_nx2, v_nx2, e_nx2);
+    have = KS ? e_cur : n_cur != OOB;
   };
 
   // The keys' segments are swept one after the other, the pipeline drained in between (carrying it across, with
@@ -1636,10 +1664,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
         if (seg > seg_lo) __syncthreads();  // everybody has left the previous segment's last tiles
       }
     }
-    pull(n_cur, v_cur);
-    pull(n_nxt, v_nxt);
-    pull(n_nx2, v_nx2);
-    have = n_cur != OOB;
+    pull(n_cur, v_cur, e_cur);
+    pull(n_nxt, v_nxt, e_nxt);
+    pull(n_nx2, v_nx2, e_nx2);
+    have = KS ? e_cur : n_cur != OOB;
+    any_key |= have;
     if (seg > seg_lo) {  // the scores left over from the previous segment's last, absent tile
 #pragma unroll
       for (int r = 0; r < 16; ++r) sn0[r] = sn1[r] = 0.f;
@@ -1665,7 +1694,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
       for (int dc = 0; dc < DC; ++dc) sn1 = T::mfma32(f[dc], qf[dc], sn1);
       if constexpr (PM == PM_BIAS) tm.add_bias(sn0, sn1, n_cur, v_cur);
       if constexpr (PM != PM_NONE && PM != PM_BIAS) {
-        tm.fetch(n_cur);
+        if (!KS || n_cur != OOB) tm.fetch(n_cur);  // (the second of two tiles may not exist)
         tm.apply(sn0, sn1);
         if (n_nxt != OOB) tm.fetch(n_nxt);
       }
@@ -1699,7 +1728,46 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
     auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_run), __float_as_uint(l_run), false, false);
     l_tot = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
   }
-  const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
+  constexpr int MINE = (DB + 1) / 2;  // KS: group 0 finishes the first MINE blocks of 32 columns, group 1 the others
+  auto is_mine = [&](int db) { return !KS || (db < MINE) == (group == 0); };
+  if constexpr (KS) {
+    // Both halves leave what the other finishes in LDS (their tiles are done with), lane by lane, and fold the two results.
+    __syncthreads();
+    char* const box = (char*)smem + lane * 16;
+    constexpr int ROOM = (DB - MINE > MINE ? DB - MINE : MINE) * 4096 + 512;
+    char* const give = box + wave_id * ROOM;
+    char* const take = box + (wave_id ^ 4) * ROOM;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+      if (is_mine(db)) continue;
+      const int at = 4096 * (db < MINE ? db : db - MINE);
+#pragma unroll
+      for (int a = 0; a < 4; ++a) *(floatx4*)(give + at + 1024 * a) = floatx4{o[db][4 * a], o[db][4 * a + 1], o[db][4 * a + 2], o[db][4 * a + 3]};
+    }
+    float* const ml = (float*)((char*)smem + wave_id * ROOM + ROOM - 512) + 2 * lane;
+    const float* const ml2 = (const float*)((char*)smem + (wave_id ^ 4) * ROOM + ROOM - 512) + 2 * lane;
+    ml[0] = m_run;
+    ml[1] = l_tot;
+    __syncthreads();
+    const float m2 = ml2[0], l2 = ml2[1];
+    const float m = fmaxf(m_run, m2), f1 = __builtin_amdgcn_exp2f(m_run - m), f2 = __builtin_amdgcn_exp2f(m2 - m);
+    l_tot = l_tot * f1 + l2 * f2;
+    m_run = m;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+      if (!is_mine(db)) continue;
+      const int at = 4096 * (db < MINE ? db : db - MINE);
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        const floatx4 x = *(const floatx4*)(take + at + 1024 * a);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[db][4 * a + i] = o[db][4 * a + i] * f1 + x[i] * f2;
+      }
+    }
+  }
+  float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
+  // without a mask, scores that are all -inf are no row without keys: a NaN, as where the running maximum begins at -inf
+  if (KS && PM == PM_NONE && any_key && l_tot == 0.f) inv = __uint_as_float(0x7fc00000u);
   if constexpr (ALL) {
     if (piece_slot >= 0) {  // partial result of one key share: fp32, into the workspace
       if (row_ok) {
@@ -1707,20 +1775,22 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
         float* wp = p.ws_out + wrow * 128;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
+          if (is_mine(db))
 #pragma unroll
           for (int a = 0; a < 4; ++a) {
             float4 w = {o[db][4 * a] * inv, o[db][4 * a + 1] * inv, o[db][4 * a + 2] * inv, o[db][4 * a + 3] * inv};
             *(float4*)(wp + 32 * db + 8 * a + 4 * hh) = w;
           }
-        if (hh == 0) p.ws_lse[wrow] = l_tot > 0.f ? (m_run + __builtin_amdgcn_logf(l_tot)) * LN2 : -INFINITY;
+        if (hh == 0 && group == 0) p.ws_lse[wrow] = l_tot > 0.f ? (m_run + __builtin_amdgcn_logf(l_tot)) * LN2 : -INFINITY;
       }
       return;
     }
     if (p.acc_out != nullptr) {  // fold into the running (out, lse) pair
+      const int64_t ridx = ((int64_t)batch * p.H + head) * p.Sq + my_row;
+      const float old = p.acc_first || !row_ok ? -INFINITY : p.acc_lse[ridx];
+      if constexpr (KS) __syncthreads();  // both halves have read it before one writes it
       if (row_ok) {
-        const int64_t ridx = ((int64_t)batch * p.H + head) * p.Sq + my_row;
         const float blk = l_tot > 0.f ? (m_run + __builtin_amdgcn_logf(l_tot)) * LN2 : -INFINITY;
-        const float old = p.acc_first ? -INFINITY : p.acc_lse[ridx];
         const float mx = fmaxf(old, blk);
         float w_old = 0.f, w_blk = 0.f, lse_new = -INFINITY;
         if (mx > -INFINITY) {
@@ -1734,6 +1804,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
         uint16_t* op = p.out ? (uint16_t*)p.out + batch * p.os_b + head * p.os_h + (int64_t)my_row * p.os_s : nullptr;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
+          if (is_mine(db))
 #pragma unroll
           for (int a = 0; a < 4; ++a) {
             const int d0 = 32 * db + 8 * a + 4 * hh;
@@ -1752,7 +1823,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
               *(float4*)(ap + d0) = r;
             }
           }
-        if (hh == 0) p.acc_lse[ridx] = lse_new;
+        if (hh == 0 && group == 0) p.acc_lse[ridx] = lse_new;
       }
       return;
     }
@@ -1761,6 +1832,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
     uint16_t* op = (uint16_t*)p.out + batch * p.os_b + head * p.os_h + (int64_t)my_row * p.os_s;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
+      if (is_mine(db))
 #pragma unroll
       for (int a = 0; a < 4; ++a) {
         u32x2 w;
@@ -1768,7 +1840,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d128_pipe_k
         w[1] = T::pack2(o[db][4 * a + 2] * inv, o[db][4 * a + 3] * inv);
         if (W == 128 || 32 * db + 8 * a < p.dt) *(u32x2*)(op + 32 * db + 8 * a + 4 * hh) = w;
       }
-    if (p.lse != nullptr && hh == 0) {
+    if (p.lse != nullptr && hh == 0 && group == 0) {
       float lse = l_tot > 0.f ? (m_run + __builtin_amdgcn_logf(l_tot)) * LN2 : -INFINITY;
       p.lse[((int64_t)batch * p.H + head) * p.Sq + my_row] = lse;
     }
@@ -1794,8 +1866,10 @@ constexpr int TILE64_BYTES = BN * 128;
 // at the parameters, because a launch with neither -- cross-attention of many rows to a few hundred keys can never split --
 // pays their decode and epilogue in every short workgroup (33 scalar registers spilled against 24): 40 heads x 32760 rows
 // against 512 keys 244.9 -> 242.0 us without them, 24 x 17776 against 256 keys 56.6 -> 55.6, 16 heads x 3000 tokens 50.5 -> 49.7.
-template <typename T, bool SPARSE, int NW, bool BOUNDED = false, int PM = PM_NONE, bool NARROW = false, bool CUT = false>
-__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_kernel(const AttnParams p) {
+template <typename T, bool SPARSE, int WAVES, bool BOUNDED = false, int PM = PM_NONE, bool NARROW = false, bool CUT = false>
+__global__ __launch_bounds__(WAVES == 4 ? 256 : 512, WAVES == 4 ? 2 : 1) void attn_fwd_d64_pipe_kernel(const AttnParams p) {
+  constexpr bool KS = WAVES == HALVES;
+  constexpr int NW = KS ? 8 : WAVES;
   // BOUNDED and the flag: as in attn_fwd_d128_pipe_kernel
   if constexpr (!SPARSE) {
     if (p.bound_flag != nullptr && (*p.bound_flag != 0) != BOUNDED) return;
@@ -1803,20 +1877,28 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
   }
   typedef typename T::vec8 vec8;
   constexpr int DC = 4, DB = 2;
-  constexpr int IPW = 8 / NW;  // copy instructions per wavefront and K (V) tile
-  constexpr int RS = 8 * NW;   // tile rows between two of them
+  static_assert(!KS || !BOUNDED, "the two halves of the keys");
+  constexpr int NWG = KS ? NW / 2 : NW;  // wavefronts that share a tile
+  constexpr int IPW = 8 / NWG;  // copy instructions per wavefront and K (V) tile
+  constexpr int RS = 8 * NWG;   // tile rows between two of them
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
-  char* const sK = (char*)smem;                      // [2][64][128 B]
-  char* const sV = (char*)smem + 2 * TILE64_BYTES;   // [2][64][128 B]
-
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave_id = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = KS ? wave_id >> 2 : 0, wave = KS ? wave_id & 3 : wave_id;  // KS: which half of the keys; the row block
+  char* const sK = (char*)smem + group * (4 * TILE64_BYTES);  // [2][64][128 B]
+  char* const sV = sK + 2 * TILE64_BYTES;                     // [2][64][128 B]
   const int l32 = lane & 31;
   const int hh = lane >> 5;
 
   int tile = blockIdx.x;
   int piece_slot = -1;  // >= 0: this workgroup computes one key share of a split query tile
+  if constexpr (!SPARSE) {
+    if (p.xcd_chunk > 0) {
+      tile = (tile & 7) * p.xcd_chunk + (tile >> 3);
+      if (tile >= p.n_wg) return;
+    }
+  }
   if constexpr (CUT) {
     if (p.split_s > 1 && tile >= p.split_main) {
       piece_slot = tile - p.split_main;
@@ -1842,7 +1924,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
   TileIter it;
   decode_block<SPARSE>(p, qt, head, batch, row_begin, row_end, it);
   TileMask<T, PM> tm;
-  if constexpr (PM != PM_NONE) tm.init(p, batch, head, lane, (char*)smem + 4 * TILE64_BYTES + wave * PM_SLOT_BYTES, min(row_begin + wave * 32 + l32, row_end - 1));
+  if constexpr (PM != PM_NONE) tm.init(p, batch, head, lane, (char*)smem + (KS ? 8 : 4) * TILE64_BYTES + wave_id * PM_SLOT_BYTES, min(row_begin + wave * 32 + l32, row_end - 1));
   if constexpr (PM == PM_BITS) {  // the key tiles this query tile keeps, as build_runs_kernel lists them
     const int nseg = p.nQ + 2, sidx = (int)((batch * p.mw_b + head * p.mw_h) / p.Sq) * nseg + 1 + qt;
     it.init_list(p.runs + (size_t)p.Hm * nseg + (size_t)sidx * p.cap * 2, p.runs[sidx], p.Skv, false);
@@ -1940,27 +2022,37 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
   for (int i = 0; i < DB; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
-  float m_run = BOUNDED ? 0.f : PM != PM_NONE ? PM_NO_MAX : -INFINITY, l_run = 0.f;
+  float m_run = BOUNDED ? 0.f : PM != PM_NONE || KS ? PM_NO_MAX : -INFINITY, l_run = 0.f;
   const float c = p.scale_log2;
 
   uint32_t n_cur, n_nxt, n_nx2;
   int v_cur, v_nxt, v_nx2;
-  auto pull = [&](uint32_t& n0, int& nv) {
+  // KS: the groups take the tiles of the list in turn; `ex` says whether the pair exists (of its two tiles the second may not)
+  bool e_cur = false, e_nxt = false, e_nx2 = false;
+  auto pull = [&](uint32_t& n0, int& nv, bool& ex) {
+    if constexpr (KS) {
+      ex = it.valid();
+      if (group != 0 && it.valid()) it.next();
+    }
     if (it.valid()) {
       int a, b;
       it.get(a, b);
       it.next();
       n0 = (uint32_t)a;
       nv = b;
+      if constexpr (KS) {
+        if (group == 0 && it.valid()) it.next();
+      }
     } else {
       n0 = OOB;
       nv = 0;
     }
   };
-  pull(n_cur, v_cur);
-  pull(n_nxt, v_nxt);
-  pull(n_nx2, v_nx2);
-  bool have = n_cur != OOB;
+  pull(n_cur, v_cur, e_cur);
+  pull(n_nxt, v_nxt, e_nxt);
+  pull(n_nx2, v_nx2, e_nx2);
+  bool have = KS ? e_cur : n_cur != OOB;
+  const bool any_key = have;
 
   const int wave_row0 = row_begin + 32 * wave;
   auto on_diagonal = [&](uint32_t n0) {
@@ -2008,7 +2100,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
     }
     if constexpr (PM == PM_BIAS) tm.add_bias(sn0, sn1, n_cur, v_cur);
     if constexpr (PM != PM_NONE && PM != PM_BIAS) {
-      tm.fetch(n_cur);
+      if (!KS || n_cur != OOB) tm.fetch(n_cur);  // (the second of two tiles may not exist)
       tm.apply(sn0, sn1);
       if (n_nxt != OOB) tm.fetch(n_nxt);
     }
@@ -2131,8 +2223,12 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
     v_cur = v_nxt;
     n_nxt = n_nx2;
     v_nxt = v_nx2;
-    pull(n_nx2, v_nx2);
-    have = n_cur != OOB;
+    if constexpr (KS) {
+      e_cur = e_nxt;
+      e_nxt = e_nx2;
+    }
+    pull(n_nx2, v_nx2, e_nx2);
+    have = KS ? e_cur : n_cur != OOB;
   };
 
   while (have) {
@@ -2147,7 +2243,46 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
     auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_run), __float_as_uint(l_run), false, false);
     l_tot = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
   }
-  const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
+  constexpr int MINE = (DB + 1) / 2;  // KS: group 0 finishes the first MINE blocks of 32 columns, group 1 the others
+  auto is_mine = [&](int db) { return !KS || (db < MINE) == (group == 0); };
+  if constexpr (KS) {
+    // Both halves leave what the other finishes in LDS (their tiles are done with), lane by lane, and fold the two results.
+    __syncthreads();
+    char* const box = (char*)smem + lane * 16;
+    constexpr int ROOM = (DB - MINE > MINE ? DB - MINE : MINE) * 4096 + 512;
+    char* const give = box + wave_id * ROOM;
+    char* const take = box + (wave_id ^ 4) * ROOM;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+      if (is_mine(db)) continue;
+      const int at = 4096 * (db < MINE ? db : db - MINE);
+#pragma unroll
+      for (int a = 0; a < 4; ++a) *(floatx4*)(give + at + 1024 * a) = floatx4{o[db][4 * a], o[db][4 * a + 1], o[db][4 * a + 2], o[db][4 * a + 3]};
+    }
+    float* const ml = (float*)((char*)smem + wave_id * ROOM + ROOM - 512) + 2 * lane;
+    const float* const ml2 = (const float*)((char*)smem + (wave_id ^ 4) * ROOM + ROOM - 512) + 2 * lane;
+    ml[0] = m_run;
+    ml[1] = l_tot;
+    __syncthreads();
+    const float m2 = ml2[0], l2 = ml2[1];
+    const float m = fmaxf(m_run, m2), f1 = __builtin_amdgcn_exp2f(m_run - m), f2 = __builtin_amdgcn_exp2f(m2 - m);
+    l_tot = l_tot * f1 + l2 * f2;
+    m_run = m;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+      if (!is_mine(db)) continue;
+      const int at = 4096 * (db < MINE ? db : db - MINE);
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        const floatx4 x = *(const floatx4*)(take + at + 1024 * a);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[db][4 * a + i] = o[db][4 * a + i] * f1 + x[i] * f2;
+      }
+    }
+  }
+  float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
+  // without a mask, scores that are all -inf are no row without keys: a NaN, as where the running maximum begins at -inf
+  if (KS && PM == PM_NONE && any_key && l_tot == 0.f) inv = __uint_as_float(0x7fc00000u);
   if constexpr (CUT) {
     if (piece_slot >= 0) {  // partial result of one key share: fp32, into the workspace
       if (row_ok) {
@@ -2155,12 +2290,13 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
         float* wp = p.ws_out + wrow * 64;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
+          if (is_mine(db))
 #pragma unroll
           for (int a = 0; a < 4; ++a) {
             float4 w = {o[db][4 * a] * inv, o[db][4 * a + 1] * inv, o[db][4 * a + 2] * inv, o[db][4 * a + 3] * inv};
             *(float4*)(wp + 32 * db + 8 * a + 4 * hh) = w;
           }
-        if (hh == 0) p.ws_lse[wrow] = l_tot > 0.f ? (m_run + __builtin_amdgcn_logf(l_tot)) * LN2 : -INFINITY;
+        if (hh == 0 && group == 0) p.ws_lse[wrow] = l_tot > 0.f ? (m_run + __builtin_amdgcn_logf(l_tot)) * LN2 : -INFINITY;
       }
       return;
     }
@@ -2169,6 +2305,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
     uint16_t* op = (uint16_t*)p.out + batch * p.os_b + head * p.os_h + (int64_t)my_row * p.os_s;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
+      if (is_mine(db))
 #pragma unroll
       for (int a = 0; a < 4; ++a) {
         u32x2 w;
@@ -2176,7 +2313,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_fwd_d64_pipe_ke
         w[1] = T::pack2(o[db][4 * a + 2] * inv, o[db][4 * a + 3] * inv);
         if (!NARROW || 32 * db + 8 * a < p.dt) *(u32x2*)(op + 32 * db + 8 * a + 4 * hh) = w;
       }
-    if (p.lse != nullptr && hh == 0) {
+    if (p.lse != nullptr && hh == 0 && group == 0) {
       float lse = l_tot > 0.f ? (m_run + __builtin_amdgcn_logf(l_tot)) * LN2 : -INFINITY;
       p.lse[((int64_t)batch * p.H + head) * p.Sq + my_row] = lse;
     }
@@ -4083,7 +4220,7 @@ static void fill_params(AttnParams& p, const void* q, const void* k, const void*
   p.order = nullptr;
   p.Hm = 0; p.nQ = 0; p.cap = 0; p.q_lo = 0; p.q_block = 0; p.pair = 0; p.tiles_left = 0; p.tiles_per_block = 0;
   p.bm = BM; p.pipe = 0;
-  p.xcd_chunk = 0;
+  p.xcd_chunk = 0; p.n_wg = 0; p.key_halves = 0;
   p.causal = 0; p.heads_first = 0;
   p.acc_out = nullptr; p.acc_lse = nullptr; p.acc_first = 0;
   p.split_main = 0; p.split_tiles = 0; p.split_s = 0; p.ws_out = nullptr; p.ws_lse = nullptr; p.ws_cols = 128;
@@ -4094,23 +4231,27 @@ static void fill_params(AttnParams& p, const void* q, const void* k, const void*
   p.st = StreamPlan{};
 }
 
-template <typename T, bool SPARSE, int NW, bool BOUNDED, int PM = PM_NONE, bool NARROW = false, bool CUT = false>
+template <typename T, bool SPARSE, int WAVES, bool BOUNDED, int PM = PM_NONE, bool NARROW = false, bool CUT = false>
 static int launch_d64(const AttnParams& p, int64_t nblocks, hipStream_t stream) {
-  const size_t smem = 4 * TILE64_BYTES + (PM == PM_KEYBIAS ? NW * PM_SLOT_BYTES : 0);
+  constexpr int NW = WAVES == HALVES ? 8 : WAVES;
+  const size_t smem = (WAVES == HALVES ? 8 : 4) * TILE64_BYTES + (PM == PM_KEYBIAS ? NW * PM_SLOT_BYTES : 0);
   static bool attr_done[PA_MAX_DEVICES] = {};  // benign race: the call is idempotent
   const int dev = current_device();
   if (dev < 0 || !attr_done[dev]) {
-    hipError_t e = hipFuncSetAttribute((const void*)attn_fwd_d64_pipe_kernel<T, SPARSE, NW, BOUNDED, PM, NARROW, CUT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    hipError_t e = hipFuncSetAttribute((const void*)attn_fwd_d64_pipe_kernel<T, SPARSE, WAVES, BOUNDED, PM, NARROW, CUT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     if (e != hipSuccess) PA_FAIL(PA_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
     if (dev >= 0) attr_done[dev] = true;
   }
-  hipLaunchKernelGGL((attn_fwd_d64_pipe_kernel<T, SPARSE, NW, BOUNDED, PM, NARROW, CUT>), dim3((unsigned)nblocks), dim3(64 * NW), smem, stream, p);
+  hipLaunchKernelGGL((attn_fwd_d64_pipe_kernel<T, SPARSE, WAVES, BOUNDED, PM, NARROW, CUT>), dim3((unsigned)nblocks), dim3(64 * NW), smem, stream, p);
   PA_CHECK_LAUNCH("attention kernel (head_dim 64)");
   return PA_OK;
 }
 
 template <typename T, bool SPARSE, bool BOUNDED>
 static int launch_d64_plain(const AttnParams& p, int64_t nblocks, hipStream_t stream) {
+  if constexpr (!BOUNDED) {
+    if (p.key_halves) return launch_d64<T, SPARSE, HALVES, false, PM_NONE, false, !SPARSE>(p, nblocks, stream);
+  }
   if constexpr (!SPARSE) {
     if (p.split_s > 1 || p.heads_first)
       return p.bm == 256 ? launch_d64<T, false, 8, BOUNDED, PM_NONE, false, true>(p, nblocks, stream)
@@ -4135,7 +4276,8 @@ static int launch_attn(const AttnParams& p, hipStream_t stream) {
   int slot;
   if constexpr (D == 128) {
     smem = 4 * TILE_BYTES;
-    if (p.pipe && p.bm == 256) { fn = (const void*)attn_fwd_d128_pipe_kernel<T, SPARSE, 8>; slot = 2; }
+    if (p.pipe && p.key_halves) { fn = (const void*)attn_fwd_d128_pipe_kernel<T, SPARSE, HALVES>; slot = 5; smem = 8 * TILE_BYTES; }
+    else if (p.pipe && p.bm == 256) { fn = (const void*)attn_fwd_d128_pipe_kernel<T, SPARSE, 8>; slot = 2; }
     else if (p.pipe) { fn = (const void*)attn_fwd_d128_pipe_kernel<T, SPARSE, 4>; slot = 1; }
     else { fn = (const void*)attn_fwd_d128_kernel<T, SPARSE>; slot = 0; }
   } else {
@@ -4146,7 +4288,7 @@ static int launch_attn(const AttnParams& p, hipStream_t stream) {
   // the attribute belongs to the function on one device: remembered per device and kernel variant
   if (p.bound_flag != nullptr && (SPARSE || slot != (D == 128 ? 2 : 1)))
     PA_FAIL(PA_ERR_UNSUPPORTED, "score bound reached a kernel that does not read it");
-  static bool attr_done[PA_MAX_DEVICES][5] = {};  // benign race: the call is idempotent
+  static bool attr_done[PA_MAX_DEVICES][6] = {};  // benign race: the call is idempotent
   const int dev = current_device();
   if (!(D == 64 && p.pipe) && (dev < 0 || !attr_done[dev][slot])) {
     hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
@@ -4184,7 +4326,9 @@ static int launch_attn(const AttnParams& p, hipStream_t stream) {
     }
   }
   if constexpr (D == 128) {
-    if (slot == 2)
+    if (slot == 5)
+      hipLaunchKernelGGL((attn_fwd_d128_pipe_kernel<T, SPARSE, HALVES>), dim3((unsigned)nblocks), dim3(512), smem, stream, p);
+    else if (slot == 2)
       hipLaunchKernelGGL((attn_fwd_d128_pipe_kernel<T, SPARSE, 8>), dim3((unsigned)nblocks), dim3(512), smem, stream, p);
     else if (slot == 1)
       hipLaunchKernelGGL((attn_fwd_d128_pipe_kernel<T, SPARSE, 4>), dim3((unsigned)nblocks), dim3(256), smem, stream, p);
@@ -4264,9 +4408,10 @@ static SplitPlan plan_split(int64_t n_tiles, int slots, int kv_tiles, int bm, bo
 //   PARAATTN_WAVE_ROWS=64    "wave_rows"     the resident-workgroup kernel as 4 wavefronts of 64 query rows instead of 8 of 32
 //   PARAATTN_SPARSE_ORDER=0  "sparse_order"  block-sparse: 0 = the query blocks of a head in their own order instead of longest list first
 //   PARAATTN_SHORT_KEYS=0|1  "short_keys"    never / wherever it applies the kernel for 449..512 keys (-1 = by the number of pieces)
+//   PARAATTN_KEY_HALVES=0|1  "key_halves"    never / wherever it applies workgroups of 8 wavefronts on 128 query rows, 4 for either half of the key tiles (-1 = by the size of the grid)
 //   PARAATTN_RESIDENT=0|1    "resident"      never / wherever it applies the kernel that keeps all keys in LDS (-1 = by size)
 struct Tuning {
-  std::atomic<int> no_pipe, no_split, no_xcd_order, forced_bm, bound, stream, stream_even, stream_dyn, stream_solo, sparse_pair, wave_rows, short_keys, sparse_order, resident;
+  std::atomic<int> no_pipe, no_split, no_xcd_order, forced_bm, bound, stream, stream_even, stream_dyn, stream_solo, sparse_pair, wave_rows, short_keys, sparse_order, resident, key_halves;
 };
 static Tuning& tuning() {
   static Tuning t;
@@ -4293,6 +4438,8 @@ static Tuning& tuning() {
     const int sk = num("PARAATTN_SHORT_KEYS", -1);
     t.short_keys = sk == 0 || sk == 1 ? sk : -1;
     t.sparse_order = num("PARAATTN_SPARSE_ORDER", 1) != 0;
+    const int kh = num("PARAATTN_KEY_HALVES", -1);
+    t.key_halves = kh == 0 || kh == 1 ? kh : -1;
     const int rs = num("PARAATTN_RESIDENT", -1);
     t.resident = rs == 0 || rs == 1 ? rs : -1;
     return true;
@@ -4319,9 +4466,34 @@ extern "C" int pa_set_tuning(const char* name, int value) {
   else if (!strcmp(name, "wave_rows")) t.wave_rows = value == 64 ? 64 : 0;
   else if (!strcmp(name, "short_keys")) t.short_keys = value == 0 || value == 1 ? value : -1;
   else if (!strcmp(name, "sparse_order")) t.sparse_order = value != 0;
+  else if (!strcmp(name, "key_halves")) t.key_halves = value == 0 || value == 1 ? value : -1;
   else if (!strcmp(name, "resident")) t.resident = value == 0 || value == 1 ? value : -1;
   else PA_FAIL(PA_ERR_INVALID, "pa_set_tuning: unknown knob '%s'", name);
   return PA_OK;
+}
+
+// Whether a launch of n workgroups of 128 query rows takes 8 wavefronts for each, 4 for either half of its key tiles (template flag
+// KS): where every compute unit gets at most one workgroup anyway, so that 4 wavefronts would leave each SIMD one and nothing to
+// run beside its softmax.  The fold of the halves in LDS and the second set of first tiles want some key tiles to be worth it.
+// Measured against what runs otherwise (B1, bf16, device time): head_dim 64 8 x 4096 tokens 54.6 -> 48.6 us, 3 x 8192 99 -> 79,
+// 16 x 1000 19.3 -> 18.8, 8 x 700 (11 tiles) 14.4 -> 14.8; head_dim 128 16 x 2000 58.8 -> 45.4, 12 x 2000 47.9 -> 41.1, 8 x 4096 80 -> 75,
+// but 8 x 2000 39.4 -> 39.0 and 3 x 3000 41 -> 49, which the key split over more compute units serves, and 3 x 8192 116 -> 120, which the
+// resident workgroups cut evenly.  is_causal: up to two workgroups per unit (the longest decide): head_dim 64 8 x 8192 110 -> 92,
+// 16 x 4096 60.8 -> 54.2, 24 x 3000 (576) 49.8 -> 53.2; head_dim 128 12 x 4096 82 -> 68, 40 x 1500 (480, 24 tiles) 42.6 -> 45.2.
+// A bias with a query dimension gains 1.03 .. 1.3 from 8 tiles on, lists of kept tiles from 32 (8 x 2000 54.9 -> 53.2).
+enum HalvesFor { HALVES_DENSE, HALVES_MASKED_KEYS, HALVES_BIAS, HALVES_LISTS };
+static bool take_halves(int64_t n, int kv_tiles, bool causal, int D, HalvesFor what) {
+  const int want = tuning().key_halves;
+  if (want >= 0) return want == 1 && kv_tiles > 1;
+  if (!mi355x_layout()) return false;
+  const int cus = device_cus();
+  if (causal) return kv_tiles >= 16 && n <= (kv_tiles >= 32 ? 2 * cus : cus + cus / 8);
+  if (n > cus) return false;
+  if (what == HALVES_BIAS) return kv_tiles >= 8;
+  if (what == HALVES_LISTS) return kv_tiles >= 32;
+  if (kv_tiles < 16) return false;
+  if (D == 64 || kv_tiles < 32) return true;
+  return 4 * n >= 3 * cus && (what == HALVES_MASKED_KEYS || kv_tiles <= 64);
 }
 
 // Bytes of workspace the key-split tail of the plan for bm rows per workgroup needs.
@@ -4347,6 +4519,19 @@ static bool pipe_fits(const AttnParams& p, int D) {
 // workgroup per CU makes a partly filled last round dearer).  The choice is the smaller estimate
 // of rounds / throughput; PARAATTN_BM=128|256 forces it, PARAATTN_NO_SPLIT=1 forbids the split.
 // `ws_bytes` is what the caller can lend (0: none); q_block limits 256 for block-sparse launches.
+static bool bound_wanted(int B, int H, int Sq, int Skv, int D);
+
+// The workgroups of a planned dense launch in an order that gives every XCD a contiguous eighth of them, so that the query tiles of a
+// head share an L2: 40 heads x 1000 tokens 42.0 -> 39.3 us (head_dim 64 26.6 -> 25.2), 24 x 1500 x 96 columns 42.4 -> 38.1; level where a
+// head has many query tiles.  Not with key shares, which cost more than whole tiles and would all lie on the last XCDs
+// (12 x 6000, head_dim 64, 135 -> 210), and not where the order of the tiles is that of their lengths.
+static void deal_to_xcds(AttnParams& p) {
+  const int64_t n = (int64_t)p.B * p.H * p.n_qtiles;
+  if (!p.pipe || p.split_s > 1 || p.causal || p.heads_first || n <= 8 || n > 0x3fffffff || !mi355x_layout() || tuning().no_xcd_order) return;
+  p.n_wg = (int)n;
+  p.xcd_chunk = (int)((n + 7) / 8);
+}
+
 static void choose_kernel(AttnParams& p, int D, int q_block, bool dense, size_t ws_bytes, size_t* ws_needed) {
   if (ws_needed) *ws_needed = 0;
   p.pipe = 0;
@@ -4372,6 +4557,10 @@ static void choose_kernel(AttnParams& p, int D, int q_block, bool dense, size_t 
   if (D == 64) {
     p.dt = p.ws_cols = 64;
     if (forced == 256 && (dense || q_block % 256 == 0)) p.bm = 256;
+    if (dense && forced == 0 && !bound_wanted(p.B, p.H, p.Sq, p.Skv, D) && take_halves((int64_t)p.B * p.H * ((p.Sq + 127) / 128), (p.Skv + BN - 1) / BN, p.causal, D, HALVES_DENSE)) {
+      p.key_halves = 1;
+      return order();
+    }
     order();
     const bool may = dense && n_cus > 0 && mi355x_layout() && !p.causal && !tuning().no_split && (ws_needed != nullptr || ws_bytes > 0);
     const int64_t tiles = (int64_t)p.B * p.H * p.n_qtiles;
@@ -4401,6 +4590,10 @@ static void choose_kernel(AttnParams& p, int D, int q_block, bool dense, size_t 
   const int kv_tiles = (p.Skv + BN - 1) / BN;
   const int64_t bh = (int64_t)p.B * p.H;
   const int64_t n128 = bh * ((p.Sq + 127) / 128), n256 = bh * ((p.Sq + 255) / 256);
+  if (forced == 0 && take_halves(n128, kv_tiles, p.causal, D, p.mask != nullptr ? HALVES_MASKED_KEYS : HALVES_DENSE)) {
+    p.key_halves = 1;
+    return order();
+  }
   SplitPlan p128 = plan_split(n128, 2 * cus, kv_tiles, 128, allow), p256 = plan_split(n256, cus, kv_tiles, 256, allow);
   if (!ws_needed) {  // the plan must fit what was lent
     if (split_ws_bytes(p128, 128) > ws_bytes) p128 = plan_split(n128, 2 * cus, kv_tiles, 128, false);
@@ -4469,7 +4662,7 @@ static bool plan_stream(AttnParams& p, int D, const KeySegs* segs, size_t ws_ava
   *ws_need = 0;
   const bool multi = segs != nullptr;
   const int want = tuning().stream;
-  if (want == 0 || (want < 0 && tuning().forced_bm != 0)) return false;  // switched off, or a workgroup size of the other kernels asked for
+  if (want == 0 || (want < 0 && (tuning().forced_bm != 0 || tuning().key_halves == 1))) return false;  // switched off, or a workgroup size of the other kernels asked for
   // per-batch key counts: only for a caller who knows that they leave nearly all keys (the plan is made for all of
   // them, and pieces that end early leave their workgroups idle), one key segment
   if (p.kv_len != nullptr && (!allow_kvlen || multi)) return false;
@@ -4490,6 +4683,7 @@ static bool plan_stream(AttnParams& p, int D, const KeySegs* segs, size_t ws_ava
   // kernels with one workgroup per query tile: this kernel would cut every piece into ranges and pay a second
   // launch to fold them, which at 30..80 us per call is 8..40 % (measured over 2..64 heads and 576..4608 tokens).
   if (want < 0 && !multi && P < cus && (int64_t)P * L <= 6144) return false;
+  if (want < 0 && !multi && p.kv_len == nullptr && tuning().forced_bm == 0 && take_halves((int64_t)p.B * p.H * ((p.Sq + 127) / 128), L, false, D, HALVES_DENSE)) return false;
   // Taken wherever it applies (measured against attn_fwd_d128_pipe_kernel + key-split tail on one box: 119056 keys
   // +0.6 %, Wan self-attention +0.9 %, a ring sweep's block +3.5 %, the sweep in one launch +1.3 %, 16k / 8k / 6k /
   // 3k tokens +1.5 / +2.4 / +7 / +7 %, FLUX +10..17 %, cross-attention to 512 keys +6 %): the hot loop is the same,
@@ -4650,7 +4844,7 @@ static int launch_short(const AttnParams& p, hipStream_t stream) {
 static bool plan_resident_call(const AttnParams& p, int D, ResidentCall& c) {
   int want = tuning().resident;
   if (tuning().no_pipe || p.causal || p.kv_len != nullptr || p.gate != nullptr) return false;
-  if (want < 0 && (tuning().forced_bm != 0 || tuning().stream == 1 || tuning().short_keys == 1)) return false;
+  if (want < 0 && (tuning().forced_bm != 0 || tuning().stream == 1 || tuning().short_keys == 1 || tuning().key_halves == 1)) return false;
   c.q = p.q; c.k = p.k; c.v = p.v; c.out = p.out; c.lse = p.lse;
   c.B = p.B; c.H = p.H; c.Sq = p.Sq; c.Skv = p.Skv;
   c.qs_b = p.qs_b; c.qs_h = p.qs_h; c.qs_s = p.qs_s;
@@ -4830,6 +5024,7 @@ static int attn_fwd_dense(const void* q, const void* k, const void* v, void* out
     return dtype == PA_DTYPE_BF16 ? launch_stream<BF16>(p, (hipStream_t)stream) : launch_stream<F16>(p, (hipStream_t)stream);
   }
   if (p.split_s > 1) lend_split_ws(p, ws_base);
+  deal_to_xcds(p);
   return dispatch_attn<false>(p, dtype, D, (hipStream_t)stream);
 }
 
@@ -4970,23 +5165,28 @@ static int launch_masked(const AttnParams& p, int mask_kind, hipStream_t stream)
 }
 
 // A pipelined kernel with its mask handling PM, or for rows narrower than D (W < D), planned by choose_kernel like a dense call with per-batch key counts.
-template <typename T, int D, int PM, int NW, int W = D>
+template <typename T, int D, int PM, int WAVES, int W = D>
 static int launch_pipe_variant(const AttnParams& p, hipStream_t stream) {
+  if constexpr (WAVES != HALVES) {
+    if (p.key_halves) return launch_pipe_variant<T, D, PM, HALVES, W>(p, stream);
+  }
+  constexpr int NW = WAVES == HALVES ? 8 : WAVES;
   int64_t nblocks = (int64_t)p.B * p.H * p.n_qtiles;
   if (p.split_s > 1) nblocks = (int64_t)p.split_main + (int64_t)p.split_tiles * p.split_s;
+  if (p.xcd_chunk > 0) nblocks = 8 * (int64_t)p.xcd_chunk;
   if constexpr (D == 128) {
-    const size_t smem = 4 * TILE_BYTES + (PM == PM_KEYBIAS ? NW * PM_SLOT_BYTES : 0);
+    const size_t smem = (WAVES == HALVES ? 8 : 4) * TILE_BYTES + (PM == PM_KEYBIAS ? NW * PM_SLOT_BYTES : 0);
     static bool attr_done[PA_MAX_DEVICES] = {};  // benign race: the call is idempotent
     const int dev = current_device();
     if (dev < 0 || !attr_done[dev]) {
-      hipError_t e = hipFuncSetAttribute((const void*)attn_fwd_d128_pipe_kernel<T, false, NW, false, false, PM, W>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+      hipError_t e = hipFuncSetAttribute((const void*)attn_fwd_d128_pipe_kernel<T, false, WAVES, false, false, PM, W>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
       if (e != hipSuccess) PA_FAIL(PA_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
       if (dev >= 0) attr_done[dev] = true;
     }
-    hipLaunchKernelGGL((attn_fwd_d128_pipe_kernel<T, false, NW, false, false, PM, W>), dim3((unsigned)nblocks), dim3(64 * NW), smem, stream, p);
+    hipLaunchKernelGGL((attn_fwd_d128_pipe_kernel<T, false, WAVES, false, false, PM, W>), dim3((unsigned)nblocks), dim3(64 * NW), smem, stream, p);
     PA_CHECK_LAUNCH("attention kernel (masked or narrow rows)");
   } else {  // (masks with a query dimension are planned without a split)
-    const int rc = launch_d64<T, false, NW, false, PM, (W < 64), PM != PM_BITS && PM != PM_BIAS>(p, nblocks, stream);
+    const int rc = launch_d64<T, false, WAVES, false, PM, (W < 64), PM != PM_BITS && PM != PM_BIAS>(p, nblocks, stream);
     if (rc != PA_OK) return rc;
   }
   if (p.split_s > 1) {
@@ -5052,6 +5252,7 @@ extern "C" int pa_attn_fwd_narrow(const void* q, const void* k, const void* v, v
   if (B <= 0 || H <= 0 || Sq <= 0 || !plan_narrow(p, D, workspace ? workspace_bytes : 0, nullptr))
     PA_FAIL(PA_ERR_UNSUPPORTED, "pa_attn_fwd_narrow does not take this call (pa_attn_fwd_narrow_plan tells)");
   if (p.split_s > 1) lend_split_ws(p, workspace);
+  deal_to_xcds(p);
   return dtype == PA_DTYPE_BF16 ? launch_narrow<BF16>(p, (hipStream_t)stream) : launch_narrow<F16>(p, (hipStream_t)stream);
 }
 
@@ -5144,6 +5345,8 @@ static int launch_masked_bits(AttnParams p, const int64_t ms[4], void* ws, hipSt
   p.bm = 128;
   p.n_qtiles = l.nQ;
   p.split_s = 0;
+  p.key_halves = take_halves((int64_t)p.B * p.H * l.nQ, l.nK, false, D, HALVES_LISTS);
+  deal_to_xcds(p);
   return launch_pipe_variant<T, D, PM_BITS, 4>(p, stream);
 }
 
@@ -5257,6 +5460,7 @@ extern "C" int pa_attn_fwd_masked(const void* q, const void* k, const void* v, v
     if (mask_kind != MASK_BOOL && plan_resident_call(p, D, rcall)) return launch_resident(rcall, dtype, D, st);
     choose_kernel(p, D, 256, true, ws ? ws_bytes : 0, nullptr);
     if (p.split_s > 1) lend_split_ws(p, ws);
+    deal_to_xcds(p);
     if (dtype == PA_DTYPE_BF16) return D == 128 ? launch_masked_pipe<BF16, 128>(p, st) : launch_masked_pipe<BF16, 64>(p, st);
     return D == 128 ? launch_masked_pipe<F16, 128>(p, st) : launch_masked_pipe<F16, 64>(p, st);
   };
@@ -5281,6 +5485,8 @@ extern "C" int pa_attn_fwd_masked(const void* q, const void* k, const void* v, v
     choose_kernel(p, D, 128, true, 0, nullptr);
     p.bm = 128;
     p.n_qtiles = (Sq + 127) / 128;
+    p.key_halves = take_halves((int64_t)B * H * p.n_qtiles, (Skv + BN - 1) / BN, false, D, HALVES_BIAS);
+    deal_to_xcds(p);
     if (dtype == PA_DTYPE_BF16) return D == 128 ? launch_pipe_variant<BF16, 128, PM_BIAS, 4>(p, st) : launch_pipe_variant<BF16, 64, PM_BIAS, 4>(p, st);
     return D == 128 ? launch_pipe_variant<F16, 128, PM_BIAS, 4>(p, st) : launch_pipe_variant<F16, 64, PM_BIAS, 4>(p, st);
   }
@@ -5501,6 +5707,7 @@ static int blocksparse_launch(const void* q, const void* k, const void* v, void*
   const int q_hi = q_lo + nQ * q_block;
   const int tiles_right = (Sq - q_hi + p.bm - 1) / p.bm;
   p.n_qtiles = p.tiles_left + nQ * p.tiles_per_block + tiles_right;
+  if (p.pipe && p.bm == 128 && !pair) p.key_halves = take_halves((int64_t)B * H * p.n_qtiles, (Skv + BN - 1) / BN, false, D, HALVES_LISTS);
   if (D == 128 && p.pipe && !tuning().no_xcd_order && mi355x_layout())
     p.xcd_chunk = (int)(((int64_t)B * H * p.n_qtiles + 7) / 8);
   return dispatch_attn<true>(p, dtype, D, (hipStream_t)stream);

@@ -1061,6 +1061,63 @@ def test_short_key_kernel(cuda, dtype, tuning):
         assert torch.equal(out_d, want[0]) and torch.equal(lse_d, want[1]), (B, H, Sq, Skv)
 
 
+@pytest.mark.parametrize("D", [128, 64, 72, 40])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_key_halves(cuda, dtype, D, tuning):
+    """Workgroups of 8 wavefronts, 4 for either half of the key tiles, forced on: one tile for one half and none for the other, odd and
+    even numbers of tiles, ragged ends; is_causal (rows whose second half is all masked); key masks, key biases, masks with a query
+    dimension as bits (with key tiles that no row keeps: lists of one tile, where the second half has none) and as biases. Against the
+    fp64 oracle and the plain form."""
+    op = torch.ops.para_attn.attention_forward_with_lse
+    tuning("resident", 0)
+    B, H = 2, 2
+    for Sq, Skv in ((1, 65), (130, 128), (257, 129), (64, 700), (300, 1000)):
+        q, k, v = inputs.qkv(B, H, Sq, Skv, D, seed=Sq + Skv, dtype=dtype)
+        g = torch.Generator().manual_seed(Skv)
+        keys = torch.rand(B, 1, 1, Skv, generator=g) < 0.5
+        keys[1] = False
+        keys[1, ..., : max(1, Skv // 5)] = True
+        bits = torch.rand(B, H, Sq, Skv, generator=g) < 0.3
+        bits[..., 64:128] = False
+        bits[0, 0, 0] = False
+        masks = [(None, False, None), (None, True, torch.ones(Sq, Skv, dtype=torch.bool).tril())]
+        if D in (64, 128):
+            masks += [(keys, False, keys), (torch.zeros(B, 1, 1, Skv).masked_fill(~keys, -math.inf), False, keys)]
+            if Sq > 1:
+                masks += [(bits, False, bits), (torch.zeros(B, H, Sq, Skv).to(dtype).masked_fill(~bits, -math.inf), False, bits)]
+        for mask, causal, keep in masks:
+            got = {}
+            for knob in (0, 1):
+                tuning("key_halves", knob)
+                got[knob] = op(q.to(cuda), k.to(cuda), v.to(cuda), None if mask is None else mask.to(cuda), is_causal=causal)
+            keep_np = None if keep is None else np.broadcast_to(keep.numpy(), (B, H, Sq, Skv))
+            ref_out, ref_lse = oattn.sdpa_lse_f64(q.double().numpy(), k.double().numpy(), v.double().numpy(), None, keep_np)
+            what = f"key halves {(Sq, Skv, D, dtype, None if mask is None else (mask.shape, mask.dtype), causal)}"
+            _check(*got[1], ref_out, ref_lse, what)
+            ok = got[0][1].isfinite()
+            assert torch.equal(ok, got[1][1].isfinite()), what
+            assert (got[0][0].float() - got[1][0].float()).abs().max().item() <= 2e-2 and (got[0][1] - got[1][1])[ok].abs().max().item() <= 1e-4, what
+
+
+def test_key_halves_block_sparse_and_ring(cuda, tuning):
+    tuning("key_halves", 1)
+    from oracle import sparse as osparse
+
+    for D in (128, 64):
+        q, k, v = inputs.qkv(1, 2, 512, 640, D, seed=D)
+        for bm in (torch.rand(2, 4, 5, generator=torch.Generator().manual_seed(D)) < 0.5, torch.eye(8, 10).bool()[None]):  # (lists of one 64-key tile)
+            keep = np.concatenate([osparse.expand_block_mask(m.numpy(), 512, 640)[None] for m in bm])
+            ref_out, ref_lse = oattn.sdpa_lse_f64(q.float().numpy(), k.float().numpy(), v.float().numpy(), None, np.broadcast_to(keep, (1, 2, 512, 640)))
+            out, lse = torch.ops.para_attn.attention_forward_block_sparse(q.to(cuda), k.to(cuda), v.to(cuda), bm.to(cuda))
+            _check(out, lse, ref_out, ref_lse, f"key halves, block-sparse {D}")
+    q, k, v = inputs.qkv(1, 3, 500, 999, 128, seed=4)
+    ref_out, ref_lse = oattn.sdpa_lse_f64(q.float().numpy(), k.float().numpy(), v.float().numpy())
+    ks, vs = ([t[:, :, i : i + 333].contiguous().to(cuda) for i in (0, 333, 666)] for t in (k, v))
+    for fused in (True, "sweep"):
+        out, lse = paraattention_amd.ring_sweep(q.to(cuda), ks, vs, fused=fused)
+        _check(out, lse, ref_out, ref_lse, f"key halves, ring {fused}")
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("D,most,most_biased", [(128, 288, 256), (64, 576, 512)])
 def test_resident_key_kernel(cuda, dtype, D, most, most_biased, tuning):
