@@ -1061,6 +1061,20 @@ def test_short_key_kernel(cuda, dtype, tuning):
         assert torch.equal(out_d, want[0]) and torch.equal(lse_d, want[1]), (B, H, Sq, Skv)
 
 
+@pytest.mark.parametrize("Skv", [1, 5, 8, 9, 63, 71, 515])
+def test_mask_packing_ends(cuda, Skv):
+    """Boolean masks with a query dimension whose rows end inside eight keys, are shorter than eight, begin at any byte, or whose keys are
+    not adjacent; query rows that end inside the 16 a wavefront has on their way."""
+    for Sq in (2, 17, 131):
+        q, k, v = inputs.qkv(1, 2, Sq, Skv, 128, seed=Sq + Skv)
+        wide = torch.rand(1, 2, Sq, Skv + 3, generator=torch.Generator().manual_seed(Skv)) < 0.6
+        for keep in (wide[..., 3:], wide[..., :Skv].transpose(2, 3).contiguous().transpose(2, 3)):
+            ref_out, ref_lse = oattn.sdpa_lse_f64(q.float().numpy(), k.float().numpy(), v.float().numpy(), None, keep.numpy())
+            mask = wide.to(cuda)[..., 3:] if keep.stride(-1) == 1 else keep.to(cuda)
+            out, lse = torch.ops.para_attn.attention_forward_with_lse(q.to(cuda), k.to(cuda), v.to(cuda), mask)
+            _check(out, lse, ref_out, ref_lse, f"mask packing {(Sq, Skv, keep.stride())}")
+
+
 @pytest.mark.parametrize("D", [128, 64, 72, 40])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_key_halves(cuda, dtype, D, tuning):
