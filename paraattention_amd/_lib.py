@@ -148,11 +148,12 @@ def host_calls():
     """The module with the host side of the ordinary calls (csrc/host_calls.cpp), on top of the same library."""
     global _host
     if _host is None:
-        load()
+        lib = load()
         try:
             from . import _host_calls
         except ImportError as e:
             raise ImportError(f"paraattention_amd/_host_calls.so cannot be loaded ({e}): build it with `make -C {os.path.join(_HERE, 'csrc')}`") from e
+        _host_calls.bind(lib._handle)
         _host = _host_calls
     return _host
 

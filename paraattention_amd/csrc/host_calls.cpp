@@ -8,6 +8,7 @@
 
 #include <ATen/ATen.h>
 #include <torch/csrc/Exceptions.h>
+#include <dlfcn.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cmath>
@@ -18,6 +19,44 @@
 namespace {
 
 using at::Tensor;
+
+// The entries of the library that _lib.py has loaded, looked up in that very one (another build of it may be in use).
+#define ENTRIES(X) \
+  X(pa_attn_fwd_blocksparse) \
+  X(pa_attn_fwd_call_workspace_bytes) \
+  X(pa_attn_fwd_lse_ws) \
+  X(pa_attn_fwd_masked) \
+  X(pa_attn_fwd_masked_call_workspace_bytes) \
+  X(pa_attn_fwd_narrow) \
+  X(pa_attn_fwd_narrow_plan) \
+  X(pa_blocksparse_workspace_bytes) \
+  X(pa_fbcache_apply_residual) \
+  X(pa_fbcache_apply_residual2) \
+  X(pa_fbcache_residual) \
+  X(pa_fbcache_residual_ratio) \
+  X(pa_fbcache_residual_ratio_strided) \
+  X(pa_taylorseer_update) \
+  X(pa_taylorseer_value)
+struct Library {
+#define MEMBER(name) decltype(&::name) name;
+  ENTRIES(MEMBER)
+#undef MEMBER
+};
+Library lib = {};
+
+// bind(handle of the loaded library): before any other function of this module
+PyObject* bind(PyObject*, PyObject* arg) {
+  void* const handle = PyLong_AsVoidPtr(arg);
+  if (PyErr_Occurred()) return nullptr;
+#define LOOK_UP(entry)                                                                                                  \
+  if ((lib.entry = (decltype(&::entry))dlsym(handle, #entry)) == nullptr) {                                             \
+    PyErr_SetString(PyExc_ImportError, #entry " is missing in the loaded library");                                     \
+    return nullptr;                                                                                                     \
+  }
+  ENTRIES(LOOK_UP)
+#undef LOOK_UP
+  Py_RETURN_NONE;
+}
 
 // None, or a tensor's C++ handle (null and an error set: neither)
 bool optional_tensor(PyObject* o, const Tensor** out) {
@@ -125,9 +164,9 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const Strides3 qs(q), ks(k), vs(v);
   const int dt = dtype_code(q.scalar_type());
   size_t bytes = 0;
-  if (pm != nullptr) bytes = pa_attn_fwd_masked_call_workspace_bytes(B, H, Sq, Skv, D, ks.v, vs.v, kind, ms);
-  else if (native) bytes = pa_attn_fwd_call_workspace_bytes(B, H, Sq, Skv, D, ks.v, vs.v, 0, causal);
-  else if (!pa_attn_fwd_narrow_plan(B, H, Sq, Skv, D, ks.v, vs.v, causal, &bytes)) Py_RETURN_NONE;
+  if (pm != nullptr) bytes = lib.pa_attn_fwd_masked_call_workspace_bytes(B, H, Sq, Skv, D, ks.v, vs.v, kind, ms);
+  else if (native) bytes = lib.pa_attn_fwd_call_workspace_bytes(B, H, Sq, Skv, D, ks.v, vs.v, 0, causal);
+  else if (!lib.pa_attn_fwd_narrow_plan(B, H, Sq, Skv, D, ks.v, vs.v, causal, &bytes)) Py_RETURN_NONE;
   Tensor out, lse;
   int rc;
   {
@@ -138,13 +177,13 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const Tensor ws = scratch(bytes, q);
     const Strides3 os(out);
     if (pm != nullptr)
-      rc = pa_attn_fwd_masked(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), (float*)ptr(lse), dt, B, H, Sq, Skv, D, qs.v, ks.v, vs.v, os.v,
+      rc = lib.pa_attn_fwd_masked(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), (float*)ptr(lse), dt, B, H, Sq, Skv, D, qs.v, ks.v, vs.v, os.v,
                               (float)scale, pm->data_ptr(), kind, ms, ptr(ws), bytes, stream);
     else if (native)
-      rc = pa_attn_fwd_lse_ws(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), (float*)ptr(lse), dt, B, H, Sq, Skv, D, qs.v, ks.v, vs.v, os.v,
+      rc = lib.pa_attn_fwd_lse_ws(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), (float*)ptr(lse), dt, B, H, Sq, Skv, D, qs.v, ks.v, vs.v, os.v,
                               (float)scale, nullptr, causal, ptr(ws), bytes, stream);
     else
-      rc = pa_attn_fwd_narrow(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), (float*)ptr(lse), dt, B, H, Sq, Skv, D, qs.v, ks.v, vs.v, os.v,
+      rc = lib.pa_attn_fwd_narrow(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), (float*)ptr(lse), dt, B, H, Sq, Skv, D, qs.v, ks.v, vs.v, os.v,
                               (float)scale, causal, ptr(ws), bytes, stream);
   }
   if (rc != PA_OK) return PyLong_FromLong(rc);
@@ -181,12 +220,12 @@ PyObject* fbcache_residual(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     ratio = at::empty({}, h->options());
     const int dt = dtype_code(h->scalar_type());
     const size_t ws_bytes = prev ? ws->numel() * ws->element_size() : 0;
-    if (!prev) rc = pa_fbcache_residual(h->data_ptr(), h0->data_ptr(), resid.data_ptr(), dt, h->numel(), ratio.data_ptr(), stream);
+    if (!prev) rc = lib.pa_fbcache_residual(h->data_ptr(), h0->data_ptr(), resid.data_ptr(), dt, h->numel(), ratio.data_ptr(), stream);
     else if (step == 1)
-      rc = pa_fbcache_residual_ratio(h->data_ptr(), h0->data_ptr(), prev->data_ptr(), resid.data_ptr(), dt, h->numel(), ratio.data_ptr(), nullptr,
+      rc = lib.pa_fbcache_residual_ratio(h->data_ptr(), h0->data_ptr(), prev->data_ptr(), resid.data_ptr(), dt, h->numel(), ratio.data_ptr(), nullptr,
                                      ws->data_ptr(), ws_bytes, stream);
     else
-      rc = pa_fbcache_residual_ratio_strided(h->data_ptr(), h0->data_ptr(), prev->data_ptr(), resid.data_ptr(), dt, h->numel() / h->size(-1), h->size(-1),
+      rc = lib.pa_fbcache_residual_ratio_strided(h->data_ptr(), h0->data_ptr(), prev->data_ptr(), resid.data_ptr(), dt, h->numel() / h->size(-1), h->size(-1),
                                              (int)step, ratio.data_ptr(), nullptr, ws->data_ptr(), ws_bytes, stream);
   }
   if (rc != PA_OK) return PyLong_FromLong(rc);
@@ -206,7 +245,7 @@ PyObject* fbcache_apply(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   {
     pybind11::gil_scoped_release no_gil;
     out = at::empty(h->sizes(), h->options());
-    rc = pa_fbcache_apply_residual(r->data_ptr(), h->data_ptr(), out.data_ptr(), dtype_code(h->scalar_type()), h->numel(), stream);
+    rc = lib.pa_fbcache_apply_residual(r->data_ptr(), h->data_ptr(), out.data_ptr(), dtype_code(h->scalar_type()), h->numel(), stream);
   }
   if (rc != PA_OK) return PyLong_FromLong(rc);
   return THPVariable_Wrap(out);
@@ -229,7 +268,7 @@ PyObject* fbcache_apply_pair(PyObject*, PyObject* const* args, Py_ssize_t nargs)
     pybind11::gil_scoped_release no_gil;
     out = at::empty(h->sizes(), h->options());
     out2 = at::empty(h2->sizes(), h2->options());
-    rc = pa_fbcache_apply_residual2(r->data_ptr(), h->data_ptr(), out.data_ptr(), h->numel(), r2->data_ptr(), h2->data_ptr(), out2.data_ptr(), h2->numel(),
+    rc = lib.pa_fbcache_apply_residual2(r->data_ptr(), h->data_ptr(), out.data_ptr(), h->numel(), r2->data_ptr(), h2->data_ptr(), out2.data_ptr(), h2->numel(),
                                     dtype_code(h->scalar_type()), stream);
   }
   if (rc != PA_OK) return PyLong_FromLong(rc);
@@ -280,7 +319,7 @@ PyObject* taylorseer_value(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   {
     pybind11::gil_scoped_release no_gil;
     out = at::empty(d[0]->sizes(), d[0]->options());
-    rc = pa_taylorseer_value(src, m, coef, pw, h ? h->data_ptr() : nullptr, out.data_ptr(), dtype_code(out.scalar_type()), out.numel(), stream);
+    rc = lib.pa_taylorseer_value(src, m, coef, pw, h ? h->data_ptr() : nullptr, out.data_ptr(), dtype_code(out.scalar_type()), out.numel(), stream);
   }
   if (rc != PA_OK) return PyLong_FromLong(rc);
   return THPVariable_Wrap(out);
@@ -309,7 +348,7 @@ PyObject* taylorseer_derivatives(PyObject*, PyObject* const* args, Py_ssize_t na
       src[i] = d[i]->data_ptr();
       dst[i] = cur[i].data_ptr();
     }
-    rc = pa_taylorseer_update(y->data_ptr(), src, dst, n, dtype_code(y->scalar_type()), y->numel(), (float)window, stream);
+    rc = lib.pa_taylorseer_update(y->data_ptr(), src, dst, n, dtype_code(y->scalar_type()), y->numel(), (float)window, stream);
   }
   if (rc != PA_OK) return PyLong_FromLong(rc);
   PyObject* list = PyList_New(n);
@@ -341,12 +380,12 @@ PyObject* block_sparse(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   int rc;
   {
     pybind11::gil_scoped_release no_gil;
-    const size_t bytes = pa_blocksparse_workspace_bytes((int)Hm, (int)nQ, (int)nK);
+    const size_t bytes = lib.pa_blocksparse_workspace_bytes((int)Hm, (int)nQ, (int)nK);
     out = out_like(q);
     lse = at::empty({B, H, Sq}, q.options().dtype(at::kFloat));
     const Tensor ws = scratch((bytes + 3) / 4 * 4, q);
     const Strides3 os(out);
-    rc = pa_attn_fwd_blocksparse(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), (float*)lse.data_ptr(), dtype_code(q.scalar_type()), B, H, Sq, Skv,
+    rc = lib.pa_attn_fwd_blocksparse(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), (float*)lse.data_ptr(), dtype_code(q.scalar_type()), B, H, Sq, Skv,
                                  D, qs.v, ks.v, vs.v, os.v, (float)scale, (const uint8_t*)m->data_ptr(), (int)Hm, (int)nQ, (int)nK, 0, (int)(Sq / nQ), 0,
                                  (int)(Skv / nK), (int32_t*)ptr(ws), bytes, stream);
   }
@@ -356,7 +395,8 @@ PyObject* block_sparse(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 }
 
 #define METHOD(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {METHOD(attention),        METHOD(block_sparse),     METHOD(fbcache_residual),       METHOD(fbcache_apply),
+PyMethodDef methods[] = {{"bind", bind, METH_O, nullptr},
+                         METHOD(attention),        METHOD(block_sparse),     METHOD(fbcache_residual),       METHOD(fbcache_apply),
                          METHOD(fbcache_apply_pair), METHOD(taylorseer_value), METHOD(taylorseer_derivatives), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_calls", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
