@@ -607,7 +607,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void attn_fwd_kernel(const AttnParams 
 // read back from LDS cost 3 and 1 %.  A tile that drops no key, or whose biases are all zero, costs
 // nothing beyond the vote that says so.  Measured against the per-score kernel (attn_fwd_kernel<MASK>, register-staged
 // tiles): two samples x 24 heads x 7800 rows against 256 keys with a bias 171 -> 104 us (0.47 PFLOP/s; bound by what a
-// workgroup does around its four key tiles), 24 heads x 4352 tokens with holes in the key mask, scan and two empty
+// workgroup does around its four key tiles; attn_resident.hip takes that call now), 24 heads x 4352 tokens with holes in the key mask, scan and two empty
 // launches included there, 390..700 -> 236 us (0.98 PFLOP/s, what the unmasked call of that size reaches, and what a mask that
 // keeps a prefix took before, in the fast kernels behind the scan); three packed samples
 // behind a common prefix, 2 x 24 heads x 8000 tokens 6.65 -> 0.88 ms, 16 heads x 3000 326 -> 94 us (about half the key tiles
