@@ -112,7 +112,8 @@ struct AttnParams {
   // tile; the last split_tiles query tiles are computed by split_s workgroups each, over
   // consecutive shares of the key tiles, which leave normalised fp32 partial outputs and their
   // LSE in the workspace (piece-major) for attn_split_merge_kernel.  split_s <= 1: no split.
-  int n_wg;        // dense pipelined kernels with xcd_chunk: workgroups that have work
+  int n_wg;        // dense pipelined kernels with xcd_chunk: workgroups that have work, in each of xcd_units
+  int xcd_units;   // the same: parts of the launch that are dealt to the XCDs one after the other (deal_to_xcds)
   int key_halves;  // pipelined kernels: 128-row workgroups of 8 wavefronts, 4 for either half of the key tiles (template flag KS)
   int xcd_chunk;  // block-sparse pipelined kernel: ceil(workgroups / 8), 0 = plain order
   // 256-row dense kernel: *bound_flag != 0 says that no score can leave [-60, 60] in the log2 domain (see
@@ -145,6 +146,21 @@ struct AttnParams {
   uint32_t gate_mask;
   StreamPlan st;  // attn_fwd_d128_stream_kernel only
 };
+
+// Workgroup number -> tile of a launch that deal_to_xcds has ordered (workgroups go to the 8 XCDs in turn: each XCD holds a contiguous
+// eighth of every unit's tiles).  False: this workgroup has no work.
+__device__ __forceinline__ bool dealt_tile(const AttnParams& p, int& tile) {
+  const int xcd = tile & 7;
+  int at = tile >> 3, first = 0;
+  if (p.xcd_units > 1) {
+    const int unit = at / p.xcd_chunk;
+    at -= unit * p.xcd_chunk;
+    first = unit * p.n_wg;
+  }
+  at += xcd * p.xcd_chunk;
+  tile = first + at;
+  return at < p.n_wg;
+}
 
 // Whether the value that an earlier launch left in *gate (0 .. 31) is one of those a launch runs for.
 __device__ __forceinline__ bool gate_open(const int* gate, uint32_t mask) { return ((mask >> (*gate & 31)) & 1u) != 0; }
@@ -1210,8 +1226,7 @@ __global__ __launch_bounds__(WAVES == 4 ? 256 : 512, WAVES == 4 ? 2 : 1) void at
       if (tile >= p.B * p.H * p.n_qtiles) return;
     }
   } else if (p.xcd_chunk > 0) {
-    tile = (tile & 7) * p.xcd_chunk + (tile >> 3);
-    if (tile >= p.n_wg) return;
+    if (!dealt_tile(p, tile)) return;
   }
   if constexpr (ALL) {
     if (p.split_s > 1 && tile >= p.split_main) {
@@ -1895,8 +1910,7 @@ __global__ __launch_bounds__(WAVES == 4 ? 256 : 512, WAVES == 4 ? 2 : 1) void at
   int piece_slot = -1;  // >= 0: this workgroup computes one key share of a split query tile
   if constexpr (!SPARSE) {
     if (p.xcd_chunk > 0) {
-      tile = (tile & 7) * p.xcd_chunk + (tile >> 3);
-      if (tile >= p.n_wg) return;
+      if (!dealt_tile(p, tile)) return;
     }
   }
   if constexpr (CUT) {
@@ -4220,7 +4234,7 @@ static void fill_params(AttnParams& p, const void* q, const void* k, const void*
   p.order = nullptr;
   p.Hm = 0; p.nQ = 0; p.cap = 0; p.q_lo = 0; p.q_block = 0; p.pair = 0; p.tiles_left = 0; p.tiles_per_block = 0;
   p.bm = BM; p.pipe = 0;
-  p.xcd_chunk = 0; p.n_wg = 0; p.key_halves = 0;
+  p.xcd_chunk = 0; p.n_wg = 0; p.xcd_units = 1; p.key_halves = 0;
   p.causal = 0; p.heads_first = 0;
   p.acc_out = nullptr; p.acc_lse = nullptr; p.acc_first = 0;
   p.split_main = 0; p.split_tiles = 0; p.split_s = 0; p.ws_out = nullptr; p.ws_lse = nullptr; p.ws_cols = 128;
@@ -4270,7 +4284,7 @@ static int launch_attn(const AttnParams& p, hipStream_t stream) {
     PA_FAIL(PA_ERR_UNSUPPORTED, "accumulation / key split reached a kernel that has neither");
   if (p.out == nullptr && p.acc_out == nullptr) PA_FAIL(PA_ERR_INVALID, "null output pointer");
   if (p.split_s > 1) nblocks = (int64_t)p.split_main + (int64_t)p.split_tiles * p.split_s;
-  if (p.xcd_chunk > 0) nblocks = 8 * (int64_t)p.xcd_chunk;
+  if (p.xcd_chunk > 0) nblocks = 8 * (int64_t)p.xcd_chunk * p.xcd_units;
   const void* fn;
   size_t smem;
   int slot;
@@ -4524,12 +4538,23 @@ static bool bound_wanted(int B, int H, int Sq, int Skv, int D);
 // The workgroups of a planned dense launch in an order that gives every XCD a contiguous eighth of them, so that the query tiles of a
 // head share an L2: 40 heads x 1000 tokens 42.0 -> 39.3 us (head_dim 64 26.6 -> 25.2), 24 x 1500 x 96 columns 42.4 -> 38.1; level where a
 // head has many query tiles.  Not with key shares, which cost more than whole tiles and would all lie on the last XCDs
-// (12 x 6000, head_dim 64, 135 -> 210), and not where the order of the tiles is that of their lengths.
+// (12 x 6000, head_dim 64, 135 -> 210), and not where the order of the tiles is that of their lengths.  Where the batch elements may keep
+// different numbers of keys (per-batch key counts, boolean key masks) every XCD gets an eighth of each of them: 2 x 24 heads x 4096
+// tokens, one element keeping 512 keys, 237..270 us (one eighth of the whole launch each 380, plain order 237..263), 2 x 24 x 12000 x 64
+// columns, one keeping 1000, 1007 (1787, 1010), and 2 x 40 x 1000, all kept, 62.8 (63.5, 71.2).
+// Their last chunk is short on the same XCDs every time, so it must not be short by more than a 64th of them; masks that differ
+// by head leave the workgroups in plain order.
 static void deal_to_xcds(AttnParams& p) {
   const int64_t n = (int64_t)p.B * p.H * p.n_qtiles;
   if (!p.pipe || p.split_s > 1 || p.causal || p.heads_first || n <= 8 || n > 0x3fffffff || !mi355x_layout() || tuning().no_xcd_order) return;
-  p.n_wg = (int)n;
-  p.xcd_chunk = (int)((n + 7) / 8);
+  const bool key_mask = p.mask != nullptr && p.mask_kind == MASK_BOOL;
+  if (key_mask && p.H > 1 && p.ms_h != 0) return;
+  const int units = p.kv_len != nullptr || (key_mask && p.ms_b != 0) ? p.B : 1;
+  const int64_t per = n / units, chunk = (per + 7) / 8;
+  if (units > 1 && (8 * chunk - per) * 64 > per) return;
+  p.n_wg = (int)per;
+  p.xcd_chunk = (int)chunk;
+  p.xcd_units = units;
 }
 
 static void choose_kernel(AttnParams& p, int D, int q_block, bool dense, size_t ws_bytes, size_t* ws_needed) {
@@ -5173,7 +5198,7 @@ static int launch_pipe_variant(const AttnParams& p, hipStream_t stream) {
   constexpr int NW = WAVES == HALVES ? 8 : WAVES;
   int64_t nblocks = (int64_t)p.B * p.H * p.n_qtiles;
   if (p.split_s > 1) nblocks = (int64_t)p.split_main + (int64_t)p.split_tiles * p.split_s;
-  if (p.xcd_chunk > 0) nblocks = 8 * (int64_t)p.xcd_chunk;
+  if (p.xcd_chunk > 0) nblocks = 8 * (int64_t)p.xcd_chunk * p.xcd_units;
   if constexpr (D == 128) {
     const size_t smem = (WAVES == HALVES ? 8 : 4) * TILE_BYTES + (PM == PM_KEYBIAS ? NW * PM_SLOT_BYTES : 0);
     static bool attr_done[PA_MAX_DEVICES] = {};  // benign race: the call is idempotent
@@ -5362,7 +5387,6 @@ static int launch_masked_bits(AttnParams p, const int64_t ms[4], void* ws, hipSt
   p.n_qtiles = l.nQ;
   p.split_s = 0;
   p.key_halves = take_halves((int64_t)p.B * p.H * l.nQ, l.nK, false, D, HALVES_LISTS);
-  deal_to_xcds(p);
   return launch_pipe_variant<T, D, PM_BITS, 4>(p, stream);
 }
 

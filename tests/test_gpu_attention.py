@@ -12,7 +12,7 @@ import torch
 import paraattention_amd  # noqa: F401
 from oracle import attention as oattn
 from oracle import inputs
-from paraattention_amd import _lib
+from paraattention_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -1130,6 +1130,58 @@ def test_key_halves_block_sparse_and_ring(cuda, tuning):
     for fused in (True, "sweep"):
         out, lse = paraattention_amd.ring_sweep(q.to(cuda), ks, vs, fused=fused)
         _check(out, lse, ref_out, ref_lse, f"key halves, ring {fused}")
+
+
+@pytest.mark.parametrize("D", [128, 64])
+@pytest.mark.parametrize("B,H,S", [(2, 24, 1400), (3, 8, 4200), (2, 37, 1800), (5, 7, 1200)])
+def test_batch_elements_of_different_length_in_any_order(cuda, B, H, S, D, tuning):
+    """Key masks and key counts that differ by batch element, with the workgroups dealt to the XCDs an eighth of every batch element at a
+    time (where a batch element's query tiles divide by 8, nearly do, and do not): the same bits as in plain order."""
+    tuning("no_split", 1)
+    g = torch.Generator(device=cuda).manual_seed(S)
+    q, k, v = (torch.randn(B, H, S, D, generator=g, device=cuda).bfloat16() for _ in range(3))
+    counts = torch.tensor([S // 8, S, 0, S - 1, 64][:B], dtype=torch.int32, device=cuda)
+    keys = (torch.arange(S, device=cuda) < counts[:, None])[:, None, None, :]
+    by_head = keys & (torch.arange(H, device=cuda) % 3 != 0)[None, :, None, None]
+    calls = [lambda m=m: torch.ops.para_attn.attention_forward_with_lse(q, k, v, m) for m in (keys, by_head)]
+    calls.append(lambda: ops._dense_forward(q, k, v, None, True, kv_len=counts))
+    for n, call in enumerate(calls):
+        got = []
+        for plain in (1, 0):
+            tuning("no_xcd_order", plain)
+            got.append(call())
+        assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]), n
+        lens = [c * (n != 1 or h % 3 != 0) for c in counts.tolist() for h in (0, 1)]
+        kept = got[1][1][:, :2].isfinite().all(-1).flatten().tolist()
+        assert kept == [x > 0 for x in lens], n
+
+
+def _device_us(call):
+    times = []
+    for _ in range(7):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        call()
+        a.record()
+        for _ in range(5):
+            call()
+        b.record()
+        b.synchronize()
+        times.append(a.elapsed_time(b) * 200)
+    return sorted(times)[3]
+
+
+@pytest.mark.parametrize("S,kept,D", [(4096, 512, 128), (12000, 1000, 64)])  # a key mask, and one with per-batch key counts behind a scan
+def test_unequal_batch_elements_fill_the_chip(cuda, S, kept, D, tuning):
+    """A batch element that keeps few keys beside one that keeps all: dealt to XCDs by whole batch elements half of the chip would idle
+    (1.45 and 1.77 times the plain order's time)."""
+    g = torch.Generator(device=cuda).manual_seed(S)
+    q, k, v = (torch.randn(2, 24, S, D, generator=g, device=cuda).bfloat16() for _ in range(3))
+    keys = (torch.arange(S, device=cuda) < torch.tensor([kept, S], device=cuda)[:, None])[:, None, None, :]
+    us = {}
+    for plain in (1, 0):
+        tuning("no_xcd_order", plain)
+        us[plain] = _device_us(lambda: torch.ops.para_attn.attention_forward_sparse_kv(q, k, v, keys))
+    assert us[0] <= 1.15 * us[1], us  # (runs of one order differ by up to 8 %)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
