@@ -1782,7 +1782,12 @@ __global__ __launch_bounds__(WAVES == 4 ? 256 : 512, WAVES == 4 ? 2 : 1) void at
   }
   float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
   // without a mask, scores that are all -inf are no row without keys: a NaN, as where the running maximum begins at -inf
-  if (KS && PM == PM_NONE && any_key && l_tot == 0.f) inv = __uint_as_float(0x7fc00000u);
+  // (its bits pass the compiler unseen: this file is compiled without NaN semantics)
+  if (KS && PM == PM_NONE && any_key && l_tot == 0.f) {
+    uint32_t nan_bits = 0x7fc00000u;
+    asm volatile("" : "+v"(nan_bits));
+    inv = __uint_as_float(nan_bits);
+  }
   if constexpr (ALL) {
     if (piece_slot >= 0) {  // partial result of one key share: fp32, into the workspace
       if (row_ok) {
@@ -2296,7 +2301,12 @@ __global__ __launch_bounds__(WAVES == 4 ? 256 : 512, WAVES == 4 ? 2 : 1) void at
   }
   float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
   // without a mask, scores that are all -inf are no row without keys: a NaN, as where the running maximum begins at -inf
-  if (KS && PM == PM_NONE && any_key && l_tot == 0.f) inv = __uint_as_float(0x7fc00000u);
+  // (its bits pass the compiler unseen: this file is compiled without NaN semantics)
+  if (KS && PM == PM_NONE && any_key && l_tot == 0.f) {
+    uint32_t nan_bits = 0x7fc00000u;
+    asm volatile("" : "+v"(nan_bits));
+    inv = __uint_as_float(nan_bits);
+  }
   if constexpr (CUT) {
     if (piece_slot >= 0) {  // partial result of one key share: fp32, into the workspace
       if (row_ok) {

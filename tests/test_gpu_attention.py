@@ -1113,6 +1113,33 @@ def test_key_halves(cuda, dtype, D, tuning):
             assert (got[0][0].float() - got[1][0].float()).abs().max().item() <= 2e-2 and (got[0][1] - got[1][1])[ok].abs().max().item() <= 1e-4, what
 
 
+@pytest.mark.parametrize("D", [128, 64, 72])
+def test_key_halves_rows_whose_scores_are_all_minus_infinity(cuda, D, tuning):
+    """Unmasked rows whose every score is -inf are NaN in the form with key halves too, where the running maximum begins at a finite value,
+    and only those rows: dense, is_causal (where a row sees one half's tile only) and block-sparse; and with resident keys."""
+    q, k, v = (t.to(cuda) for t in inputs.qkv(1, 2, 256, 288, D, seed=D))
+    rows = [0, 70, 255]
+    q[..., 7] = 0.0
+    q[:, 1, rows] = 0.0
+    q[:, 1, rows, 7] = 3e38
+    k[..., 7] = -3e38  # times 3e38: -inf; times 0: 0
+    op = torch.ops.para_attn.attention_forward_with_lse
+    calls = [lambda: op(q, k, v), lambda: op(q, k, v, is_causal=True)]
+    if D in (64, 128):
+        keep = torch.tensor([[1, 0, 1, 1, 0, 0, 1, 1, 1], [0, 0, 0, 1, 0, 0, 0, 0, 0]], dtype=torch.bool, device=cuda)
+        calls.append(lambda: torch.ops.para_attn.attention_forward_block_sparse(q, k, v, keep))
+    want = torch.zeros(1, 2, 256, D, dtype=torch.bool, device=cuda)
+    want[:, 1, rows] = True
+    for n, call in enumerate(calls):
+        got = []
+        for resident, halves in ((0, 0), (0, 1), (1, 0)):
+            tuning("resident", resident)
+            tuning("key_halves", halves)
+            got.append(call())
+            assert torch.equal(got[-1][0].isnan(), want), (n, resident, halves)
+            assert torch.equal(got[0][1].isfinite(), got[-1][1].isfinite()), (n, resident, halves)
+
+
 def test_key_halves_block_sparse_and_ring(cuda, tuning):
     tuning("key_halves", 1)
     from oracle import sparse as osparse
