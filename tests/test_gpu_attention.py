@@ -1140,6 +1140,32 @@ def test_key_halves_rows_whose_scores_are_all_minus_infinity(cuda, D, tuning):
             assert torch.equal(got[0][1].isfinite(), got[-1][1].isfinite()), (n, resident, halves)
 
 
+@pytest.mark.parametrize("D", [128, 64])
+def test_key_halves_with_key_counts(cuda, D, tuning):
+    """Per-batch key counts of none, part of one tile, one tile, two, and many in one launch of the form with key halves."""
+    counts = [0, 5, 64, 65, 128, 700]
+    q, k, v = inputs.qkv(len(counts), 2, 200, 700, D, seed=D)
+    keep = (torch.arange(700) < torch.tensor(counts)[:, None])[:, None, None, :].expand(-1, 2, 200, -1)
+    ref_out, ref_lse = oattn.sdpa_lse_f64(q.double().numpy(), k.double().numpy(), v.double().numpy(), None, keep.numpy())
+    tuning("key_halves", 1)
+    out, lse = ops._dense_forward(q.to(cuda), k.to(cuda), v.to(cuda), None, True, kv_len=torch.tensor(counts, dtype=torch.int32, device=cuda))
+    _check(out, lse, ref_out, ref_lse, f"key halves, key counts {D}")
+    assert not out[0].any() and lse[0].eq(-math.inf).all()
+
+
+@pytest.mark.parametrize("length", [1, 40, 64, 65, 129])
+def test_key_halves_ring_of_short_blocks(cuda, length, tuning):
+    """Ring blocks of one key tile (the plain form where a launch has no more; in one launch over all blocks the second half of a
+    workgroup has none of any block), of two, and of three, folded into the running pair block by block and in one launch."""
+    tuning("key_halves", 1)
+    q, k, v = inputs.qkv(2, 2, 150, 3 * length, 128, seed=length)
+    ref_out, ref_lse = oattn.sdpa_lse_f64(q.float().numpy(), k.float().numpy(), v.float().numpy())
+    ks, vs = ([t[:, :, i * length : (i + 1) * length].contiguous().to(cuda) for i in range(3)] for t in (k, v))
+    for fused in (True, "sweep"):
+        out, lse = paraattention_amd.ring_sweep(q.to(cuda), ks, vs, fused=fused)
+        _check(out, lse, ref_out, ref_lse, f"key halves, ring {fused} of {length}")
+
+
 def test_key_halves_block_sparse_and_ring(cuda, tuning):
     tuning("key_halves", 1)
     from oracle import sparse as osparse
