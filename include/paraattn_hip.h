@@ -40,7 +40,7 @@ extern "C" {
 #define PA_DTYPE_F16 1
 #define PA_DTYPE_F32 2
 
-/* ABI version of this header (bumped on any signature change). */
+/* ABI version of this header (bumped with any change of a signature or of the set of entries). */
 PA_API int pa_abi_version(void);
 
 /* Text of the last error raised on the calling thread ("" if none). */

@@ -28,7 +28,7 @@ PA_MASK_BOOL = 1
 PA_MASK_F32 = 2
 PA_MASK_ACT = 3
 
-ABI_VERSION = 4
+ABI_VERSION = 5
 
 _vp = ctypes.c_void_p
 _i = ctypes.c_int
@@ -130,13 +130,13 @@ def load():
                 "(hipcc, --offload-arch=gfx950). paraattention_amd has no CPU or eager fallback."
             )
         lib = ctypes.CDLL(LIB_PATH)
+        got = lib.pa_abi_version()  # before the entries are looked up: another version may lack some
+        if got != ABI_VERSION:
+            raise ImportError(f"{LIB_PATH}: ABI version {got}, this package expects {ABI_VERSION}; rebuild it")
         for name, (res, args) in SIGNATURES.items():
             fn = getattr(lib, name)  # AttributeError if the symbol is not exported
             fn.restype = res
             fn.argtypes = args
-        got = lib.pa_abi_version()
-        if got != ABI_VERSION:
-            raise ImportError(f"{LIB_PATH}: ABI version {got}, this package expects {ABI_VERSION}; rebuild it")
         _lib = lib
     return _lib
 

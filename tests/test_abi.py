@@ -115,3 +115,14 @@ def test_missing_library_is_loud():
     env = dict(os.environ, PARAATTN_HIP_LIB="/nonexistent/libparaattn_hip.so", PYTHONPATH=ROOT)
     out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, env=env)
     assert "IMPORTERROR True" in out.stdout, out.stdout + out.stderr
+
+
+def test_another_abi_version_is_named(tmp_path):
+    """A library of another version, which may lack entries of this one, is refused by its version."""
+    src, lib = tmp_path / "old.c", tmp_path / "old.so"
+    src.write_text("int pa_abi_version(void) { return 4; }\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(lib), str(src)], check=True)
+    code = "import paraattention_amd._lib as l\ntry:\n    l.load()\nexcept ImportError as e:\n    print('IMPORTERROR', e)\n"
+    env = dict(os.environ, PARAATTN_HIP_LIB=str(lib), PYTHONPATH=ROOT)
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, env=env)
+    assert f"ABI version 4, this package expects {_lib.ABI_VERSION}" in out.stdout, out.stdout + out.stderr
