@@ -7,6 +7,7 @@ missing, loading raises and every op of this package raises with it.
 import ctypes
 import os
 import threading
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # PARAATTN_HIP_LIB points at another build of the same ABI (kernel experiments); default = in-tree
@@ -141,21 +142,34 @@ def load():
     return _lib
 
 
-_host = None
+_host = None  # the module once it is loaded, False where it cannot be used
 
 
 def host_calls():
-    """The module with the host side of the ordinary calls (csrc/host_calls.cpp), on top of the same library."""
+    """The module with the host side of the ordinary calls (csrc/host_calls.cpp), on top of the same library.  It is compiled against
+    one torch; where it is missing or belongs to another one this says so once and returns None, and the calls take the Python
+    code of ops.py, which needs the library alone."""
     global _host
     if _host is None:
         lib = load()
+        why = None
         try:
             from . import _host_calls
+
+            import torch
+
+            if _host_calls.torch_version != str(torch.__version__):
+                why = f"built against torch {_host_calls.torch_version}, this is {torch.__version__}"
         except ImportError as e:
-            raise ImportError(f"paraattention_amd/_host_calls.so cannot be loaded ({e}): build it with `make -C {os.path.join(_HERE, 'csrc')}`") from e
-        _host_calls.bind(lib._handle)
-        _host = _host_calls
-    return _host
+            why = str(e)
+        if why is None:
+            _host_calls.bind(lib._handle)
+            _host = _host_calls
+        else:
+            warnings.warn(f"paraattention_amd/_host_calls.so is not used ({why}): every call takes about 10 us more of the host's time; "
+                          f"build it with `make -C {os.path.join(_HERE, 'csrc')}`", RuntimeWarning, stacklevel=3)
+            _host = False
+    return _host or None
 
 
 def check(rc, what):

@@ -402,4 +402,11 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_calls", nullptr, -1, methods
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host_calls(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__host_calls(void) {
+  PyObject* const m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "torch_version", BUILT_WITH_TORCH) < 0) {  // whose C++ interface this is
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

@@ -66,11 +66,12 @@ def _native(name, device, *args):
     """The ordinary call in native code (csrc/host_calls.cpp), which takes operands that lie on the current device ready for the kernels;
     None where it is another kind of call, to be looked at by the code below each use."""
     index = device.index
-    if index is None or torch._C._cuda_getDevice() != index:
+    host = _lib.host_calls()
+    if host is None or index is None or torch._C._cuda_getDevice() != index:
         return None
     if args[-1] is _fb_workspace:
         args = (*args[:-1], _fb_workspace(device))
-    res = getattr(_lib.host_calls(), name)(*args, torch._C._cuda_getCurrentRawStream(index))
+    res = getattr(host, name)(*args, torch._C._cuda_getCurrentRawStream(index))
     if type(res) is int:
         _lib.check(res, name)
     return res

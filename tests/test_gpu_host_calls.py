@@ -110,3 +110,11 @@ def test_a_library_error_becomes_the_ops_exception(cuda):
     with pytest.raises(NotImplementedError, match="scale"):
         NS.attention_forward(q, k, v, scale=0.0)
     assert _lib.host_calls().attention(q.cpu(), k, v, None, None, False, False, 0) is None
+
+
+def test_the_ops_run_without_the_module(cuda, monkeypatch):
+    q, k, v = (t.cuda() for t in inputs.qkv(1, 2, 64, 96, 128, seed=4))
+    want = NS.attention_forward_with_lse(q, k, v)
+    monkeypatch.setattr(_lib, "_host", False)  # what host_calls() leaves where the module cannot be used
+    got = NS.attention_forward_with_lse(q, k, v)
+    assert torch.equal(want[0], got[0]) and torch.equal(want[1], got[1])

@@ -1,6 +1,9 @@
 """Host layer without a GPU: op names and schemas equal the reference's, fake (meta) implementations give
 the reference's output contract, config flags, cache-context gates and the no-fallback rule."""
 import os
+import sys
+import types
+import warnings
 
 import pytest
 import torch
@@ -353,3 +356,32 @@ def test_cache_context_module_level_accessors():
     assert [ctx.get_incremental_name(), ctx.get_incremental_name(), ctx.get_incremental_name("a")] == ["default_0", "default_1", "a_0"]
     ctx.reset_incremental_names()
     assert ctx.get_incremental_name() == "default_0"
+
+
+@pytest.mark.parametrize("kind", ["missing", "another torch's"])
+def test_ops_do_without_the_native_host_path(monkeypatch, kind):
+    """Without _host_calls.so, or with one built against another torch, the calls take the Python code: said once, raised never."""
+    from paraattention_amd import _lib
+
+    def bind(handle):
+        raise AssertionError("a module of another torch is not called")
+
+    stale = types.SimpleNamespace(torch_version="1.0.0", bind=bind) if kind != "missing" else None
+    monkeypatch.setattr(_lib, "_host", None)
+    monkeypatch.setitem(sys.modules, "paraattention_amd._host_calls", stale)  # None: the import fails
+    if stale is None:
+        monkeypatch.delattr(paraattention_amd, "_host_calls", raising=False)
+    else:
+        monkeypatch.setattr(paraattention_amd, "_host_calls", stale, raising=False)
+    with pytest.warns(RuntimeWarning, match="_host_calls.so is not used"):
+        assert _lib.host_calls() is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert _lib.host_calls() is None
+        assert ops._native("attention", torch.device("cuda", 0), None) is None
+
+
+def test_native_host_path_is_of_this_torch():
+    from paraattention_amd import _lib
+
+    assert _lib.host_calls() is not None and _lib.host_calls().torch_version == str(torch.__version__)
