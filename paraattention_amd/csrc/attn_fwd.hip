@@ -4875,8 +4875,8 @@ static int launch_short(const AttnParams& p, hipStream_t stream) {
 }
 
 // The call as the kernel that keeps all keys in LDS takes it (attn_resident.hip), for a dense call or one with an additive
-// mask that has no query dimension.  Asking for another kernel by knob switches it off.
-static bool plan_resident_call(const AttnParams& p, int D, ResidentCall& c) {
+// mask that has no query dimension.  Asking for another kernel by knob switches it off.  sizing: only whether it takes the call.
+static bool plan_resident_call(const AttnParams& p, int D, ResidentCall& c, bool sizing = false) {
   int want = tuning().resident;
   if (tuning().no_pipe || p.causal || p.kv_len != nullptr || p.gate != nullptr) return false;
   if (want < 0 && (tuning().forced_bm != 0 || tuning().stream == 1 || tuning().short_keys == 1 || tuning().key_halves == 1)) return false;
@@ -4889,7 +4889,7 @@ static bool plan_resident_call(const AttnParams& p, int D, ResidentCall& c) {
   c.scale_log2 = p.scale_log2;
   c.bias = p.mask; c.ms_b = p.ms_b; c.ms_h = p.ms_h; c.ms_k = p.ms_k;
   c.bias_act = p.mask_kind == MASK_ACT;
-  return plan_resident(c, D, want);
+  return sizing ? resident_takes(c, D, want) : plan_resident(c, D, want);
 }
 
 template <typename T, int RB, bool KVLEN>
@@ -5148,7 +5148,7 @@ static size_t dense_ws_need(int B, int H, int Sq, int Skv, int D, const int64_t 
     p.causal = plan == 2;
     size_t need = 0;
     ResidentCall rcall;
-    if (plan == 0 && plan_resident_call(p, D, rcall)) continue;  // takes none
+    if (plan == 0 && plan_resident_call(p, D, rcall, true)) continue;  // takes none
     if (plan != 0 || !plan_stream(p, D, nullptr, 0, true, &need, allow_drawn)) {
       need = 0;
       choose_kernel(p, D, 256, true, 0, &need);

@@ -27,8 +27,9 @@ struct ResidentCall {
   int xcd_chunk;     // workgroups per XCD, 0: plain order
 };
 
-// Whether the kernel takes the call (fills the plan's fields).  want: -1 where it is expected to be the fastest,
-// 1 wherever it can run.
+// Whether the kernel takes the call.  want: -1 where it is expected to be the fastest, 1 wherever it can run.
+bool resident_takes(ResidentCall& c, int D, int want);
+// The same, and fills the plan's fields.
 bool plan_resident(ResidentCall& c, int D, int want);
 int launch_resident(const ResidentCall& c, int dtype, int D, hipStream_t stream);
 

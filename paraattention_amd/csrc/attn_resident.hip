@@ -14,6 +14,8 @@
 // 62, without reading new Q 66, without both 58 us; touching the next block's Q a block ahead gains nothing.
 #include "attn_resident.h"
 
+#include "resident_plan.h"
+
 #include <type_traits>
 
 namespace pa {
@@ -489,7 +491,7 @@ int launch_form(const ResidentCall& c, hipStream_t stream) {
 
 }  // namespace
 
-bool plan_resident(ResidentCall& c, int D, int want) {
+bool resident_takes(ResidentCall& c, int D, int want) {
   if (want == 0 || (D != 128 && D != 64) || c.Skv <= 0 || c.Sq <= 0 || c.B <= 0 || c.H <= 0) return false;
   if (c.Skv > 1024 || lds_bytes(D, c.Skv, c.bias != nullptr) > (size_t)LDS_BYTES) return false;
   // 32-bit offsets of the copies (rows past the last key included)
@@ -499,7 +501,7 @@ bool plan_resident(ResidentCall& c, int D, int want) {
   const int64_t heads = (int64_t)c.B * c.H;
   c.n_units = (c.Sq + 31) / 32;
   c.n_full = key_blocks(c.Skv, c.bias != nullptr) / 2;
-  if (heads * c.n_units > 0x7fffffff) return false;
+  if (heads * c.n_units > 0x7fffffff || heads * ((c.n_units + 3) / 4) > 0x3fffffff) return false;
   if (want < 0) {
     // Copying all keys in before the first product must pay.  Where the other kernel is one with a workgroup per query tile that streams
     // them, it does not for one tile of 128 rows while all heads together hold more than 8 MB of keys and values (80 heads x
@@ -512,23 +514,15 @@ bool plan_resident(ResidentCall& c, int D, int want) {
     if (heads > cus && c.n_units <= 16 && (tiled || (heads > 2 * cus && c.n_units > 8))) return false;
     if (D == 64 && (c.Skv > 512 || (c.Skv > 384 && heads > 160))) return false;
   }
-  // Workgroups per head: rounds of workgroups times what one takes, in passes of its 8 wavefronts over the keys.  Copying K and
-  // V in is priced at 3/4 of one, a pass that leaves every SIMD at most one wavefront at 0.6.
-  int best = 1;
-  double best_cost = 1e30;
-  const int most = (c.n_units + 3) / 4;
-  for (int parts = 1; parts <= most && parts <= 4 * cus; ++parts) {
-    const double rounds = (double)((heads * parts + cus - 1) / cus);
-    const int units = (c.n_units + parts - 1) / parts, rest = units % 8;
-    const double cost = rounds * (0.75 + units / 8 + (rest == 0 ? 0. : rest <= 4 ? 0.6 : 1.));
-    if (cost < best_cost * 0.999) {
-      best_cost = cost;
-      best = parts;
-    }
-  }
-  c.parts = best;
-  if (heads * best > 0x3fffffff) return false;
-  c.xcd_chunk = cus == 256 ? (int)((heads * best + 7) / 8) : 0;
+  return true;
+}
+
+bool plan_resident(ResidentCall& c, int D, int want) {
+  if (!resident_takes(c, D, want)) return false;
+  const int cus = device_cus();
+  const int64_t heads = (int64_t)c.B * c.H;
+  c.parts = resident_parts(heads, c.n_units, cus);
+  c.xcd_chunk = cus == 256 ? (int)((heads * c.parts + 7) / 8) : 0;
   return true;
 }
 
