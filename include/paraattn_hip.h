@@ -55,7 +55,7 @@ PA_API const char* pa_last_error(void);
  *   "no_pipe"      PARAATTN_NO_PIPE=1       1: the kernels without 32-bit offset limits
  *   "bm"           PARAATTN_BM=128|256      query rows per workgroup, 0 = chosen per launch
  *   "no_split"     PARAATTN_NO_SPLIT=1      1: no key-split tail
- *   "no_xcd_order" PARAATTN_NO_XCD_ORDER=1  1: block-sparse workgroups in plain order
+ *   "no_xcd_order" PARAATTN_NO_XCD_ORDER=1  1: workgroups of the pipelined kernels (one per query tile) in plain order
  *   "bound"        PARAATTN_BOUND=0|1       0 / 1: never / always compute the score bound, -1 = by size
  *   "stream"       PARAATTN_STREAM=0|1      0 / 1: never / wherever possible the kernel with resident workgroups, -1 = by shape
  *   "stream_even"  PARAATTN_STREAM_EVEN=0|1 that kernel's tail cut into shares that begin at the same keys / into equal ranges, -1 = by size

@@ -108,14 +108,14 @@ struct AttnParams {
   int q_lo, q_block;
   int pair;  // block-sparse: each 256-row workgroup holds two 128-row query blocks and walks the union of their ranges
   int tiles_left, tiles_per_block;
+  int key_halves;  // pipelined kernels: 128-row workgroups of 8 wavefronts, 4 for either half of the key tiles (template flag KS)
+  // pipelined kernels: an eighth of the workgroups, of each of xcd_units parts of the launch where it is not block-sparse, so that every
+  // XCD gets a contiguous run of them (deal_to_xcds); 0 = plain order.  Not block-sparse: n_wg workgroups of each part have work.
+  int xcd_chunk, xcd_units, n_wg;
   // dense pipelined kernel only: key-split tail.  Workgroups below split_main own a whole query
   // tile; the last split_tiles query tiles are computed by split_s workgroups each, over
   // consecutive shares of the key tiles, which leave normalised fp32 partial outputs and their
   // LSE in the workspace (piece-major) for attn_split_merge_kernel.  split_s <= 1: no split.
-  int n_wg;        // dense pipelined kernels with xcd_chunk: workgroups that have work, in each of xcd_units
-  int xcd_units;   // the same: parts of the launch that are dealt to the XCDs one after the other (deal_to_xcds)
-  int key_halves;  // pipelined kernels: 128-row workgroups of 8 wavefronts, 4 for either half of the key tiles (template flag KS)
-  int xcd_chunk;  // block-sparse pipelined kernel: ceil(workgroups / 8), 0 = plain order
   // 256-row dense kernel: *bound_flag != 0 says that no score can leave [-60, 60] in the log2 domain (see
   // score_bound_*_kernel), so the running maximum is not needed; null = not known, keep the maximum
   const int* bound_flag;
@@ -4422,7 +4422,7 @@ static SplitPlan plan_split(int64_t n_tiles, int slots, int kv_tiles, int bm, bo
 //   PARAATTN_NO_PIPE=1       "no_pipe"       the kernels without 32-bit offset limits
 //   PARAATTN_BM=128|256      "bm"            query rows per workgroup (0 = choose)
 //   PARAATTN_NO_SPLIT=1      "no_split"      no key-split tail
-//   PARAATTN_NO_XCD_ORDER=1  "no_xcd_order"  block-sparse workgroups in plain order
+//   PARAATTN_NO_XCD_ORDER=1  "no_xcd_order"  workgroups of the pipelined kernels (block-sparse, dense, masked, narrow) in plain order
 //   PARAATTN_BOUND=0|1       "bound"         never / always compute the score bound (-1 = by size)
 //   PARAATTN_STREAM=0|1      "stream"        never / wherever possible the resident-workgroup kernel (-1 = by shape)
 //   PARAATTN_STREAM_EVEN=0|1 "stream_even"   its tail cut into shares that begin at the same keys / into equal ranges (-1 = by size)
@@ -4536,13 +4536,6 @@ static bool pipe_fits(const AttnParams& p, int D) {
   return !tuning().no_pipe;  // test aid: the kernels without offset limits
 }
 
-// Picks the kernel, the query rows per workgroup and the key-split tail.  The pipelined
-// head_dim-128 kernel needs K and V to span less than 4 GiB (32-bit buffer offsets).  128 rows = 4
-// wavefronts, two workgroups per CU; 256 rows = 8 wavefronts sharing one K/V stream (half the tile
-// copies per flop: measured 5.5 % more throughput per full round at the 119k-token shape, but one
-// workgroup per CU makes a partly filled last round dearer).  The choice is the smaller estimate
-// of rounds / throughput; PARAATTN_BM=128|256 forces it, PARAATTN_NO_SPLIT=1 forbids the split.
-// `ws_bytes` is what the caller can lend (0: none); q_block limits 256 for block-sparse launches.
 static bool bound_wanted(int B, int H, int Sq, int Skv, int D);
 
 // The workgroups of a planned dense launch in an order that gives every XCD a contiguous eighth of them, so that the query tiles of a
@@ -4567,6 +4560,13 @@ static void deal_to_xcds(AttnParams& p) {
   p.xcd_units = units;
 }
 
+// Picks the kernel, the query rows per workgroup and the key-split tail.  The pipelined
+// head_dim-128 kernel needs K and V to span less than 4 GiB (32-bit buffer offsets).  128 rows = 4
+// wavefronts, two workgroups per CU; 256 rows = 8 wavefronts sharing one K/V stream (half the tile
+// copies per flop: measured 5.5 % more throughput per full round at the 119k-token shape, but one
+// workgroup per CU makes a partly filled last round dearer).  The choice is the smaller estimate
+// of rounds / throughput; PARAATTN_BM=128|256 forces it, PARAATTN_NO_SPLIT=1 forbids the split.
+// `ws_bytes` is what the caller can lend (0: none); q_block limits 256 for block-sparse launches.
 static void choose_kernel(AttnParams& p, int D, int q_block, bool dense, size_t ws_bytes, size_t* ws_needed) {
   if (ws_needed) *ws_needed = 0;
   p.pipe = 0;
@@ -5148,7 +5148,10 @@ static size_t dense_ws_need(int B, int H, int Sq, int Skv, int D, const int64_t 
     p.causal = plan == 2;
     size_t need = 0;
     ResidentCall rcall;
-    if (plan == 0 && plan_resident_call(p, D, rcall, true)) continue;  // takes none
+    // The kernel with resident keys takes none.  (Neither does a ring step over so few keys ask for any, which goes to the resident
+    // workgroups instead: without room for partial results they leave the last round uncut, and that is the faster plan -- 24 heads x
+    // 7800 rows x 256 keys 55 us against 72, 24 x 2816 x 288, whose last round is nearly empty, 38.5 against 56.9.)
+    if (plan == 0 && plan_resident_call(p, D, rcall, true)) continue;
     if (plan != 0 || !plan_stream(p, D, nullptr, 0, true, &need, allow_drawn)) {
       need = 0;
       choose_kernel(p, D, 256, true, 0, &need);

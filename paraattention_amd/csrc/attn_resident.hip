@@ -1,17 +1,19 @@
 // Attention of many query rows to keys that fit the LDS of one compute unit: cross-attention to a text prompt or to an
-// image's tokens, short self-attention (up to 288 keys at head_dim 128, 256 with a bias; 512 at head_dim 64).
+// image's tokens, short self-attention.  It takes up to 288 keys at head_dim 128, 256 with a bias; 576 and 512 at head_dim 64, where it is
+// chosen up to 512.
 //
 // A workgroup copies all keys and values of one (batch, head) into LDS once and keeps them; its 8 wavefronts then take
 // blocks of 32 query rows on their own: no barrier, no tile copies, and while one of a SIMD's two wavefronts changes
 // blocks (output stores, the next block's Q) the other is somewhere else in its sweep.  The kernels that stream K and V
 // through LDS pay a workgroup's ends (Q, first tiles, last stores, all wavefronts at once) around every 256 rows.
 // Against them (attn_fwd_d128_pipe / _stream_kernel, attn_fwd_d64_pipe_kernel; device time per call, bf16):
-//   2 x 24 heads x 7800 rows x 256 keys, padding as a bias 107 -> 69 us     40 x 32760 x 257       299 -> 226 us
-//   the same without                                      96 -> 69          2 x 24 x 5598 x 77     69 -> 36
-//   24 x 4000 x 256                                       42 -> 22          24 x 257 x 257       13.3 -> 10.1
-//   head_dim 64: 2 x 40 x 31316 x 457                    464 -> 379         24 x 17776 x 226       60 -> 43
+//   2 x 24 heads x 7800 rows x 256 keys   96 -> 69 us                     40 x 32760 x 257       299 -> 226 us
+//   the same, padding as a bias          101 -> 57 (with the far key      2 x 24 x 5598 x 77     69 -> 36
+//     tiles computed too                 107 -> 69)                       24 x 257 x 257       13.3 -> 10.1
+//   24 x 4000 x 256                       42 -> 22
+//   head_dim 64: 2 x 40 x 31316 x 457    464 -> 379                       24 x 17776 x 226       60 -> 43
 // What bounds it is the traffic of Q and the output together with the clock that leaves: without stores the first of these takes
-// 62, without reading new Q 66, without both 58 us; touching the next block's Q a block ahead gains nothing.
+// 60, without reading new Q 62, without both 53 us; touching the next block's Q a block ahead gains nothing.
 #include "attn_resident.h"
 
 #include "resident_plan.h"
@@ -78,7 +80,7 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_resident_kernel(const Residen
     const u32x4 krs = rsrc((const uint16_t*)p.k + batch * p.ks_b + head * p.ks_h, ks_bytes);
     const u32x4 vrs = rsrc((const uint16_t*)p.v + batch * p.vs_b + head * p.vs_h, vs_bytes);
     const int r0 = lane / CHUNKS, pc = lane % CHUNKS;
-    const int row = 8 * RPC * 0 + RPC * wave + r0;  // + 8 RPC i: the swizzles below repeat every 16 rows
+    const int row = RPC * wave + r0;  // + 8 RPC i: the swizzles below repeat every 16 rows
     const int k_chunk = pc ^ (D == 128 ? row & 15 : (row >> 1) & 7);
     const int v_chunk = pc ^ (4 * (D == 128 ? row & 3 : (row >> 1) & 1));
     const uint32_t k_off = row * ks_bytes + 16 * k_chunk, v_off = row * vs_bytes + 16 * v_chunk;
@@ -503,16 +505,21 @@ bool resident_takes(ResidentCall& c, int D, int want) {
   c.n_full = key_blocks(c.Skv, c.bias != nullptr) / 2;
   if (heads * c.n_units > 0x7fffffff || heads * ((c.n_units + 3) / 4) > 0x3fffffff) return false;
   if (want < 0) {
-    // Copying all keys in before the first product must pay.  Where the other kernel is one with a workgroup per query tile that streams
-    // them, it does not for one tile of 128 rows while all heads together hold more than 8 MB of keys and values (80 heads x
-    // 128 rows, head_dim 64, 512 keys 11.7 -> 12.5 us; 24 heads 10.5 -> 9.8), nor for up to 512 rows with more heads than compute
-    // units (300 x 128 x 512 16.2 -> 23.0, 300 x 256 x 226 17.5 -> 19.6), nor at head_dim 64 and more than 384 keys in a second round of
-    // workgroups (257 x 2000 x 512 112 -> 119, 40 x 32760 x 512 248 -> 219); against the resident workgroups of head_dim 128 only
-    // for a few hundred rows of more than 512 heads (640 x 500 x 128 57.8 -> 61.8, 640 x 1000 x 128 105.8 -> 101.5).
+    // Copying all keys in before the first product must pay.  Each line lies between the points measured on its sides (before -> with
+    // this kernel, inputs that change from call to call); with everything in the caches this kernel still gains 1.05 .. 1.4 beyond some
+    // of them (300 x 128 x 64, head_dim 64, 7.4 -> 6.7; 224 x 4000 x 400 146 -> 126; 520 x 300 x 288, head_dim 128, 84 -> 57).
+    // Where the other kernel is one with a workgroup per query tile that streams the keys:
+    // - one tile of 128 rows, and the LDS of all heads together (keys, values and 16 KB of staging each) above 8 MB: head_dim 64, 512 keys,
+    //   80 heads 11.7 -> 12.5 us, 24 heads (3.5 MB) 10.5 -> 9.8
+    // - up to 512 rows and more heads than compute units: 300 x 128 x 512 16.2 -> 23.0, 300 x 256 x 226 17.5 -> 19.6
+    // - head_dim 64 and more than 384 keys, from five eighths as many heads as compute units on: 257 x 2000 x 512 112 -> 119, 40 x 32760 x 512
+    //   248 -> 219, 2 x 40 x 31316 x 457 464 -> 379
+    // Where it is the one with resident workgroups (head_dim 128, no bias):
+    // - 257 to 512 rows and more than two heads per compute unit: 640 x 500 x 128 57.8 -> 61.8, 640 x 1000 x 128 105.8 -> 101.5
     const bool tiled = D == 64 || c.bias != nullptr;
     if (tiled && c.n_units <= 4 && heads * (double)lds_bytes(D, c.Skv, false) > 8.0e6) return false;
     if (heads > cus && c.n_units <= 16 && (tiled || (heads > 2 * cus && c.n_units > 8))) return false;
-    if (D == 64 && (c.Skv > 512 || (c.Skv > 384 && heads > 160))) return false;
+    if (D == 64 && (c.Skv > 512 || (c.Skv > 384 && 8 * heads > 5 * cus))) return false;
   }
   return true;
 }

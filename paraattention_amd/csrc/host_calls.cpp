@@ -58,7 +58,7 @@ PyObject* bind(PyObject*, PyObject* arg) {
   Py_RETURN_NONE;
 }
 
-// None, or a tensor's C++ handle (null and an error set: neither)
+// The C++ handle of a tensor, null for None; false (and no error set): neither
 bool optional_tensor(PyObject* o, const Tensor** out) {
   *out = nullptr;
   if (o == Py_None) return true;
