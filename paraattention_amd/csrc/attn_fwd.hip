@@ -109,9 +109,9 @@ struct AttnParams {
   int pair;  // block-sparse: each 256-row workgroup holds two 128-row query blocks and walks the union of their ranges
   int tiles_left, tiles_per_block;
   int key_halves;  // pipelined kernels: 128-row workgroups of 8 wavefronts, 4 for either half of the key tiles (template flag KS)
-  // pipelined kernels: an eighth of the workgroups, of each of xcd_units parts of the launch where it is not block-sparse, so that every
-  // XCD gets a contiguous run of them (deal_to_xcds); 0 = plain order.  Not block-sparse: n_wg workgroups of each part have work.
-  int xcd_chunk, xcd_units, n_wg;
+  // pipelined kernels: ceil(workgroups / 8), so that every XCD gets a contiguous run of them; 0 = plain order.  Where the launch is not
+  // block-sparse this is of every n_wg workgroups (deal_to_xcds): all of them, or those of one batch element.
+  int xcd_chunk, n_wg;
   // dense pipelined kernel only: key-split tail.  Workgroups below split_main own a whole query
   // tile; the last split_tiles query tiles are computed by split_s workgroups each, over
   // consecutive shares of the key tiles, which leave normalised fp32 partial outputs and their
@@ -148,17 +148,10 @@ struct AttnParams {
 };
 
 // Workgroup number -> tile of a launch that deal_to_xcds has ordered (workgroups go to the 8 XCDs in turn: each XCD holds a contiguous
-// eighth of every unit's tiles).  False: this workgroup has no work.
+// eighth of every n_wg tiles, which are the grid's y).  False: this workgroup has no work.
 __device__ __forceinline__ bool dealt_tile(const AttnParams& p, int& tile) {
-  const int xcd = tile & 7;
-  int at = tile >> 3, first = 0;
-  if (p.xcd_units > 1) {
-    const int unit = at / p.xcd_chunk;
-    at -= unit * p.xcd_chunk;
-    first = unit * p.n_wg;
-  }
-  at += xcd * p.xcd_chunk;
-  tile = first + at;
+  const int at = (tile & 7) * p.xcd_chunk + (tile >> 3);
+  tile = blockIdx.y * p.n_wg + at;
   return at < p.n_wg;
 }
 
@@ -4244,7 +4237,7 @@ static void fill_params(AttnParams& p, const void* q, const void* k, const void*
   p.order = nullptr;
   p.Hm = 0; p.nQ = 0; p.cap = 0; p.q_lo = 0; p.q_block = 0; p.pair = 0; p.tiles_left = 0; p.tiles_per_block = 0;
   p.bm = BM; p.pipe = 0;
-  p.xcd_chunk = 0; p.n_wg = 0; p.xcd_units = 1; p.key_halves = 0;
+  p.xcd_chunk = 0; p.n_wg = 0; p.key_halves = 0;
   p.causal = 0; p.heads_first = 0;
   p.acc_out = nullptr; p.acc_lse = nullptr; p.acc_first = 0;
   p.split_main = 0; p.split_tiles = 0; p.split_s = 0; p.ws_out = nullptr; p.ws_lse = nullptr; p.ws_cols = 128;
@@ -4255,8 +4248,13 @@ static void fill_params(AttnParams& p, const void* q, const void* k, const void*
   p.st = StreamPlan{};
 }
 
+// The grid of a pipelined launch of n workgroups, in plain order or as deal_to_xcds (or the block-sparse launch) has dealt them.
+static dim3 launch_grid(const AttnParams& p, int64_t n) {
+  return p.xcd_chunk > 0 ? dim3(8u * (unsigned)p.xcd_chunk, p.n_wg > 0 ? (unsigned)(n / p.n_wg) : 1u) : dim3((unsigned)n);
+}
+
 template <typename T, bool SPARSE, int WAVES, bool BOUNDED, int PM = PM_NONE, bool NARROW = false, bool CUT = false>
-static int launch_d64(const AttnParams& p, int64_t nblocks, hipStream_t stream) {
+static int launch_d64(const AttnParams& p, dim3 grid, hipStream_t stream) {
   constexpr int NW = WAVES == HALVES ? 8 : WAVES;
   const size_t smem = (WAVES == HALVES ? 8 : 4) * TILE64_BYTES + (PM == PM_KEYBIAS ? NW * PM_SLOT_BYTES : 0);
   static bool attr_done[PA_MAX_DEVICES] = {};  // benign race: the call is idempotent
@@ -4266,22 +4264,22 @@ static int launch_d64(const AttnParams& p, int64_t nblocks, hipStream_t stream) 
     if (e != hipSuccess) PA_FAIL(PA_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
     if (dev >= 0) attr_done[dev] = true;
   }
-  hipLaunchKernelGGL((attn_fwd_d64_pipe_kernel<T, SPARSE, WAVES, BOUNDED, PM, NARROW, CUT>), dim3((unsigned)nblocks), dim3(64 * NW), smem, stream, p);
+  hipLaunchKernelGGL((attn_fwd_d64_pipe_kernel<T, SPARSE, WAVES, BOUNDED, PM, NARROW, CUT>), grid, dim3(64 * NW), smem, stream, p);
   PA_CHECK_LAUNCH("attention kernel (head_dim 64)");
   return PA_OK;
 }
 
 template <typename T, bool SPARSE, bool BOUNDED>
-static int launch_d64_plain(const AttnParams& p, int64_t nblocks, hipStream_t stream) {
+static int launch_d64_plain(const AttnParams& p, dim3 grid, hipStream_t stream) {
   if constexpr (!BOUNDED) {
-    if (p.key_halves) return launch_d64<T, SPARSE, HALVES, false, PM_NONE, false, !SPARSE>(p, nblocks, stream);
+    if (p.key_halves) return launch_d64<T, SPARSE, HALVES, false, PM_NONE, false, !SPARSE>(p, grid, stream);
   }
   if constexpr (!SPARSE) {
     if (p.split_s > 1 || p.heads_first)
-      return p.bm == 256 ? launch_d64<T, false, 8, BOUNDED, PM_NONE, false, true>(p, nblocks, stream)
-                         : launch_d64<T, false, 4, BOUNDED, PM_NONE, false, true>(p, nblocks, stream);
+      return p.bm == 256 ? launch_d64<T, false, 8, BOUNDED, PM_NONE, false, true>(p, grid, stream)
+                         : launch_d64<T, false, 4, BOUNDED, PM_NONE, false, true>(p, grid, stream);
   }
-  return p.bm == 256 ? launch_d64<T, SPARSE, 8, BOUNDED>(p, nblocks, stream) : launch_d64<T, SPARSE, 4, BOUNDED>(p, nblocks, stream);
+  return p.bm == 256 ? launch_d64<T, SPARSE, 8, BOUNDED>(p, grid, stream) : launch_d64<T, SPARSE, 4, BOUNDED>(p, grid, stream);
 }
 
 template <typename T, int D, bool SPARSE>
@@ -4294,7 +4292,7 @@ static int launch_attn(const AttnParams& p, hipStream_t stream) {
     PA_FAIL(PA_ERR_UNSUPPORTED, "accumulation / key split reached a kernel that has neither");
   if (p.out == nullptr && p.acc_out == nullptr) PA_FAIL(PA_ERR_INVALID, "null output pointer");
   if (p.split_s > 1) nblocks = (int64_t)p.split_main + (int64_t)p.split_tiles * p.split_s;
-  if (p.xcd_chunk > 0) nblocks = 8 * (int64_t)p.xcd_chunk * p.xcd_units;
+  const dim3 grid = launch_grid(p, nblocks);
   const void* fn;
   size_t smem;
   int slot;
@@ -4328,9 +4326,9 @@ static int launch_attn(const AttnParams& p, hipStream_t stream) {
           if (e != hipSuccess) PA_FAIL(PA_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
           if (dev >= 0) attr_done[dev][3] = true;
         }
-        hipLaunchKernelGGL((attn_fwd_d128_pipe_kernel<T, false, 8, true>), dim3((unsigned)nblocks), dim3(512), smem, stream, p);
+        hipLaunchKernelGGL((attn_fwd_d128_pipe_kernel<T, false, 8, true>), grid, dim3(512), smem, stream, p);
       } else {
-        const int rc = launch_d64_plain<T, false, true>(p, nblocks, stream);
+        const int rc = launch_d64_plain<T, false, true>(p, grid, stream);
         if (rc != PA_OK) return rc;
       }
       PA_CHECK_LAUNCH("attention kernel (bounded scores)");
@@ -4344,26 +4342,26 @@ static int launch_attn(const AttnParams& p, hipStream_t stream) {
         if (e != hipSuccess) PA_FAIL(PA_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
         if (dev >= 0) attr_done[dev][4] = true;
       }
-      hipLaunchKernelGGL((attn_fwd_d128_pipe_kernel<T, true, 8, false, true>), dim3((unsigned)nblocks), dim3(512), smem, stream, p);
+      hipLaunchKernelGGL((attn_fwd_d128_pipe_kernel<T, true, 8, false, true>), grid, dim3(512), smem, stream, p);
       PA_CHECK_LAUNCH("attention kernel (paired query blocks)");
       return PA_OK;
     }
   }
   if constexpr (D == 128) {
     if (slot == 5)
-      hipLaunchKernelGGL((attn_fwd_d128_pipe_kernel<T, SPARSE, HALVES>), dim3((unsigned)nblocks), dim3(512), smem, stream, p);
+      hipLaunchKernelGGL((attn_fwd_d128_pipe_kernel<T, SPARSE, HALVES>), grid, dim3(512), smem, stream, p);
     else if (slot == 2)
-      hipLaunchKernelGGL((attn_fwd_d128_pipe_kernel<T, SPARSE, 8>), dim3((unsigned)nblocks), dim3(512), smem, stream, p);
+      hipLaunchKernelGGL((attn_fwd_d128_pipe_kernel<T, SPARSE, 8>), grid, dim3(512), smem, stream, p);
     else if (slot == 1)
-      hipLaunchKernelGGL((attn_fwd_d128_pipe_kernel<T, SPARSE, 4>), dim3((unsigned)nblocks), dim3(256), smem, stream, p);
+      hipLaunchKernelGGL((attn_fwd_d128_pipe_kernel<T, SPARSE, 4>), grid, dim3(256), smem, stream, p);
     else
-      hipLaunchKernelGGL((attn_fwd_d128_kernel<T, SPARSE>), dim3((unsigned)nblocks), dim3(NTHREADS), smem, stream, p);
+      hipLaunchKernelGGL((attn_fwd_d128_kernel<T, SPARSE>), grid, dim3(NTHREADS), smem, stream, p);
   } else {
     if (p.pipe) {
-      const int rc = launch_d64_plain<T, SPARSE, false>(p, nblocks, stream);
+      const int rc = launch_d64_plain<T, SPARSE, false>(p, grid, stream);
       if (rc != PA_OK) return rc;
     } else
-      hipLaunchKernelGGL((attn_fwd_kernel<T, D, SPARSE>), dim3((unsigned)nblocks), dim3(NTHREADS), smem, stream, p);
+      hipLaunchKernelGGL((attn_fwd_kernel<T, D, SPARSE>), grid, dim3(NTHREADS), smem, stream, p);
   }
   PA_CHECK_LAUNCH("attention kernel");
   if constexpr (!SPARSE) {
@@ -4542,9 +4540,9 @@ static bool bound_wanted(int B, int H, int Sq, int Skv, int D);
 // head share an L2: 40 heads x 1000 tokens 42.0 -> 39.3 us (head_dim 64 26.6 -> 25.2), 24 x 1500 x 96 columns 42.4 -> 38.1; level where a
 // head has many query tiles.  Not with key shares, which cost more than whole tiles and would all lie on the last XCDs
 // (12 x 6000, head_dim 64, 135 -> 210), and not where the order of the tiles is that of their lengths.  Where the batch elements may keep
-// different numbers of keys (per-batch key counts, boolean key masks) every XCD gets an eighth of each of them: 2 x 24 heads x 4096
-// tokens, one element keeping 512 keys, 237..270 us (one eighth of the whole launch each 380, plain order 237..263), 2 x 24 x 12000 x 64
-// columns, one keeping 1000, 1007 (1787, 1010), and 2 x 40 x 1000, all kept, 62.8 (63.5, 71.2).
+// different numbers of keys (per-batch key counts, boolean key masks) and workgroups wait for a place, every XCD gets an eighth of each
+// of them: 2 x 24 heads x 4096 tokens, one element keeping 512 keys, 235..275 us (one eighth of the whole launch each 380, plain order
+// 234..262), 2 x 24 x 12000 x 64 columns, one keeping 1000, 997 (1787, 998), and 2 x 40 x 1000, all kept, 61.7 (63.5, 71.2).
 // Their last chunk is short on the same XCDs every time, so it must not be short by more than a 64th of them; masks that differ
 // by head leave the workgroups in plain order.
 static void deal_to_xcds(AttnParams& p) {
@@ -4552,12 +4550,11 @@ static void deal_to_xcds(AttnParams& p) {
   if (!p.pipe || p.split_s > 1 || p.causal || p.heads_first || n <= 8 || n > 0x3fffffff || !mi355x_layout() || tuning().no_xcd_order) return;
   const bool key_mask = p.mask != nullptr && p.mask_kind == MASK_BOOL;
   if (key_mask && p.H > 1 && p.ms_h != 0) return;
-  const int units = p.kv_len != nullptr || (key_mask && p.ms_b != 0) ? p.B : 1;
+  const int units = n > device_cus() && (p.kv_len != nullptr || (key_mask && p.ms_b != 0)) ? p.B : 1;
   const int64_t per = n / units, chunk = (per + 7) / 8;
-  if (units > 1 && (8 * chunk - per) * 64 > per) return;
+  if (units > 1 && ((8 * chunk - per) * 64 > per || units > 65535)) return;
   p.n_wg = (int)per;
   p.xcd_chunk = (int)chunk;
-  p.xcd_units = units;
 }
 
 // Picks the kernel, the query rows per workgroup and the key-split tail.  The pipelined
@@ -5211,7 +5208,7 @@ static int launch_pipe_variant(const AttnParams& p, hipStream_t stream) {
   constexpr int NW = WAVES == HALVES ? 8 : WAVES;
   int64_t nblocks = (int64_t)p.B * p.H * p.n_qtiles;
   if (p.split_s > 1) nblocks = (int64_t)p.split_main + (int64_t)p.split_tiles * p.split_s;
-  if (p.xcd_chunk > 0) nblocks = 8 * (int64_t)p.xcd_chunk * p.xcd_units;
+  const dim3 grid = launch_grid(p, nblocks);
   if constexpr (D == 128) {
     const size_t smem = (WAVES == HALVES ? 8 : 4) * TILE_BYTES + (PM == PM_KEYBIAS ? NW * PM_SLOT_BYTES : 0);
     static bool attr_done[PA_MAX_DEVICES] = {};  // benign race: the call is idempotent
@@ -5221,10 +5218,10 @@ static int launch_pipe_variant(const AttnParams& p, hipStream_t stream) {
       if (e != hipSuccess) PA_FAIL(PA_ERR_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
       if (dev >= 0) attr_done[dev] = true;
     }
-    hipLaunchKernelGGL((attn_fwd_d128_pipe_kernel<T, false, WAVES, false, false, PM, W>), dim3((unsigned)nblocks), dim3(64 * NW), smem, stream, p);
+    hipLaunchKernelGGL((attn_fwd_d128_pipe_kernel<T, false, WAVES, false, false, PM, W>), grid, dim3(64 * NW), smem, stream, p);
     PA_CHECK_LAUNCH("attention kernel (masked or narrow rows)");
   } else {  // (masks with a query dimension are planned without a split)
-    const int rc = launch_d64<T, false, WAVES, false, PM, (W < 64), PM != PM_BITS && PM != PM_BIAS>(p, nblocks, stream);
+    const int rc = launch_d64<T, false, WAVES, false, PM, (W < 64), PM != PM_BITS && PM != PM_BIAS>(p, grid, stream);
     if (rc != PA_OK) return rc;
   }
   if (p.split_s > 1) {
