@@ -108,7 +108,9 @@ struct AttnParams {
   int q_lo, q_block;
   int pair;  // block-sparse: each 256-row workgroup holds two 128-row query blocks and walks the union of their ranges
   int tiles_left, tiles_per_block;
-  int key_halves;  // pipelined kernels: 128-row workgroups of 8 wavefronts, 4 for either half of the key tiles (template flag KS)
+  // pipelined kernels: > 0: 128-row workgroups of 8 wavefronts, 4 for either half of the key tiles (template flag KS); a
+  // workgroup with less than that many key tiles leaves them all to the first 4
+  int key_halves;
   // pipelined kernels: ceil(workgroups / 8), so that every XCD gets a contiguous run of them; 0 = plain order.  Where the launch is not
   // block-sparse this is of every n_wg workgroups (deal_to_xcds): all of them, or those of one batch element.
   int xcd_chunk, n_wg;
@@ -219,6 +221,21 @@ struct TileIter {
     }
   }
   __device__ __forceinline__ bool valid() const { return ri < nranges; }
+  // Whether the whole walk has at most n tiles, asked before it begins (n <= MOST, else no).  The ranges' ends are fetched at once.
+  static constexpr int MOST = 10;
+  __device__ __forceinline__ bool at_most(int n) const {
+    if (n <= 0 || n > MOST || nranges > n) return false;  // (a range holds a tile or more)
+    if (nranges <= 1 || ranges == nullptr) return !valid() || end - pos <= n * BN;
+    int tiles = 0;
+#pragma unroll
+    for (int i = 0; i < MOST; ++i) {
+      const int j = i < nranges ? i : nranges - 1;
+      const int b = ranges[2 * j], e = ranges[2 * j + 1];
+      const int len = (e < limit ? e : limit) - b;
+      if (i < nranges && len > 0) tiles += (len + BN - 1) / BN;
+    }
+    return tiles <= n;
+  }
   // current tile: rows [n0, n0 + nvalid), clamp row index to last
   __device__ __forceinline__ void get(int& n0, int& nvalid) const {
     n0 = pos;
@@ -1246,6 +1263,12 @@ __global__ __launch_bounds__(WAVES == 4 ? 256 : 512, WAVES == 4 ? 2 : 1) void at
     it.init_list(p.runs + (size_t)p.Hm * nseg + (size_t)sidx * p.cap * 2, p.runs[sidx], p.Skv, false);
   }
   if constexpr (PM == PM_KEYS) it.init_dense(__builtin_amdgcn_readfirstlane(tm.kept_end(p.Skv)));
+  // KS, few key tiles: the second half's wavefronts leave (a barrier waits for the ones that are left)
+  bool alone = false;
+  if constexpr (KS) {
+    alone = (!ALL || p.st.nseg <= 1) && it.at_most(p.key_halves - 1);
+    if (alone && group != 0) return;
+  }
   // Keys in segments (the blocks of a ring sweep, StreamPlan::kseg / vseg): the sweep below runs once per
   // segment, with the softmax state carried over in registers.  A key share of a split piece is then a run of
   // whole segments; with one segment it is a range of key tiles.
@@ -1394,7 +1417,7 @@ __global__ __launch_bounds__(WAVES == 4 ? 256 : 512, WAVES == 4 ? 2 : 1) void at
       n0 = (uint32_t)a;
       nv = b;
       if constexpr (KS) {
-        if (group == 0 && it.valid()) it.next();
+        if (group == 0 && !alone && it.valid()) it.next();
       }
     } else {
       n0 = OOB;
@@ -1737,8 +1760,8 @@ __global__ __launch_bounds__(WAVES == 4 ? 256 : 512, WAVES == 4 ? 2 : 1) void at
     l_tot = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
   }
   constexpr int MINE = (DB + 1) / 2;  // KS: group 0 finishes the first MINE blocks of 32 columns, group 1 the others
-  auto is_mine = [&](int db) { return !KS || (db < MINE) == (group == 0); };
-  if constexpr (KS) {
+  auto is_mine = [&](int db) { return !KS || alone || (db < MINE) == (group == 0); };
+  if constexpr (KS) if (!alone) {
     // Both halves leave what the other finishes in LDS (their tiles are done with), lane by lane, and fold the two results.
     __syncthreads();
     char* const box = (char*)smem + lane * 16;
@@ -1942,6 +1965,11 @@ __global__ __launch_bounds__(WAVES == 4 ? 256 : 512, WAVES == 4 ? 2 : 1) void at
     it.init_list(p.runs + (size_t)p.Hm * nseg + (size_t)sidx * p.cap * 2, p.runs[sidx], p.Skv, false);
   }
   if constexpr (PM == PM_KEYS) it.init_dense(__builtin_amdgcn_readfirstlane(tm.kept_end(p.Skv)));
+  bool alone = false;  // KS, few key tiles: the second half's wavefronts leave (a barrier waits for the ones that are left)
+  if constexpr (KS) {
+    alone = it.at_most(p.key_halves - 1);
+    if (alone && group != 0) return;
+  }
 
   if constexpr (CUT) {
     if (piece_slot >= 0) {
@@ -2053,7 +2081,7 @@ __global__ __launch_bounds__(WAVES == 4 ? 256 : 512, WAVES == 4 ? 2 : 1) void at
       n0 = (uint32_t)a;
       nv = b;
       if constexpr (KS) {
-        if (group == 0 && it.valid()) it.next();
+        if (group == 0 && !alone && it.valid()) it.next();
       }
     } else {
       n0 = OOB;
@@ -2256,8 +2284,8 @@ __global__ __launch_bounds__(WAVES == 4 ? 256 : 512, WAVES == 4 ? 2 : 1) void at
     l_tot = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
   }
   constexpr int MINE = (DB + 1) / 2;  // KS: group 0 finishes the first MINE blocks of 32 columns, group 1 the others
-  auto is_mine = [&](int db) { return !KS || (db < MINE) == (group == 0); };
-  if constexpr (KS) {
+  auto is_mine = [&](int db) { return !KS || alone || (db < MINE) == (group == 0); };
+  if constexpr (KS) if (!alone) {
     // Both halves leave what the other finishes in LDS (their tiles are done with), lane by lane, and fold the two results.
     __syncthreads();
     char* const box = (char*)smem + lane * 16;
@@ -4502,20 +4530,27 @@ extern "C" int pa_set_tuning(const char* name, int value) {
 // but 8 x 2000 39.4 -> 39.0 and 3 x 3000 41 -> 49, which the key split over more compute units serves, and 3 x 8192 116 -> 120, which the
 // resident workgroups cut evenly.  is_causal: up to two workgroups per unit (the longest decide): head_dim 64 8 x 8192 110 -> 92,
 // 16 x 4096 60.8 -> 54.2, 24 x 3000 (576) 49.8 -> 53.2; head_dim 128 12 x 4096 82 -> 68, 40 x 1500 (480, 24 tiles) 42.6 -> 45.2.
-// A bias with a query dimension gains 1.03 .. 1.3 from 8 tiles on, lists of kept tiles from 32 (8 x 2000 54.9 -> 53.2).
+// A bias with a query dimension gains 1.03 .. 1.3 from 8 tiles on.
+// Lists of kept tiles, key masks and key counts may leave a workgroup few of the tiles there are.  The second half's start and the fold cost
+// 2 .. 3 us, so a workgroup with less tiles than the number returned (0: the plain form) leaves them all to the first half (plain / this
+// way / in two halves, us; a launch whose key mask keeps 1, 4, 8, 16, 31 tiles of 31): head_dim 128, 64 workgroups 8.8 / 9.0 / 12.2, 11.8 / 12.2 /
+// 13.0, 15.8 / 16.6 / 16.0, 22.9 / - / 21.4, 37.2 / - / 33.0; 256 workgroups 10.0 / 10.2 / 13.4, 13.0 / 13.5 / 14.7, 17.2 / 17.9 / 18.7, 25.2 / - / 24.9,
+// 41.2 / - / 40.3 (9 to 14 tiles lose up to 6 % there, 13: 22.6 / - / 23.9); head_dim 64, 64 workgroups 6.9 / 7.1 / 9.3, 9.1 / 9.5 / 9.8, 11.9 / 12.8 / 12.0, 17.1 / - / 16.3, 27.8 / - / 25.5.  Lists gain 1.05 .. 1.1
+// from 24 tiles on where there are at least 32, at head_dim 128 not beyond three quarters of the units (256 workgroups, 31 tiles 45.4 / - / 45.3).
 enum HalvesFor { HALVES_DENSE, HALVES_MASKED_KEYS, HALVES_BIAS, HALVES_LISTS };
-static bool take_halves(int64_t n, int kv_tiles, bool causal, int D, HalvesFor what) {
+static int take_halves(int64_t n, int kv_tiles, bool causal, int D, HalvesFor what) {
   const int want = tuning().key_halves;
   if (want >= 0) return want == 1 && kv_tiles > 1;
-  if (!mi355x_layout()) return false;
+  if (!mi355x_layout()) return 0;
   const int cus = device_cus();
-  if (causal) return kv_tiles >= 16 && n <= (kv_tiles >= 32 ? 2 * cus : cus + cus / 8);
-  if (n > cus) return false;
-  if (what == HALVES_BIAS) return kv_tiles >= 8;
-  if (what == HALVES_LISTS) return kv_tiles >= 32;
-  if (kv_tiles < 16) return false;
-  if (D == 64 || kv_tiles < 32) return true;
-  return 4 * n >= 3 * cus && (what == HALVES_MASKED_KEYS || kv_tiles <= 64);
+  const int from = D == 64 ? 6 : 4 * n > 3 * cus ? 11 : 7;
+  if (causal) return kv_tiles >= 16 && n <= (kv_tiles >= 32 ? 2 * cus : cus + cus / 8) ? from : 0;
+  if (n > cus) return 0;
+  if (what == HALVES_BIAS) return kv_tiles >= 8;  // (every workgroup walks them all)
+  if (what == HALVES_LISTS) return kv_tiles >= 32 && !(D == 128 && 4 * n > 3 * cus) ? from : 0;
+  if (kv_tiles < 16) return 0;
+  if (D == 64 || kv_tiles < 32) return from;
+  return 4 * n >= 3 * cus && (what == HALVES_MASKED_KEYS || kv_tiles <= 64) ? from : 0;
 }
 
 // Bytes of workspace the key-split tail of the plan for bm rows per workgroup needs.
@@ -4589,9 +4624,9 @@ static void choose_kernel(AttnParams& p, int D, int q_block, bool dense, size_t 
   if (D == 64) {
     p.dt = p.ws_cols = 64;
     if (forced == 256 && (dense || q_block % 256 == 0)) p.bm = 256;
-    if (dense && forced == 0 && !bound_wanted(p.B, p.H, p.Sq, p.Skv, D) && take_halves((int64_t)p.B * p.H * ((p.Sq + 127) / 128), (p.Skv + BN - 1) / BN, p.causal, D, HALVES_DENSE)) {
-      p.key_halves = 1;
-      return order();
+    if (dense && forced == 0 && !bound_wanted(p.B, p.H, p.Sq, p.Skv, D)) {
+      p.key_halves = take_halves((int64_t)p.B * p.H * ((p.Sq + 127) / 128), (p.Skv + BN - 1) / BN, p.causal, D, HALVES_DENSE);
+      if (p.key_halves) return order();
     }
     order();
     const bool may = dense && n_cus > 0 && mi355x_layout() && !p.causal && !tuning().no_split && (ws_needed != nullptr || ws_bytes > 0);
@@ -4622,9 +4657,9 @@ static void choose_kernel(AttnParams& p, int D, int q_block, bool dense, size_t 
   const int kv_tiles = (p.Skv + BN - 1) / BN;
   const int64_t bh = (int64_t)p.B * p.H;
   const int64_t n128 = bh * ((p.Sq + 127) / 128), n256 = bh * ((p.Sq + 255) / 256);
-  if (forced == 0 && take_halves(n128, kv_tiles, p.causal, D, p.mask != nullptr ? HALVES_MASKED_KEYS : HALVES_DENSE)) {
-    p.key_halves = 1;
-    return order();
+  if (forced == 0) {
+    p.key_halves = take_halves(n128, kv_tiles, p.causal, D, p.mask != nullptr ? HALVES_MASKED_KEYS : HALVES_DENSE);
+    if (p.key_halves) return order();
   }
   SplitPlan p128 = plan_split(n128, 2 * cus, kv_tiles, 128, allow), p256 = plan_split(n256, cus, kv_tiles, 256, allow);
   if (!ws_needed) {  // the plan must fit what was lent

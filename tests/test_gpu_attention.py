@@ -1166,6 +1166,74 @@ def test_key_halves_ring_of_short_blocks(cuda, length, tuning):
         _check(out, lse, ref_out, ref_lse, f"key halves, ring {fused} of {length}")
 
 
+@pytest.mark.parametrize("D", [128, 64])
+def test_key_halves_leave_short_lists_to_one_half(cuda, D, tuning):
+    """Workgroups whose key mask, key count or block list leaves them 0 to 12 key tiles of 31 or 33, where the launch takes key halves: those up
+    to the line run in the first half's wavefronts alone, the others in both, in one launch.  Lists of one run, of several, ragged ones."""
+    B, H, Sq, Skv = 6, 1, 300, 31 * 64 - 10
+    q, k, v = inputs.qkv(B, H, Sq, Skv, D, seed=D)
+    qc, kc, vc = q.to(cuda), k.to(cuda), v.to(cuda)
+    op = torch.ops.para_attn.attention_forward_with_lse
+    for counts in ([0, 1, 64, 65, 4 * 64, 5 * 64], [5 * 64 + 1, 6 * 64, 7 * 64, 10 * 64 + 3, 12 * 64, Skv]):
+        keep = (torch.arange(Skv) < torch.tensor(counts)[:, None])[:, None, None, :]
+        ref_out, ref_lse = oattn.sdpa_lse_f64(q.double().numpy(), k.double().numpy(), v.double().numpy(), None, np.broadcast_to(keep.numpy(), (B, H, Sq, Skv)))
+        kv_len = torch.tensor(counts, dtype=torch.int32, device=cuda)
+        for what, call in (("mask", lambda: op(qc, kc, vc, keep.to(cuda))), ("counts", lambda: ops._dense_forward(qc, kc, vc, None, True, kv_len=kv_len))):
+            _check(*call(), ref_out, ref_lse, f"short lists by {what} {(D, counts)}")
+    # block lists and packed masks: row block i keeps tiles i, i + step, ... (a run each, or one run for step 1)
+    from oracle import sparse as osparse
+
+    Sq, Skv = 13 * 128, 33 * 64
+    q, k, v = inputs.qkv(1, 2, Sq, Skv, D, seed=D + 1)
+    qc, kc, vc = q.to(cuda), k.to(cuda), v.to(cuda)
+    for step in (1, 2):
+        bm = torch.zeros(13, 33, dtype=torch.bool)
+        for i in range(13):
+            bm[i, [(i + step * j) % 33 for j in range(i)]] = True
+        keep = torch.from_numpy(osparse.expand_block_mask(bm.numpy(), Sq, Skv))
+        ref_out, ref_lse = oattn.sdpa_lse_f64(q.double().numpy(), k.double().numpy(), v.double().numpy(), None, np.broadcast_to(keep.numpy(), (1, 2, Sq, Skv)))
+        _check(*torch.ops.para_attn.attention_forward_block_sparse(qc, kc, vc, bm.to(cuda)), ref_out, ref_lse, f"short block lists {(D, step)}")
+        _check(*op(qc, kc, vc, keep.to(cuda)), ref_out, ref_lse, f"short lists of a packed mask {(D, step)}")
+
+
+def _device_us(call):
+    times = []
+    for _ in range(7):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        call()
+        a.record()
+        for _ in range(5):
+            call()
+        b.record()
+        b.synchronize()
+        times.append(a.elapsed_time(b) * 200)
+    return sorted(times)[3]
+
+
+@pytest.mark.parametrize("what", ["keys", "blocks"])
+def test_short_lists_cost_no_more_than_the_plain_form(cuda, what, tuning):
+    """128 workgroups of head_dim 64 with one key tile each, of the 32 there are: in two halves 1.25 to 1.3 times the plain form's time."""
+    B, H, S = (8, 1, 2048) if what == "keys" else (1, 8, 2048)
+    g = torch.Generator(device=cuda).manual_seed(1)
+    q, k, v = (torch.randn(B, H, S, 64, generator=g, device=cuda).bfloat16() for _ in range(3))
+    if what == "keys":
+        keep = (torch.arange(S, device=cuda) < 64).expand(B, 1, 1, S)
+        call = lambda: torch.ops.para_attn.attention_forward(q, k, v, keep)
+    else:
+        runs = torch.ops.para_attn.block_sparse_key_runs(torch.eye(16, 32, dtype=torch.bool, device=cuda), S)
+        call = lambda: torch.ops.para_attn.attention_forward_block_sparse_runs(q, k, v, runs, 1, 16, 32)
+    us = {}
+    for halves in (0, -1):
+        tuning("key_halves", halves)
+        call()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(20):
+                call()
+        us[halves] = _device_us(graph.replay) / 20
+    assert us[-1] <= 1.12 * us[0], us
+
+
 def test_key_halves_block_sparse_and_ring(cuda, tuning):
     tuning("key_halves", 1)
     from oracle import sparse as osparse
@@ -1207,20 +1275,6 @@ def test_batch_elements_of_different_length_in_any_order(cuda, B, H, S, D, tunin
         lens = [c * (n != 1 or h % 3 != 0) for c in counts.tolist() for h in (0, 1)]
         kept = got[1][1][:, :2].isfinite().all(-1).flatten().tolist()
         assert kept == [x > 0 for x in lens], n
-
-
-def _device_us(call):
-    times = []
-    for _ in range(7):
-        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        call()
-        a.record()
-        for _ in range(5):
-            call()
-        b.record()
-        b.synchronize()
-        times.append(a.elapsed_time(b) * 200)
-    return sorted(times)[3]
 
 
 @pytest.mark.parametrize("S,kept,D", [(4096, 512, 128), (12000, 1000, 64)])  # a key mask, and one with per-batch key counts behind a scan
