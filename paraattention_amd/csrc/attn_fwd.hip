@@ -4579,13 +4579,19 @@ static bool bound_wanted(int B, int H, int Sq, int Skv, int D);
 // of them: 2 x 24 heads x 4096 tokens, one element keeping 512 keys, 235..275 us (one eighth of the whole launch each 380, plain order
 // 234..262), 2 x 24 x 12000 x 64 columns, one keeping 1000, 997 (1787, 998), and 2 x 40 x 1000, all kept, 61.7 (63.5, 71.2).
 // Their last chunk is short on the same XCDs every time, so it must not be short by more than a 64th of them; masks that differ
-// by head leave the workgroups in plain order.
+// by head leave the workgroups in plain order.  The same for a bias with a query dimension that the batch elements share: its rows are
+// then read by one XCD (4 x 8 heads x 2000 x 64 columns, fp32 bias per head, 66.5 us, plain order 67.5, dealt as a whole
+// 90.3; 2 x 16 x 1500 x 128 63.8, 76.2, -).  One that the heads share is in plain order, which deals a head's query tiles round the XCDs as the
+// next head's.
 static void deal_to_xcds(AttnParams& p) {
   const int64_t n = (int64_t)p.B * p.H * p.n_qtiles;
   if (!p.pipe || p.split_s > 1 || p.causal || p.heads_first || n <= 8 || n > 0x3fffffff || !mi355x_layout() || tuning().no_xcd_order) return;
   const bool key_mask = p.mask != nullptr && p.mask_kind == MASK_BOOL;
   if (key_mask && p.H > 1 && p.ms_h != 0) return;
-  const int units = n > device_cus() && (p.kv_len != nullptr || (key_mask && p.ms_b != 0)) ? p.B : 1;
+  const bool full_bias = p.mask != nullptr && !key_mask && p.ms_q != 0 && p.Sq > 1;
+  if (full_bias && p.H > 1 && p.ms_h == 0) return;
+  const bool lengths = n > device_cus() && (p.kv_len != nullptr || (key_mask && p.ms_b != 0));
+  const int units = lengths || (full_bias && p.ms_b == 0) ? p.B : 1;
   const int64_t per = n / units, chunk = (per + 7) / 8;
   if (units > 1 && ((8 * chunk - per) * 64 > per || units > 65535)) return;
   p.n_wg = (int)per;

@@ -1196,6 +1196,21 @@ def test_key_halves_leave_short_lists_to_one_half(cuda, D, tuning):
         _check(*op(qc, kc, vc, keep.to(cuda)), ref_out, ref_lse, f"short lists of a packed mask {(D, step)}")
 
 
+@pytest.mark.parametrize("D", [128, 64])
+def test_biases_shared_by_batch_or_heads_in_any_order(cuda, D, tuning):
+    """A bias with a query dimension of every way of sharing it, dealt to the XCDs and in plain order: the same bits."""
+    B, H, S = 3, 8, 1100  # 9 query tiles: 216 workgroups, 72 a batch element
+    g = torch.Generator(device=cuda).manual_seed(D)
+    q, k, v = (torch.randn(B, H, S, D, generator=g, device=cuda).bfloat16() for _ in range(3))
+    for shape in ((1, H, S, S), (B, H, S, S), (1, 1, S, S), (B, 1, S, S)):
+        bias = torch.randn(shape, generator=g, device=cuda)
+        got = []
+        for plain in (1, 0):
+            tuning("no_xcd_order", plain)
+            got.append(torch.ops.para_attn.attention_forward_with_lse(q, k, v, bias))
+        assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]), shape
+
+
 def _device_us(call):
     times = []
     for _ in range(7):
@@ -1208,6 +1223,19 @@ def _device_us(call):
         b.synchronize()
         times.append(a.elapsed_time(b) * 200)
     return sorted(times)[3]
+
+
+def test_a_shared_bias_is_read_by_one_xcd(cuda, tuning):
+    """A bias per head that four batch elements share: dealt to XCDs by whole batch elements it is read by four of them (1.3 times the plain
+    order's time)."""
+    g = torch.Generator(device=cuda).manual_seed(1)
+    q, k, v = (torch.randn(4, 8, 2000, 64, generator=g, device=cuda).bfloat16() for _ in range(3))
+    bias = torch.randn(1, 8, 2000, 2000, generator=g, device=cuda)
+    us = {}
+    for plain in (1, 0):
+        tuning("no_xcd_order", plain)
+        us[plain] = _device_us(lambda: torch.ops.para_attn.attention_forward(q, k, v, bias))
+    assert us[0] <= 1.12 * us[1], us
 
 
 @pytest.mark.parametrize("what", ["keys", "blocks"])
