@@ -114,13 +114,13 @@ struct AttnParams {
   // pipelined kernels: ceil(workgroups / 8), so that every XCD gets a contiguous run of them; 0 = plain order.  Where the launch is not
   // block-sparse this is of every n_wg workgroups (deal_to_xcds): all of them, or those of one batch element.
   int xcd_chunk, n_wg;
+  // 256-row dense kernel: *bound_flag != 0 says that no score can leave [-60, 60] in the log2 domain (see
+  // score_bound_*_kernel), so the running maximum is not needed; null = not known, keep the maximum
+  const int* bound_flag;
   // dense pipelined kernel only: key-split tail.  Workgroups below split_main own a whole query
   // tile; the last split_tiles query tiles are computed by split_s workgroups each, over
   // consecutive shares of the key tiles, which leave normalised fp32 partial outputs and their
   // LSE in the workspace (piece-major) for attn_split_merge_kernel.  split_s <= 1: no split.
-  // 256-row dense kernel: *bound_flag != 0 says that no score can leave [-60, 60] in the log2 domain (see
-  // score_bound_*_kernel), so the running maximum is not needed; null = not known, keep the maximum
-  const int* bound_flag;
   int split_main, split_tiles, split_s;
   float* ws_out;  // [split_s * split_tiles][bm][ws_cols]
   float* ws_lse;  // [split_s * split_tiles][bm]
