@@ -1393,12 +1393,13 @@ __global__ __launch_bounds__(WAVES == 4 ? 256 : 512, WAVES == 4 ? 2 : 1) void at
   // upper); a range's first key carries the bits in its two low bits (ranges begin at multiples of 4 there).
   int m_cur = 3, m_nxt = 3, m_nx2 = 3;
   const int my_bit = wave < NW / 2 ? 1 : 2;
-  // KS: the groups take the tiles of the list in turn; `ex` says whether the pair exists (of its two tiles the second may not)
-  bool e_cur = false, e_nxt = false, e_nx2 = false;
-  auto pull = [&](uint32_t& n0, int& nv, bool& ex) {
+  // KS: the groups take the tiles of the list in turn.  Of a pair's two tiles the second may not exist: it has -1 valid keys,
+  // where one of no pair has 0
+  auto pull = [&](uint32_t& n0, int& nv) {
+    bool pair = false;
     if constexpr (KS) {
-      ex = it.valid();
-      if (group != 0 && it.valid()) it.next();
+      pair = it.valid();
+      if (group != 0 && pair) it.next();
     }
     if constexpr (PAIR) {
       m_cur = m_nxt;
@@ -1421,7 +1422,7 @@ __global__ __launch_bounds__(WAVES == 4 ? 256 : 512, WAVES == 4 ? 2 : 1) void at
       }
     } else {
       n0 = OOB;
-      nv = 0;
+      nv = pair ? -1 : 0;
       if constexpr (PAIR) m_nx2 = 0;
     }
   };
@@ -1674,12 +1675,8 @@ __global__ __launch_bounds__(WAVES == 4 ? 256 : 512, WAVES == 4 ? 2 : 1) void at
     v_cur = v_nxt;
     n_nxt = n_nx2;
     v_nxt = v_nx2;
-    if constexpr (KS) {
-      e_cur = e_nxt;
-      e_nxt = e_nx2;
-    }
-    pull(n_nx2, v_nx2, e_nx2);
-    have = KS ? e_cur : n_cur != OOB;
+    pull(n_nx2, v_nx2);
+    have = n_cur != OOB || (KS && v_cur < 0);
   };
 
   // The keys' segments are swept one after the other, the pipeline drained in between (carrying it across, with
@@ -1695,10 +1692,10 @@ __global__ __launch_bounds__(WAVES == 4 ? 256 : 512, WAVES == 4 ? 2 : 1) void at
         if (seg > seg_lo) __syncthreads();  // everybody has left the previous segment's last tiles
       }
     }
-    pull(n_cur, v_cur, e_cur);
-    pull(n_nxt, v_nxt, e_nxt);
-    pull(n_nx2, v_nx2, e_nx2);
-    have = KS ? e_cur : n_cur != OOB;
+    pull(n_cur, v_cur);
+    pull(n_nxt, v_nxt);
+    pull(n_nx2, v_nx2);
+    have = n_cur != OOB || (KS && v_cur < 0);
     any_key |= have;
     if (seg > seg_lo) {  // the scores left over from the previous segment's last, absent tile
 #pragma unroll
@@ -2067,12 +2064,13 @@ __global__ __launch_bounds__(WAVES == 4 ? 256 : 512, WAVES == 4 ? 2 : 1) void at
 
   uint32_t n_cur, n_nxt, n_nx2;
   int v_cur, v_nxt, v_nx2;
-  // KS: the groups take the tiles of the list in turn; `ex` says whether the pair exists (of its two tiles the second may not)
-  bool e_cur = false, e_nxt = false, e_nx2 = false;
-  auto pull = [&](uint32_t& n0, int& nv, bool& ex) {
+  // KS: the groups take the tiles of the list in turn.  Of a pair's two tiles the second may not exist: it has -1 valid keys,
+  // where one of no pair has 0
+  auto pull = [&](uint32_t& n0, int& nv) {
+    bool pair = false;
     if constexpr (KS) {
-      ex = it.valid();
-      if (group != 0 && it.valid()) it.next();
+      pair = it.valid();
+      if (group != 0 && pair) it.next();
     }
     if (it.valid()) {
       int a, b;
@@ -2085,13 +2083,13 @@ __global__ __launch_bounds__(WAVES == 4 ? 256 : 512, WAVES == 4 ? 2 : 1) void at
       }
     } else {
       n0 = OOB;
-      nv = 0;
+      nv = pair ? -1 : 0;
     }
   };
-  pull(n_cur, v_cur, e_cur);
-  pull(n_nxt, v_nxt, e_nxt);
-  pull(n_nx2, v_nx2, e_nx2);
-  bool have = KS ? e_cur : n_cur != OOB;
+  pull(n_cur, v_cur);
+  pull(n_nxt, v_nxt);
+  pull(n_nx2, v_nx2);
+  bool have = n_cur != OOB || (KS && v_cur < 0);
   const bool any_key = have;
 
   const int wave_row0 = row_begin + 32 * wave;
@@ -2263,12 +2261,8 @@ __global__ __launch_bounds__(WAVES == 4 ? 256 : 512, WAVES == 4 ? 2 : 1) void at
     v_cur = v_nxt;
     n_nxt = n_nx2;
     v_nxt = v_nx2;
-    if constexpr (KS) {
-      e_cur = e_nxt;
-      e_nxt = e_nx2;
-    }
-    pull(n_nx2, v_nx2, e_nx2);
-    have = KS ? e_cur : n_cur != OOB;
+    pull(n_nx2, v_nx2);
+    have = n_cur != OOB || (KS && v_cur < 0);
   };
 
   while (have) {
