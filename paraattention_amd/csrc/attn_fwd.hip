@@ -4531,13 +4531,14 @@ extern "C" int pa_set_tuning(const char* name, int value) {
 // 13.0, 15.8 / 16.6 / 16.0, 22.9 / - / 21.4, 37.2 / - / 33.0; 256 workgroups 10.0 / 10.2 / 13.4, 13.0 / 13.5 / 14.7, 17.2 / 17.9 / 18.7, 25.2 / - / 24.9,
 // 41.2 / - / 40.3 (9 to 14 tiles lose up to 6 % there, 13: 22.6 / - / 23.9); head_dim 64, 64 workgroups 6.9 / 7.1 / 9.3, 9.1 / 9.5 / 9.8, 11.9 / 12.8 / 12.0, 17.1 / - / 16.3, 27.8 / - / 25.5.  Lists gain 1.05 .. 1.1
 // from 24 tiles on where there are at least 32, at head_dim 128 not beyond three quarters of the units (256 workgroups, 31 tiles 45.4 / - / 45.3).
+// Two halves walk 7 tiles in as many steps as 8: 120 workgroups of head_dim 128 15.1 / 15.6 / 16.4 at 7, 16.0 / - / 16.5 at 8.
 enum HalvesFor { HALVES_DENSE, HALVES_MASKED_KEYS, HALVES_BIAS, HALVES_LISTS };
 static int take_halves(int64_t n, int kv_tiles, bool causal, int D, HalvesFor what) {
   const int want = tuning().key_halves;
   if (want >= 0) return want == 1 && kv_tiles > 1;
   if (!mi355x_layout()) return 0;
   const int cus = device_cus();
-  const int from = D == 64 ? 6 : 4 * n > 3 * cus ? 11 : 7;
+  const int from = D == 64 ? 6 : 4 * n > 3 * cus ? 11 : 8;
   if (causal) return kv_tiles >= 16 && n <= (kv_tiles >= 32 ? 2 * cus : cus + cus / 8) ? from : 0;
   if (n > cus) return 0;
   if (what == HALVES_BIAS) return kv_tiles >= 8;  // (every workgroup walks them all)
