@@ -520,10 +520,17 @@ bool resident_takes(ResidentCall& c, int D, int want) {
     // - head_dim 64 and more than 384 keys, from five eighths as many heads as compute units on: 257 x 2000 x 512 112 -> 119, 40 x 32760 x 512
     //   248 -> 219, 2 x 40 x 31316 x 457 464 -> 379
     // Where it is the one with resident workgroups (head_dim 128, no bias):
-    // - 257 to 512 rows and more than two heads per compute unit: 640 x 500 x 128 57.8 -> 61.8, 640 x 1000 x 128 105.8 -> 101.5
+    // - its pieces of 256 rows make whole rounds (it cuts the last round otherwise, which costs it 20 us: 510 x 256 x 128 63 -> 31) and are more
+    //   than half full, up to two of them per head and more heads than compute units: 512 x 256 x 128 25.2 -> 30.6, 768 x 150 x 230 41.8 -> 49.8,
+    //   384 x 440 x 230 42.6 -> 46.7, 640 x 500 x 128 50.0 -> 55.8.  Not with up to 96 keys (384 x 440 x 77 31.4 -> 29.8), nor half-full ones
+    //   (512 x 300 rows), nor two each of whole rounds of heads beyond 192 keys (768 x 440 x 230 83.8 -> 79.8)
     const bool tiled = D == 64 || c.bias != nullptr;
     if (tiled && c.n_units <= 4 && heads * (double)lds_bytes(D, c.Skv, false) > 8.0e6) return false;
-    if (heads > cus && c.n_units <= 16 && (tiled || (heads > 2 * cus && c.n_units > 8))) return false;
+    if (heads > cus && c.n_units <= 16) {
+      if (tiled) return false;
+      const bool whole = heads * ((c.n_units + 7) / 8) % cus == 0, filled = (c.n_units - 1) % 8 >= 4;
+      if (whole && filled && c.Skv > 96 && (c.n_units <= 8 || heads % cus != 0 || c.Skv <= 192)) return false;
+    }
     if (D == 64 && (c.Skv > 512 || (c.Skv > 384 && 8 * heads > 5 * cus))) return false;
   }
   return true;

@@ -1401,6 +1401,26 @@ def test_padding_in_small_calls_costs_no_search(cuda, tuning):
     assert us[-1] <= 1.02 * us[0], us
 
 
+@pytest.mark.parametrize("heads,rows,keys,most", [(512, 256, 128, 1.05), (384, 440, 230, 1.05), (600, 350, 128, 0.8)])
+def test_resident_keys_where_heads_outnumber_compute_units(cuda, heads, rows, keys, most, tuning):
+    """More heads than compute units and few rows: resident keys take 1.21 and 1.10 times as long as whole rounds of pieces of 256 rows, and 0.62
+    of the time of rounds that have to be cut.  The output is that of both kernels."""
+    g = torch.Generator(device=cuda).manual_seed(heads)
+    q, k, v = (torch.randn(2, heads // 2, n, 128, generator=g, device=cuda).bfloat16() for n in (rows, keys, keys))
+    call = lambda: torch.ops.para_attn.attention_forward(q, k, v)
+    us, out = {}, {}
+    for resident in (0, 1, -1):
+        tuning("resident", resident)
+        out[resident] = call()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(10):
+                call()
+        us[resident] = _device_us(graph.replay) / 10
+    assert all(torch.allclose(out[-1].float(), out[r].float(), atol=2e-2, rtol=2e-2) for r in (0, 1))
+    assert us[-1] <= most * us[0], us
+
+
 @pytest.mark.parametrize("scale", [1.0, 0.3])
 def test_short_key_kernel_large_logits(cuda, scale, tuning):
     """Logits of a few hundred through the kernel for short key sequences: the running maximum rises from tile to
